@@ -118,13 +118,22 @@ def _rows(case, gen, rows):
     return X.to(getattr(torch, case["dtype"]))
 
 
+def _centres(case, X, gen):
+    """Distinct rows of the data, each moved a little: centres as a fit would have left them."""
+    pick = torch.randperm(X.shape[0], device="cuda", generator=gen)[:case["k"]]
+    C = X[pick]
+    C += 0.25 * X.std() * torch.randn(C.shape, device="cuda", generator=gen, dtype=C.dtype)
+    return C.contiguous()
+
+
 def _fitted(case, gen):
-    """A model fitted on a sample of the distribution, and rows it has not seen."""
+    """A fitted model, and rows of its distribution. (The fit has the centres for its rows, each
+    the nearest to itself by far, so the model is these centres whatever the rounding.)"""
     X = _rows(case, gen, case["rows"])
-    sample = X[torch.randint(0, X.shape[0], (2 * case["k"],), device="cuda", generator=gen)].contiguous()
-    model = KMeans(n_clusters=case["k"], init="random", max_iter=2, tol=0.0, random_state=1)
-    model.fit(sample)
-    return X, model
+    C = _centres(case, X, gen)
+    model = KMeans(n_clusters=case["k"], init=C.cpu().numpy(), max_iter=1, tol=0.0, random_state=1)
+    model.fit(C)
+    return X, model, C
 
 
 def prepare(case, seed):
@@ -139,7 +148,7 @@ def prepare(case, seed):
     if kind == "fit":
         return dict(case=case, X=_rows(case, gen, case["rows"]), seed=int(seed) % 30000)
     if kind in ("predict", "transform"):
-        X, model = _fitted(case, gen)
+        X, model, _ = _fitted(case, gen)
         return dict(case=case, X=X, model=model)
     return dict(case=case, X=_rows(case, gen, case["rows"]).cpu().numpy(), seed=int(seed) % 30000)
 
@@ -163,6 +172,30 @@ def run(state):
     if kind == "host":
         out["predicted"] = model.predict(state["X"])
     return out
+
+
+def exact(case, seed):
+    """Distances (or the nearest centres) of the rows in float64; a fit has none: its start rows
+    come from the framework's own random generator."""
+    kind = case["kind"]
+    if kind not in ("serve", "predict", "transform"):
+        return None
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1000 + int(seed))
+    X = _rows(case, gen, case["rows"])
+    if kind == "serve":
+        C = X[torch.randint(0, X.shape[0], (case["k"],), device="cuda", generator=gen)]
+    else:
+        C = _centres(case, X, gen)
+    C = C.double()
+    cc = (C * C).sum(1)
+    out = []
+    step = max(1, int(2e8) // case["k"])
+    for lo in range(0, X.shape[0], step):
+        x = X[lo:lo + step].double()
+        dist = torch.addmm((x * x).sum(1, keepdim=True) + cc, x, C.t(), alpha=-2.0).abs()
+        out.append(dist if kind == "transform" else dist.argmin(1).to(torch.int32))
+    return torch.cat(out)
 
 
 def work(case):
