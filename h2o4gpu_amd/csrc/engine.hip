@@ -1069,7 +1069,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     KM_TRY(regrow(&dhist, &cap_hist, (size_t)M));
     std::vector<int> hist((size_t)M);
     int rc = hipMemsetAsync(dhist, 0, (size_t)M * sizeof(int), stream) == hipSuccess ? 0 : H2O4GPU_KMEANS_EDEVICE;
-    if (rc == 0) rc = launch_label_histogram(stream, *near, dhist, n);
+    if (rc == 0) rc = launch_label_histogram(stream, *near, dhist, n, M);
     if (rc == 0 && hipMemcpyAsync(hist.data(), dhist, (size_t)M * sizeof(int), hipMemcpyDeviceToHost, stream) != hipSuccess)
       rc = H2O4GPU_KMEANS_EDEVICE;
     if (rc == 0 && hipStreamSynchronize(stream) != hipSuccess) rc = H2O4GPU_KMEANS_EDEVICE;

@@ -243,7 +243,7 @@ int launch_fold_min(hipStream_t s, const T *cur, T *cost, double *bsums, int64_t
 template <typename T>
 int launch_select_rows(hipStream_t s, const T *cost, T total, uint32_t state0, int k, int *list,
                        int *count, int cap, int64_t n);
-int launch_label_histogram(hipStream_t s, const int *labels, int *counts, int64_t n);
+int launch_label_histogram(hipStream_t s, const int *labels, int *counts, int64_t n, int m);
 // CcT: column-major copy of the m candidate rows Cc (launch_transpose_candidates): the dot
 // products are then summed over the features in ascending order, as a scalar loop sums them.
 // CcT null: several lanes share a candidate (strided partial sums and a tree; much faster,
