@@ -710,7 +710,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       KM_TRY(dalloc(&order, n));
       KM_TRY(dalloc(&order_label, n));
       KM_TRY(dalloc(&bucket_offsets, k));
-      KM_TRY(dalloc(&bucket_hist, (size_t)bucket_blocks(n) * k));
+      KM_TRY(dalloc(&bucket_hist, (size_t)bucket_blocks(n, k) * k));
       KM_TRY(dalloc(&bucket_seg, (size_t)32 * k));
       KM_TRY(dalloc(&bucket_total, 1));
       KM_TRY(dalloc(&bucket_partials, bucket_partial_slots(n, k) * d));

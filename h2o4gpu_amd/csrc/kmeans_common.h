@@ -175,12 +175,12 @@ int launch_accumulate(hipStream_t s, const UpdatePlan &p, const T *X,
                       int d, int k);
 // Pass 1 for shapes whose sums need many LDS chunks: the rows are ordered by label with a
 // stable counting sort (order / order_label: [n] int32 each, offsets: [k] int32,
-// block_hist: [bucket_blocks(n)][k] int32, seg_hist: [32][k] int32) and summed in fixed
+// block_hist: [bucket_blocks(n, k)][k] int32, seg_hist: [32][k] int32) and summed in fixed
 // windows of the ordered rows (partials: [bucket_partial_slots(n, k)][d] double) into
 // gsum [k][d] double; counts receives the bucket sizes. Run-to-run reproducible for
 // both precisions. The result is consumed by launch_finalize with slots = 1.
 bool bucketed_update_applies(int k_chunks, int k, int d);
-int bucket_blocks(int64_t n);
+int bucket_blocks(int64_t n, int k);
 size_t bucket_partial_slots(int64_t n, int k);
 template <typename T>
 int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int *order,
