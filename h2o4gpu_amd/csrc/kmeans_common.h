@@ -153,6 +153,10 @@ int launch_transform(hipStream_t s, const T *X, const T *xnorm, const T *C,
                      const T *cnorm, T *D, int64_t n, int64_t ldn, int d, int k,
                      int num_cu, int split = 0, SplitScratch split_scratch = SplitScratch());
 
+// out[0 .. n-1] = value
+template <typename T>
+int launch_fill(hipStream_t s, T *out, T value, int64_t n);
+
 // out[i] = sum_j X[i][j]^2, j ascending, no contraction.
 template <typename T>
 int launch_row_norms(hipStream_t s, const T *X, T *out, int64_t n, int d);

@@ -207,6 +207,21 @@ __global__ __launch_bounds__(WG) void row_norms_long_kernel(const T *__restrict_
 }
 
 template <typename T>
+__global__ __launch_bounds__(WG) void fill_kernel(T *__restrict__ out, T value, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x;
+  if (i < n) out[i] = value;
+}
+template <typename T>
+int launch_fill(hipStream_t s, T *out, T value, int64_t n) {
+  if (n <= 0) return 0;
+  hipLaunchKernelGGL((fill_kernel<T>), dim3((unsigned)((n + WG - 1) / WG)), dim3(WG), 0, s, out, value, n);
+  KM_HIP_TRY(hipGetLastError());
+  return 0;
+}
+template int launch_fill<float>(hipStream_t, float *, float, int64_t);
+template int launch_fill<double>(hipStream_t, double *, double, int64_t);
+
+template <typename T>
 int launch_row_norms(hipStream_t s, const T *X, T *out, int64_t n, int d) {
   if (n <= 0) return 0;
   if (d >= 4 && d <= 64 && n * (int64_t)d >= (1 << 22)) {
