@@ -91,14 +91,26 @@ __global__ __launch_bounds__(WG) void assign_valu_kernel(
 #pragma unroll
     for (int j = 0; j < DREG; j++) xr[j] = (valid && j < d) ? x[j] : (T)0;
   }
-  const T xx = valid ? xnorm[row] : (T)0;
+  // no norm buffers given: the values row_norms would have stored, from the row and the centroid
+  // themselves (j ascending, multiply and add rounded separately)
+  T xx = 0;
+  if (xnorm) {
+    xx = valid ? xnorm[row] : (T)0;
+  } else if (DREG > 0) {
+#pragma unroll
+    for (int j = 0; j < DREG; j++)
+      if (j < d) xx = xx + xr[j] * xr[j];
+  } else if (valid) {
+    xx = row_sqnorm<T>(x, d);
+  }
   T best = argmin_start<T>();
   int bidx = -1;
   for (int c0 = 0; c0 < k; c0 += kc) {
     const int nc = min(kc, k - c0);
     __syncthreads();
     for (int e = tid; e < nc * d; e += WG) Cs[e] = C[(size_t)c0 * d + e];
-    for (int c = tid; c < nc; c += WG) ccs[c] = cnorm[c0 + c];
+    for (int c = tid; c < nc; c += WG)
+      ccs[c] = cnorm ? cnorm[c0 + c] : row_sqnorm<T>(C + (size_t)(c0 + c) * d, d);
     __syncthreads();
     if (!valid) continue;
     for (int c = 0; c < nc; c++) {
@@ -358,7 +370,7 @@ __global__ __launch_bounds__(WG) void lloyd_valu_anyd_kernel(
       if (tid < VEC && el < (n - base) * d) pre_tail = xb[el];
     }
     const int64_t r = base + tid;
-    pre_xx = xnorm[r < n ? r : n - 1];
+    if (xnorm) pre_xx = xnorm[r < n ? r : n - 1];
   };
   const int64_t stride = (int64_t)gridDim.x * WG;
   int64_t base = (int64_t)blockIdx.x * WG;
@@ -416,12 +428,13 @@ __global__ __launch_bounds__(WG) void lloyd_valu_anyd_kernel(
       const int el = vlim * VEC + tid;
       if (tid < VEC && el < rows * d) Xs[el + row_of(el) * pad] = pre_tail;
     }
-    const T xx = pre_xx;
+    T xx = pre_xx;
     __syncthreads();
     fetch(base + stride < n ? base + stride : base);
     const int64_t row = base + tid;
     if (tid < rows) {
       const T *xrow = Xs + tid * sx;
+      if (!xnorm) xx = row_sqnorm<T>(xrow, d);
       T dot[KREG];
 #pragma unroll
       for (int c = 0; c < KREG; c++) dot[c] = 0;
@@ -2556,6 +2569,16 @@ int launch_assign(hipStream_t s, int variant, const T *X, const T *xnorm,
   }
   return H2O4GPU_KMEANS_EARG;
 }
+
+template <typename T>
+AssignInputs assign_inputs(int64_t n, int d, int k) {
+  const int v = pick_assign_variant<T>(ASSIGN_AUTO, n, d, k);
+  if (v == ASSIGN_VALU) return ASSIGN_FROM_ROWS;
+  if (v == ASSIGN_ROWSTAT && rowstat_chunk<T>(d, k) >= k) return ASSIGN_FROM_ROW_NORMS;
+  return ASSIGN_FROM_MODEL;
+}
+template AssignInputs assign_inputs<float>(int64_t, int, int);
+template AssignInputs assign_inputs<double>(int64_t, int, int);
 
 template <typename T>
 int launch_transform(hipStream_t s, const T *X, const T *xnorm, const T *C,

@@ -101,6 +101,14 @@ int launch_assign(hipStream_t s, int variant, const T *X, const T *xnorm,
                   const T *C, const T *cnorm, int *labels, T *mindist,
                   int64_t n, int d, int k, int num_cu, int *used, bool exact = false,
                   StackShape st = StackShape(), int split = 0, SplitScratch split_scratch = SplitScratch());
+// What launch_assign (variant ASSIGN_AUTO) needs beside the rows and the k centroids for a shape:
+enum AssignInputs {
+  ASSIGN_FROM_ROWS,       // nothing: xnorm and cnorm may be null, C need not be padded
+  ASSIGN_FROM_ROW_NORMS,  // xnorm; cnorm may be null, C need not be padded
+  ASSIGN_FROM_MODEL       // both norms, and the padding described at CENTROID_PAD
+};
+template <typename T>
+AssignInputs assign_inputs(int64_t n, int d, int k);
 template <typename T>
 int pick_assign_variant(int requested, int64_t n, int d, int k);
 // The one-pass kernel for long rows and at most 16 centroids (longrow_kernels.hip): whether a
