@@ -266,6 +266,23 @@ template <typename T>
 int launch_candidate_dists(hipStream_t s, const T *Cc, const T *CcT, const T *ccn, int centre, T *best,
                            T *mirror, int m, int d, int first);
 
+// The draws of a random permutation that its first k entries depend on. positions draws of
+// minstd_rand0 follow state x; draw q serves step first_step + q of the permutation, less the
+// draws turned down before it, of which there are at most shuffle_slack(first_step + q) (the
+// caller checks). Those that could be turned down (at or past the largest multiple of step + 1) or land in
+// [0, k) go to list as (q, value), a block's draws together and in order, table[block] saying where
+// they start and how many there are; *total, zero at the start, counts them all (beyond cap they are
+// counted and not written).
+static const int64_t SHUFFLE_MAX_ROWS = (int64_t)1 << 27;  // beyond, more draws are turned down than the slack
+static const int SHUFFLE_BLOCK_DRAWS = 8192;
+__host__ __device__ static inline int64_t shuffle_slack(int64_t step) { return step / 32 + 64; }
+static inline int shuffle_draw_blocks(int64_t positions) {
+  return (int)((positions + SHUFFLE_BLOCK_DRAWS - 1) / SHUFFLE_BLOCK_DRAWS);
+}
+static inline size_t shuffle_draw_capacity(int64_t n) { return (size_t)n / 16 + 16384; }
+int launch_shuffle_draws(hipStream_t s, uint32_t x, int64_t first_step, int64_t positions, int k, uint2 *table,
+                         uint2 *list, unsigned cap, unsigned *total);
+
 // Copy rows idx[0..k-1] of X into C ([k][d]).
 template <typename T>
 int launch_gather_rows(hipStream_t s, const T *X, const int *idx, T *C, int k,

@@ -302,34 +302,43 @@ __device__ __forceinline__ uint32_t mulmod_m31(uint32_t a, uint32_t b) {
 // state0 * 48271^(row+1); the distribution maps x to float(x - 1) / (1.0f + float(m - 2)).
 // Rows taken are appended to list in arrival order (the host sorts them); *count may
 // exceed cap, in which case only cap entries were written.
+// A thread jumps to its first row's draw (some 24 modular products and squarings) and from there
+// from row to row by one product with `hop` = 48271^(threads of the launch): a jump for every row
+// was nine tenths of the kernel (10M rows: 133 us).
 template <typename T>
 __global__ __launch_bounds__(WG) void select_rows_kernel(const T *__restrict__ cost, T total,
-                                                        uint32_t state0, int k,
+                                                        uint32_t state0, uint32_t hop, int k,
                                                         int *__restrict__ list,
                                                         int *__restrict__ count, int cap,
                                                         int64_t n) {
-  const int64_t row = (int64_t)blockIdx.x * WG + threadIdx.x;
-  if (row >= n) return;
+  const int64_t first = (int64_t)blockIdx.x * WG + threadIdx.x, stride = (int64_t)gridDim.x * WG;
+  if (first >= n) return;
   uint32_t acc = state0, base = 48271u;
-  for (uint64_t e = (uint64_t)row + 1; e != 0; e >>= 1) {
+  for (uint64_t e = (uint64_t)first + 1; e != 0; e >>= 1) {
     if (e & 1) acc = mulmod_m31(acc, base);
     base = mulmod_m31(base, base);
   }
-  float u = static_cast<float>(acc - 1u);
-  u /= (1.0f + static_cast<float>(2147483645u));
-  const T threshold = (T)u;
-  const T prob = (T)((2.0 * k * (double)cost[row]) / (double)total);
-  if (prob > threshold) {
-    const int pos = atomicAdd(count, 1);
-    if (pos < cap) list[pos] = (int)row;
+  for (int64_t row = first; row < n; row += stride, acc = mulmod_m31(acc, hop)) {
+    float u = static_cast<float>(acc - 1u);
+    u /= (1.0f + static_cast<float>(2147483645u));
+    const T threshold = (T)u;
+    const T prob = (T)((2.0 * k * (double)cost[row]) / (double)total);
+    if (prob > threshold) {
+      const int pos = atomicAdd(count, 1);
+      if (pos < cap) list[pos] = (int)row;
+    }
   }
 }
 template <typename T>
 int launch_select_rows(hipStream_t s, const T *cost, T total, uint32_t state0, int k, int *list,
                        int *count, int cap, int64_t n) {
   if (n <= 0) return 0;
-  hipLaunchKernelGGL((select_rows_kernel<T>), dim3((unsigned)((n + WG - 1) / WG)), dim3(WG), 0, s,
-                     cost, total, state0, k, list, count, cap, n);
+  const unsigned blocks = (unsigned)std::min<int64_t>((n + WG - 1) / WG, 2048);
+  uint64_t hop = 1, base = 48271;
+  for (uint64_t e = (uint64_t)blocks * WG; e != 0; e >>= 1, base = base * base % 2147483647u)
+    if (e & 1) hop = hop * base % 2147483647u;
+  hipLaunchKernelGGL((select_rows_kernel<T>), dim3(blocks), dim3(WG), 0, s, cost, total, state0, (uint32_t)hop, k,
+                     list, count, cap, n);
   KM_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -340,8 +349,8 @@ int launch_select_rows(hipStream_t s, const T *cost, T total, uint32_t state0, i
 // A few dozen to a few thousand counters that every wavefront of the chip adds to: as global
 // atomics they queue up at the cache lines that hold them (10M rows, some 200 candidates:
 // 10.9 ms). STAGED: every workgroup counts into LDS and adds its totals to the global counters
-// once, so a counter sees one global add per workgroup and the kernel runs at the speed of
-// reading the labels (HIST_MEASURED).
+// once, so a counter sees one global add per workgroup (0.04 ms; a fit of 10.1M x 3, k = 27 with this
+// seeding 38.1 -> 26.5 ms, 1M x 64, k = 64 2.81 -> 2.08 ms).
 template <bool STAGED>
 __global__ __launch_bounds__(WG) void label_histogram_kernel(const int *__restrict__ labels,
                                                             int *__restrict__ counts, int64_t n, int m) {
@@ -380,6 +389,74 @@ int launch_label_histogram(hipStream_t s, const int *labels, int *counts, int64_
     hipLaunchKernelGGL((label_histogram_kernel<false>), dim3((unsigned)std::min<int64_t>(want, 2048)), dim3(WG), 0,
                        s, labels, counts, n, m);
   }
+  KM_HIP_TRY(hipGetLastError());
+  return 0;
+}
+
+// One thread per 32 consecutive draws, twice through them: once to count, once to write, the
+// block's place in the list taken with a single atomic in between.
+__global__ __launch_bounds__(WG) void shuffle_draws_kernel(uint32_t x0, int64_t first_step, int64_t positions,
+                                                          int k, uint2 *__restrict__ table,
+                                                          uint2 *__restrict__ list, unsigned cap,
+                                                          unsigned *__restrict__ total) {
+  constexpr int PER = SHUFFLE_BLOCK_DRAWS / WG;
+  constexpr uint32_t M = 2147483647u, R = M - 2;
+  auto mul = [](uint32_t a, uint32_t b) -> uint32_t {
+    const uint64_t p = (uint64_t)a * b;
+    uint32_t r = (uint32_t)(p & M) + (uint32_t)(p >> 31);
+    return r >= M ? r - M : r;
+  };
+  __shared__ unsigned part[WG];
+  __shared__ unsigned base_s;
+  const int tid = threadIdx.x;
+  const int64_t q0 = (int64_t)blockIdx.x * SHUFFLE_BLOCK_DRAWS + (int64_t)tid * PER;
+  const int mine = (int)max((int64_t)0, min((int64_t)PER, positions - q0));
+  // state before draw q0: 16807^q0 steps on
+  uint32_t x = x0;
+  for (uint32_t e = (uint32_t)q0, pw = 16807u; e != 0; e >>= 1, pw = mul(pw, pw))
+    if (e & 1) x = mul(x, pw);
+  // lands in the first k entries only below k * floor(R / (step + 1)): the smallest step that the
+  // thread's draws can serve bounds it for all of them
+  const int64_t at = first_step + q0;
+  const uint32_t ue_low = (uint32_t)max((int64_t)1, at - shuffle_slack(at + PER) + 1);
+  const uint64_t low = (uint64_t)k * (R / ue_low);
+  auto matters = [&](uint32_t ret, int j) {
+    return (uint64_t)ret < low || ret >= R - (uint32_t)(at + j);
+  };
+  unsigned cnt = 0;
+  uint32_t y = x;
+  for (int j = 0; j < mine; j++) {
+    y = mul(y, 16807u);
+    cnt += matters(y - 1, j) ? 1 : 0;
+  }
+  part[tid] = cnt;
+  __syncthreads();
+  for (int off = 1; off < WG; off <<= 1) {  // inclusive scan
+    const unsigned v = tid >= off ? part[tid - off] : 0;
+    __syncthreads();
+    part[tid] += v;
+    __syncthreads();
+  }
+  if (tid == WG - 1) {
+    base_s = atomicAdd(total, part[tid]);
+    table[blockIdx.x] = make_uint2(base_s, part[tid]);
+  }
+  __syncthreads();
+  unsigned w = base_s + part[tid] - cnt;
+  y = x;
+  for (int j = 0; j < mine; j++) {
+    y = mul(y, 16807u);
+    if (matters(y - 1, j)) {
+      if (w < cap) list[w] = make_uint2((unsigned)(q0 + j), y - 1);
+      w++;
+    }
+  }
+}
+int launch_shuffle_draws(hipStream_t s, uint32_t x, int64_t first_step, int64_t positions, int k, uint2 *table,
+                         uint2 *list, unsigned cap, unsigned *total) {
+  if (positions < 1 || first_step + positions >= ((int64_t)1 << 30) || k < 1) return H2O4GPU_KMEANS_EARG;
+  hipLaunchKernelGGL(shuffle_draws_kernel, dim3((unsigned)shuffle_draw_blocks(positions)), dim3(WG), 0, s, x,
+                     first_step, positions, k, table, list, cap, total);
   KM_HIP_TRY(hipGetLastError());
   return 0;
 }

@@ -219,6 +219,7 @@ int launch_fill(hipStream_t s, T *out, T value, int64_t n) {
   return 0;
 }
 template int launch_fill<float>(hipStream_t, float *, float, int64_t);
+template int launch_fill<int>(hipStream_t, int *, int, int64_t);
 template int launch_fill<double>(hipStream_t, double *, double, int64_t);
 
 template <typename T>
