@@ -645,6 +645,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   uint2 *draw_table = nullptr, *draw_list = nullptr;
   T *kpp_dcc = nullptr;     // [k] distances newest centre -> earlier centres
   bool have_data = false, have_centroids = false, have_mindist = false;
+  unsigned *finalize_done = nullptr;  // workgroups of a finalize launch that have ended
   int *d_frozen = nullptr;  // [sets] flags of a stacked handle's sets that have converged
   // (option fp32_split, tiled kernel) the centroids' bfloat16 parts, rewritten by every launch
   unsigned char *d_split = nullptr;
@@ -750,6 +751,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     want(list, &C[1], kpad * d);
     want(list, &counts, k);
     want(list, &d_frozen, sets);
+    want(list, &finalize_done, 1);
     want(list, &labels, (size_t)n * sets);  // the reference's label vector starts zeroed (thrust::device_vector<int>)
     want(list, &cnorm, kpad);
     want(list, &xnorm, n);
@@ -1338,24 +1340,25 @@ struct Engine : h2o4gpu_kmeans_handle {
     return 0;
   }
 
-  int update_async(bool want_shift = true) {
+  int update_async(bool want_shift = true, T *shift_host = nullptr) {
     KM_TRY(ensure_work());
     if (use_buckets && opt_buckets) {
       PROFILED("accumulate", launch_bucketed_accumulate<T>(stream, X, labels, order, order_label,
                                                            bucket_offsets, bucket_hist, bucket_seg,
                                                            bucket_total, bucket_partials, psums,
                                                            pcounts, n, d, k));
-      return finish_update(1, want_shift);
+      return finish_update(1, want_shift, shift_host);
     }
     PROFILED("accumulate", launch_accumulate<T>(stream, plan, X, labels, psums, pcounts, n, d, k));
-    return finish_update(plan.row_blocks, want_shift);
+    return finish_update(plan.row_blocks, want_shift, shift_host);
   }
 
   // one Lloyd step: labels against the current centroids, then the update.
   // want_shift: the caller will read the convergence scalar of this step.
   // want_mindist false: the step need not leave the rows' minimum distances behind (a later
   // assignment pass will, before anyone reads them): one store per row less in the fused step.
-  int step_async(bool want_shift, bool want_mindist = true) {
+  // shift_host: pinned memory that receives the scalar as well (want_shift only).
+  int step_async(bool want_shift, bool want_mindist = true, T *shift_host = nullptr) {
     // (the exact-compare argmin exists in the assignment-only kernels)
     KM_TRY(ensure_work());
     const int fam = pick_assign_variant<T>(opt_assign, n, d, k);
@@ -1368,18 +1371,19 @@ struct Engine : h2o4gpu_kmeans_handle {
                                            k, num_cu, psums, pcounts, &slots, &last_variant, shape(),
                                            opt_split));
       have_mindist = want_mindist || sets > 1;
-      return finish_update(slots, want_shift);
+      return finish_update(slots, want_shift, shift_host);
     }
     if (sets > 1) return H2O4GPU_KMEANS_ESTATE;  // a stacked handle has no other step
     KM_TRY(assign());
-    return update_async(want_shift);
+    return update_async(want_shift, shift_host);
   }
 
-  // post: also run pass 3 (norms of the new centroids + the shift scalar). Without it the
-  // norms are marked stale and the scalar of this step does not exist.
-  int finish_update(int slots, bool post) {
+  // want_shift: the scalar sum((old - new)^2) of this step is left in shift2 (and in shift_host).
+  // The norms of the new centroids are made by whoever needs them (ensure_cnorm): the fused kernels
+  // do not.
+  int finish_update(int slots, bool want_shift, T *shift_host = nullptr) {
     int nsp = 0;
-    if (sets > 1 && post) {
+    if (sets > 1 && want_shift) {
       // per-set convergence: frozen sets keep their centroids; every set's squared shift is
       // the ordered sum of its own partials
       PROFILED("finalize", launch_finalize<T>(stream, slots, psums, pcounts, C[cur], C[cur ^ 1],
@@ -1394,11 +1398,9 @@ struct Engine : h2o4gpu_kmeans_handle {
       return 0;
     }
     PROFILED("finalize", launch_finalize<T>(stream, slots, psums, pcounts, C[cur], C[cur ^ 1],
-                                            counts, shift_partials, &nsp, d, k));
-    if (post)
-      PROFILED("post_update", launch_post_update<T>(stream, C[cur ^ 1], cnorm, shift_partials,
-                                                    nsp, shift2, d, k));
-    cnorm_stale = !post;
+                                            counts, shift_partials, &nsp, d, k, nullptr, 1,
+                                            want_shift ? finalize_done : (unsigned *)nullptr, shift2, shift_host));
+    cnorm_stale = true;
     cur ^= 1;
     return 0;
   }
@@ -1559,8 +1561,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     auto queue_iteration = [&](int i) -> int {
       log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
-      KM_TRY(step_async(true));
-      KM_HIP_TRY(hipMemcpyAsync(host_shift + (i & 1), shift2, sizeof(T), hipMemcpyDeviceToHost, stream));
+      KM_TRY(step_async(true, true, host_shift + (i & 1)));
       KM_HIP_TRY(hipEventRecord(shift_ready[i & 1], stream));
       return 0;
     };

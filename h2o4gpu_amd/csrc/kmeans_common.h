@@ -206,6 +206,8 @@ int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int
 // [k / kps] flags): centroids of a set of a stacked model whose flag is set stay as they
 // are; each block of 32 coordinates then lies inside one set (kps is a multiple of 32), so
 // a set's squared shift is the sum of its own partials.
+// done (nullable): a counter that is zero between launches; the launch then also leaves the sum of
+// its shift partials in *shift2 and, where given, in *shift_host (pinned host memory).
 static const int64_t FINALIZE_NARROW_KD = 4096;
 static inline int max_shift_partials(int d, int k) {
   const int64_t kd = (int64_t)k * d;
@@ -215,7 +217,8 @@ template <typename T>
 int launch_finalize(hipStream_t s, int slots, const double *psums,
                     const int *pcounts, const T *c_old, T *c_new, int *counts,
                     T *shift_partials, int *n_shift_partials, int d, int k,
-                    const int *frozen = nullptr, int kps = 1);
+                    const int *frozen = nullptr, int kps = 1, unsigned *done = nullptr,
+                    T *shift2 = nullptr, T *shift_host = nullptr);
 // Pass 3: cnorm of the new centroids and the fixed-order sum of the shift
 // partials into *shift2.
 template <typename T>

@@ -906,11 +906,38 @@ int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int
 // order), then group 0 adds the RS range sums in range order. EPW is 32, or 4
 // for a small model with many slots, where 32 would leave a handful of
 // workgroups walking thousands of slots one after the other.
+// Fixed-order sum of n partials by the whole workgroup, valid in thread 0.
+template <typename T>
+__device__ __forceinline__ T sum_shift_partials(const T *shift_partials, int n) {
+#pragma clang fp contract(off)
+  __shared__ T red[WG];
+  const int tid = threadIdx.x;
+  // eight loads in flight per thread, added in index order
+  T acc = 0;
+  int i = tid;
+  for (; i + 7 * WG < n; i += 8 * WG) {
+    T v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = shift_partials[i + u * WG];
+#pragma unroll
+    for (int u = 0; u < 8; u++) acc = acc + v[u];
+  }
+  for (; i < n; i += WG) acc = acc + shift_partials[i];
+  red[tid] = acc;
+  __syncthreads();
+  for (int off = WG / 2; off > 0; off >>= 1) {
+    if (tid < off) red[tid] = red[tid] + red[tid + off];
+    __syncthreads();
+  }
+  return red[0];
+}
+
 template <typename T, int EPW>
 __global__ __launch_bounds__(WG) void finalize_kernel(
     const double *__restrict__ psums, const int *__restrict__ pcounts, int row_blocks,
     const T *__restrict__ c_old, T *__restrict__ c_new, int *__restrict__ counts,
-    T *__restrict__ shift_partials, int d, int k, const int *__restrict__ frozen, int kps) {
+    T *__restrict__ shift_partials, int d, int k, const int *__restrict__ frozen, int kps,
+    unsigned *__restrict__ done, T *__restrict__ shift2, T *__restrict__ shift_host) {
 #pragma clang fp contract(off)
   constexpr int RS = WG / EPW;
   __shared__ double part[RS][EPW];
@@ -977,26 +1004,23 @@ __global__ __launch_bounds__(WG) void finalize_kernel(
     for (int q = 0; q < EPW; q++) acc = acc + red[q];
     shift_partials[blockIdx.x] = acc;
   }
-}
-
-template <typename T>
-int launch_finalize(hipStream_t s, int slots, const double *psums,
-                    const int *pcounts, const T *c_old, T *c_new, int *counts,
-                    T *shift_partials, int *n_shift_partials, int d, int k, const int *frozen,
-                    int kps) {
-  const int64_t kd = (int64_t)k * d;
-  // (a stacked model always takes the wide form: its sets' partials must not share a block)
-  const bool narrow = kd <= FINALIZE_NARROW_KD && slots >= 256 && frozen == nullptr;
-  const int blocks = narrow ? (int)((kd + 3) / 4) : (int)((kd + 31) / 32);
-  if (narrow)
-    hipLaunchKernelGGL((finalize_kernel<T, 4>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
-                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps);
-  else
-    hipLaunchKernelGGL((finalize_kernel<T, 32>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
-                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps);
-  KM_HIP_TRY(hipGetLastError());
-  *n_shift_partials = blocks;
-  return 0;
+  if (done == nullptr) return;
+  // The workgroup that finishes last adds the blocks' partials up, in the order of
+  // sum_shift_partials whichever it is, and leaves the scalar on the device and, where the host
+  // waits for it, in pinned memory: a loop with a convergence test ran a kernel and a copy command
+  // for that, some 12 us of an iteration that may have 60.
+  __shared__ bool last;
+  if (tid == 0)
+    last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  const T sum = sum_shift_partials<T>(shift_partials, (int)gridDim.x);
+  if (tid == 0) {
+    *shift2 = sum;
+    if (shift_host) *shift_host = sum;
+    *done = 0;  // for the next launch
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1008,29 +1032,15 @@ template <typename T>
 __global__ __launch_bounds__(WG) void post_update_kernel(
     const T *__restrict__ c_new, T *__restrict__ cnorm,
     const T *__restrict__ shift_partials, int n_partials, T *__restrict__ shift2,
-    int d, int k) {
+    T *__restrict__ shift_host, int d, int k) {
 #pragma clang fp contract(off)
   const int tid = threadIdx.x;
   if (blockIdx.x == gridDim.x - 1) {
-    __shared__ T red[WG];
-    // eight loads in flight per thread, added in index order
-    T acc = 0;
-    int i = tid;
-    for (; i + 7 * WG < n_partials; i += 8 * WG) {
-      T v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = shift_partials[i + u * WG];
-#pragma unroll
-      for (int u = 0; u < 8; u++) acc = acc + v[u];
+    const T sum = sum_shift_partials<T>(shift_partials, n_partials);
+    if (tid == 0) {
+      *shift2 = sum;
+      if (shift_host) *shift_host = sum;
     }
-    for (; i < n_partials; i += WG) acc = acc + shift_partials[i];
-    red[tid] = acc;
-    __syncthreads();
-    for (int off = WG / 2; off > 0; off >>= 1) {
-      if (tid < off) red[tid] = red[tid] + red[tid + off];
-      __syncthreads();
-    }
-    if (tid == 0) *shift2 = red[0];
     return;
   }
   const int c = blockIdx.x * WG + tid;
@@ -1045,6 +1055,33 @@ __global__ __launch_bounds__(WG) void post_update_kernel(
 }
 
 template <typename T>
+int launch_finalize(hipStream_t s, int slots, const double *psums,
+                    const int *pcounts, const T *c_old, T *c_new, int *counts,
+                    T *shift_partials, int *n_shift_partials, int d, int k, const int *frozen,
+                    int kps, unsigned *done, T *shift2, T *shift_host) {
+  const int64_t kd = (int64_t)k * d;
+  // (a stacked model always takes the wide form: its sets' partials must not share a block)
+  const bool narrow = kd <= FINALIZE_NARROW_KD && slots >= 256 && frozen == nullptr;
+  const int blocks = narrow ? (int)((kd + 3) / 4) : (int)((kd + 31) / 32);
+  // the last workgroup adds up the shift only while there are few: every one releases its writes and
+  // adds to one counter on the way (1024 workgroups: 32 us instead of 8; 48: 6 instead of 4 + 2)
+  T *const sum_to = done && blocks > 64 ? shift2 : nullptr;
+  if (sum_to) done = nullptr;
+  if (narrow)
+    hipLaunchKernelGGL((finalize_kernel<T, 4>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
+                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host);
+  else
+    hipLaunchKernelGGL((finalize_kernel<T, 32>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
+                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host);
+  if (sum_to)
+    hipLaunchKernelGGL((post_update_kernel<T>), dim3(1), dim3(WG), 0, s, c_new, (T *)nullptr, shift_partials,
+                       blocks, sum_to, shift_host, d, k);
+  KM_HIP_TRY(hipGetLastError());
+  *n_shift_partials = blocks;
+  return 0;
+}
+
+template <typename T>
 int launch_post_update(hipStream_t s, const T *c_new, T *cnorm,
                        const T *shift_partials, int n_shift_partials, T *shift2,
                        int d, int k) {
@@ -1054,7 +1091,7 @@ int launch_post_update(hipStream_t s, const T *c_new, T *cnorm,
   const int blocks = separate_norms ? 1 : (k + WG - 1) / WG + 1;
   hipLaunchKernelGGL((post_update_kernel<T>), dim3(blocks), dim3(WG), 0, s, c_new,
                      separate_norms ? (T *)nullptr : cnorm, shift_partials, n_shift_partials,
-                     shift2, d, k);
+                     shift2, (T *)nullptr, d, k);
   KM_HIP_TRY(hipGetLastError());
   if (separate_norms) return launch_row_norms<T>(s, c_new, cnorm, k, d);
   return 0;
@@ -1141,7 +1178,7 @@ template int launch_bucketed_accumulate<double>(hipStream_t, const double *, con
   template UpdatePlan plan_update<T>(int64_t, int, int, int);                        \
   template int launch_finalize<T>(hipStream_t, int, const double *,                  \
                                   const int *, const T *, T *, int *, T *, int *,    \
-                                  int, int, const int *, int);                       \
+                                  int, int, const int *, int, unsigned *, T *, T *);                       \
   template int launch_post_update<T>(hipStream_t, const T *, T *, const T *, int,    \
                                      T *, int, int);                                 \
   template int launch_sum<T>(hipStream_t, const T *, int64_t, double *, int,         \
