@@ -29,8 +29,20 @@ namespace kmhip {
 
 namespace {
 
-constexpr int LR_WG = 512;  // 8 wavefronts
-constexpr int LR_NW = LR_WG / 64;
+// Threads per workgroup. The sums of a long model leave room for one workgroup per CU, so its size is
+// the number of wavefronts that can hide each other's loads and LDS reads: 12 of them from 513
+// float32 features on, which their registers just allow (500k x 784, a step, k = 10: 562 -> 508 us,
+// k = 16: 615 -> 507, 500k x 600, k = 8: 341 -> 250), 8 for shorter rows, of which several workgroups fit
+// (1M x 132, k = 8: 244 against 258 us with 12) and for float64 (500k x 256, k = 16: 440 against 1409).
+template <typename T>
+constexpr int lr_threads(int nvl) { return sizeof(T) == 4 && nvl >= 3 ? 768 : 512; }
+// Whether the rows of the next step are fetched into a second set of registers while the current
+// ones are worked on: float64 rows beyond 128 features (500k x 256, k = 8: 289 -> 240 us, k = 16:
+// 440 -> 400), where a workgroup of 8 wavefronts has a CU to itself and the registers hold both sets.
+// (1M x 96, k = 8: 317 without, 366 with; float32 1M x 256, k = 16: 381 and 454, and from 513
+// features on more wavefronts are worth more.)
+template <typename T>
+constexpr bool lr_ahead(int nvl, int kp) { return sizeof(T) == 8 && nvl >= 2 && nvl * kp <= 32; }
 constexpr int LR_R = 4;    // rows per wavefront and step
 constexpr int LR_KP = 16;  // centroids at most (a launch pads k to 4, 8 or 16)
 constexpr int LR_MAX_NVL = 4;
@@ -53,11 +65,12 @@ size_t longrow_lds(int d, int k, bool sums) {
 }
 
 template <typename T, int NVL, int KP, bool SUMS>
-__global__ __launch_bounds__(LR_WG) void lloyd_longrow_kernel(
+__global__ __launch_bounds__(lr_threads<T>(NVL)) void lloyd_longrow_kernel(
     const T *__restrict__ X, const T *__restrict__ xnorm, const T *__restrict__ C,
     const T *__restrict__ cnorm, int *__restrict__ labels, T *__restrict__ mindist,
     double *__restrict__ psums, int *__restrict__ pcounts, int64_t n, int d, int k) {
 #pragma clang fp contract(off)
+  constexpr int LR_WG = lr_threads<T>(NVL), LR_NW = LR_WG / 64;
   typedef Mfma<T> M;
   constexpr int VW = M::VW;
   typedef typename M::vec_t vec_t;
@@ -111,9 +124,12 @@ __global__ __launch_bounds__(LR_WG) void lloyd_longrow_kernel(
   const int mine = butterfly_index<NB>(lane);
   const int my_r = mine / KP, my_k = mine % KP;
   const bool last_valid = lane + 64 * (NVL - 1) < dq;  // the last vector of this lane exists
-  for (int64_t g = (int64_t)blockIdx.x * LR_NW + wave; g < ngroups; g += (int64_t)gridDim.x * LR_NW) {
+  // (two bodies, so that nothing is moved between the sets)
+  constexpr bool AHEAD = lr_ahead<T>(NVL, KP);
+  const int64_t g_step = (int64_t)gridDim.x * LR_NW;
+  auto fetch = [&](vec_t (&x)[LR_R][NVL], T &xx, int64_t g) {
     const int64_t row0 = g * LR_R;
-    vec_t x[LR_R][NVL];
+    xx = xnorm[min(row0 + my_r, n - 1)];
 #pragma unroll
     for (int r = 0; r < LR_R; r++) {
       const T *xr = X + min(row0 + r, n - 1) * (int64_t)d;
@@ -125,6 +141,9 @@ __global__ __launch_bounds__(LR_WG) void lloyd_longrow_kernel(
         for (int q = 0; q < VW; q++) x[r][j][q] = u[q];
       }
     }
+  };
+  auto step = [&](const vec_t (&x)[LR_R][NVL], T xx, int64_t g) {
+    const int64_t row0 = g * LR_R;
     T val[NV];
 #pragma unroll
     for (int i = 0; i < NV; i++) val[i] = 0;
@@ -166,7 +185,7 @@ __global__ __launch_bounds__(LR_WG) void lloyd_longrow_kernel(
     T best = argmin_start<T>();
     int bidx = -1;
     if (my_k < k) {
-      const T t = xnorm[min(my_row, n - 1)] + ccs[my_k];
+      const T t = xx + ccs[my_k];
       const T dist = fabs(t - (T)2 * val[0]);
       if (dist < best) {
         best = dist;
@@ -203,6 +222,29 @@ __global__ __launch_bounds__(LR_WG) void lloyd_longrow_kernel(
           if (lane == 0) atomicAdd(&cnt[lab], 1);
         }
       }
+    }
+  };
+  vec_t xa[LR_R][NVL];
+  T na;
+  int64_t g = (int64_t)blockIdx.x * LR_NW + wave;
+  if constexpr (AHEAD) {
+    vec_t xb[LR_R][NVL];
+    T nb;
+    // (a fetch past the last group re-reads the last row)
+    if (g < ngroups) fetch(xa, na, g);
+    while (g < ngroups) {
+      fetch(xb, nb, g + g_step);
+      step(xa, na, g);
+      g += g_step;
+      if (g >= ngroups) break;
+      fetch(xa, na, g + g_step);
+      step(xb, nb, g);
+      g += g_step;
+    }
+  } else {
+    for (; g < ngroups; g += g_step) {
+      fetch(xa, na, g);
+      step(xa, na, g);
     }
   }
   if (!SUMS) return;
@@ -253,6 +295,7 @@ int launch_longrow(hipStream_t s, const T *X, const T *xnorm, const T *C, const 
   do {                                                                                             \
     auto kern = lloyd_longrow_kernel<T, NVL, KP, SUMS>;                                            \
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                         \
+    constexpr int LR_WG = lr_threads<T>(NVL), LR_NW = LR_WG / 64;                                  \
     int per_cu = resident_blocks_per_cu(reinterpret_cast<const void *>(kern), LR_WG, lds);         \
     if (per_cu < 1) per_cu = 1;                                                                    \
     if (SUMS) per_cu = std::min(per_cu, longrow_max_slots<T>(d, k, 1));                            \

@@ -833,14 +833,16 @@ __global__ __launch_bounds__(WG) void bucket_sum_kernel(const double *__restrict
 
 size_t bucket_lds_bytes(int k) { return (size_t)bucket_waves(k) * k * sizeof(int); }
 bool bucketed_update_applies(int k_chunks, int k, int d) {
-  // Measured: up to 8 chunks the LDS kernel is ahead (10M x 32, k = 4096: 0.61 vs 0.83 ms;
-  // 8M x 16, k = 8192: 0.40 vs 0.66), from 11 chunks on bucketing is (2M x 256, k = 1024:
-  // 0.49 vs 0.62; 500k x 784, k = 256: 0.36 vs 0.52). With a handful of centroids a bucket
-  // spans thousands of windows and the per-label sum has no parallelism left, so bucketing
-  // is never used while the sums fit LDS.
-  (void)d;
-
-  return k_chunks > KM_MAX_LDS_CHUNKS && (size_t)k * sizeof(int) <= 128 * 1024;
+  if ((size_t)k * sizeof(int) > 128 * 1024) return false;
+  // Short rows: up to 8 chunks of centroids the LDS kernel is ahead (2M x 32, k = 4096: 0.15 vs
+  // 0.21 ms, 2M x 64, k = 1000: 0.19 vs 0.22).
+  if (k_chunks > KM_MAX_LDS_CHUNKS) return true;
+  // From rows of about 100 features on, a gathered row is a few whole cache lines and bucketing
+  // is ahead as soon as there is more than one chunk (2M x 101, k = 256: 0.30 vs 0.27 ms, 2M x 256,
+  // k = 100: 0.57 vs 0.45, 640k x 784, k = 100: 0.54 vs 0.45). With a single chunk (298 features, k = 48
+  // 0.59 vs 0.47; 256, k = 48 0.47 vs 0.45) it would need counts that a handful of centroids, whose
+  // buckets span thousands of windows each, does not have.
+  return d >= 96 && k_chunks > 1;
 }
 
 template <typename T>
