@@ -1044,10 +1044,18 @@ struct Engine : h2o4gpu_kmeans_handle {
     std::vector<int> all(1, dis(gen));
     std::vector<int> recent = all;
     T *cost = nullptr, *Cc = nullptr, *ccn = nullptr, *best = nullptr;
-    int *list = nullptr, *didx = nullptr, *dcount = nullptr, *near = nullptr;
-    int rc = parallel_rounds(seed, all, recent, &cost, &Cc, &ccn, &best, &list, &didx, &dcount, &near);
+    int *list = nullptr, *didx = nullptr, *dcount = nullptr, *near = nullptr, *spare = nullptr;
+    std::vector<Want> wants;
+    want(wants, &cost, n);
+    want(wants, &near, n);
+    want(wants, &list, n);
+    want(wants, &didx, n);
+    want(wants, &dcount, 1);
+    unsigned char *seed_slab = nullptr;
+    int rc = allocate(wants, &seed_slab);
+    if (rc == 0) rc = parallel_rounds(seed, all, recent, cost, &Cc, &ccn, &best, list, didx, dcount, near, &spare);
     (void)hipStreamSynchronize(stream);
-    void *ptrs[] = {cost, Cc, ccn, best, list, didx, dcount, near};
+    void *ptrs[] = {seed_slab, Cc, ccn, best, spare};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
     have_mindist = false;  // mindist served as scratch
@@ -1067,30 +1075,28 @@ struct Engine : h2o4gpu_kmeans_handle {
     *have = count;
     return 0;
   }
-  int parallel_rounds(int seed, std::vector<int> &all, std::vector<int> &recent, T **cost, T **Cc,
-                      T **ccn, T **best, int **list, int **didx, int **dcount, int **near) {
+  int parallel_rounds(int seed, std::vector<int> &all, std::vector<int> &recent, T *cost, T **Cc,
+                      T **ccn, T **best, int *list, int *didx, int *dcount, int *near,
+                      int **spare) {
     const int k = kk();
     const int64_t nb = (n + KPP_BLOCK - 1) / KPP_BLOCK;
-    size_t cap_model = 0, cap_norm = 0, cap_idx = 0, cap_best = 0;
+    size_t cap_model = 0, cap_norm = 0, cap_best = 0;
     const int list_cap = (int)n;
     // per-row scratch of the rounds: the selected set's own block of a stacked handle (the
     // block that init_parallel clears afterwards)
     T *const md = mindist + row_off();
     int *const lb = labels + row_off();
-    KM_TRY(dalloc(cost, n));
-    KM_TRY(dalloc(near, n));
-    KM_TRY(dalloc(list, list_cap));
-    KM_TRY(dalloc(dcount, 1));
     std::vector<double> bs((size_t)nb);
     // stage m candidate rows as a padded model
     auto stage = [&](const std::vector<int> &rows) -> int {
       const size_t m = rows.size();
       const size_t mpad = (m + CENTROID_PAD - 1) / CENTROID_PAD * CENTROID_PAD;
-      KM_TRY(regrow(Cc, &cap_model, mpad * d));
-      KM_TRY(regrow(ccn, &cap_norm, mpad));
-      KM_TRY(regrow(didx, &cap_idx, m));
-      KM_HIP_TRY(hipMemcpyAsync(*didx, rows.data(), m * sizeof(int), hipMemcpyHostToDevice, stream));
-      return launch_gather_model<T>(stream, X, xnorm, *didx, (int)m, (int)mpad, *Cc, *ccn, d);
+      // (room for what a run usually ends with at once: the candidates come to a little over 2k)
+      const size_t room = cap_norm == 0 ? std::max(mpad, ((size_t)k * 9 / 4 + 511) / CENTROID_PAD * CENTROID_PAD) : mpad;
+      KM_TRY(regrow(Cc, &cap_model, room * d));
+      KM_TRY(regrow(ccn, &cap_norm, room));
+      KM_HIP_TRY(hipMemcpyAsync(didx, rows.data(), m * sizeof(int), hipMemcpyHostToDevice, stream));
+      return launch_gather_model<T>(stream, X, xnorm, didx, (int)m, (int)mpad, *Cc, *ccn, d);
     };
     uint32_t state0 = (uint32_t)seed % 2147483647u;  // thrust seeds minstd_rand like this
     if (state0 == 0) state0 = 1;
@@ -1121,7 +1127,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       PROFILED("seed_assign", launch_assign<T>(stream, opt_assign, X, xnorm, *Cc, *ccn, lb, md,
                                                n, d, (int)recent.size(), num_cu, nullptr, true, StackShape(),
                                                opt_split, split_scratch((int)recent.size())));
-      PROFILED("seed_fold", launch_fold_min<T>(stream, md, *cost, kpp_bsums, n, counter == 0, lb, *near,
+      PROFILED("seed_fold", launch_fold_min<T>(stream, md, cost, kpp_bsums, n, counter == 0, lb, near,
                                                recent_off));
       measured = true;
       KM_HIP_TRY(hipMemcpyAsync(bs.data(), kpp_bsums, (size_t)nb * sizeof(double), hipMemcpyDeviceToHost,
@@ -1136,11 +1142,11 @@ struct Engine : h2o4gpu_kmeans_handle {
         settled = true;
         continue;
       }
-      KM_HIP_TRY(hipMemsetAsync(*dcount, 0, sizeof(int), stream));
-      PROFILED("seed_select", launch_select_rows<T>(stream, *cost, total, state0, k, *list, *dcount,
+      KM_HIP_TRY(hipMemsetAsync(dcount, 0, sizeof(int), stream));
+      PROFILED("seed_select", launch_select_rows<T>(stream, cost, total, state0, k, list, dcount,
                                                     list_cap, n));
       int count = 0;
-      KM_HIP_TRY(hipMemcpyAsync(&count, *dcount, sizeof(int), hipMemcpyDeviceToHost, stream));
+      KM_HIP_TRY(hipMemcpyAsync(&count, dcount, sizeof(int), hipMemcpyDeviceToHost, stream));
       KM_HIP_TRY(hipStreamSynchronize(stream));
       if (count > list_cap) count = list_cap;  // (cannot happen: one entry per row at most)
       seed_info.round_count[counter] = count;
@@ -1148,7 +1154,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       if (count == 0) settled = true;
       if (count > 0) {
         recent.resize((size_t)count);
-        KM_HIP_TRY(hipMemcpyAsync(recent.data(), *list, (size_t)count * sizeof(int), hipMemcpyDeviceToHost,
+        KM_HIP_TRY(hipMemcpyAsync(recent.data(), list, (size_t)count * sizeof(int), hipMemcpyDeviceToHost,
                                   stream));
         KM_HIP_TRY(hipStreamSynchronize(stream));
         std::sort(recent.begin(), recent.end());  // the reference's copy_if keeps row order
@@ -1159,13 +1165,20 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     seed_info.cand_rows = all;
     const int M = (int)all.size();
+    // (the last list has been read: the counts per candidate go there. A row may become a candidate
+    // again where its distance to itself is not quite zero, so M may pass n on tiny data.)
+    int *dhist = list;
+    if (M > n) {
+      KM_TRY(dalloc(spare, (size_t)2 * M));
+      didx = *spare;
+      dhist = *spare + M;
+    }
     seed_info.chosen.assign((size_t)k, -1);
     if (M <= k) {  // kmeans_h2o4gpu.cu:536-540: the candidates, then zero rows
       for (int c = 0; c < M; c++) seed_info.chosen[(size_t)c] = c;
       KM_HIP_TRY(hipMemsetAsync(C[cur] + set_off() * d, 0, (size_t)k * d * sizeof(T), stream));
-      KM_TRY(regrow(didx, &cap_idx, (size_t)M));
-      KM_HIP_TRY(hipMemcpyAsync(*didx, all.data(), (size_t)M * sizeof(int), hipMemcpyHostToDevice, stream));
-      KM_TRY(launch_gather_rows<T>(stream, X, *didx, C[cur] + set_off() * d, M, d));
+      KM_HIP_TRY(hipMemcpyAsync(didx, all.data(), (size_t)M * sizeof(int), hipMemcpyHostToDevice, stream));
+      KM_TRY(launch_gather_rows<T>(stream, X, didx, C[cur] + set_off() * d, M, d));
       last_seed_rows.assign((size_t)k, -1);
       std::copy(all.begin(), all.end(), last_seed_rows.begin());
       KM_TRY(centroids_changed());
@@ -1180,19 +1193,15 @@ struct Engine : h2o4gpu_kmeans_handle {
       PROFILED("seed_weights", launch_assign<T>(stream, opt_assign, X, xnorm, *Cc, *ccn, lb, md, n, d,
                                                 (int)recent.size(), num_cu, nullptr, true, StackShape(),
                                                 opt_split, split_scratch((int)recent.size())));
-      PROFILED("seed_fold", launch_fold_min<T>(stream, md, *cost, kpp_bsums, n, 0, lb, *near, recent_off));
+      PROFILED("seed_fold", launch_fold_min<T>(stream, md, cost, kpp_bsums, n, 0, lb, near, recent_off));
     }
     KM_TRY(stage(all));  // the picks below read all candidates
-    int *dhist = nullptr;
-    size_t cap_hist = 0;
-    KM_TRY(regrow(&dhist, &cap_hist, (size_t)M));
     std::vector<int> hist((size_t)M);
     int rc = hipMemsetAsync(dhist, 0, (size_t)M * sizeof(int), stream) == hipSuccess ? 0 : H2O4GPU_KMEANS_EDEVICE;
-    if (rc == 0) rc = launch_label_histogram(stream, *near, dhist, n, M);
+    if (rc == 0) rc = launch_label_histogram(stream, near, dhist, n, M);
     if (rc == 0 && hipMemcpyAsync(hist.data(), dhist, (size_t)M * sizeof(int), hipMemcpyDeviceToHost, stream) != hipSuccess)
       rc = H2O4GPU_KMEANS_EDEVICE;
     if (rc == 0 && hipStreamSynchronize(stream) != hipSuccess) rc = H2O4GPU_KMEANS_EDEVICE;
-    (void)hipFree(dhist);
     KM_TRY(rc);
     std::vector<T> w((size_t)M);
     seed_info.weights.resize((size_t)M);
@@ -1201,7 +1210,6 @@ struct Engine : h2o4gpu_kmeans_handle {
       seed_info.weights[(size_t)c] = (double)hist[(size_t)c];
     }
     // the host k-means++ (kmeans_h2o4gpu.cu:201-279); its distances run on the device
-    KM_TRY(regrow(best, &cap_best, (size_t)M));
     std::vector<T> thr((size_t)M), share((size_t)M);
     {
       std::mt19937 mt(seed);  // the sampler makes a fresh one on every call: same draws
@@ -1283,6 +1291,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       }
       (void)hipGetLastError();  // no room for the matrix: one kernel per pick, below
     }
+    KM_TRY(regrow(best, &cap_best, (size_t)M));
     T *CcT = nullptr;
     int prc = 0;
     if (opt_assign == ASSIGN_VALU) {
