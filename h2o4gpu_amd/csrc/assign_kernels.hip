@@ -9,6 +9,7 @@
 // when nothing is below it.
 #include <type_traits>
 
+#include "bf16_parts.h"
 #include "kmeans_common.h"
 #include "mfma_traits.h"
 
@@ -23,20 +24,6 @@ __host__ __device__ static inline int staged_row_stride(int d) {
   int sx = d | 1;
   if (((sx + 1) & sx) == 0) sx += 2;
   return sx;
-}
-
-// Squared norm of one centroid row, j ascending, multiply and add rounded separately:
-// the value row_norms / post_update would store (kmeans_labels.h:187-199). The fused
-// kernels call it when they are given no norm buffer, which spares the Lloyd loop a launch.
-template <typename T>
-__device__ __forceinline__ T row_sqnorm(const T *__restrict__ x, int d) {
-#pragma clang fp contract(off)
-  T acc = 0;
-  for (int j = 0; j < d; j++) {
-    const T v = x[j];
-    acc = acc + v * v;
-  }
-  return acc;
 }
 
 // Features [j, j + VW) of a row of d >= VW values that is aligned to its elements only;
@@ -497,59 +484,6 @@ __global__ __launch_bounds__(WG) void lloyd_valu_anyd_kernel(
   for (int c = tid; c < k; c += WG) cdst[c] = cnt[c];
 }
 
-// Three-input unsigned minimum as ONE instruction. Written as inline assembly
-// because the optimiser otherwise re-associates a chain of them into pairs of
-// two-input minima and spends 12 instead of 8 instructions on 16 keys.
-__device__ __forceinline__ unsigned umin3(unsigned a, unsigned b, unsigned c) {
-  unsigned r;
-  asm("v_min3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
-// centroid row of accumulator v (runtime v) of the 32x32 float tile
-__device__ __forceinline__ int key_row(unsigned v, int g) {
-  return (int)((v >> 2) * 8 + (unsigned)g * 4 + (v & 3));
-}
-
-// float32 products on the bfloat16 matrix pipe. A float is the exact sum of three
-// bfloat16 values (8 significant bits each: the float rounded to bfloat16, the remainder
-// rounded to bfloat16, and what is left of it, which has at most 8 significant bits; every
-// subtraction is exact), so x * c is the exact sum of the nine products of their parts, each
-// of which a float holds exactly (16 bits). v_mfma_f32_32x32x16_bf16 adds such products
-// into float accumulators: the result carries float rounding of the running sum only, as
-// the float32 instruction's does. On gfx950 the instruction runs at 16 times the float32
-// rate (nine of them per 16 features take 288 cycles where eight v_mfma_f32_32x32x2_f32
-// take 512). The parts are rounded to nearest (v_cvt_pk_bf16_f32), not cut off: the
-// remainders then carry either sign, and the products the 6-product form leaves out cancel
-// on average instead of adding up to a bias of the distances (cut-off parts all have the
-// sign of the float they come from; measured on 6000 x 200 blobs far from the origin, the
-// sum of the minimum distances came out 1.6e-5 too large).
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
-// two floats rounded to bfloat16 in one register: a in bits 0-15, b in bits 16-31
-__device__ __forceinline__ unsigned cvt_pk_bf16(float a, float b) {
-  const floatx2 f = {a, b};
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(f, bf16x2));
-}
-// The three parts of two floats, each pair packed like cvt_pk_bf16 packs it: 11 vector
-// instructions (three conversions, four unpackings, four subtractions).
-struct Bf16x3Pair {
-  unsigned h, m, l;
-};
-__device__ __forceinline__ Bf16x3Pair split_pair_bf16x3(float a, float b) {
-  Bf16x3Pair p;
-  p.h = cvt_pk_bf16(a, b);
-  const float ra = a - __uint_as_float(p.h << 16), rb = b - __uint_as_float(p.h & 0xFFFF0000u);
-  p.m = cvt_pk_bf16(ra, rb);
-  p.l = cvt_pk_bf16(ra - __uint_as_float(p.m << 16), rb - __uint_as_float(p.m & 0xFFFF0000u));
-  return p;
-}
-__device__ __forceinline__ floatx16 mma_bf16(uintx4 a, uintx4 b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
 // ---------------------------------------------------------------------------
 // MFMA row-stationary variant (d <= DP, all centroids resident in LDS).
 //
@@ -584,7 +518,7 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
     const T *__restrict__ C, const T *__restrict__ cnorm,
     int *__restrict__ labels, T *__restrict__ mindist, int64_t n, int d, int k,
     int kp, double *__restrict__ psums, int *__restrict__ pcounts, int c_off, int merge,
-    int sets, int kps, int kset) {
+    int sets, int kps, int kset, int ncopy) {
   constexpr int TPB = NW * 64;
   typedef Mfma<T> M;
   constexpr int MT = M::MT, KL = M::KL, NACC = M::NACC, VW = M::VW;
@@ -602,12 +536,19 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
 
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *Cs = reinterpret_cast<T *>(smem_raw);  // [KT][NV][64][VW], see cs_slot
-  // (SPLIT: [KT][NS][3][64] vectors of 8 bfloat16, 6 bytes per element instead of 4)
-  T *ccs = SPLIT ? reinterpret_cast<T *>(smem_raw + (size_t)kp * DP * 6) : Cs + (size_t)kp * DP;  // [kp]
+  // (SPLIT: [KT][NS][3][64] vectors of 8 bfloat16, 6 bytes per element instead of 4, and behind
+  // them [KT][64] vectors with the norms' parts, see below)
+  T *ccs = Cs + (size_t)kp * DP;  // [kp] (not SPLIT)
+  uintx4 *nps = reinterpret_cast<uintx4 *>(smem_raw + (size_t)kp * DP * 6);  // (SPLIT)
   constexpr int SD = DP + 1;
   // (FUSE) sums in double: ds_add_f64 is the fast LDS floating-point atomic on gfx950
-  double *sums = reinterpret_cast<double *>(ccs + kp + (kp & 1));  // [k][SD], 8-byte aligned
-  int *cnt = reinterpret_cast<int *>(sums + (size_t)k * SD);       // [k]
+  // The 32 rows of a tile add their feature f at the same moment; rows of one centroid then queue up
+  // at one address. With a few dozen centroids that is most of a fused step, so lane l adds into copy
+  // l % ncopy (a power of two) of the sums (2M x 64, k = 17: 165 -> 131 us a step, k = 40 201 -> 165,
+  // 2M x 16, k = 20 56 -> 44).
+  double *sums = SPLIT ? reinterpret_cast<double *>(nps + kp * 2)
+                       : reinterpret_cast<double *>(ccs + kp + (kp & 1));  // [ncopy][k][SD], 8-byte aligned
+  int *cnt = reinterpret_cast<int *>(sums + (size_t)ncopy * k * SD);       // [ncopy][k]
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -626,9 +567,11 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
   };
 
   if (FUSE) {
-    for (int e = tid; e < k * SD; e += TPB) sums[e] = 0.0;
-    for (int c = tid; c < k; c += TPB) cnt[c] = 0;
+    for (int e = tid; e < ncopy * k * SD; e += TPB) sums[e] = 0.0;
+    for (int c = tid; c < ncopy * k; c += TPB) cnt[c] = 0;
   }
+  double *const my_sums = sums + (size_t)(lane & (ncopy - 1)) * k * SD;
+  int *const my_cnt = cnt + (size_t)(lane & (ncopy - 1)) * k;
 
   if constexpr (SPLIT != 0) {
     // one (centroid, step, lane group) per thread and turn: its 8 features, times -2
@@ -637,9 +580,17 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
       const int c = e / (NS * KL), rem = e - c * (NS * KL), st = rem / KL, gg = rem - st * KL;
       float v[8];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const int f = ((2 * st + j / VW) * KL + gg) * VW + j % VW;
-        v[j] = (c < k && f < d) ? -2.0f * (float)C[(size_t)c * d + f] : 0.0f;
+      for (int h = 0; h < 2; h++) {
+        const int f = ((2 * st + h) * KL + gg) * VW;
+        const T *src = C + (size_t)c * d + f;
+        if (c < k && f + VW <= d) {
+          const typename M::uvec_t u = *reinterpret_cast<const typename M::uvec_t *>(src);
+#pragma unroll
+          for (int j = 0; j < 4; j++) v[4 * h + j] = -2.0f * (float)u[j % VW];
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; j++) v[4 * h + j] = (c < k && f + j < d) ? -2.0f * (float)src[j] : 0.0f;
+        }
       }
       uintx4 ph, pm, pl;
 #pragma unroll
@@ -694,24 +645,45 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
   // Stacked model (sets > 1): `sets` independent centroid sets laid end to end, each padded
   // to kps rows (a multiple of the tile height) of which the first kset are centroids; a
   // padding row's norm is +inf, so it can never win. One set: kps = kp, kset = k.
-  for (int c = tid; c < kp; c += TPB)
-    ccs[c] = (c < k && (c % kps) < kset && cnorm) ? cnorm[c] : pos_inf<T>();
-  __syncthreads();
-  if (cnorm == nullptr) {
-    // No norm buffer given: take the norms from the staged centroids. A staged value is
-    // -2c; halving it is exact, so the sum below (j ascending, multiply and add rounded
-    // separately) is bit for bit what row_norms / post_update would have stored.
-#pragma clang fp contract(off)
-    for (int c = tid; c < k; c += TPB) {
-      if ((c % kps) >= kset) continue;
-      T acc = 0;
-      for (int j = 0; j < d; j++) {
-        const T v = SPLIT ? C[(size_t)c * d + j] : (T)-0.5 * Cs[cs_slot(c, j)];
-        acc = acc + v * v;
+  if constexpr (SPLIT != 0) {
+    // xx + cc joins the accumulators as one more matrix instruction per tile, the last one: lane
+    // group 0's step holds the three parts of cc against ones and ones against the three parts
+    // of xx, group 1's is zero. The accumulators start at zero (an inline constant), so the
+    // products are summed at their own size, and 16 vector additions per tile are gone.
+    for (int e = tid; e < kp * 2; e += TPB) {
+      const int t = e / 64, slot = e - t * 64, c = t * MT + slot % MT;
+      uintx4 v = {0, 0, 0, 0};
+      if (slot < MT) {
+        float cc = pos_inf<float>();
+        if (c < k && (c % kps) < kset) cc = cnorm ? (float)cnorm[c] : (float)row_sqnorm<T>(C + (size_t)c * d, d);
+        const Bf16x3 p = split_norm_bf16x3(cc);
+        v[0] = p.h | (p.m << 16);
+        v[1] = p.l | (0x3F80u << 16);
+        v[2] = 0x3F803F80u;
       }
-      ccs[c] = acc;
+      nps[e] = v;
     }
     __syncthreads();
+  } else {
+    for (int c = tid; c < kp; c += TPB)
+      ccs[c] = (c < k && (c % kps) < kset && cnorm) ? cnorm[c] : pos_inf<T>();
+    __syncthreads();
+    if (cnorm == nullptr) {
+      // No norm buffer given: take the norms from the staged centroids. A staged value is
+      // -2c; halving it is exact, so the sum below (j ascending, multiply and add rounded
+      // separately) is bit for bit what row_norms / post_update would have stored.
+#pragma clang fp contract(off)
+      for (int c = tid; c < k; c += TPB) {
+        if ((c % kps) >= kset) continue;
+        T acc = 0;
+        for (int j = 0; j < d; j++) {
+          const T v = (T)-0.5 * Cs[cs_slot(c, j)];
+          acc = acc + v * v;
+        }
+        ccs[c] = acc;
+      }
+      __syncthreads();
+    }
   }
 
   constexpr int ROWS_PER_WAVE = ROWT * MT;
@@ -817,18 +789,29 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
         }
       }
     }
+    // (SPLIT) the row side of the instruction that adds xx + cc
+    uintx4 xnp[SPLIT ? ROWT : 1];
+    if constexpr (SPLIT != 0) {
+#pragma unroll
+      for (int rt = 0; rt < ROWT; rt++) {
+        const Bf16x3 p = split_norm_bf16x3((float)xx[rt]);
+        xnp[rt][0] = g == 0 ? 0x3F803F80u : 0u;
+        xnp[rt][1] = g == 0 ? 0x3F80u | (p.h << 16) : 0u;
+        xnp[rt][2] = g == 0 ? p.m | (p.l << 16) : 0u;
+        xnp[rt][3] = 0u;
+      }
+    }
     T best[ROWT];
     int bidx[ROWT];
     unsigned bkey[ROWT];  // float32 path: running minimum key and its tile
     int btile[ROWT];
     auto tile_mma = [&](acc_t (&acc)[ROWT], int t) {
-#pragma unroll
-      for (int v = 0; v < NACC; v++) {
-        const T cc = ccs[t * MT + M::acc_row(v, g)];
-#pragma unroll
-        for (int rt = 0; rt < ROWT; rt++) acc[rt][v] = xx[rt] + cc;
-      }
       if constexpr (SPLIT != 0) {
+#pragma unroll
+        for (int rt = 0; rt < ROWT; rt++) {
+#pragma unroll
+          for (int v = 0; v < NACC; v++) acc[rt][v] = 0;
+        }
         const uintx4 *ap = reinterpret_cast<const uintx4 *>(smem_raw) + (size_t)t * NS * 3 * 64 + lane;
 #pragma unroll
         for (int st = 0; st < NS; st++) {
@@ -851,7 +834,16 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
             }
           }
         }
+        const uintx4 an = nps[t * 64 + lane];
+#pragma unroll
+        for (int rt = 0; rt < ROWT; rt++) acc[rt] = mma_bf16(an, xnp[rt], acc[rt]);
         return;
+      }
+#pragma unroll
+      for (int v = 0; v < NACC; v++) {
+        const T cc = ccs[t * MT + M::acc_row(v, g)];
+#pragma unroll
+        for (int rt = 0; rt < ROWT; rt++) acc[rt][v] = xx[rt] + cc;
       }
       const vec_t *ap = reinterpret_cast<const vec_t *>(Cs) + (size_t)t * NV * 64 + lane;
 #pragma unroll
@@ -980,7 +972,7 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
           if (mindist) mindist[(int64_t)set * n + row] = bv;
         }
         if (FUSE && row < n && bidx[rt] >= 0) {
-          double *srow = sums + (size_t)bidx[rt] * SD;
+          double *srow = my_sums + (size_t)bidx[rt] * SD;
 #pragma unroll
           for (int q = 0; q < NV; q++) {
             if (LOAD == 1 || q < nq) {
@@ -991,7 +983,7 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
               }
             }
           }
-          if (g == 0) atomicAdd(&cnt[bidx[rt]], 1);
+          if (g == 0) atomicAdd(&my_cnt[bidx[rt]], 1);
         }
       }
     }  // centroid sets
@@ -1001,10 +993,16 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
     double *dst = psums + (size_t)blockIdx.x * k * d;
     for (int e = tid; e < k * d; e += TPB) {
       const int c = e / d, j = e - c * d;
-      dst[e] = sums[(size_t)c * SD + j];
+      double v = sums[(size_t)c * SD + j];
+      for (int cp = 1; cp < ncopy; cp++) v += sums[((size_t)cp * k + c) * SD + j];  // copy order
+      dst[e] = v;
     }
     int *cdst = pcounts + (size_t)blockIdx.x * k;
-    for (int c = tid; c < k; c += TPB) cdst[c] = cnt[c];
+    for (int c = tid; c < k; c += TPB) {
+      int v = cnt[c];
+      for (int cp = 1; cp < ncopy; cp++) v += cnt[(size_t)cp * k + c];
+      cdst[c] = v;
+    }
   }
 }
 
@@ -1039,7 +1037,8 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
 // turn: vector 0 and 2 to lane group 0, 1 and 3 to lane group 1). Rows past k and features
 // past d are zero, so the tiled kernel needs no bounds on this operand.
 __global__ void split_centroids_kernel(const float *__restrict__ C, uintx4 *__restrict__ out, int k,
-                                       int d, int bc, int nstage, int nblocks) {
+                                       int d, int bc, int nstage, int nblocks, int *fix_count) {
+  if (fix_count && blockIdx.x == 0 && threadIdx.x == 0) *fix_count = 0;  // (NearTies of the launch behind)
   const int tiles = bc / 32;
   const int64_t total = (int64_t)nblocks * nstage * tiles * 64;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
@@ -1073,9 +1072,14 @@ __global__ void split_centroids_kernel(const float *__restrict__ C, uintx4 *__re
   }
 }
 
-template <typename T, int BCW, bool WIDE = false, int SPLIT = 0>
+// XB (with SPLIT): every data value is a bfloat16 itself (8-bit pixels, small integers, indicators):
+// its middle and low parts are zeros, so three of the six products are left, the row side needs no
+// splitting and a third of the LDS. The wavefronts then stand side by side along the centroids only
+// (RW = 1): each reads its centroid parts, the larger operand now, for 128 rows instead of 64.
+template <typename T, int BCW, bool WIDE = false, int SPLIT = 0, bool XB = false>
 struct TiledCfg {
-  static constexpr int TPB = 2 * BCW * 64;
+  static constexpr int RW = XB ? 1 : 2;  // wavefronts along the rows
+  static constexpr int TPB = RW * BCW * 64;
   // WIDE: every wavefront holds twice as many centroid tiles (a 256-centroid block for four
   // wavefronts) at half the stage depth: the same matrix work per stage and barrier, half as
   // many passes over the workgroup's row slice.
@@ -1091,20 +1095,22 @@ struct TiledCfg {
   // one 16-feature step of the bfloat16 instruction; its three parts per element take 6 bytes
   // of LDS where the float takes 4.
   static constexpr int BK = SPLIT ? 16 : (sizeof(T) == 4 ? 32 : 16) / (BCW == 1 || WIDE ? 2 : 1);
-  static constexpr size_t OPERAND_BYTES = (size_t)2 * (BC + BR) * BK * (SPLIT ? 6 : sizeof(T));
+  static constexpr size_t OPERAND_BYTES =
+      SPLIT ? (size_t)2 * (BC * 6 + BR * (XB ? 2 : 6)) * BK : (size_t)2 * (BC + BR) * BK * sizeof(T);
   // two copies of a block's centroid norms behind the operand stages
   static constexpr size_t LDS_BYTES = OPERAND_BYTES + (size_t)2 * BC * sizeof(T);
 };
 
 template <typename T, int MODE, bool VECLOAD, bool DTAIL, int BCW, bool EXACT = false, bool WIDE = false,
-          int SPLIT = 0>
-__global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_kernel(
+          int SPLIT = 0, bool XB = false>
+__global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) void assign_tiled_kernel(
     const T *__restrict__ X, const T *__restrict__ xnorm,
     const T *__restrict__ C, const T *__restrict__ cnorm,
     int *__restrict__ labels, T *__restrict__ mindist, T *__restrict__ D,
-    int64_t n, int64_t ldn, int d, int k, const uintx4 *__restrict__ Cparts) {
+    int64_t n, int64_t ldn, int d, int k, const uintx4 *__restrict__ Cparts, NearTies ties) {
   typedef Mfma<T> M;
-  typedef TiledCfg<T, BCW, WIDE, SPLIT> Cfg;
+  typedef TiledCfg<T, BCW, WIDE, SPLIT, XB> Cfg;
+  static_assert(!XB || SPLIT == 6, "bfloat16 rows: a form of the split kernel");
   static_assert(SPLIT == 0 || (sizeof(T) == 4 && VECLOAD && (SPLIT == 6 || SPLIT == 9)),
                 "bfloat16 parts: float32 rows fetched as vectors");
   constexpr int MT = M::MT, KL = M::KL, NACC = M::NACC, VW = M::VW;
@@ -1112,7 +1118,7 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
   constexpr int DCH = BK / KL;       // features per lane group per stage
   constexpr int NV = DCH / VW;       // 16-byte vectors per lane per tile per stage
   constexpr int CT = BC / BCW / MT;  // centroid tiles per wavefront
-  constexpr int RT = BR / 2 / MT;    // row tiles per wavefront
+  constexpr int RT = BR / Cfg::RW / MT;  // row tiles per wavefront
   constexpr int TILE_ELEMS = MT * BK;               // one operand tile, one stage
   constexpr int A_ELEMS = (BC / MT) * TILE_ELEMS;   // = BC*BK
   constexpr int B_ELEMS = (BR / MT) * TILE_ELEMS;
@@ -1130,7 +1136,7 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
   // after the main loop the same memory is reused for the cross-wave merge
   // SPLIT: [2][tile][16-feature step][part][64 lanes] vectors of 8 bfloat16 for either operand
   constexpr int NSB = SPLIT ? NV / 2 : 1;  // 16-feature steps per stage
-  constexpr int A_BYTES = BC * BK * 6, B_BYTES = BR * BK * 6;
+  constexpr int A_BYTES = BC * BK * 6, B_BYTES = BR * BK * (XB ? 2 : 6);
   unsigned char *Ab = smem_raw, *Bb = smem_raw + 2 * A_BYTES;
   // The accumulators start at zero and -(xx + cc)/2 is added when a block is complete, as in
   // assign_tiled_dma_kernel and for its reason (the partial sums of the dot product are then
@@ -1145,7 +1151,7 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wc = wave % BCW;  // which part of the centroid block
-  const int wr = wave / BCW;  // which half of the row block
+  const int wr = wave / BCW;  // which part of the row block
   const int r = lane % MT;
   const int g = lane / MT;
   // MODE 0: one workgroup per row block. MODE 1: one per (row block, centroid block) pair
@@ -1208,7 +1214,7 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
       // threads of a wavefront write 16 consecutive lane slots of 2 lane groups and both
       // halves: every bank equally often, no swizzle needed.)
       const int sf = s / VW;
-      lds_off[q] = ((((t * NSB + sf / 2) * 3) * 64 + gg * MT + i) * 16) + (sf % 2) * 8;
+      lds_off[q] = ((((t * NSB + sf / 2) * (XB ? 1 : 3)) * 64 + gg * MT + i) * 16) + (sf % 2) * 8;
     }
   }
   int rd_slot[NV];  // this lane's (swizzled) slot when it reads vector q of a tile
@@ -1233,8 +1239,12 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
   int bidx[RT];
   unsigned bkey[RT];
   int bblk[RT];
+  // (SPLIT, float compare) the second smallest distance of the row, for the near-tie test at the end
+  constexpr bool SECOND = SPLIT != 0 && MODE == 0 && EXACT;
+  T second[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; rt++) {
+    second[rt] = pos_inf<T>();
     best[rt] = (T)0.5 * argmin_start<T>();  // the start value FLT_MAX on the accumulators' scale
     bidx[rt] = -1;
     bkey[rt] = 0x7EFFFFF0u;  // FLT_MAX / 2 with the index bits cleared
@@ -1295,6 +1305,14 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
   auto store_parts = [&](unsigned char *dst, const vec_t &v) {
     if constexpr (SPLIT != 0) {
       typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+      if constexpr (XB) {
+        uintx2 p;
+#pragma unroll
+        for (int w = 0; w < 2; w++)
+          p[w] = (__float_as_uint((float)v[2 * w]) >> 16) | (__float_as_uint((float)v[2 * w + 1]) & 0xFFFF0000u);
+        *reinterpret_cast<uintx2 *>(dst) = p;
+        return;
+      }
       uintx2 ph, pm, pl;
 #pragma unroll
       for (int w = 0; w < 2; w++) {
@@ -1368,10 +1386,12 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
           uintx4 bh[RT], bm[RT], bl[RT];
 #pragma unroll
           for (int rt = 0; rt < RT; rt++) {
-            const int o = (((wr * RT + rt) * NSB + sb) * 3) * 64;
+            const int o = (((wr * RT + rt) * NSB + sb) * (XB ? 1 : 3)) * 64;
             bh[rt] = bp[o];
-            bm[rt] = bp[o + 64];
-            bl[rt] = bp[o + 128];
+            if constexpr (!XB) {
+              bm[rt] = bp[o + 64];
+              bl[rt] = bp[o + 128];
+            }
           }
 #pragma unroll
           for (int ct = 0; ct < CT; ct++) {
@@ -1386,10 +1406,12 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
                 acc[ct][rt] = mma_bf16(am, bl[rt], acc[ct][rt]);
               }
               acc[ct][rt] = mma_bf16(al, bh[rt], acc[ct][rt]);
-              acc[ct][rt] = mma_bf16(ah, bl[rt], acc[ct][rt]);
-              acc[ct][rt] = mma_bf16(am, bm[rt], acc[ct][rt]);
+              if constexpr (!XB) {
+                acc[ct][rt] = mma_bf16(ah, bl[rt], acc[ct][rt]);
+                acc[ct][rt] = mma_bf16(am, bm[rt], acc[ct][rt]);
+              }
               acc[ct][rt] = mma_bf16(am, bh[rt], acc[ct][rt]);
-              acc[ct][rt] = mma_bf16(ah, bm[rt], acc[ct][rt]);
+              if constexpr (!XB) acc[ct][rt] = mma_bf16(ah, bm[rt], acc[ct][rt]);
               acc[ct][rt] = mma_bf16(ah, bh[rt], acc[ct][rt]);
             }
           }
@@ -1488,6 +1510,8 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
 #pragma unroll
           for (int rt = 0; rt < RT; rt++) {
             const T a = acc[ct][rt][v] + fma((T)-0.5, cc, xx[rt]);
+            if constexpr (SECOND)
+              second[rt] = __builtin_amdgcn_fmed3f((float)fabs(a), (float)fabs(best[rt]), (float)second[rt]);
             if (fabs(a) < fabs(best[rt])) {
               best[rt] = a;
               loc[rt] = ct * NACC + v;
@@ -1526,18 +1550,24 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
       for (int off = MT; off < 64; off <<= 1) {
         const T ob = __shfl_xor(best[rt], off, 64);
         const int oi = __shfl_xor(bidx[rt], off, 64);
+        if constexpr (SECOND) {
+          const T os = __shfl_xor(second[rt], off, 64);
+          second[rt] = fmin(fmax(best[rt], ob), fmin(second[rt], os));
+        }
         argmin_merge(best[rt], bidx[rt], ob, oi);
       }
     }
     __syncthreads();  // all waves are past their last LDS operand read
     T *mb = reinterpret_cast<T *>(smem_raw);                   // [BCW-1][BR]
     int *mi = reinterpret_cast<int *>(mb + (BCW - 1) * BR);    // [BCW-1][BR]
+    T *ms = reinterpret_cast<T *>(mi + (BCW - 1) * BR);        // (SECOND) [BCW-1][BR]
     if (wc > 0 && g == 0) {
 #pragma unroll
       for (int rt = 0; rt < RT; rt++) {
         const int lr = (wr * RT + rt) * MT + r;
         mb[(wc - 1) * BR + lr] = best[rt];
         mi[(wc - 1) * BR + lr] = bidx[rt];
+        if constexpr (SECOND) ms[(wc - 1) * BR + lr] = second[rt];
       }
     }
     __syncthreads();
@@ -1546,12 +1576,26 @@ __global__ __launch_bounds__(2 * BCW * 64, BCW == 4 ? 1 : 2) void assign_tiled_k
       for (int rt = 0; rt < RT; rt++) {
         const int lr = (wr * RT + rt) * MT + r;
 #pragma unroll
-        for (int w = 0; w < BCW - 1; w++)
+        for (int w = 0; w < BCW - 1; w++) {
+          if constexpr (SECOND)
+            second[rt] = fmin(fmax(best[rt], mb[w * BR + lr]), fmin(second[rt], ms[w * BR + lr]));
           argmin_merge(best[rt], bidx[rt], mb[w * BR + lr], mi[w * BR + lr]);
+        }
         const int64_t row = row0 + lr;
         if (row < n) {
           labels[row] = bidx[rt];
           if (mindist) mindist[row] = (T)2 * best[rt];
+          if constexpr (SECOND) {
+            // (all on the accumulators' scale of half a distance; xx[rt] is -xx / 2, and a centroid
+            // this close has a norm of at most 2 xx + 2 distances)
+            if (ties.count && second[rt] - best[rt] <= ties.margin * (4 * best[rt] - 3 * xx[rt])) {
+              const int at = atomicAdd(ties.count, 1);
+              if (at < ties.cap) {
+                ties.rows[at] = (int)row;
+                ties.keys[at] = ~0ull;
+              }
+            }
+          }
         }
       }
     }
@@ -1927,6 +1971,110 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// Near ties of the split tiled kernel, settled as the float32 instructions settle them.
+//
+// The split products and the float32 instructions round differently, so a row whose two nearest
+// centroids lie within rounding of each other may get either label, and over the iterations of a fit
+// such rows carry on into different centroids. The main kernel lists the rows whose two smallest
+// distances are that close (a few in a thousand); their distances are then formed here with the
+// float32 matrix instructions' own chain of fused multiply-adds: v_mfma_f32_32x32x2_f32 adds its two
+// products one after the other, each rounded, so with the tiled kernels' order of features (of every
+// eight 0 4 1 5 2 6 3 7) and their closing expression a scalar chain gives the same bits, and the row
+// the same label. Lists longer than `cap` (data full of equal centroids) are left as they are: either
+// label is right to rounding.
+// A workgroup takes 16 listed rows and 256 centroids at a time, a centroid per thread, the rows' values
+// broadcast from LDS, the winners combined by one 64-bit minimum per row and wavefront (distance bits
+// above the centroid's index: the lowest index wins a tie). 261k x 298, k = 1000: 38 us beside
+// the 754 of the main kernel (1355 on the float32 instructions), 500k x 784, k = 4096: 291 beside 8224.
+// ---------------------------------------------------------------------------
+static constexpr int TIE_ROWS = 16, TIE_PIECE = 128;
+__global__ __launch_bounds__(WG) void near_ties_kernel(const float *__restrict__ X, const float *__restrict__ xnorm,
+                                                      const float *__restrict__ C, const float *__restrict__ cnorm,
+                                                      int d, int k, NearTies ties) {
+  __shared__ floatx4 xs[TIE_ROWS][TIE_PIECE / 4];
+  const int m = *ties.count;
+  if (m > ties.cap) return;
+  const int groups = (m + TIE_ROWS - 1) / TIE_ROWS, blocks = (k + WG - 1) / WG;
+  const int tid = threadIdx.x;
+  for (int unit = blockIdx.x; unit < groups * blocks; unit += gridDim.x) {
+    const int g = unit / blocks, c = (unit - g * blocks) * WG + tid;
+    const float *crow = C + (size_t)min(c, k - 1) * d;
+    float acc[TIE_ROWS];
+#pragma unroll
+    for (int r = 0; r < TIE_ROWS; r++) acc[r] = 0;
+    auto load8 = [&](float (&v)[8], int f) {
+      if (f + 8 <= d) {
+        const floatx4_u a = *reinterpret_cast<const floatx4_u *>(crow + f);
+        const floatx4_u b = *reinterpret_cast<const floatx4_u *>(crow + f + 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          v[e] = a[e];
+          v[4 + e] = b[e];
+        }
+      } else {  // features past the end: zeros, which leave a chain as it is
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = f + e < d ? crow[f + e] : 0.0f;
+      }
+    };
+    float nx[8];
+    load8(nx, 0);
+    for (int d0 = 0; d0 < d; d0 += TIE_PIECE) {
+      __syncthreads();  // the piece before has been read
+      for (int e = tid; e < TIE_ROWS * TIE_PIECE; e += WG) {
+        const int r = e / TIE_PIECE, f = d0 + e % TIE_PIECE;
+        const int64_t row = ties.rows[min(g * TIE_ROWS + r, m - 1)];
+        reinterpret_cast<float *>(xs)[e] = f < d ? X[row * d + f] : 0.0f;
+      }
+      __syncthreads();
+      const int lim = min(TIE_PIECE, d - d0);
+      for (int f = 0; f < lim; f += 8) {
+        float cv[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) cv[e] = nx[e];
+        if (d0 + f + 8 < d) load8(nx, d0 + f + 8);  // travels while these eight are used
+#pragma unroll
+        for (int r = 0; r < TIE_ROWS; r++) {
+          const floatx4 a = xs[r][f / 4], b = xs[r][f / 4 + 1];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            acc[r] = fmaf(cv[e], a[e], acc[r]);
+            acc[r] = fmaf(cv[4 + e], b[e], acc[r]);
+          }
+        }
+      }
+    }
+    const float cc = c < k ? cnorm[c] : pos_inf<float>();
+#pragma unroll
+    for (int r = 0; r < TIE_ROWS; r++) {
+      const int at = g * TIE_ROWS + r;
+      if (at < m) {  // (the same for the whole workgroup)
+        const float a = fabsf(acc[r] + fmaf(-0.5f, cc, -0.5f * xnorm[ties.rows[at]]));
+        unsigned long long key = ((unsigned long long)__float_as_uint(a) << 32) | (unsigned)c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const unsigned long long o = __shfl_xor(key, off, 64);
+          key = o < key ? o : key;
+        }
+        if ((tid & 63) == 0) atomicMin(&ties.keys[at], key);
+      }
+    }
+  }
+}
+__global__ __launch_bounds__(WG) void near_ties_labels_kernel(int *__restrict__ labels, float *__restrict__ mindist,
+                                                             NearTies ties) {
+  const int m = *ties.count;
+  if (m > ties.cap) return;
+  for (int at = blockIdx.x * WG + threadIdx.x; at < m; at += gridDim.x * WG) {
+    const unsigned long long key = ties.keys[at];
+    const float start = 0.5f * argmin_start<float>();
+    const unsigned bits = (unsigned)(key >> 32);
+    const bool found = bits < __float_as_uint(start);  // (a NaN compares above)
+    labels[ties.rows[at]] = found ? (int)(unsigned)key : -1;
+    if (mindist) mindist[ties.rows[at]] = 2.0f * (found ? __uint_as_float(bits) : start);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 const char *assign_variant_name(int variant) {
@@ -1952,7 +2100,8 @@ template <typename T>
 static size_t rowstat_lds(int d, int k, int split = 0) {
   const int MT = Mfma<T>::MT;
   const int kp = (k + MT - 1) / MT * MT;
-  return (size_t)kp * rowstat_dp<T>(d) * (split ? 6 : sizeof(T)) + (size_t)kp * sizeof(T);
+  // (split: and the norms' parts take a 16-byte vector per lane of a tile)
+  return (size_t)kp * rowstat_dp<T>(d) * (split ? 6 : sizeof(T)) + (size_t)kp * (split ? 32 : sizeof(T));
 }
 
 static const size_t ROWSTAT_LDS_MAX = 96 * 1024;
@@ -1961,7 +2110,7 @@ template <typename T>
 static int rowstat_chunk(int d, int k, int split = 0) {
   if (rowstat_lds<T>(d, k, split) <= ROWSTAT_LDS_MAX) return k;
   const int MT = Mfma<T>::MT;
-  const size_t per = (size_t)rowstat_dp<T>(d) * (split ? 6 : sizeof(T)) + sizeof(T);
+  const size_t per = (size_t)rowstat_dp<T>(d) * (split ? 6 : sizeof(T)) + (split ? 32 : sizeof(T));
   const int kc_max = (int)(ROWSTAT_LDS_MAX / per) / MT * MT;
   const int chunks = (k + kc_max - 1) / kc_max;
   const int kc = ((k + chunks - 1) / chunks + MT - 1) / MT * MT;  // balanced
@@ -2055,6 +2204,16 @@ static int launch_rowstat_nw(hipStream_t s, const T *X, const T *xnorm, const T 
                              const T *cnorm, int *labels, T *mindist, int64_t n, int d,
                              int k, int num_cu, double *psums, int *pcounts, int *slots,
                              size_t lds, int c_off, int merge, bool exact, const StackShape &st) {
+  int ncopy = 1;
+  // (the one workgroup of a CU; two 4-wave ones share its LDS. From 2048 rows a workgroup on: clearing
+  // and adding up the copies costs a microsecond or two.)
+  if (FUSE && NW > 4 && n >= (int64_t)2048 * num_cu) {
+    const size_t copy = lds - rowstat_lds<T>(d, k, SPLIT);
+    while (ncopy < 8 && lds + (size_t)ncopy * copy <= ROWSTAT_FUSED_LDS_MAX) {
+      lds += (size_t)ncopy * copy;
+      ncopy *= 2;
+    }
+  }
   const int MT = Mfma<T>::MT;
   const int kp = (k + MT - 1) / MT * MT;
   const int sets = st.sets > 1 ? st.sets : 1;
@@ -2078,7 +2237,7 @@ static int launch_rowstat_nw(hipStream_t s, const T *X, const T *xnorm, const T 
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                    \
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), lds, s, X, xnorm, C, cnorm, \
                        labels, mindist, n, d, k, kp, psums, pcounts, c_off, merge, sets, kps, \
-                       kset);                                                                 \
+                       kset, ncopy);                                                          \
   } while (0)
   // the exact-compare form exists for the float32 assignment-only kernels
 #define KM_RS_LAUNCH(LOAD)                                       \
@@ -2369,12 +2528,12 @@ static int launch_tiled_dma(hipStream_t s, const T *X, const T *xnorm, const T *
   return 0;
 }
 
-template <typename T, int MODE, int BCW, bool WIDE = false, int SPLIT = 0>
+template <typename T, int MODE, int BCW, bool WIDE = false, int SPLIT = 0, bool XB = false>
 static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *C,
                             const T *cnorm, int *labels, T *mindist, T *D, int64_t n,
                             int64_t ldn, int d, int k, bool exact, void *cparts = nullptr,
-                            bool direct = true) {
-  typedef TiledCfg<T, BCW, WIDE, SPLIT> Cfg;
+                            bool direct = true, NearTies ties = NearTies()) {
+  typedef TiledCfg<T, BCW, WIDE, SPLIT, XB> Cfg;
   const size_t lds = Cfg::LDS_BYTES;
   if constexpr (SPLIT != 0) {
     // the centroids' parts, once per launch, as the LDS images the kernel stages
@@ -2383,7 +2542,7 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
     const int64_t items = (int64_t)nblocks * nstage * (Cfg::BC / 32) * 64;
     hipLaunchKernelGGL(split_centroids_kernel, dim3((unsigned)std::min<int64_t>((items + 255) / 256, 4096)),
                        dim3(256), 0, s, reinterpret_cast<const float *>(C), static_cast<uintx4 *>(cparts), k,
-                       d, Cfg::BC, nstage, nblocks);
+                       d, Cfg::BC, nstage, nblocks, ties.count);
   }
   if constexpr (SPLIT == 0 && BCW == 2) if (direct) {
     // Stage depth, ring size and issue order per shape, each measured against the others and
@@ -2413,10 +2572,10 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
   const bool tail = (d % Cfg::BK) != 0;
 #define KM_TILED_X(VEC, TAIL, EXACT)                                                         \
   do {                                                                                       \
-    auto kern = assign_tiled_kernel<T, MODE, VEC, TAIL, BCW, EXACT, WIDE, SPLIT>;            \
+    auto kern = assign_tiled_kernel<T, MODE, VEC, TAIL, BCW, EXACT, WIDE, SPLIT, XB>;            \
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                   \
     hipLaunchKernelGGL(kern, grid, dim3(Cfg::TPB), lds, s, X, xnorm, C, cnorm, labels,       \
-                       mindist, D, n, ldn, d, k, static_cast<const uintx4 *>(cparts));       \
+                       mindist, D, n, ldn, d, k, static_cast<const uintx4 *>(cparts), ties); \
   } while (0)
   // From 128 features on the float32 argmin compares the distances themselves: the
   // epilogue is then about one per cent of the matrix work (2M x 256, k = 1024: 8.30 ->
@@ -2438,6 +2597,13 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
   else return H2O4GPU_KMEANS_EARG;
 #undef KM_TILED
 #undef KM_TILED_X
+  if constexpr (SPLIT != 0 && MODE == 0) {
+    if (ties.count && exact) {
+      hipLaunchKernelGGL(near_ties_kernel, dim3(512), dim3(WG), 0, s, X, xnorm, C, cnorm, d, k, ties);
+      hipLaunchKernelGGL(near_ties_labels_kernel, dim3((unsigned)std::min(64, (ties.cap + WG - 1) / WG)), dim3(WG), 0, s,
+                         labels, mindist, ties);
+    }
+  }
   KM_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -2463,6 +2629,23 @@ size_t tiled_split_scratch_bytes(int split, int d, int k) {
   const int bc = tiled_split_wide(k) ? 256 : 128;
   return (size_t)((k + bc - 1) / bc) * bc * ((d + 15) / 16) * 16 * 6;
 }
+// Rows listed at most, and the bytes their list takes behind the parts.
+static int near_ties_cap(int64_t n) { return (int)std::min<int64_t>(n / 16 + 64, 1 << 26); }
+size_t near_ties_bytes(int64_t n) { return 256 + ((size_t)near_ties_cap(n) * 4 + 255) / 256 * 256 + (size_t)near_ties_cap(n) * 8; }
+static NearTies near_ties_at(const SplitScratch &scratch, size_t parts, int64_t n, int d) {
+  NearTies t;
+  const size_t at = (parts + 255) / 256 * 256;
+  if (!scratch.near_ties || !scratch.ptr || scratch.bytes < at + near_ties_bytes(n)) return t;
+  unsigned char *p = static_cast<unsigned char *>(scratch.ptr) + at;
+  t.cap = near_ties_cap(n);
+  t.count = reinterpret_cast<int *>(p);
+  t.rows = reinterpret_cast<int *>(p + 256);
+  t.keys = reinterpret_cast<unsigned long long *>(p + 256 + ((size_t)t.cap * 4 + 255) / 256 * 256);
+  // Rounding noise between the two forms: measured over the shapes above, the difference of two distances
+  // has an rms of about half an eps of xx + cc per form and grows with the square root of the features
+  t.margin = (6.0f + 0.5f * sqrtf((float)d)) * 1.1920929e-7f;
+  return t;
+}
 template size_t tiled_split_scratch_bytes<float>(int, int, int);
 template size_t tiled_split_scratch_bytes<double>(int, int, int);
 
@@ -2476,14 +2659,22 @@ static int launch_tiled(hipStream_t s, const T *X, const T *xnorm, const T *C,
     const bool wide = tiled_split_wide(k);
     const size_t need = tiled_split_scratch_bytes<T>(split, d, k);
     void *split_scratch = scratch.ptr;
-    switch (need > 0 && scratch.ptr && scratch.bytes >= need ? split : 0) {
+    // the list of near ties lies behind the parts, where the caller asks for one
+    const NearTies ties = MODE == 0 && d >= 128 ? near_ties_at(scratch, need, n, d) : NearTies();
+    const int products = need > 0 && scratch.ptr && scratch.bytes >= need ? split : 0;
+    // rows of bfloat16 values: three products (500k x 784 8-bit pixels, k = 4096: 24.0 ms on
+    // the float32 instructions, 12.9 with six products, 8.2 with three)
+    if (products == 6 && wide && scratch.rows_bf16)
+      return launch_tiled_bcw<T, MODE, 4, false, 6, true>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k,
+                                                          exact, split_scratch, true, ties);
+    switch (products) {
 #define KM_TILED_SPLIT(SP)                                                                         \
   case SP:                                                                                         \
     if (wide)                                                                                      \
       return launch_tiled_bcw<T, MODE, 2, true, SP>(s, X, xnorm, C, cnorm, labels, mindist, D, n,  \
-                                                    ldn, d, k, exact, split_scratch);              \
+                                                    ldn, d, k, exact, split_scratch, true, ties);  \
     return launch_tiled_bcw<T, MODE, 2, false, SP>(s, X, xnorm, C, cnorm, labels, mindist, D, n,   \
-                                                   ldn, d, k, exact, split_scratch)
+                                                   ldn, d, k, exact, split_scratch, true, ties)
       KM_TILED_SPLIT(6);
       KM_TILED_SPLIT(9);
 #undef KM_TILED_SPLIT
@@ -2570,11 +2761,36 @@ int launch_assign(hipStream_t s, int variant, const T *X, const T *xnorm,
   return H2O4GPU_KMEANS_EARG;
 }
 
+// The six products are the default of the float32 matrix-core kernels where they are the faster form.
+// Their distances are as close to float64 as the float32 instructions' or closer: over 4 to 784
+// features, 17 to 4096 centroids, centred and offset data the rms error of all distances was 0.82 to
+// 1.00, of the minimum distances 0.6 to 1.02 times theirs (a product is exact to 2^-25 and the
+// accumulators round half as often).
+template <typename T>
+int default_split(SplitUse use, int64_t n, int d, int k) {
+  if (sizeof(T) != 4) return 0;
+  if (d < Mfma<T>::VW) return 0;
+  if (use == SPLIT_TRANSFORM) return tiled_split<T>(6, d, k);
+  const int v = pick_assign_variant<T>(ASSIGN_AUTO, n, d, k);
+  if (v == ASSIGN_TILED) return use == SPLIT_ASSIGN ? tiled_split<T>(6, d, k) : 0;
+  if (v != ASSIGN_ROWSTAT) return 0;
+  // Row-stationary: once the matrix work outweighs splitting a row tile (measured at 2M rows, fused
+  // step: 1.4 to 1.8 times for 65 centroids and more up to 32 features, 1.05 to 1.4 for 33 to 64 of them;
+  // 64 features 1.05, 1.07, 1.23, 1.28 times for 40, 65, 100, 256; 17 centroids 0.98 to 1.1).
+  return k > 64 || d * k > 2048 ? 6 : 0;
+}
+template int default_split<float>(SplitUse, int64_t, int, int);
+template int default_split<double>(SplitUse, int64_t, int, int);
+
 template <typename T>
 AssignInputs assign_inputs(int64_t n, int d, int k) {
   const int v = pick_assign_variant<T>(ASSIGN_AUTO, n, d, k);
   if (v == ASSIGN_VALU) return ASSIGN_FROM_ROWS;
-  if (v == ASSIGN_ROWSTAT && rowstat_chunk<T>(d, k) >= k) return ASSIGN_FROM_ROW_NORMS;
+  // (a model swept in chunks takes the norms of a chunk from the buffer; the staged parts of the
+  // bfloat16 products are larger than the floats, so their chunks are smaller)
+  if (v == ASSIGN_ROWSTAT && rowstat_chunk<T>(d, k) >= k &&
+      rowstat_chunk<T>(d, k, default_split<T>(SPLIT_ASSIGN, n, d, k)) >= k)
+    return ASSIGN_FROM_ROW_NORMS;
   return ASSIGN_FROM_MODEL;
 }
 template AssignInputs assign_inputs<float>(int64_t, int, int);

@@ -1,0 +1,105 @@
+// Building blocks the matrix-core distance kernels share: float32 products on the bfloat16
+// matrix pipe, integer argmin keys, the norm of a staged row.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "mfma_traits.h"
+
+namespace kmhip {
+
+// Squared norm of one centroid row, j ascending, multiply and add rounded separately:
+// the value row_norms / post_update would store (kmeans_labels.h:187-199). The fused
+// kernels call it when they are given no norm buffer, which spares the Lloyd loop a launch.
+template <typename T>
+__device__ __forceinline__ T row_sqnorm(const T *__restrict__ x, int d) {
+#pragma clang fp contract(off)
+  T acc = 0;
+  int j = 0;
+  for (; j + 8 <= d; j += 8) {  // (eight loads under way at a time)
+    T v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = x[j + e];
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc = acc + v[e] * v[e];
+  }
+  for (; j < d; j++) {
+    const T v = x[j];
+    acc = acc + v * v;
+  }
+  return acc;
+}
+
+// Three-input unsigned minimum as ONE instruction. Written as inline assembly
+// because the optimiser otherwise re-associates a chain of them into pairs of
+// two-input minima and spends 12 instead of 8 instructions on 16 keys.
+__device__ __forceinline__ unsigned umin3(unsigned a, unsigned b, unsigned c) {
+  unsigned r;
+  asm("v_min3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+// centroid row of accumulator v (runtime v) of the 32x32 float tile
+__device__ __forceinline__ int key_row(unsigned v, int g) {
+  return (int)((v >> 2) * 8 + (unsigned)g * 4 + (v & 3));
+}
+
+// float32 products on the bfloat16 matrix pipe. A float is the exact sum of three
+// bfloat16 values (8 significant bits each: the float rounded to bfloat16, the remainder
+// rounded to bfloat16, and what is left of it, which has at most 8 significant bits; every
+// subtraction is exact), so x * c is the exact sum of the nine products of their parts, each
+// of which a float holds exactly (16 bits). v_mfma_f32_32x32x16_bf16 adds such products
+// into float accumulators: the result carries float rounding of the running sum only, as
+// the float32 instruction's does. On gfx950 the instruction runs at 16 times the float32
+// rate (nine of them per 16 features take 288 cycles where eight v_mfma_f32_32x32x2_f32
+// take 512). The parts are rounded to nearest (v_cvt_pk_bf16_f32), not cut off: the
+// remainders then carry either sign, and the products the 6-product form leaves out cancel
+// on average instead of adding up to a bias of the distances (cut-off parts all have the
+// sign of the float they come from; measured on 6000 x 200 blobs far from the origin, the
+// sum of the minimum distances came out 1.6e-5 too large).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+// two floats rounded to bfloat16 in one register: a in bits 0-15, b in bits 16-31
+__device__ __forceinline__ unsigned cvt_pk_bf16(float a, float b) {
+  const floatx2 f = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f, bf16x2));
+}
+// The three parts of two floats, each pair packed like cvt_pk_bf16 packs it: 11 vector
+// instructions (three conversions, four unpackings, four subtractions).
+struct Bf16x3Pair {
+  unsigned h, m, l;
+};
+__device__ __forceinline__ Bf16x3Pair split_pair_bf16x3(float a, float b) {
+  Bf16x3Pair p;
+  p.h = cvt_pk_bf16(a, b);
+  const float ra = a - __uint_as_float(p.h << 16), rb = b - __uint_as_float(p.h & 0xFFFF0000u);
+  p.m = cvt_pk_bf16(ra, rb);
+  p.l = cvt_pk_bf16(ra - __uint_as_float(p.m << 16), rb - __uint_as_float(p.m & 0xFFFF0000u));
+  return p;
+}
+// A squared norm as an exact sum of three bfloat16 values with their bits in the low halves of
+// h, m and l. Cut off instead of rounded: the largest floats would round to an infinity, and all
+// parts have the norm's sign here anyway. Infinities and NaN stay whole in the first part.
+struct Bf16x3 {
+  unsigned h, m, l;
+};
+__device__ __forceinline__ Bf16x3 split_norm_bf16x3(float v) {
+  Bf16x3 p;
+  const unsigned u = __float_as_uint(v);
+  p.h = u >> 16;
+  const float r = v - __uint_as_float(u & 0xFFFF0000u);
+  const unsigned ur = __float_as_uint(r);
+  p.m = ur >> 16;
+  p.l = __float_as_uint(r - __uint_as_float(ur & 0xFFFF0000u)) >> 16;
+  if ((u & 0x7F800000u) == 0x7F800000u) {
+    if ((u & 0xFFFFu) != 0) p.h |= 0x40u;  // (a NaN whose payload lies in the low half)
+    p.m = p.l = 0;
+  }
+  return p;
+}
+__device__ __forceinline__ floatx16 mma_bf16(uintx4 a, uintx4 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+}  // namespace kmhip

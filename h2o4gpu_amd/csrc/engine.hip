@@ -237,7 +237,7 @@ struct h2o4gpu_kmeans_handle {
   int opt_fuse = 1;  // 1: use the fused assign+accumulate kernel where the shape allows
   int opt_buckets = 1;  // 1: bucketed centroid sums where the sums do not fit LDS
   int opt_exact = 0;    // 1: float32 MFMA argmin on the float distances, not on 16-ulp keys
-  int opt_split = 0;    // 6 or 9: float32 matrix-core kernels as that many bfloat16 products per feature pair
+  int opt_split = SPLIT_DEFAULT;  // 6 or 9: float32 matrix-core kernels as that many bfloat16 products per feature pair
   int opt_transform_buffers = 2;  // sets of device buffers of a transform in several batches
   int opt_seed_matrix = 1;  // k-means||: distances between candidates as one matrix (0: a kernel per pick)
   int opt_tiled_direct = 1;  // tiled kernels: operands by direct-to-LDS loads where the shape allows
@@ -288,6 +288,8 @@ struct h2o4gpu_kmeans_handle {
   virtual int transform_host(size_t rows, const void *X, void *dist) = 0;
   virtual int transform_resident(void *d_dist) = 0;
   virtual int release() = 0;
+  // bfloat16 products per feature pair of the kernel a Lloyd step labels the rows with (0: none)
+  virtual int step_products() const = 0;
   int kk() const { return sets > 1 ? kset : k; }  // centroids of one set
 
   hipEvent_t get_event() {
@@ -645,6 +647,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   uint2 *draw_table = nullptr, *draw_list = nullptr;
   T *kpp_dcc = nullptr;     // [k] distances newest centre -> earlier centres
   bool have_data = false, have_centroids = false, have_mindist = false;
+  int *rows_inexact = nullptr;
   unsigned *finalize_done = nullptr;  // workgroups of a finalize launch that have ended
   int *d_frozen = nullptr;  // [sets] flags of a stacked handle's sets that have converged
   // (option fp32_split, tiled kernel) the centroids' bfloat16 parts, rewritten by every launch
@@ -654,12 +657,31 @@ struct Engine : h2o4gpu_kmeans_handle {
   // may still read the old one: the stream is drained before it is replaced); null when the
   // option is off or does not apply, and when the allocation fails (the launch then runs the
   // float32 instructions).
-  SplitScratch split_scratch() { return split_scratch(k); }
-  SplitScratch split_scratch(int model_rows) {  // (the seeding runs models of other sizes)
+  // bfloat16 products per feature pair a launch is asked to run with: the option's number or, left
+  // alone, the rule of default_split() (which a kernel family or the exact compare asked for by
+  // name switches off: they stand for the float32 instructions)
+  int split_for(SplitUse use, int model_rows, bool stacked = false) const {
+    if (opt_split != SPLIT_DEFAULT) return opt_split;
+    if (opt_assign != ASSIGN_AUTO || opt_exact || stacked) return 0;
+    return default_split<T>(use, n, d, model_rows);
+  }
+  int step_products() const override {
+    const bool fused = (opt_fuse || sets > 1) && !opt_exact && fused_slots<T>(opt_assign, n, d, k, num_cu) > 0;
+    const int split = split_for(fused ? SPLIT_FUSED : SPLIT_ASSIGN, k, sets > 1);
+    const int products = assign_split_products<T>(opt_assign, split, n, d, k, fused);
+    return products == 6 && rows_bf16 && k > 128 && pick_assign_variant<T>(opt_assign, n, d, k) == ASSIGN_TILED
+               ? 3 : products;
+  }
+  // resident: the launch reads the handle's rows
+  // ties: rows of an assignment whose near ties are settled (default rule only; 0: none)
+  SplitScratch split_scratch(int split, int model_rows, bool resident, int64_t ties) {  // (the seeding runs models of other sizes)
     SplitScratch sc;
     sc.through_registers = opt_tiled_direct == 0;
-    const size_t need = opt_split ? tiled_split_scratch_bytes<T>(opt_split, d, model_rows) : 0;
+    sc.rows_bf16 = resident && rows_bf16;
+    size_t need = split ? tiled_split_scratch_bytes<T>(split, d, model_rows) : 0;
     if (need == 0) return sc;
+    sc.near_ties = ties > 0 && opt_split == SPLIT_DEFAULT && d >= 128;
+    if (sc.near_ties) need = (need + 255) / 256 * 256 + near_ties_bytes(ties);
     if (need > split_bytes) {
       (void)hipStreamSynchronize(stream);
       if (d_split) (void)hipFree(d_split);
@@ -752,6 +774,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     want(list, &counts, k);
     want(list, &d_frozen, sets);
     want(list, &finalize_done, 1);
+    want(list, &rows_inexact, 1);
     want(list, &labels, (size_t)n * sets);  // the reference's label vector starts zeroed (thrust::device_vector<int>)
     want(list, &cnorm, kpad);
     want(list, &xnorm, n);
@@ -833,10 +856,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       own_X = true;
     }
     KM_TRY(upload_rows(dev, stream, X, hX, (size_t)n * d * sizeof(T)));
-    PROFILED("row_norms", launch_row_norms<T>(stream, X, xnorm, n, d));
-    KM_HIP_TRY(hipStreamSynchronize(stream));
-    have_data = true;
-    return 0;
+    return data_changed();
   }
 
   int set_data_device(const void *dX) override {
@@ -845,8 +865,20 @@ struct Engine : h2o4gpu_kmeans_handle {
     if (own_X && X) (void)hipFree(X);
     X = const_cast<T *>(static_cast<const T *>(dX));
     own_X = false;
-    PROFILED("row_norms", launch_row_norms<T>(stream, X, xnorm, n, d));
+    return data_changed();
+  }
+
+  // Norms of the rows, and whether they are bfloat16 values (8-bit pixels, small integers), which the
+  // split kernels need half the products for: the pass over long rows looks at them on its way.
+  bool rows_bf16 = false;
+  int data_changed() {
+    const bool look = row_norms_check<T>(n, d);
+    if (look) KM_TRY(launch_fill<int>(stream, rows_inexact, 0, 1));
+    PROFILED("row_norms", launch_row_norms<T>(stream, X, xnorm, n, d, look ? rows_inexact : (int *)nullptr));
+    int inexact = 1;
+    if (look) KM_HIP_TRY(hipMemcpyAsync(&inexact, rows_inexact, sizeof(int), hipMemcpyDeviceToHost, stream));
     KM_HIP_TRY(hipStreamSynchronize(stream));
+    rows_bf16 = inexact == 0;
     have_data = true;
     return 0;
   }
@@ -1123,10 +1155,11 @@ struct Engine : h2o4gpu_kmeans_handle {
         continue;
       }
       KM_TRY(stage(recent));
+      const int split = split_for(SPLIT_ASSIGN, (int)recent.size());
       // minimum distance to this round's candidates, compared as floats (no integer keys)
       PROFILED("seed_assign", launch_assign<T>(stream, opt_assign, X, xnorm, *Cc, *ccn, lb, md,
                                                n, d, (int)recent.size(), num_cu, nullptr, true, StackShape(),
-                                               opt_split, split_scratch((int)recent.size())));
+                                               split, split_scratch(split, (int)recent.size(), true, 0)));
       PROFILED("seed_fold", launch_fold_min<T>(stream, md, cost, kpp_bsums, n, counter == 0, lb, near,
                                                recent_off));
       measured = true;
@@ -1190,9 +1223,10 @@ struct Engine : h2o4gpu_kmeans_handle {
     // not been through a pass yet.
     if (!measured) {
       KM_TRY(stage(recent));
+      const int split = split_for(SPLIT_ASSIGN, (int)recent.size());
       PROFILED("seed_weights", launch_assign<T>(stream, opt_assign, X, xnorm, *Cc, *ccn, lb, md, n, d,
                                                 (int)recent.size(), num_cu, nullptr, true, StackShape(),
-                                                opt_split, split_scratch((int)recent.size())));
+                                                split, split_scratch(split, (int)recent.size(), true, 0)));
       PROFILED("seed_fold", launch_fold_min<T>(stream, md, cost, kpp_bsums, n, 0, lb, near, recent_off));
     }
     KM_TRY(stage(all));  // the picks below read all candidates
@@ -1262,9 +1296,10 @@ struct Engine : h2o4gpu_kmeans_handle {
       T *G = nullptr;
       if (hG && dalloc(&G, (size_t)M * M) == 0) {
         int grc = 0;
+        const int split = split_for(SPLIT_TRANSFORM, M);
         prof_begin("seed_gram");
         grc = launch_transform<T>(stream, *Cc, *ccn, *Cc, *ccn, G, (int64_t)M, (int64_t)M, d, M, num_cu,
-                                  opt_split, split_scratch(M));
+                                  split, split_scratch(split, M, true, 0));
         prof_end();
         if (grc == 0) grc = download_rows(dev, stream, hG.get(), G, (size_t)M * M * sizeof(T));
         if (grc == 0 && hipStreamSynchronize(stream) != hipSuccess) grc = H2O4GPU_KMEANS_EDEVICE;
@@ -1342,9 +1377,10 @@ struct Engine : h2o4gpu_kmeans_handle {
     KM_HIP_TRY(hipSetDevice(dev));
     if (!have_data || !have_centroids) return H2O4GPU_KMEANS_ESTATE;
     KM_TRY(ensure_cnorm());
+    const int split = split_for(SPLIT_ASSIGN, k, sets > 1);
     PROFILED("assign", launch_assign<T>(stream, opt_assign, X, xnorm, C[cur], cnorm,
                                         labels, mindist, n, d, k, num_cu, &last_variant,
-                                        opt_exact != 0, shape(), opt_split, split_scratch()));
+                                        opt_exact != 0, shape(), split, split_scratch(split, k, true, n)));
     have_mindist = true;
     return 0;
   }
@@ -1378,7 +1414,7 @@ struct Engine : h2o4gpu_kmeans_handle {
                launch_assign_accumulate<T>(stream, opt_assign, X, xnorm, C[cur], (const T *)nullptr,
                                            labels, (want_mindist || sets > 1) ? mindist : (T *)nullptr, n, d,
                                            k, num_cu, psums, pcounts, &slots, &last_variant, shape(),
-                                           opt_split));
+                                           split_for(SPLIT_FUSED, k, sets > 1)));
       have_mindist = want_mindist || sets > 1;
       return finish_update(slots, want_shift, shift_host);
     }
@@ -1525,6 +1561,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     KM_TRY(dalloc(&Cp, kpad * d));
     int rc = dalloc(&cn, kpad);
     const std::vector<T> inf(kpad, std::numeric_limits<T>::infinity());
+    const int split = split_for(SPLIT_ASSIGN, kset);
     for (int s = 0; s < sets && rc == 0; s++) {
       // padded like an ordinary model: zero rows with +inf norms past the last centroid
       if (hipMemsetAsync(Cp, 0, kpad * d * sizeof(T), stream) != hipSuccess ||
@@ -1542,7 +1579,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       prof_begin("assign");
       rc = launch_assign<T>(stream, opt_assign, X, xnorm, Cp, cn, labels + (size_t)s * n,
                             mindist + (size_t)s * n, n, d, kset, num_cu, &last_variant, opt_exact != 0,
-                            StackShape(), opt_split, split_scratch(kset));
+                            StackShape(), split, split_scratch(split, kset, true, n));
       prof_end();
     }
     (void)hipStreamSynchronize(stream);
@@ -1673,14 +1710,15 @@ struct Engine : h2o4gpu_kmeans_handle {
       piece = std::max<size_t>((rows + 7) / 8, ((size_t)32 << 20) / row_bytes);
       piece = (piece + 1023) / 1024 * 1024;
     }
-    const SplitScratch scratch = split_scratch();  // (before the first launch: it may drain the stream)
+    const int split = split_for(SPLIT_ASSIGN, k);
+    const SplitScratch scratch = split_scratch(split, k, false, (int64_t)piece);  // (before the first launch: it may drain the stream)
     for (size_t lo = 0; lo < rows; lo += piece) {
       const size_t cnt = std::min(piece, rows - lo);
       KM_TRY(upload_rows(dev, stream, dX + lo * d, static_cast<const T *>(hX) + lo * d, cnt * row_bytes, lo == 0));
       PROFILED("row_norms", launch_row_norms<T>(stream, dX + lo * d, dxn + lo, (int64_t)cnt, d));
       PROFILED("assign", launch_assign<T>(stream, opt_assign, dX + lo * d, dxn + lo, C[cur], cnorm, dl + lo,
                                           dmin + lo, (int64_t)cnt, d, k, num_cu, &last_variant,
-                                          opt_exact != 0, StackShape(), opt_split, scratch));
+                                          opt_exact != 0, StackShape(), split, scratch));
     }
     KM_TRY(download_rows(dev, stream, out, dl, rows * sizeof(int)));
     KM_HIP_TRY(hipStreamSynchronize(stream));
@@ -1728,7 +1766,8 @@ struct Engine : h2o4gpu_kmeans_handle {
       }
       rc = arc;
     }
-    const SplitScratch scratch = rc == 0 ? split_scratch() : SplitScratch();
+    const int split = split_for(SPLIT_TRANSFORM, k);
+    const SplitScratch scratch = rc == 0 ? split_scratch(split, k, false, 0) : SplitScratch();
     // upload + kernels of batch i, left running
     auto queue_batch = [&](size_t i) -> int {
       const size_t lo = i * batch, cur_rows = std::min(batch, rows - lo);
@@ -1740,7 +1779,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       PROFILED("row_norms", launch_row_norms<T>(stream, dX[b], dxn[b], (int64_t)cur_rows, d));
       PROFILED("transform", launch_transform<T>(stream, dX[b], dxn[b], C[cur], cnorm, dD[b],
                                                 (int64_t)cur_rows, (int64_t)cur_rows, d, k, num_cu,
-                                                opt_split, scratch));
+                                                split, scratch));
       KM_HIP_TRY(hipEventRecord(ready[b], stream));
       return 0;
     };
@@ -1773,9 +1812,10 @@ struct Engine : h2o4gpu_kmeans_handle {
     KM_HIP_TRY(hipSetDevice(dev));
     if (!have_data || !have_centroids || !d_dist || sets > 1) return H2O4GPU_KMEANS_ESTATE;
     KM_TRY(ensure_cnorm());
+    const int split = split_for(SPLIT_TRANSFORM, k);
     PROFILED("transform", launch_transform<T>(stream, X, xnorm, C[cur], cnorm,
-                                              static_cast<T *>(d_dist), n, n, d, k, num_cu, opt_split,
-                                              split_scratch()));
+                                              static_cast<T *>(d_dist), n, n, d, k, num_cu, split,
+                                              split_scratch(split, k, true, 0)));
     KM_HIP_TRY(hipStreamSynchronize(stream));
     return 0;
   }
@@ -1802,11 +1842,11 @@ static int create_engine(h2o4gpu_kmeans_handle **out, size_t rows, size_t cols, 
     e->k = sets * e->kps;
   }
   e->verbose = verbose;
-  // The reference's entry points have no argument for it: H2O4GPU_KMEANS_FP32_SPLIT=6 (or 9)
-  // in the environment turns the "fp32_split" option on for every handle created afterwards.
+  // The reference's entry points have no argument for it: H2O4GPU_KMEANS_FP32_SPLIT=6 (9, 0)
+  // in the environment sets the "fp32_split" option of every handle created afterwards.
   if (const char *env = getenv("H2O4GPU_KMEANS_FP32_SPLIT")) {
     const int v = atoi(env);
-    if (v == 6 || v == 9) e->opt_split = v;
+    if (v == 6 || v == 9 || strcmp(env, "0") == 0) e->opt_split = v;
   }
   if (gpu_id < 0) gpu_id = 0;
   e->dev = gpu_id % nvis;  // kmeans_init: gpu_id = gpu_idtry % n_gpuvis
@@ -2023,16 +2063,30 @@ static void forget_noalloc(int dev) {
   if (dev >= 0 && dev < StagingPool::MAX_DEV) g_noalloc[dev] = NoAllocDevice();
 }
 
-// Cpad [kpad][d] = C [k][d] followed by zero rows; cnorm [k, kpad) = +inf.
+// Cpad [kpad][d] = C [k][d] followed by zero rows; cnorm = the squared norms of the k rows (j ascending,
+// multiply and add rounded separately, the value row_norms stores) followed by +inf. A wavefront per
+// row: coalesced loads, and one lane adds the squares in order from LDS.
 template <typename T>
 __global__ __launch_bounds__(256) void stage_model_kernel(const T *__restrict__ C, T *__restrict__ Cpad,
                                                           T *__restrict__ cnorm, int k, int kpad, int d) {
-  const size_t kd = (size_t)k * d, total = (size_t)kpad * d;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  const size_t t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (size_t e = t0; e < total; e += stride) Cpad[e] = e < kd ? C[e] : (T)0;
-  for (size_t c = (size_t)k + t0; c < (size_t)kpad; c += stride)
-    cnorm[c] = std::numeric_limits<T>::infinity();
+#pragma clang fp contract(off)
+  __shared__ T sq[4][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int c = blockIdx.x * 4 + w;  // (kpad is a multiple of 4)
+  T acc = 0;
+  for (int j0 = 0; j0 < d; j0 += 64) {
+    const int j = j0 + lane;
+    const T v = (c < k && j < d) ? C[(size_t)c * d + j] : (T)0;
+    if (j < d) Cpad[(size_t)c * d + j] = v;
+    __syncthreads();
+    sq[w][lane] = v * v;
+    __syncthreads();
+    if (lane == 0) {
+      const int lim = min(64, d - j0);
+      for (int e = 0; e < lim; e++) acc = acc + sq[w][e];
+    }
+  }
+  if (lane == 0) cnorm[c] = c < k ? acc : std::numeric_limits<T>::infinity();
 }
 
 // Address of this device's copy of `scratch` and the device's CU count, looked up on the
@@ -2085,20 +2139,25 @@ static int predict_device_noalloc(size_t rows, size_t cols, int k, const T *dX, 
   // they read anyway and the row-stationary ones the centroids', so their calls are one and two
   // launches instead of four (1000 x 16, k = 8: 15.0 -> 5.2 us).
   const AssignInputs in = assign_inputs<T>((int64_t)rows, d, k);
+  const int split = default_split<T>(SPLIT_ASSIGN, (int64_t)rows, d, k);
   if (in != ASSIGN_FROM_MODEL) {
     if (in == ASSIGN_FROM_ROW_NORMS) KM_TRY(launch_row_norms<T>(stream, dX, xnorm, (int64_t)rows, d));
     return launch_assign<T>(stream, ASSIGN_AUTO, dX, in == ASSIGN_FROM_ROW_NORMS ? xnorm : (const T *)nullptr, dC,
-                            (const T *)nullptr, d_labels, mind, (int64_t)rows, d, k, nd.num_cu, nullptr);
+                            (const T *)nullptr, d_labels, mind, (int64_t)rows, d, k, nd.num_cu, nullptr, false,
+                            StackShape(), split);
   }
-  const size_t total = kpad * cols;
-  const unsigned blocks = (unsigned)std::min<size_t>((total + 255) / 256, 2048);
-  hipLaunchKernelGGL((stage_model_kernel<T>), dim3(blocks), dim3(256), 0, stream, dC, Cpad, cnorm, k,
+  hipLaunchKernelGGL((stage_model_kernel<T>), dim3((unsigned)(kpad / 4)), dim3(256), 0, stream, dC, Cpad, cnorm, k,
                      (int)kpad, d);
   KM_HIP_TRY(hipGetLastError());
-  KM_TRY(launch_row_norms<T>(stream, Cpad, cnorm, k, d));
   KM_TRY(launch_row_norms<T>(stream, dX, xnorm, (int64_t)rows, d));
+  // the centroids' bfloat16 parts go behind the rest where the array has room for them (without,
+  // the launch runs the float32 instructions)
+  SplitScratch parts;
+  parts.ptr = nd.ptr + need;
+  parts.bytes = (size_t)H2O4GPU_KMEANS_NOALLOC_SCRATCH_BYTES - need;
+  parts.near_ties = true;
   return launch_assign<T>(stream, ASSIGN_AUTO, dX, xnorm, Cpad, cnorm, d_labels, mind, (int64_t)rows, d,
-                          k, nd.num_cu, nullptr);
+                          k, nd.num_cu, nullptr, false, StackShape(), split, parts);
 }
 
 // Largest number of centroid sets (at most max_sets) of k centroids each that one stacked
@@ -2444,6 +2503,8 @@ KM_API const char *h2o4gpu_kmeans_assign_variant(h2o4gpu_kmeans_handle *h) {
   }
   return assign_variant_name(v);
 }
+
+KM_API int h2o4gpu_kmeans_step_products(h2o4gpu_kmeans_handle *h) { return h ? h->step_products() : 0; }
 
 KM_API int h2o4gpu_kmeans_bandwidth_probe(int gpu_id, int kind, size_t bytes, int reps, float *ms) {
   if (!ms || reps < 1 || bytes < 16 || kind < 0 || kind > 3) return H2O4GPU_KMEANS_EARG;

@@ -79,12 +79,34 @@ struct StackShape {
   int kset = 0;
 };
 
+// The number of bfloat16 products per feature pair (0: the float32 instructions) a launch runs
+// with when nobody asked for a number, for each of the three uses of the distance kernels.
+static const int SPLIT_DEFAULT = -1;
+enum SplitUse { SPLIT_ASSIGN, SPLIT_FUSED, SPLIT_TRANSFORM };
+template <typename T>
+int default_split(SplitUse use, int64_t n, int d, int k);
+
+// Rows a split launch of the tiled kernel has found within rounding of a tie (near_ties_kernel).
+struct NearTies {
+  int *count = nullptr;  // null: none are listed
+  int *rows = nullptr;
+  unsigned long long *keys = nullptr;
+  int cap = 0;
+  float margin = 0;  // relative to xx + cc
+};
+size_t near_ties_bytes(int64_t n);
+
 // Device memory a launch with the bfloat16-parts option may write the centroids' parts to
 // (tiled kernel only; tiled_split_scratch_bytes() says how much a shape needs). A launch that
 // is given less runs the float32 instructions.
 struct SplitScratch {
   void *ptr = nullptr;
   size_t bytes = 0;
+  // assignments that compare the distances themselves (128 features and more): settle near ties as the
+  // float32 instructions do; the scratch then holds near_ties_bytes(n) behind the parts (256-aligned)
+  bool near_ties = false;
+  // every value of X is a bfloat16 (row_norms' check): the products with its other parts are zeros
+  bool rows_bf16 = false;
   // tiled kernels: stage the operands through registers also where the direct-to-LDS form
   // applies (handle option "tiled_direct" = 0)
   bool through_registers = false;
@@ -166,8 +188,12 @@ template <typename T>
 int launch_fill(hipStream_t s, T *out, T value, int64_t n);
 
 // out[i] = sum_j X[i][j]^2, j ascending, no contraction.
+// inexact (nullable, device, zero before the call): receives 1 when some value of X is not a
+// bfloat16. Only the pass over many long float32 rows looks (row_norms_check tells); others leave it.
 template <typename T>
-int launch_row_norms(hipStream_t s, const T *X, T *out, int64_t n, int d);
+int launch_row_norms(hipStream_t s, const T *X, T *out, int64_t n, int d, int *inexact = nullptr);
+template <typename T>
+bool row_norms_check(int64_t n, int d);
 
 // Centroid update, pass 1: per-row-block partial sums (always double) and counts.
 struct UpdatePlan {

@@ -157,7 +157,7 @@ __global__ __launch_bounds__(WG) void row_norms_staged_kernel(const T *__restric
 // Bound by the read of X: 500k x 784 1.40 -> 0.314 ms (5.0 TB/s), 261k x 298 0.078 ms.
 template <typename T>
 __global__ __launch_bounds__(WG) void row_norms_long_kernel(const T *__restrict__ X, T *__restrict__ out,
-                                                           int64_t n, int d) {
+                                                           int64_t n, int d, int *__restrict__ inexact) {
 #pragma clang fp contract(off)
   constexpr int VW = 16 / sizeof(T);
   constexpr int PIECE = 128 / sizeof(T);  // features per step
@@ -182,6 +182,7 @@ __global__ __launch_bounds__(WG) void row_norms_long_kernel(const T *__restrict_
   };
   fetch(0);
   T acc = 0;
+  unsigned low = 0;  // bits of the row values below a bfloat16's
   for (int j0 = 0; j0 < d; j0 += PIECE) {
     const int skip = j0 + lj - min(j0 + lj, d - VW);
     __syncthreads();  // the piece before has been consumed
@@ -191,6 +192,10 @@ __global__ __launch_bounds__(WG) void row_norms_long_kernel(const T *__restrict_
 #pragma unroll
       for (int e = 0; e < VW; e++)
         if (e >= skip) dst[e] = pre[i][e];
+      if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int e = 0; e < VW; e++) low |= __float_as_uint(pre[i][e]);
+      }
     }
     __syncthreads();
     if (j0 + PIECE < d) fetch(j0 + PIECE);
@@ -204,6 +209,8 @@ __global__ __launch_bounds__(WG) void row_norms_long_kernel(const T *__restrict_
     }
   }
   if (row0 + tid < n) out[row0 + tid] = acc;
+  // (every writer writes the same value; one per wavefront at most)
+  if (inexact && __ballot((low & 0xFFFFu) != 0) != 0 && (tid & 63) == 0) *inexact = 1;
 }
 
 template <typename T>
@@ -222,8 +229,14 @@ template int launch_fill<float>(hipStream_t, float *, float, int64_t);
 template int launch_fill<int>(hipStream_t, int *, int, int64_t);
 template int launch_fill<double>(hipStream_t, double *, double, int64_t);
 
+static bool row_norms_long(int64_t n, int d) { return d > 64 && n >= 256 * 192; }
 template <typename T>
-int launch_row_norms(hipStream_t s, const T *X, T *out, int64_t n, int d) {
+bool row_norms_check(int64_t n, int d) { return sizeof(T) == 4 && row_norms_long(n, d); }
+template bool row_norms_check<float>(int64_t, int);
+template bool row_norms_check<double>(int64_t, int);
+
+template <typename T>
+int launch_row_norms(hipStream_t s, const T *X, T *out, int64_t n, int d, int *inexact) {
   if (n <= 0) return 0;
   if (d >= 4 && d <= 64 && n * (int64_t)d >= (1 << 22)) {
     int sx = d | 1;
@@ -243,9 +256,9 @@ int launch_row_norms(hipStream_t s, const T *X, T *out, int64_t n, int d) {
   }
   // Many long rows: enough workgroups of 256 rows to give most CUs one. Below that (the
   // centroids of a model, a short batch) a row per wavefront spreads further over the chip.
-  if (d > 64 && n >= 256 * 192) {
+  if (row_norms_long(n, d)) {
     hipLaunchKernelGGL((row_norms_long_kernel<T>), dim3((unsigned)((n + WG - 1) / WG)), dim3(WG), 0, s, X, out, n,
-                       d);
+                       d, inexact);
     KM_HIP_TRY(hipGetLastError());
     return 0;
   }
@@ -1176,7 +1189,7 @@ template int launch_bucketed_accumulate<double>(hipStream_t, const double *, con
                                                 int64_t, int, int);
 
 #define KM_INSTANTIATE(T)                                                            \
-  template int launch_row_norms<T>(hipStream_t, const T *, T *, int64_t, int);       \
+  template int launch_row_norms<T>(hipStream_t, const T *, T *, int64_t, int, int *);       \
   template UpdatePlan plan_update<T>(int64_t, int, int, int);                        \
   template int launch_finalize<T>(hipStream_t, int, const double *,                  \
                                   const int *, const T *, T *, int *, T *, int *,    \

@@ -77,6 +77,7 @@ PROTOTYPES = {
     "h2o4gpu_kmeans_profile": (c_int, [c_void_p, c_int]),
     "h2o4gpu_kmeans_kernel_time": (c_int, [c_void_p, c_char_p, P(c_int), P(c_double)]),
     "h2o4gpu_kmeans_assign_variant": (c_char_p, [c_void_p]),
+    "h2o4gpu_kmeans_step_products": (c_int, [c_void_p]),
     "h2o4gpu_kmeans_copy_probe": (c_int, [c_int, c_size_t, c_int, P(c_float)]),
     "h2o4gpu_kmeans_bandwidth_probe": (c_int, [c_int, c_int, c_size_t, c_int, P(c_float)]),
     "h2o4gpu_kmeans_predict_device_noalloc": (c_int, [c_int, c_size_t, c_size_t, c_int, c_void_p,
@@ -309,6 +310,10 @@ class Handle:
 
     def assign_variant(self):
         return lib().h2o4gpu_kmeans_assign_variant(self._h).decode()
+
+    def step_products(self):
+        """Bfloat16 products per pair of float32 values in a Lloyd step's distance kernel (0: none)."""
+        return lib().h2o4gpu_kmeans_step_products(self._h)
 
     def timer_start(self):
         _check("timer_start", lib().h2o4gpu_kmeans_timer_start(self._h))

@@ -236,16 +236,20 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * themselves instead of 16-ulp integer keys (slower, never fused; 0 is the default).
  * "transform_batch_mb" (default 4096) bounds the device buffer transform_host fills per
  * batch of rows; smaller values force more, shorter batches.
- * "fp32_split" = 9 or 6 (default 0) makes the float32 matrix-core kernels form their dot
+ * "fp32_split" = 6 or 9 makes the float32 matrix-core kernels form their dot
  * products on the bfloat16 matrix pipe: every float is the exact sum of three bfloat16
  * parts (rounded to nearest), 9 runs all nine products of the parts (each exact,
- * accumulated in float32), 6
- * leaves out the three smallest (below one ulp of xx + cc per distance). 1.4 to 1.9 times
- * faster on matrix-bound shapes, same parity bars; shapes it does not apply to (float64,
- * k <= 16 && d <= 64, rows of fewer than 4 features, ...) run as without it, and
- * h2o4gpu_kmeans_assign_variant() names what runs ("mfma_tiled_bf16x6", ...). The
- * environment variable H2O4GPU_KMEANS_FP32_SPLIT=6|9 sets it for every handle created
- * afterwards, the reference's four entry points included.
+ * accumulated in float32), 6 leaves out the three smallest (2^-25 of |x||c| and below); 0 runs the
+ * float32 matrix instructions. A handle that nobody sets it for, and that asks for no kernel family
+ * and no exact compare, runs 6 wherever that is the faster form (more than 64 centroids,
+ * or d * k > 2048; from 17 centroids on for 3 or 4 features, 49 for 5 to 8): 1.4 to 2 times on
+ * matrix-bound shapes, with distances as close to float64 as the float32 instructions' or
+ * closer. Rows whose every value is a bfloat16 (8-bit pixels, small integers) need three of the six.
+ * Shapes it does not apply to (float64, k <= 16 && d <= 64, ...) run as without it.
+ * h2o4gpu_kmeans_assign_variant() names a form that was asked for ("mfma_tiled_bf16x6", ...),
+ * h2o4gpu_kmeans_step_products() says what runs. The environment variable
+ * H2O4GPU_KMEANS_FP32_SPLIT=6|9|0 sets it for every handle created afterwards, the reference's four
+ * entry points included.
  * "transform_buffers" = 2 (default) gives a transform in several batches two sets of device
  * buffers, so that a batch is computed while the previous one is downloaded (this is also
  * what happens with 1, one batch at a time, when the second set cannot be allocated).
@@ -278,6 +282,9 @@ int h2o4gpu_kmeans_kernel_time(h2o4gpu_kmeans_handle *h, const char *kernel,
                                int *launches, double *milliseconds);
 /* Name of the assign kernel variant the handle's shape dispatches to. */
 const char *h2o4gpu_kmeans_assign_variant(h2o4gpu_kmeans_handle *h);
+/* Bfloat16 products per pair of float32 values that the distance kernel of a Lloyd step runs
+ * with (see "fp32_split"): 9, 6, 3, or 0 where it runs the float32 or float64 instructions. */
+int h2o4gpu_kmeans_step_products(h2o4gpu_kmeans_handle *h);
 
 /* Device-to-device copy bandwidth probe: copies `bytes` from one scratch
  * buffer to another `reps` times and returns the average milliseconds of one

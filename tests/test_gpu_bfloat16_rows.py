@@ -1,0 +1,38 @@
+"""Rows whose every value is a bfloat16 (8-bit pixels) run half the products of the split tiled
+kernel; the other half are products with zeros, so labels and distances are the same bits as
+those of rows the handle does not look at (host rows of a predict or transform call)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,d,k", [(49152, 65, 129), (50001, 100, 300), (49153, 784, 257), (60000, 128, 1024)])
+@pytest.mark.parametrize("odd", [None, "first", "last", "middle"])
+def test_same_bits_as_the_general_form(hip, n, d, k, odd):
+    rng = np.random.default_rng(n + d + k)
+    X = rng.integers(0, 256, size=(n, d)).astype(np.float32) * (rng.random((n, d)) < 0.4)
+    X = np.ascontiguousarray(X, np.float32)
+    if odd is not None:  # one value that is not a bfloat16, wherever the pass over the rows may end
+        i, j = {"first": (0, 0), "last": (n - 1, d - 1), "middle": (n // 2 + 1, d - 3)}[odd]
+        X[i, j] = 200.1234
+    C = (X[rng.choice(n, size=k, replace=False)] + rng.standard_normal((k, d))).astype(np.float32)
+    m = 3000
+    part = np.concatenate([X[:m // 3], X[n // 2:n // 2 + m // 3], X[n - m // 3:]])
+    with hip.Handle(n, d, k, np.float32) as h:
+        h.set_data(X)
+        h.set_centroids(C)
+        h.assign()
+        got = h.labels()
+        out = torch.empty((k, n), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        h.transform_resident(out.data_ptr())
+        want, D = h.predict(part), h.transform(part)
+        out = out.cpu().numpy()
+    pick = np.r_[0:m // 3, n // 2:n // 2 + m // 3, n - m // 3:n]
+    assert np.array_equal(got[pick], want)
+    assert np.array_equal(out[:, pick], D)
+    D64 = ((X[pick[::50]].astype(np.float64)[:, None, :] - C.astype(np.float64)[None, :64]) ** 2).sum(2).T
+    scale = (X.astype(np.float64) ** 2).sum(1).max() + (C.astype(np.float64) ** 2).sum(1).max()
+    assert np.abs(out[:64, pick[::50]] - D64).max() <= (4 * np.sqrt(d) + 40) * np.finfo(np.float32).eps * scale

@@ -1,0 +1,73 @@
+"""Rows within rounding of a tie between two centroids: the split tiled kernel lists them and
+settles them with the float32 instructions' own arithmetic, so the labels are those of the float32
+instructions bit for bit, as long as the list (a sixteenth of the rows) holds them."""
+import numpy as np
+import pytest
+
+from parity import label_report
+
+pytestmark = pytest.mark.gpu
+
+
+def labels_of(hip, X, C, split=None, steps=0):
+    n, d = X.shape
+    with hip.Handle(n, d, C.shape[0], np.float32) as h:
+        h.set_data(X)
+        h.set_centroids(C)
+        if split is not None:
+            h.set_option("fp32_split", split)
+        if steps:
+            h.fit(steps, 0.0)
+        else:
+            h.assign()
+        return h.labels(), h.min_distances(), h.centroids()
+
+
+@pytest.mark.parametrize("n,d,k", [(5000, 128, 129), (4097, 131, 300), (20011, 298, 257), (3000, 784, 100), (60001, 256, 1000),
+                                   (129, 136, 70)])
+@pytest.mark.parametrize("whole", [False, True])
+def test_labels_are_the_float32_instructions(hip, n, d, k, whole):
+    rng = np.random.default_rng(n + d + k)
+    C = rng.uniform(0, 200, size=(k, d)).astype(np.float32)
+    # a few centroids within a hair of another one: about three rows in a hundred have both nearest
+    for c in range(0, k - 1, max(2, k // 2)):
+        C[c + 1] = C[c] + (1e-4 * rng.standard_normal(d)).astype(np.float32)
+    X = (C[rng.integers(0, k, size=n)] + 30 * rng.standard_normal((n, d))).astype(np.float32)
+    if whole:  # (rows of bfloat16 values: half the products where the rows are many)
+        X = np.clip(np.rint(X), 0, 255).astype(np.float32)
+    got, mind, _ = labels_of(hip, X, C)
+    want, wmind, _ = labels_of(hip, X, C, split=0)
+    assert np.array_equal(got, want)
+    eps = np.finfo(np.float32).eps
+    scale = (X.astype(np.float64) ** 2).sum(1).max() + (C.astype(np.float64) ** 2).sum(1).max()
+    assert np.abs(mind - wmind).max() <= (4 * np.sqrt(d) + 40) * eps * scale
+
+
+def test_a_fit_takes_the_same_course(hip):
+    rng = np.random.default_rng(4)
+    n, d, k = 60000, 200, 150
+    X = (rng.uniform(0, 50, size=(40, d))[rng.integers(0, 40, size=n)] + 9 * rng.standard_normal((n, d))).astype(np.float32)
+    C = X[rng.choice(n, size=k, replace=False)]
+    got, want = labels_of(hip, X, C, steps=25), labels_of(hip, X, C, split=0, steps=25)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[2], want[2])
+
+
+def test_more_ties_than_the_list_holds(hip, oracle):
+    """Every centroid twice: every row is a tie; either label is right, the lower index wins."""
+    rng = np.random.default_rng(8)
+    n, d, k = 9000, 160, 140
+    C = np.repeat(rng.standard_normal((k // 2, d)).astype(np.float32) * 10, 2, axis=0)
+    X = (C[rng.integers(0, k, size=n)] + rng.standard_normal((n, d))).astype(np.float32)
+    got, _, _ = labels_of(hip, X, C)
+    label_report(oracle, X, C, got, oracle.assign(X, C))
+    assert (got % 2 == 0).all()
+
+
+def test_rows_no_distance_exists_for(hip):
+    rng = np.random.default_rng(9)
+    n, d, k = 3000, 150, 90
+    X, C = rng.standard_normal((n, d)).astype(np.float32), rng.standard_normal((k, d)).astype(np.float32)
+    X[[3, 77, 2999], [0, 149, 20]] = np.nan, np.inf, -np.inf
+    C[11, 5] = np.nan
+    got, want = labels_of(hip, X, C)[0], labels_of(hip, X, C, split=0)[0]
+    assert np.array_equal(got, want) and (got[[3, 77, 2999]] == -1).all()
