@@ -2491,6 +2491,10 @@ int launch_assign_accumulate(hipStream_t s, int variant, const T *X, const T *xn
     return launch_longrow<T, true>(s, X, xnorm, C, cnorm, labels, mindist, n, d, k, num_cu, psums, pcounts,
                                    slots);
   if (v != ASSIGN_ROWSTAT) return H2O4GPU_KMEANS_EARG;
+  if constexpr (sizeof(T) == 4) {
+    if (variant == ASSIGN_AUTO && split == 6 && st.sets <= 1 && shortrow_applies(d, k, true))
+      return launch_shortrow(s, X, C, labels, mindist, n, d, k, num_cu, true, psums, pcounts, slots);
+  }
   return RowstatDispatch<T, true>::run(s, X, xnorm, C, cnorm, labels, mindist, n, d, k,
                                        num_cu, psums, pcounts, slots, 0, 0, false, st, split);
 }
@@ -2734,6 +2738,10 @@ int launch_assign(hipStream_t s, int variant, const T *X, const T *xnorm,
                                            nullptr, nullptr, nullptr);
       return launch_valu<T, 0>(s, X, xnorm, C, cnorm, labels, mindist, nullptr, n, n, d, k);
     case ASSIGN_ROWSTAT: {
+      if constexpr (sizeof(T) == 4) {
+        if (variant == ASSIGN_AUTO && split == 6 && !exact && shortrow_applies(d, k, false))
+          return launch_shortrow(s, X, C, labels, mindist, n, d, k, num_cu, false, nullptr, nullptr, nullptr);
+      }
       // (the staged bfloat16 parts are half as large again as the floats: smaller chunks)
       const int split_dp = rowstat_dp<T>(d);
       const bool split_ok = sizeof(T) == 4 && (split == 6 || split == 9) && !exact && split_dp >= 16 &&
@@ -2769,6 +2777,7 @@ int launch_assign(hipStream_t s, int variant, const T *X, const T *xnorm,
 template <typename T>
 int default_split(SplitUse use, int64_t n, int d, int k) {
   if (sizeof(T) != 4) return 0;
+  if (use != SPLIT_TRANSFORM && shortrow_applies(d, k, use == SPLIT_FUSED)) return 6;
   if (d < Mfma<T>::VW) return 0;
   if (use == SPLIT_TRANSFORM) return tiled_split<T>(6, d, k);
   const int v = pick_assign_variant<T>(ASSIGN_AUTO, n, d, k);
@@ -2786,6 +2795,7 @@ template <typename T>
 AssignInputs assign_inputs(int64_t n, int d, int k) {
   const int v = pick_assign_variant<T>(ASSIGN_AUTO, n, d, k);
   if (v == ASSIGN_VALU) return ASSIGN_FROM_ROWS;
+  if (v == ASSIGN_ROWSTAT && sizeof(T) == 4 && shortrow_applies(d, k, false)) return ASSIGN_FROM_ROWS;
   // (a model swept in chunks takes the norms of a chunk from the buffer; the staged parts of the
   // bfloat16 products are larger than the floats, so their chunks are smaller)
   if (v == ASSIGN_ROWSTAT && rowstat_chunk<T>(d, k) >= k &&

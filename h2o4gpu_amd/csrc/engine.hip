@@ -668,6 +668,9 @@ struct Engine : h2o4gpu_kmeans_handle {
   int step_products() const override {
     const bool fused = (opt_fuse || sets > 1) && !opt_exact && fused_slots<T>(opt_assign, n, d, k, num_cu) > 0;
     const int split = split_for(fused ? SPLIT_FUSED : SPLIT_ASSIGN, k, sets > 1);
+    if (sizeof(T) == 4 && split == 6 && opt_assign == ASSIGN_AUTO && sets == 1 && !opt_exact &&
+        pick_assign_variant<T>(ASSIGN_AUTO, n, d, k) == ASSIGN_ROWSTAT && shortrow_applies(d, k, fused))
+      return 6;
     const int products = assign_split_products<T>(opt_assign, split, n, d, k, fused);
     return products == 6 && rows_bf16 && k > 128 && pick_assign_variant<T>(opt_assign, n, d, k) == ASSIGN_TILED
                ? 3 : products;

@@ -145,6 +145,12 @@ template <typename T, bool SUMS>
 int launch_longrow(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm, int *labels,
                    T *mindist, int64_t n, int d, int k, int num_cu, double *psums, int *pcounts,
                    int *slots);
+// The kernel for rows of three to eight float32 features and more than 16 centroids
+// (shortrow_kernels.hip): whether a shape is its, and the launch. It makes both norms itself and
+// reads the k centroids only; fused: partial sums and counts per workgroup, at most 2 * num_cu slots.
+bool shortrow_applies(int d, int k, bool fused);
+int launch_shortrow(hipStream_t s, const float *X, const float *C, int *labels, float *mindist, int64_t n, int d,
+                    int k, int num_cu, bool fused, double *psums, int *pcounts, int *slots);
 const char *assign_variant_name(int variant);
 // split (float32 matrix-core kernels; 0, 6 or 9): run the dot products on the bfloat16
 // matrix pipe as that many products of bfloat16 parts per feature pair (9: every product

@@ -1,0 +1,296 @@
+// Rows of three to eight float32 features against more than 16 centroids (pixels, coordinates).
+//
+// The row-stationary kernel of assign_kernels.hip pads such rows to eight features and spends
+// four 64-cycle matrix instructions and 16 vector additions on a 32 x 32 tile of distances. Here
+// the tile comes from three (up to four features) or four 32-cycle bfloat16 instructions: a float
+// is the exact sum of three bfloat16 parts (bf16_parts.h), six products of parts make a product of
+// floats to float32 accuracy, and with so few features the six products of all of them lie side by
+// side in the 16-wide k-steps. A lane group holds NP pairs of features, group 0 the features
+// 0 .. 2NP-1, group 1 the rest, and its k-slots are, for every pair (a, b), twelve halves in six
+// registers
+//     row side       h h  m m  l l  h h  m m  h h      (h, m, l: the parts of a and of b)
+//     centroid side  H H  H H  H H  M M  M M  L L      (parts of -2c)
+// which is what splitting a pair yields in packed form anyway. The accumulators start at cc (the
+// instruction takes them from the registers that hold the tile's norms, nothing is moved), the
+// products bring them to the size of xx, and an instruction of its own adds the three parts of xx
+// against ones: every partial sum is rounded at half the size of xx + cc or below. Up to four
+// features the smallest products come after that, at the size of the distance itself. (Distances
+// against float64 at three to eight features, rms, over the float32 instructions': 0.89 to
+// 0.94 centred on the origin, 0.73 to 0.85 at an offset of three times the spread.)
+// Labels (16-ulp integer keys, lowest index on ties), minimum distances, -1 where nothing is
+// below FLT_MAX: as in the row-stationary kernel. xx is summed from the row in feature order with
+// separate multiply and add, the value row_norms stores, so the norm buffer is not read.
+//
+// FUSE: sums in LDS in double, [copy][centroid][4 NP + 1]: every lane adds the 2NP features it
+// holds, lane group 0 counts the row in the last slot (a double counts exactly); lane l adds into
+// copy l % ncopy, so that rows of one wavefront that share a centroid meet less often.
+// Bound by the vector instructions per row (splitting, keys), not by memory. 10.1M rows, a fused step,
+// against the row-stationary kernel: 3 features, k = 27 124 -> 85 us, k = 64 182 -> 111; 4, k = 100
+// 277 -> 165; 8, k = 100 287 -> 196.
+#include <algorithm>
+
+#include "bf16_parts.h"
+#include "kmeans_common.h"
+#include "mfma_traits.h"
+
+namespace kmhip {
+
+namespace {
+
+constexpr int SR_TPB = 1024;
+constexpr int SR_NW = SR_TPB / 64;
+constexpr int SR_MAX_D = 8;
+constexpr size_t SR_LDS_MAX = 150 * 1024;
+__host__ __device__ constexpr int sr_pairs(int d) { return d <= 4 ? 1 : 2; }
+__host__ __device__ constexpr int sr_steps(int d) { return d <= 4 ? 2 : 3; }  // k-steps of the products
+
+// row tiles a wavefront keeps in flight: as many as its 128 registers hold beside the work
+__host__ __device__ constexpr int sr_ahead(int d) { return d <= 3 ? 8 : d == 4 ? 6 : d == 5 ? 4 : 2; }
+
+size_t sr_model_lds(int d, int k) { return (size_t)((k + 31) / 32) * (sr_steps(d) * 64 * 16 + 32 * 4); }
+size_t sr_sums_lds(int d, int k) { return (size_t)k * (4 * sr_pairs(d) + 1) * sizeof(double); }
+
+template <int D, bool FUSE>
+__global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
+    const float *__restrict__ X, const float *__restrict__ C, int *__restrict__ labels,
+    float *__restrict__ mindist, int64_t n, int k, double *__restrict__ psums, int *__restrict__ pcounts,
+    int ncopy) {
+  constexpr int NP = sr_pairs(D), NM = sr_steps(D), NV = 2 * NP;
+  constexpr int SD = 2 * NV + 1;  // doubles per centroid of the sums, the count last
+  constexpr int MT = 32, NACC = 16, ROWT = 2;
+  static_assert(D >= 1 && D <= 2 * NV && NM * 4 >= 6 * NP, "the features' products fit the k-steps");
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int KT = (k + MT - 1) / MT;
+  uintx4 *cs = reinterpret_cast<uintx4 *>(smem_raw);                        // [KT][NM][64]
+  floatx4 *ccs = reinterpret_cast<floatx4 *>(cs + (size_t)KT * NM * 64);    // [KT][8] norms, four centroids each
+  double *sums = reinterpret_cast<double *>(ccs + (size_t)KT * 8);          // (FUSE) [ncopy][k][SD]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane % MT, g = lane / MT;
+  if (FUSE)
+    for (int e = tid; e < ncopy * k * SD; e += SR_TPB) sums[e] = 0.0;
+  // the centroid side, one (tile, lane) per thread and turn
+  for (int e = tid; e < KT * 64; e += SR_TPB) {
+    const int t = e >> 6, l = e & 63, c = t * MT + l % MT, gg = l / MT;
+    float v[NV];
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+      const int f = gg * NV + q;
+      v[q] = (c < k && f < D) ? -2.0f * C[(size_t)c * D + f] : 0.0f;
+    }
+    unsigned w[NM * 4];
+#pragma unroll
+    for (int q = 0; q < NM * 4; q++) w[q] = 0;
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+      const Bf16x3Pair s = split_pair_bf16x3(v[2 * p], v[2 * p + 1]);
+      w[6 * p] = w[6 * p + 1] = w[6 * p + 2] = s.h;
+      w[6 * p + 3] = w[6 * p + 4] = s.m;
+      w[6 * p + 5] = s.l;
+    }
+    // (a padding centroid is infinitely far)
+    if (gg == 0)
+      reinterpret_cast<float *>(ccs)[c] = c < k ? row_sqnorm<float>(C + (size_t)c * D, D) : pos_inf<float>();
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+      const uintx4 q = {w[4 * m], w[4 * m + 1], w[4 * m + 2], w[4 * m + 3]};
+      cs[(size_t)(t * NM + m) * 64 + l] = q;
+    }
+  }
+  __syncthreads();
+
+  double *const my_sums = sums + (size_t)(lane & (ncopy - 1)) * k * SD;
+  // PF row tiles are under way while two are worked on: with two in flight per wavefront the
+  // kernel waited for memory (three features: 1.6 TB/s).
+  constexpr int PF = sr_ahead(D);
+  float xn[PF][D];
+  // rows past the end re-read the last one; their results are never stored
+  auto fetch = [&](float (&x)[D], int64_t row0) {
+    const float *src = X + min(row0 + r, n - 1) * D;
+#pragma unroll
+    for (int j = 0; j < D; j++) x[j] = src[j];
+  };
+  // the centroid side of the instruction that adds xx
+  const uintx4 ones = {g == 0 ? 0x3F803F80u : 0u, g == 0 ? 0x3F80u : 0u, 0u, 0u};
+  auto work = [&](const float (&xr)[ROWT][D], int64_t row0) {
+    float val[ROWT][NV];  // what this lane group holds of the row
+    uintx4 b[ROWT][NM], bn[ROWT];
+#pragma unroll
+    for (int rt = 0; rt < ROWT; rt++) {
+      float x[4 * NP];
+#pragma unroll
+      for (int j = 0; j < 4 * NP; j++) x[j] = j < D ? xr[rt][j] : 0.0f;
+      float xx;
+      {
+#pragma clang fp contract(off)
+        xx = 0;
+#pragma unroll
+        for (int j = 0; j < D; j++) xx = xx + x[j] * x[j];
+      }
+#pragma unroll
+      for (int q = 0; q < NV; q++) val[rt][q] = g == 0 ? x[q] : x[NV + q];
+      unsigned w[NM * 4];
+#pragma unroll
+      for (int q = 0; q < NM * 4; q++) w[q] = 0;
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        const Bf16x3Pair s = split_pair_bf16x3(val[rt][2 * p], val[rt][2 * p + 1]);
+        w[6 * p] = w[6 * p + 3] = w[6 * p + 5] = s.h;
+        w[6 * p + 1] = w[6 * p + 4] = s.m;
+        w[6 * p + 2] = s.l;
+      }
+#pragma unroll
+      for (int m = 0; m < NM; m++) {
+        const uintx4 q = {w[4 * m], w[4 * m + 1], w[4 * m + 2], w[4 * m + 3]};
+        b[rt][m] = q;
+      }
+      const Bf16x3 xp = split_norm_bf16x3(xx);
+      const uintx4 q = {g == 0 ? xp.h | (xp.m << 16) : 0u, g == 0 ? xp.l : 0u, 0u, 0u};
+      bn[rt] = q;
+    }
+    unsigned bkey[ROWT];
+    int btile[ROWT];
+#pragma unroll
+    for (int rt = 0; rt < ROWT; rt++) {
+      bkey[rt] = 0x7F7FFFF0u;  // FLT_MAX with the index bits cleared
+      btile[rt] = -1;
+    }
+    for (int t = 0; t < KT; t++) {
+      uintx4 a[NM];
+#pragma unroll
+      for (int m = 0; m < NM; m++) a[m] = cs[(size_t)(t * NM + m) * 64 + lane];
+      floatx16 cc;  // accumulator v is centroid 8 (v / 4) + 4 g + v % 4 of the tile
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const floatx4 c4 = ccs[t * 8 + 2 * q + g];
+#pragma unroll
+        for (int e = 0; e < 4; e++) cc[4 * q + e] = c4[e];
+      }
+#pragma unroll
+      for (int rt = 0; rt < ROWT; rt++) {
+        floatx16 acc = mma_bf16(a[0], b[rt][0], cc);
+        if constexpr (NP == 1) {
+          acc = mma_bf16(ones, bn[rt], acc);
+          acc = mma_bf16(a[1], b[rt][1], acc);
+        } else {
+#pragma unroll
+          for (int m = 1; m < NM; m++) acc = mma_bf16(a[m], b[rt][m], acc);
+          acc = mma_bf16(ones, bn[rt], acc);
+        }
+        unsigned key[NACC];
+#pragma unroll
+        for (int v = 0; v < NACC; v++) key[v] = (__float_as_uint(acc[v]) & 0x7FFFFFF0u) | (unsigned)v;
+        unsigned m = umin3(key[0], key[1], key[2]);
+#pragma unroll
+        for (int v = 3; v + 1 < NACC; v += 2) m = umin3(m, key[v], key[v + 1]);
+        m = min(m, key[NACC - 1]);
+        if ((m | 15u) < bkey[rt]) {
+          bkey[rt] = m;
+          btile[rt] = t;
+        }
+      }
+    }
+#pragma unroll
+    for (int rt = 0; rt < ROWT; rt++) {
+      float best = __uint_as_float(bkey[rt] & 0xFFFFFFF0u);
+      int bidx = btile[rt] < 0 ? -1 : btile[rt] * MT + key_row(bkey[rt] & 15u, g);
+      argmin_merge(best, bidx, __shfl_xor(best, MT, 64), __shfl_xor(bidx, MT, 64));
+      const int64_t row = row0 + rt * MT + r;
+      if (g == 0 && row < n) {
+        labels[row] = bidx;
+        if (mindist) mindist[row] = best;
+      }
+      if (FUSE && row < n && bidx >= 0) {
+        double *srow = my_sums + (size_t)bidx * SD;
+#pragma unroll
+        for (int q = 0; q < NV; q++) {
+          // (a slot that no feature fills in either lane group is left out)
+          if (q < D) unsafeAtomicAdd(srow + g * NV + q, (double)val[rt][q]);
+        }
+        if (g == 0) unsafeAtomicAdd(srow + SD - 1, 1.0);
+      }
+    }
+  };
+  constexpr int ROWS = PF * MT;
+  const int64_t stride = (int64_t)gridDim.x * SR_NW * ROWS;
+  const int64_t first = ((int64_t)wave * gridDim.x + blockIdx.x) * ROWS;
+  if (first < n) {
+#pragma unroll
+    for (int rt = 0; rt < PF; rt++) fetch(xn[rt], first + rt * MT);
+  }
+  for (int64_t row0 = first; row0 < n; row0 += stride) {
+#pragma unroll
+    for (int p = 0; p < PF; p += ROWT) {
+      float x[ROWT][D];
+#pragma unroll
+      for (int rt = 0; rt < ROWT; rt++) {
+#pragma unroll
+        for (int j = 0; j < D; j++) x[rt][j] = xn[p + rt][j];
+        fetch(xn[p + rt], row0 + stride + (p + rt) * MT);
+      }
+      if (row0 + p * MT < n) work(x, row0 + p * MT);
+    }
+  }
+  if (!FUSE) return;
+  __syncthreads();
+  double *dst = psums + (size_t)blockIdx.x * k * D;
+  for (int e = tid; e < k * SD; e += SR_TPB) {
+    const int c = e / SD, f = e - c * SD;
+    double v = 0;
+    for (int cp = 0; cp < ncopy; cp++) v += sums[(size_t)cp * k * SD + e];  // copy order
+    if (f < D) dst[(size_t)c * D + f] = v;
+    else if (f == SD - 1) pcounts[(size_t)blockIdx.x * k + c] = (int)v;
+  }
+}
+
+}  // namespace
+
+// One or two features stay with the float32 instructions, whose two or three roundings per
+// distance are hard to beat. Up to four features every model of more
+// than 16 centroids is ahead (2M x 4, k = 17: 32.9 -> 29.8 us a fused step, k = 100: 66 -> 44); five to eight from
+// about 48 (2M x 8, k = 40: 42.5 -> 43.3, k = 65: 54 -> 47, k = 100: 66 -> 53).
+bool shortrow_applies(int d, int k, bool fused) {
+  return d >= 3 && d <= SR_MAX_D && k > (d <= 4 ? 16 : 48) &&
+         sr_model_lds(d, k) + (fused ? sr_sums_lds(d, k) : 0) <= SR_LDS_MAX;
+}
+
+int launch_shortrow(hipStream_t s, const float *X, const float *C, int *labels, float *mindist, int64_t n, int d,
+                    int k, int num_cu, bool fused, double *psums, int *pcounts, int *slots) {
+  if (!shortrow_applies(d, k, fused)) return H2O4GPU_KMEANS_EARG;
+  // copies of the sums: what fits beside the model in half a CU's LDS, eight at most (one is
+  // always there)
+  int ncopy = 1;
+  const size_t model = sr_model_lds(d, k), sums = sr_sums_lds(d, k);
+  while (fused && ncopy < 8 && model + 2 * ncopy * sums <= 72 * 1024) ncopy *= 2;
+  const size_t lds = model + (fused ? ncopy * sums : 0);
+  const int rows_per_wave = sr_ahead(d) * 32;
+  const int64_t tiles = (n + rows_per_wave - 1) / rows_per_wave;
+  int grid = 1;
+#define KM_SR_X(D, FUSE)                                                                                   \
+  do {                                                                                                     \
+    auto kern = assign_shortrow_kernel<D, FUSE>;                                                           \
+    KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                                 \
+    const int per_cu = std::min(2, resident_blocks_per_cu(reinterpret_cast<const void *>(kern), SR_TPB, lds)); \
+    grid = (int)std::min<int64_t>((int64_t)num_cu * per_cu, tiles);                                        \
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(SR_TPB), lds, s, X, C, labels, mindist, n, k, psums, pcounts, ncopy); \
+  } while (0)
+#define KM_SR(D)                    \
+  case D:                           \
+    if (fused) KM_SR_X(D, true);    \
+    else KM_SR_X(D, false);         \
+    break
+  switch (d) {
+    KM_SR(3);
+    KM_SR(4);
+    KM_SR(5);
+    KM_SR(6);
+    KM_SR(7);
+    KM_SR(8);
+  }
+#undef KM_SR
+#undef KM_SR_X
+  KM_HIP_TRY(hipGetLastError());
+  if (slots) *slots = grid;
+  return 0;
+}
+
+}  // namespace kmhip
