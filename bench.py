@@ -248,7 +248,7 @@ def extra_step(workload, scale, steps, warmup=2):
             h.init_plusplus(seed)   # the benchmark's start for this shape: k-means++, fixed seed
         else:
             h.set_centroids(datasets.seeded_row_init(X, k, seed))
-        variant = h.assign_variant()
+        variant = running_variant(h)
         h.iterate(warmup)
         h.timer_start()
         h.iterate(steps)
@@ -274,9 +274,19 @@ def extra_step(workload, scale, steps, warmup=2):
                     "unit": "GB/s", "frac": gbps / PEAK_HBM_GBPS})
     else:
         tf = 2.0 * n * k * d / (kern[dom] * 1e-3) / 1e12
-        out.update({"bound": "mfma", "algorithmic_flops": 2.0 * n * k * d, "achieved": tf,
-                    "peak": PEAK_MFMA_TFLOPS["f32"], "unit": "TFLOP/s", "frac": tf / PEAK_MFMA_TFLOPS["f32"]})
+        products = int(variant[-1]) if "_bf16x" in variant else 1
+        peak = PEAK_BF16_TFLOPS if products > 1 else PEAK_MFMA_TFLOPS["f32"]
+        out.update({"bound": "mfma", "algorithmic_flops": 2.0 * n * k * d, "algorithmic_tflops": tf,
+                    "products": products, "achieved": products * tf, "peak": peak, "unit": "TFLOP/s",
+                    "frac": products * tf / peak})
     return out
+
+
+def running_variant(h):
+    """The kernel a Lloyd step labels the rows with: its family and, where its float32 products are
+    formed on the bfloat16 matrix pipe, how many bfloat16 products make one."""
+    variant, products = h.assign_variant(), h.step_products()
+    return variant if "_bf16x" in variant or not products else "%s_bf16x%d" % (variant, products)
 
 
 def main():
@@ -377,7 +387,7 @@ def main():
         h.set_option("exact_argmin", 1)
     if args.fp32_split is not None:
         h.set_option("fp32_split", args.fp32_split)
-    variant = h.assign_variant()
+    variant = running_variant(h)
     log("upload %.3f s (%.1f GB/s incl. pageable staging; first call of the process %.3f s); "
         "assign variant %s" % (h2d_s, n * d * s / h2d_s / 1e9, h2d_first_s, variant))
 
@@ -405,11 +415,11 @@ def main():
     assign_ms = kern[dom]["avg_ms"]
     tflops = flops_per_iter / (assign_ms * 1e-3) / 1e12
     peak = PEAK_MFMA_TFLOPS[args.dtype]
+    products = int(variant[-1]) if "_bf16x" in variant else 1
     mfma_bound = variant not in ("valu", "wave_row")   # (the kernels without matrix instructions stream X)
     if mfma_bound and "_bf16x" in variant:
-        # the option that forms each float32 product from bfloat16 parts: the kernel executes
-        # 6 or 9 times the algorithmic flop, on the bfloat16 matrix pipe, and is priced there
-        products = int(variant[-1])
+        # each float32 product formed from bfloat16 parts: the kernel executes that many times the
+        # algorithmic flop, on the bfloat16 matrix pipe, and is priced there
         roofline = {"bound": "mfma", "kernel": "%s (%s)" % (dom, variant), "achieved": products * tflops,
                     "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": products * tflops / PEAK_BF16_TFLOPS,
                     "traffic": traffic, "algorithmic_tflops": tflops,
@@ -449,27 +459,22 @@ def main():
         transform = {"rows": int(H.shape[0]), "kernel_ms": ms, "launches": cnt, "tflops": tf,
                      "mfma_frac": tf / peak, "end_to_end_seconds": wall,
                      "output_bytes": float(H.shape[0]) * k * s}
-    # the same steps with the float32 dot products on the bfloat16 matrix pipe (an option of
-    # the matrix-core kernels, off by default; never part of `value`)
-    split_leg = None
-    if args.dtype == "f32" and variant in ("mfma_rowstat", "mfma_tiled"):  # (i.e. the main run was without it)
-        h.set_option("fp32_split", 6)
-        if h.assign_variant() == variant + "_bf16x6":
-            h.set_centroids(C0)
-            h.iterate(args.warmup)
-            h.timer_start()
-            h.iterate(args.steps)
-            ms6 = h.timer_stop() / args.steps
-            h.profile(True)
-            h.iterate(args.steps)
-            cnt6, kms6 = h.kernel_time(dom)
-            h.profile(False)
-            h.assign()
-            split_leg = {"option": "fp32_split=6", "assign_variant": variant + "_bf16x6",
-                         "ms_per_step": ms6, "iterations_per_s": 1000.0 / ms6,
-                         "kernel_avg_ms": kms6 / max(cnt6, 1), "inertia": h.inertia(),
-                         "note": "products of bfloat16 parts, float32 accumulation; same parity bars"}
+    # the same steps on the float32 matrix instructions, where the run above did not use them
+    f32_leg = None
+    if args.dtype == "f32" and "_bf16x" in variant and args.fp32_split is None:
         h.set_option("fp32_split", 0)
+        h.set_centroids(C0)
+        h.iterate(args.warmup)
+        h.timer_start()
+        h.iterate(args.steps)
+        ms0 = h.timer_stop() / args.steps
+        h.profile(True)
+        h.iterate(args.steps)
+        cnt0, kms0 = h.kernel_time(dom)
+        h.profile(False)
+        h.assign()
+        f32_leg = {"option": "fp32_split=0", "assign_variant": h.assign_variant(), "ms_per_step": ms0,
+                   "iterations_per_s": 1000.0 / ms0, "kernel_avg_ms": kms0 / max(cnt0, 1), "inertia": h.inertia()}
     h.close()
 
     out = {
@@ -488,7 +493,8 @@ def main():
         "iteration": {"algorithmic_bytes": bytes_per_iter, "algorithmic_flops": flops_per_iter,
                       "gbps": iter_gbps, "hbm_frac": iter_gbps / PEAK_HBM_GBPS,
                       "tflops": flops_per_iter / (ms_step * 1e-3) / 1e12,
-                      "mfma_frac": flops_per_iter / (ms_step * 1e-3) / 1e12 / peak},
+                      "mfma_frac": products * flops_per_iter / (ms_step * 1e-3) / 1e12
+                                   / (PEAK_BF16_TFLOPS if products > 1 else peak)},
         "kernels_avg_ms": {kname: round(v["avg_ms"], 5) for kname, v in kern.items()},
         "copy_probe_gbps": 2.0 * copy_bytes / (copy_ms * 1e-3) / 1e9,
         "hbm_probes": probes,
@@ -498,8 +504,8 @@ def main():
     }
     if transform:
         out["transform"] = transform
-    if split_leg:
-        out["fp32_split"] = split_leg
+    if f32_leg:
+        out["fp32_instructions"] = f32_leg
     if args.extras and args.workload == "C3" and args.scale == 1.0 and args.dtype == "f32" and not args.shape:
         # the north star's two regimes under the same clock as the headline shape; extras, never
         # the reason a bench line is missing
