@@ -457,7 +457,7 @@ def main():
         h.profile(False)
         tf = 2.0 * H.shape[0] * k * d / (ms * 1e-3) / 1e12
         transform = {"rows": int(H.shape[0]), "kernel_ms": ms, "launches": cnt, "tflops": tf,
-                     "mfma_frac": tf / peak, "end_to_end_seconds": wall,
+                     "mfma_frac": 6 * tf / PEAK_BF16_TFLOPS if products > 1 else tf / peak, "end_to_end_seconds": wall,
                      "output_bytes": float(H.shape[0]) * k * s}
     # the same steps on the float32 matrix instructions, where the run above did not use them
     f32_leg = None

@@ -1101,6 +1101,21 @@ struct TiledCfg {
   static constexpr size_t LDS_BYTES = OPERAND_BYTES + (size_t)2 * BC * sizeof(T);
 };
 
+// The distance the float32 matrix instructions of the tiled kernels give (xxh = -xx / 2): one chain of
+// fused multiply-adds, of every eight features 0 4 1 5 2 6 3 7.
+__device__ __forceinline__ float float32_distance(const float *x, const float *c, int d, float xxh, float cc) {
+  float acc = 0;
+#pragma unroll 1
+  for (int f = 0; f < d; f += 8) {
+#pragma unroll 1
+    for (int e = 0; e < 8; e++) {
+      const int j = f + (e & 1) * 4 + (e >> 1);
+      if (j < d) acc = fmaf(c[j], x[j], acc);
+    }
+  }
+  return 2.0f * fabsf(acc + fmaf(-0.5f, cc, xxh));
+}
+
 template <typename T, int MODE, bool VECLOAD, bool DTAIL, int BCW, bool EXACT = false, bool WIDE = false,
           int SPLIT = 0, bool XB = false>
 __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) void assign_tiled_kernel(
@@ -1463,7 +1478,15 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
           for (int rt = 0; rt < RT; rt++) {
             const int64_t row = row0 + (wr * RT + rt) * MT + r;
             const T a = acc[ct][rt][v] + fma((T)-0.5, cc, xx[rt]);
-            if (c < k && row < n) D[(size_t)c * ldn + row] = (T)2 * fabs(a);
+            if (c < k && row < n) {
+              T dist = (T)2 * fabs(a);
+              // (SPLIT) the parts of an infinity are not finite either, and a float just below it rounds up
+              // to one: such distances come from the float32 chain, infinite or NaN as it has them
+              if constexpr (SPLIT != 0) {
+                if (!(dist <= argmin_start<T>())) dist = float32_distance((const float *)X + row * d, (const float *)C + (size_t)c * d, d, (float)xx[rt], (float)cc);
+              }
+              D[(size_t)c * ldn + row] = dist;
+            }
           }
         }
       }

@@ -71,3 +71,21 @@ def test_rows_no_distance_exists_for(hip):
     C[11, 5] = np.nan
     got, want = labels_of(hip, X, C)[0], labels_of(hip, X, C, split=0)[0]
     assert np.array_equal(got, want) and (got[[3, 77, 2999]] == -1).all()
+
+
+@pytest.mark.parametrize("d,k", [(20, 70), (150, 90), (130, 300)])
+def test_transform_of_rows_that_are_not_finite(hip, d, k):
+    """Infinite and NaN distances come out as the float32 instructions have them."""
+    rng = np.random.default_rng(d)
+    X, C = rng.standard_normal((300, d)).astype(np.float32), rng.standard_normal((k, d)).astype(np.float32)
+    X[[3, 77, 150, 299], [0, 7, 2, 5]] = np.nan, np.inf, -np.inf, 3.4e38
+    C[[11, 60], [5, 1]] = np.inf, -3.4e38
+    with hip.Handle(300, d, k, np.float32) as h:
+        h.set_data(X)
+        h.set_centroids(C)
+        got = h.transform(X)
+        h.set_option("fp32_split", 0)
+        want = h.transform(X)
+    finite = np.isfinite(want)
+    assert np.array_equal(got[~finite], want[~finite], equal_nan=True) and np.isfinite(got[finite]).all()
+    assert (~finite).sum() > 4 * k
