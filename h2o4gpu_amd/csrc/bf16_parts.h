@@ -37,6 +37,49 @@ __device__ __forceinline__ unsigned umin3(unsigned a, unsigned b, unsigned c) {
   asm("v_min3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
+// The middle one of three, likewise.
+__device__ __forceinline__ unsigned umed3(unsigned a, unsigned b, unsigned c) {
+  unsigned r;
+  asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+// The smallest of the 16 keys of a tile; `second` becomes the second smallest of them, the running
+// minimum `best` and the running second minimum. Triples give their two smallest with two
+// instructions, so the second minimum costs 12 instructions on top of the 8 of the minimum alone.
+__device__ __forceinline__ unsigned two_smallest_keys(const unsigned (&key)[16], unsigned best, unsigned &second) {
+  unsigned lo[5], mid[5];
+#pragma unroll
+  for (int i = 0; i < 5; i++) {
+    lo[i] = umin3(key[3 * i], key[3 * i + 1], key[3 * i + 2]);
+    mid[i] = umed3(key[3 * i], key[3 * i + 1], key[3 * i + 2]);
+  }
+  const unsigned a = umin3(lo[0], lo[1], lo[2]), b = umin3(lo[3], lo[4], key[15]);
+  const unsigned am = umed3(lo[0], lo[1], lo[2]), bm = umed3(lo[3], lo[4], key[15]);
+  second = umin3(umin3(mid[0], mid[1], mid[2]), umin3(mid[3], mid[4], am), umin3(bm, umed3(a, b, best), second));
+  return min(a, b);
+}
+// Whether two distances of a row, compared at 16 ulp, lie so close that the bfloat16 products and the
+// float32 instructions may order them differently. settle_margin() bounds the rounding of both forms
+// relative to xx + cc, and a centroid at a distance `second` has a norm of at most 2 xx + 2 second; two
+// buckets of 16 ulp come on top. (A row whose norm is infinite counts as tied, a NaN never does.)
+struct TieBound {
+  float of_norm, of_second;  // tied when of_second * second - best <= of_norm * xx; of_norm -infinity: never
+};
+__device__ __forceinline__ bool near_tie(float best, float second, float xx, TieBound b) {
+  return fmaf(b.of_second, second, -best) <= b.of_norm * xx;
+}
+// Each form's d roundings are 0.3 ulp of a partial sum of at most xx + cc, so the difference of two
+// distances in two forms has an rms of about 0.3 sqrt(d) eps (xx + cc) (measured without the norms' own
+// error, which both share: 0.4 to 1.3 eps a distance at 3 to 64 features). Five times that and more: the
+// bound on cc makes xx + cc half again as large as it is, and a constant is there for the roundings that
+// do not depend on d.
+static inline TieBound settle_margin(int d, bool settle) {
+  const float m = (3.0f + sqrtf((float)d)) * 1.1920929e-7f;
+  return settle ? TieBound{3.0f * m, 1.0f - 2.0f * m - 3.9e-6f} : TieBound{-__builtin_huge_valf(), 1.0f};
+}
+// the floats whose upper halves are the low and the high half of a packed pair
+__device__ __forceinline__ float bf16_low(unsigned p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float bf16_high(unsigned p) { return __uint_as_float(p & 0xFFFF0000u); }
 // centroid row of accumulator v (runtime v) of the 32x32 float tile
 __device__ __forceinline__ int key_row(unsigned v, int g) {
   return (int)((v >> 2) * 8 + (unsigned)g * 4 + (v & 3));

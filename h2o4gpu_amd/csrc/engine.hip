@@ -665,6 +665,9 @@ struct Engine : h2o4gpu_kmeans_handle {
     if (opt_assign != ASSIGN_AUTO || opt_exact || stacked) return 0;
     return default_split<T>(use, n, d, model_rows);
   }
+  // Whether labels found with bfloat16 products are the float32 instructions' (near ties settled):
+  // always where nobody asked for a number of products.
+  bool settles() const { return opt_split == SPLIT_DEFAULT; }
   int step_products() const override {
     const bool fused = (opt_fuse || sets > 1) && !opt_exact && fused_slots<T>(opt_assign, n, d, k, num_cu) > 0;
     const int split = split_for(fused ? SPLIT_FUSED : SPLIT_ASSIGN, k, sets > 1);
@@ -681,9 +684,9 @@ struct Engine : h2o4gpu_kmeans_handle {
     SplitScratch sc;
     sc.through_registers = opt_tiled_direct == 0;
     sc.rows_bf16 = resident && rows_bf16;
+    sc.near_ties = ties > 0 && settles();
     size_t need = split ? tiled_split_scratch_bytes<T>(split, d, model_rows) : 0;
     if (need == 0) return sc;
-    sc.near_ties = ties > 0 && opt_split == SPLIT_DEFAULT && d >= 128;
     if (sc.near_ties) need = (need + 255) / 256 * 256 + near_ties_bytes(ties);
     if (need > split_bytes) {
       (void)hipStreamSynchronize(stream);
@@ -1417,7 +1420,7 @@ struct Engine : h2o4gpu_kmeans_handle {
                launch_assign_accumulate<T>(stream, opt_assign, X, xnorm, C[cur], (const T *)nullptr,
                                            labels, (want_mindist || sets > 1) ? mindist : (T *)nullptr, n, d,
                                            k, num_cu, psums, pcounts, &slots, &last_variant, shape(),
-                                           split_for(SPLIT_FUSED, k, sets > 1)));
+                                           split_for(SPLIT_FUSED, k, sets > 1), settles()));
       have_mindist = want_mindist || sets > 1;
       return finish_update(slots, want_shift, shift_host);
     }

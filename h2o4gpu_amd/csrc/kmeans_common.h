@@ -93,6 +93,7 @@ struct NearTies {
   unsigned long long *keys = nullptr;
   int cap = 0;
   float margin = 0;  // relative to xx + cc
+  unsigned mask = ~0u;  // bits of a distance that are compared (keys: 16 ulp)
 };
 size_t near_ties_bytes(int64_t n);
 
@@ -102,8 +103,8 @@ size_t near_ties_bytes(int64_t n);
 struct SplitScratch {
   void *ptr = nullptr;
   size_t bytes = 0;
-  // assignments that compare the distances themselves (128 features and more): settle near ties as the
-  // float32 instructions do; the scratch then holds near_ties_bytes(n) behind the parts (256-aligned)
+  // assignments: settle near ties as the float32 instructions do (tiled kernel: the scratch then holds
+  // near_ties_bytes(n) behind the parts, 256-aligned)
   bool near_ties = false;
   // every value of X is a bfloat16 (row_norms' check): the products with its other parts are zeros
   bool rows_bf16 = false;
@@ -150,7 +151,7 @@ int launch_longrow(hipStream_t s, const T *X, const T *xnorm, const T *C, const 
 // reads the k centroids only; fused: partial sums and counts per workgroup, at most 2 * num_cu slots.
 bool shortrow_applies(int d, int k, bool fused);
 int launch_shortrow(hipStream_t s, const float *X, const float *C, int *labels, float *mindist, int64_t n, int d,
-                    int k, int num_cu, bool fused, double *psums, int *pcounts, int *slots);
+                    int k, int num_cu, bool fused, double *psums, int *pcounts, int *slots, bool settle);
 const char *assign_variant_name(int variant);
 // split (float32 matrix-core kernels; 0, 6 or 9): run the dot products on the bfloat16
 // matrix pipe as that many products of bfloat16 parts per feature pair (9: every product
@@ -181,7 +182,7 @@ template <typename T>
 int launch_assign_accumulate(hipStream_t s, int variant, const T *X, const T *xnorm, const T *C,
                              const T *cnorm, int *labels, T *mindist, int64_t n, int d,
                              int k, int num_cu, double *psums, int *pcounts, int *slots,
-                             int *used, StackShape st = StackShape(), int split = 0);
+                             int *used, StackShape st = StackShape(), int split = 0, bool settle = false);
 
 // Full squared-distance matrix, centroid-major: D[c * ldn + i], i < n.
 template <typename T>

@@ -17,16 +17,17 @@
 // features the smallest products come after that, at the size of the distance itself. (Distances
 // against float64 at three to eight features, rms, over the float32 instructions': 0.89 to
 // 0.94 centred on the origin, 0.73 to 0.85 at an offset of three times the spread.)
-// Labels (16-ulp integer keys, lowest index on ties), minimum distances, -1 where nothing is
-// below FLT_MAX: as in the row-stationary kernel. xx is summed from the row in feature order with
+// Labels (16-ulp integer keys, lowest index on ties; near ties settled by the float32 instructions),
+// minimum distances, -1 where nothing is below FLT_MAX: as in the row-stationary kernel. xx is summed from the row in feature order with
 // separate multiply and add, the value row_norms stores, so the norm buffer is not read.
 //
 // FUSE: sums in LDS in double, [copy][centroid][4 NP + 1]: every lane adds the 2NP features it
 // holds, lane group 0 counts the row in the last slot (a double counts exactly); lane l adds into
 // copy l % ncopy, so that rows of one wavefront that share a centroid meet less often.
 // Bound by the vector instructions per row (splitting, keys), not by memory. 10.1M rows, a fused step,
-// against the row-stationary kernel: 3 features, k = 27 124 -> 85 us, k = 64 182 -> 111; 4, k = 100
-// 277 -> 165; 8, k = 100 287 -> 196.
+// against the row-stationary kernel on the float32 instructions: 3 features, k = 27 124 -> 98 us; 10M
+// rows: 4, k = 100 285 -> 200; 5, k = 60 188 -> 151; 8, k = 100 293 -> 235 (85, 160, 136 and 206 without
+// the second minimum that near ties are found by).
 #include <algorithm>
 
 #include "bf16_parts.h"
@@ -54,7 +55,7 @@ template <int D, bool FUSE>
 __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
     const float *__restrict__ X, const float *__restrict__ C, int *__restrict__ labels,
     float *__restrict__ mindist, int64_t n, int k, double *__restrict__ psums, int *__restrict__ pcounts,
-    int ncopy) {
+    int ncopy, TieBound bound) {
   constexpr int NP = sr_pairs(D), NM = sr_steps(D), NV = 2 * NP;
   constexpr int SD = 2 * NV + 1;  // doubles per centroid of the sums, the count last
   constexpr int MT = 32, NACC = 16, ROWT = 2;
@@ -113,6 +114,7 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
   const uintx4 ones = {g == 0 ? 0x3F803F80u : 0u, g == 0 ? 0x3F80u : 0u, 0u, 0u};
   auto work = [&](const float (&xr)[ROWT][D], int64_t row0) {
     float val[ROWT][NV];  // what this lane group holds of the row
+    float nrm[ROWT];
     uintx4 b[ROWT][NM], bn[ROWT];
 #pragma unroll
     for (int rt = 0; rt < ROWT; rt++) {
@@ -126,6 +128,7 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
 #pragma unroll
         for (int j = 0; j < D; j++) xx = xx + x[j] * x[j];
       }
+      nrm[rt] = xx;
 #pragma unroll
       for (int q = 0; q < NV; q++) val[rt][q] = g == 0 ? x[q] : x[NV + q];
       unsigned w[NM * 4];
@@ -147,11 +150,11 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
       const uintx4 q = {g == 0 ? xp.h | (xp.m << 16) : 0u, g == 0 ? xp.l : 0u, 0u, 0u};
       bn[rt] = q;
     }
-    unsigned bkey[ROWT];
+    unsigned bkey[ROWT], skey[ROWT];
     int btile[ROWT];
 #pragma unroll
     for (int rt = 0; rt < ROWT; rt++) {
-      bkey[rt] = 0x7F7FFFF0u;  // FLT_MAX with the index bits cleared
+      bkey[rt] = skey[rt] = 0x7F7FFFF0u;  // FLT_MAX with the index bits cleared
       btile[rt] = -1;
     }
     for (int t = 0; t < KT; t++) {
@@ -179,10 +182,7 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
         unsigned key[NACC];
 #pragma unroll
         for (int v = 0; v < NACC; v++) key[v] = (__float_as_uint(acc[v]) & 0x7FFFFFF0u) | (unsigned)v;
-        unsigned m = umin3(key[0], key[1], key[2]);
-#pragma unroll
-        for (int v = 3; v + 1 < NACC; v += 2) m = umin3(m, key[v], key[v + 1]);
-        m = min(m, key[NACC - 1]);
+        const unsigned m = two_smallest_keys(key, bkey[rt], skey[rt]);
         if ((m | 15u) < bkey[rt]) {
           bkey[rt] = m;
           btile[rt] = t;
@@ -193,7 +193,58 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
     for (int rt = 0; rt < ROWT; rt++) {
       float best = __uint_as_float(bkey[rt] & 0xFFFFFFF0u);
       int bidx = btile[rt] < 0 ? -1 : btile[rt] * MT + key_row(bkey[rt] & 15u, g);
-      argmin_merge(best, bidx, __shfl_xor(best, MT, 64), __shfl_xor(bidx, MT, 64));
+      const float ob = __shfl_xor(best, MT, 64);
+      const float second = fminf(fmaxf(best, ob), __uint_as_float(skey[rt] & 0xFFFFFFF0u));
+      argmin_merge(best, bidx, ob, __shfl_xor(bidx, MT, 64));
+      // Near ties, settled as the float32 instructions settle them (assign_rowstat_kernel): a tile with
+      // such a row is swept again by them, with the operands the row-stationary kernel gives them
+      // (lane group 0 the features 0 to 3, group 1 the rest).
+      const unsigned long long ties = __ballot(near_tie(best, second, nrm[rt], bound));
+      if (__builtin_expect(ties != 0, 0)) {
+        const bool tie = (((ties | ties >> 32) >> r) & 1) != 0;
+        unsigned fkey = 0x7F7FFFF0u;
+        int ftile = -1;
+#pragma unroll 1
+        for (int t = 0; t < KT; t++) {
+          floatx16 acc;
+#pragma unroll
+          for (int v = 0; v < NACC; v++)
+            acc[v] = nrm[rt] + reinterpret_cast<const float *>(ccs)[t * MT + Mfma<float>::acc_row(v, g)];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            // feature 4 g + e of this lane's centroid, from its parts' words 6 p, 6 p + 3 and 6 p + 5
+            auto part = [&](int w) {
+              const uintx4 *slot = cs + (size_t)(t * NM + w / 4) * 64 + (NP == 2 ? lane : r + e / 2 * MT);
+              const unsigned u = reinterpret_cast<const unsigned *>(slot)[w % 4];
+              return e % 2 ? bf16_high(u) : bf16_low(u);
+            };
+            constexpr int P = 6;
+            const int p = NP == 2 ? e / 2 : 0;
+            float a = (part(P * p) + part(P * p + 3)) + part(P * p + 5);
+            float b = NP == 2 ? val[rt][e % NV] : (e < D ? xr[rt][e < D ? e : 0] : 0.0f);
+            if (NP == 1 && g == 1) a = b = 0.0f;
+            acc = Mfma<float>::mma(a, b, acc);
+          }
+          unsigned key[NACC];
+#pragma unroll
+          for (int v = 0; v < NACC; v++) key[v] = (__float_as_uint(acc[v]) & 0x7FFFFFF0u) | (unsigned)v;
+          unsigned m = umin3(key[0], key[1], key[2]);
+#pragma unroll
+          for (int v = 3; v + 1 < NACC; v += 2) m = umin3(m, key[v], key[v + 1]);
+          m = min(m, key[NACC - 1]);
+          if ((m | 15u) < fkey) {
+            fkey = m;
+            ftile = t;
+          }
+        }
+        float fbest = __uint_as_float(fkey & 0xFFFFFFF0u);
+        int fidx = ftile < 0 ? -1 : ftile * MT + key_row(fkey & 15u, g);
+        argmin_merge(fbest, fidx, __shfl_xor(fbest, MT, 64), __shfl_xor(fidx, MT, 64));
+        if (tie) {
+          best = fbest;
+          bidx = fidx;
+        }
+      }
       const int64_t row = row0 + rt * MT + r;
       if (g == 0 && row < n) {
         labels[row] = bidx;
@@ -254,7 +305,8 @@ bool shortrow_applies(int d, int k, bool fused) {
 }
 
 int launch_shortrow(hipStream_t s, const float *X, const float *C, int *labels, float *mindist, int64_t n, int d,
-                    int k, int num_cu, bool fused, double *psums, int *pcounts, int *slots) {
+                    int k, int num_cu, bool fused, double *psums, int *pcounts, int *slots, bool settle) {
+  const TieBound bound = settle_margin(d, settle);
   if (!shortrow_applies(d, k, fused)) return H2O4GPU_KMEANS_EARG;
   // copies of the sums: what fits beside the model in half a CU's LDS, eight at most (one is
   // always there)
@@ -271,7 +323,8 @@ int launch_shortrow(hipStream_t s, const float *X, const float *C, int *labels, 
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                                 \
     const int per_cu = std::min(2, resident_blocks_per_cu(reinterpret_cast<const void *>(kern), SR_TPB, lds)); \
     grid = (int)std::min<int64_t>((int64_t)num_cu * per_cu, tiles);                                        \
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(SR_TPB), lds, s, X, C, labels, mindist, n, k, psums, pcounts, ncopy); \
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(SR_TPB), lds, s, X, C, labels, mindist, n, k, psums, pcounts, ncopy, \
+                       bound);                                                                             \
   } while (0)
 #define KM_SR(D)                    \
   case D:                           \
