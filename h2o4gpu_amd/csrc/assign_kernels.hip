@@ -1156,8 +1156,8 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
 // turn: vector 0 and 2 to lane group 0, 1 and 3 to lane group 1). Rows past k and features
 // past d are zero, so the tiled kernel needs no bounds on this operand.
 __global__ void split_centroids_kernel(const float *__restrict__ C, uintx4 *__restrict__ out, int k,
-                                       int d, int bc, int nstage, int nblocks, int *fix_count) {
-  if (fix_count && blockIdx.x == 0 && threadIdx.x == 0) *fix_count = 0;  // (NearTies of the launch behind)
+                                       int d, int bc, int nstage, int nblocks, unsigned *ties) {
+  if (ties && blockIdx.x == 0 && threadIdx.x == 0) *ties = 0;  // (NearTies of the launch behind)
   const int tiles = bc / 32;
   const int64_t total = (int64_t)nblocks * nstage * tiles * 64;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
@@ -1242,6 +1242,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
     const T *__restrict__ C, const T *__restrict__ cnorm,
     int *__restrict__ labels, T *__restrict__ mindist, T *__restrict__ D,
     int64_t n, int64_t ldn, int d, int k, const uintx4 *__restrict__ Cparts, NearTies ties) {
+  if (SPLIT == 0 && ties.count && *ties.count <= ties.cap) return;
   typedef Mfma<T> M;
   typedef TiledCfg<T, BCW, WIDE, SPLIT, XB> Cfg;
   static_assert(!XB || SPLIT == 6, "bfloat16 rows: a form of the split kernel");
@@ -1740,7 +1741,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
             // this close has a norm of at most 2 xx + 2 distances; keys: and two buckets of 16 ulp)
             if (ties.count && second[rt] - best[rt] <= ties.margin * (4 * best[rt] - 3 * xx[rt]) +
                                                            (EXACT ? (T)0 : (T)3.9e-6f * second[rt])) {
-              const int at = atomicAdd(ties.count, 1);
+              const unsigned at = atomicAdd(ties.count, 1u);
               if (at < ties.cap) {
                 ties.rows[at] = (int)row;
                 ties.keys[at] = ~0ull;
@@ -1808,7 +1809,8 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
     const T *__restrict__ X, const T *__restrict__ xnorm,
     const T *__restrict__ C, const T *__restrict__ cnorm,
     int *__restrict__ labels, T *__restrict__ mindist, T *__restrict__ D,
-    int64_t n, int64_t ldn, int d, int k) {
+    int64_t n, int64_t ldn, int d, int k, NearTies gate) {
+  if (gate.count && *gate.count <= gate.cap) return;
   typedef Mfma<T> M;
   typedef DmaCfg<T, BCW, WIDE, BK, NBUF> Cfg;
   constexpr int MT = M::MT, KL = M::KL, NACC = M::NACC, VW = M::VW;
@@ -2131,8 +2133,9 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
 // float32 matrix instructions' own chain of fused multiply-adds: v_mfma_f32_32x32x2_f32 adds its two
 // products one after the other, each rounded, so with the tiled kernels' order of features (of every
 // eight 0 4 1 5 2 6 3 7) and their closing expression a scalar chain gives the same bits, and the row
-// the same label. Lists longer than `cap` (data full of equal centroids) are left as they are: either
-// label is right to rounding.
+// the same label. A list that does not hold them all (data far from the origin, or full of equal
+// centroids) is left alone: the pass is then run again, whole, by the float32 instructions, whose launch
+// behind these two looks at the count and ends at once otherwise.
 // A workgroup takes 16 listed rows and 256 centroids at a time, a centroid per thread, the rows' values
 // broadcast from LDS, the winners combined by one 64-bit minimum per row and wavefront (distance bits
 // above the centroid's index: the lowest index wins a tie). 261k x 298, k = 1000: 38 us beside
@@ -2143,8 +2146,8 @@ __global__ __launch_bounds__(WG) void near_ties_kernel(const float *__restrict__
                                                       const float *__restrict__ C, const float *__restrict__ cnorm,
                                                       int d, int k, NearTies ties) {
   __shared__ floatx4 xs[TIE_ROWS][TIE_PIECE / 4];
-  const int m = *ties.count;
-  if (m > ties.cap) return;
+  if (*ties.count > ties.cap) return;
+  const int m = (int)*ties.count;
   const int groups = (m + TIE_ROWS - 1) / TIE_ROWS, blocks = (k + WG - 1) / WG;
   const int tid = threadIdx.x;
   for (int unit = blockIdx.x; unit < groups * blocks; unit += gridDim.x) {
@@ -2213,8 +2216,8 @@ __global__ __launch_bounds__(WG) void near_ties_kernel(const float *__restrict__
 }
 __global__ __launch_bounds__(WG) void near_ties_labels_kernel(int *__restrict__ labels, float *__restrict__ mindist,
                                                              NearTies ties) {
-  const int m = *ties.count;
-  if (m > ties.cap) return;
+  if (*ties.count > ties.cap) return;
+  const int m = (int)*ties.count;
   for (int at = blockIdx.x * WG + threadIdx.x; at < m; at += gridDim.x * WG) {
     const unsigned long long key = ties.keys[at];
     const unsigned start = __float_as_uint(0.5f * argmin_start<float>()) & ties.mask;
@@ -2659,7 +2662,7 @@ int launch_assign_accumulate(hipStream_t s, int variant, const T *X, const T *xn
 template <typename T, int MODE, int BCW, bool WIDE, int BK, int NBUF, bool SPREAD>
 static int launch_tiled_dma(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm,
                             int *labels, T *mindist, T *D, int64_t n, int64_t ldn, int d, int k,
-                            bool exact) {
+                            bool exact, const NearTies &gate) {
   typedef DmaCfg<T, BCW, WIDE, BK, NBUF> Cfg;
   const uintptr_t bits = reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(C) |
                          reinterpret_cast<uintptr_t>(cnorm);
@@ -2673,7 +2676,7 @@ static int launch_tiled_dma(hipStream_t s, const T *X, const T *xnorm, const T *
     auto kern = assign_tiled_dma_kernel<T, MODE, BCW, EXACT, WIDE, BK, NBUF, SPREAD>;        \
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                   \
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(Cfg::TPB), lds, s, X, xnorm, C,     \
-                       cnorm, labels, mindist, D, n, ldn, d, k);                             \
+                       cnorm, labels, mindist, D, n, ldn, d, k, gate);                       \
   } while (0)
   if (d >= 128) exact = true;  // as in launch_tiled_bcw
   if constexpr (MODE == 0 && sizeof(T) == 4) {
@@ -2714,13 +2717,13 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
     int rc = 1;
     if constexpr (sizeof(T) == 8)
       rc = launch_tiled_dma<T, MODE, BCW, WIDE, 16, 2, false>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn,
-                                                              d, k, exact);
+                                                              d, k, exact, ties);
     else if constexpr (!WIDE)
       rc = launch_tiled_dma<T, MODE, BCW, WIDE, 32, 2, false>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn,
-                                                              d, k, exact);
+                                                              d, k, exact, ties);
     else
       rc = launch_tiled_dma<T, MODE, BCW, WIDE, 16, 2, MODE == 0>(s, X, xnorm, C, cnorm, labels, mindist, D, n,
-                                                                  ldn, d, k, exact);
+                                                                  ldn, d, k, exact, ties);
     if (rc != 1) return rc;
   }
   const int64_t row_tiles = (n + Cfg::BR - 1) / Cfg::BR;
@@ -2758,9 +2761,8 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
 #undef KM_TILED_X
   if constexpr (SPLIT != 0 && MODE == 0) {
     if (ties.count) {
-      ties.mask = exact ? ~0u : 0x7FFFFFF0u;
       hipLaunchKernelGGL(near_ties_kernel, dim3(512), dim3(WG), 0, s, X, xnorm, C, cnorm, d, k, ties);
-      hipLaunchKernelGGL(near_ties_labels_kernel, dim3((unsigned)std::min(64, (ties.cap + WG - 1) / WG)), dim3(WG), 0, s,
+      hipLaunchKernelGGL(near_ties_labels_kernel, dim3(std::min(64u, (ties.cap + WG - 1) / WG)), dim3(WG), 0, s,
                          labels, mindist, ties);
     }
   }
@@ -2778,74 +2780,52 @@ static int tiled_split(int split, int d, int k) {
   return split;
 }
 
-// Bytes of device scratch the tiled kernel needs for the centroids' parts (0: the option
-// does not apply to the shape).
 // (with the parts the 256-centroid block is ahead whenever it has the centroids to fill it:
 // 2M x 256, k = 1024 5.87 -> 5.37 ms, 500k x 784, k = 4096 14.96 -> 13.52 ms)
 static bool tiled_split_wide(int k) { return k > 128; }
-template <typename T>
-size_t tiled_split_scratch_bytes(int split, int d, int k) {
-  if (tiled_split<T>(split, d, k) == 0) return 0;
+// Rows listed at most, and the scratch: a block of 256 bytes with the count, the parts, the list.
+static int64_t near_ties_cap(int64_t n) { return std::min<int64_t>(n / 16 + 64, 1 << 26); }
+static size_t round256(size_t bytes) { return (bytes + 255) / 256 * 256; }
+static size_t split_parts_bytes(int d, int k) {
   const int bc = tiled_split_wide(k) ? 256 : 128;
-  return (size_t)((k + bc - 1) / bc) * bc * ((d + 15) / 16) * 16 * 6;
+  return round256((size_t)((k + bc - 1) / bc) * bc * ((d + 15) / 16) * 16 * 6);
 }
-// Rows listed at most, and the bytes their list takes behind the parts.
-static int near_ties_cap(int64_t n) { return (int)std::min<int64_t>(n / 16 + 64, 1 << 26); }
-size_t near_ties_bytes(int64_t n) { return 256 + ((size_t)near_ties_cap(n) * 4 + 255) / 256 * 256 + (size_t)near_ties_cap(n) * 8; }
-static NearTies near_ties_at(const SplitScratch &scratch, size_t parts, int64_t n, int d) {
+template <typename T>
+size_t tiled_split_scratch_bytes(int split, int d, int k, int64_t ties) {
+  if (tiled_split<T>(split, d, k) == 0) return 0;
+  const size_t cap = ties > 0 ? (size_t)near_ties_cap(ties) : 0;
+  return 256 + split_parts_bytes(d, k) + round256(cap * sizeof(int)) + cap * sizeof(unsigned long long);
+}
+static NearTies near_ties_at(void *scratch, int64_t n, int d, int k, bool exact) {
   NearTies t;
-  const size_t at = (parts + 255) / 256 * 256;
-  if (!scratch.near_ties || !scratch.ptr || scratch.bytes < at + near_ties_bytes(n)) return t;
-  unsigned char *p = static_cast<unsigned char *>(scratch.ptr) + at;
-  t.cap = near_ties_cap(n);
-  t.count = reinterpret_cast<int *>(p);
-  t.rows = reinterpret_cast<int *>(p + 256);
-  t.keys = reinterpret_cast<unsigned long long *>(p + 256 + ((size_t)t.cap * 4 + 255) / 256 * 256);
+  unsigned char *p = static_cast<unsigned char *>(scratch);
+  t.cap = (unsigned)near_ties_cap(n);
+  t.count = reinterpret_cast<unsigned *>(p);
+  p += 256 + split_parts_bytes(d, k);
+  t.rows = reinterpret_cast<int *>(p);
+  t.keys = reinterpret_cast<unsigned long long *>(p + round256(t.cap * sizeof(int)));
   // Rounding noise between the two forms: measured over the shapes above, the difference of two distances
   // has an rms of about half an eps of xx + cc per form and grows with the square root of the features
   t.margin = (6.0f + 0.5f * sqrtf((float)d)) * 1.1920929e-7f;
+  t.mask = exact || d >= 128 ? ~0u : 0x7FFFFFF0u;  // (see launch_tiled_bcw)
   return t;
 }
-template size_t tiled_split_scratch_bytes<float>(int, int, int);
-template size_t tiled_split_scratch_bytes<double>(int, int, int);
+template size_t tiled_split_scratch_bytes<float>(int, int, int, int64_t);
+template size_t tiled_split_scratch_bytes<double>(int, int, int, int64_t);
 
+// The launch on the float32 (or float64) instructions. gate: run it only where a split launch before
+// it counted more ties than its list holds.
 template <typename T, int MODE>
-static int launch_tiled(hipStream_t s, const T *X, const T *xnorm, const T *C,
-                        const T *cnorm, int *labels, T *mindist, T *D, int64_t n,
-                        int64_t ldn, int d, int k, bool exact = false, int split = 0,
-                        SplitScratch scratch = SplitScratch()) {
-  const bool direct = !scratch.through_registers;
-  if constexpr (sizeof(T) == 4) {
-    const bool wide = tiled_split_wide(k);
-    const size_t need = tiled_split_scratch_bytes<T>(split, d, k);
-    void *split_scratch = scratch.ptr;
-    // the list of near ties lies behind the parts, where the caller asks for one
-    const NearTies ties = MODE == 0 ? near_ties_at(scratch, need, n, d) : NearTies();
-    const int products = need > 0 && scratch.ptr && scratch.bytes >= need ? split : 0;
-    // rows of bfloat16 values: three products (500k x 784 8-bit pixels, k = 4096: 24.0 ms on
-    // the float32 instructions, 12.9 with six products, 8.2 with three)
-    if (products == 6 && wide && scratch.rows_bf16)
-      return launch_tiled_bcw<T, MODE, 4, false, 6, true>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k,
-                                                          exact, split_scratch, true, ties);
-    switch (products) {
-#define KM_TILED_SPLIT(SP)                                                                         \
-  case SP:                                                                                         \
-    if (wide)                                                                                      \
-      return launch_tiled_bcw<T, MODE, 2, true, SP>(s, X, xnorm, C, cnorm, labels, mindist, D, n,  \
-                                                    ldn, d, k, exact, split_scratch, true, ties);  \
-    return launch_tiled_bcw<T, MODE, 2, false, SP>(s, X, xnorm, C, cnorm, labels, mindist, D, n,   \
-                                                   ldn, d, k, exact, split_scratch, true, ties)
-      KM_TILED_SPLIT(6);
-      KM_TILED_SPLIT(9);
-#undef KM_TILED_SPLIT
-    }
-  }
+static int launch_tiled_plain(hipStream_t s, const T *X, const T *xnorm, const T *C,
+                              const T *cnorm, int *labels, T *mindist, T *D, int64_t n,
+                              int64_t ldn, int d, int k, bool exact, bool direct, const NearTies &gate = NearTies()) {
   // Measured at 2M x 256, k = 1024 and 500k x 784, k = 4096: two 4-wave workgroups per CU
   // (BCW = 2) beat one 8-wave workgroup with the wider centroid block (BCW = 4) by 5-10 %,
   // so the 128-centroid form is used for large models. Up to 64 centroids a 64-wide block
   // (two wavefronts) halves the matrix work spent on padding; such shapes are bandwidth-bound.
   if (k <= 64)
-    return launch_tiled_bcw<T, MODE, 1>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact);
+    return launch_tiled_bcw<T, MODE, 1>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact,
+                                        nullptr, direct, gate);
   // A float32 model beyond one XCD's 4 MB of L2 (500k x 784, k = 4096: 12.8 MB): the centroid
   // stream misses L2 as well as the row slices, and the 256-centroid block, which passes over
   // a workgroup's row slice half as often, is ahead (26.9 -> 26.3 ms, 53 -> 30 GB through the
@@ -2853,7 +2833,7 @@ static int launch_tiled(hipStream_t s, const T *X, const T *xnorm, const T *C,
   if constexpr (sizeof(T) == 4) {
     if ((size_t)k * d * sizeof(T) > ((size_t)4 << 20))
       return launch_tiled_bcw<T, MODE, 2, true>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact,
-                                                nullptr, direct);
+                                                nullptr, direct, gate);
     // With the operands staged by direct loads the 256-centroid block is ahead for models that
     // stay in L2 as well (2M x 256, k = 1024: 7.95 against 8.11 ms in alternating runs): half as
     // many bytes fetched and read back from LDS per matrix instruction. Taken whenever its
@@ -2863,10 +2843,41 @@ static int launch_tiled(hipStream_t s, const T *X, const T *xnorm, const T *C,
     const int64_t pad256 = ((int64_t)k + 255) / 256 * 256, pad128 = ((int64_t)k + 127) / 128 * 128;
     if (direct && MODE == 0 && d % 16 == 0 && (bits & 15) == 0 && pad256 * 50 <= pad128 * 51)
       return launch_tiled_bcw<T, MODE, 2, true>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact,
-                                                nullptr, true);
+                                                nullptr, true, gate);
   }
   return launch_tiled_bcw<T, MODE, 2>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact, nullptr,
-                                      direct);
+                                      direct, gate);
+}
+
+template <typename T, int MODE>
+static int launch_tiled(hipStream_t s, const T *X, const T *xnorm, const T *C,
+                        const T *cnorm, int *labels, T *mindist, T *D, int64_t n,
+                        int64_t ldn, int d, int k, bool exact = false, int split = 0,
+                        SplitScratch scratch = SplitScratch()) {
+  const bool direct = !scratch.through_registers;
+  if constexpr (sizeof(T) == 4) {
+    const bool settle = MODE == 0 && scratch.near_ties;
+    const size_t need = tiled_split_scratch_bytes<T>(split, d, k, settle ? n : 0);
+    if (need > 0 && scratch.ptr && scratch.bytes >= need) {
+      const bool wide = tiled_split_wide(k);
+      void *const parts = static_cast<unsigned char *>(scratch.ptr) + 256;
+      const NearTies ties = settle ? near_ties_at(scratch.ptr, n, d, k, exact) : NearTies();
+      // rows of bfloat16 values: three products (500k x 784 8-bit pixels, k = 4096: 24.0 ms on
+      // the float32 instructions, 12.9 with six products, 8.2 with three)
+#define KM_TILED_SPLIT(BCW, WIDE, SP, XB)                                                                   \
+  KM_TRY((launch_tiled_bcw<T, MODE, BCW, WIDE, SP, XB>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, \
+                                                       k, exact, parts, true, ties)))
+      if (split == 6 && wide && scratch.rows_bf16) KM_TILED_SPLIT(4, false, 6, true);
+      else if (split == 6 && wide) KM_TILED_SPLIT(2, true, 6, false);
+      else if (split == 6) KM_TILED_SPLIT(2, false, 6, false);
+      else if (wide) KM_TILED_SPLIT(2, true, 9, false);
+      else KM_TILED_SPLIT(2, false, 9, false);
+#undef KM_TILED_SPLIT
+      if (!settle) return 0;
+      return launch_tiled_plain<T, MODE>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact, direct, ties);
+    }
+  }
+  return launch_tiled_plain<T, MODE>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact, direct);
 }
 
 template <typename T>

@@ -685,9 +685,10 @@ struct Engine : h2o4gpu_kmeans_handle {
     sc.through_registers = opt_tiled_direct == 0;
     sc.rows_bf16 = resident && rows_bf16;
     sc.near_ties = ties > 0 && settles();
-    size_t need = split ? tiled_split_scratch_bytes<T>(split, d, model_rows) : 0;
+    // (an assignment whose rows the tiled kernel does not see needs no memory)
+    if (ties > 0 && pick_assign_variant<T>(opt_assign, n, d, model_rows) != ASSIGN_TILED) return sc;
+    const size_t need = split ? tiled_split_scratch_bytes<T>(split, d, model_rows, sc.near_ties ? ties : 0) : 0;
     if (need == 0) return sc;
-    if (sc.near_ties) need = (need + 255) / 256 * 256 + near_ties_bytes(ties);
     if (need > split_bytes) {
       (void)hipStreamSynchronize(stream);
       if (d_split) (void)hipFree(d_split);
@@ -768,7 +769,6 @@ struct Engine : h2o4gpu_kmeans_handle {
           fused_slots<T>(ASSIGN_AUTO, n, d, k, num_cu) <= 0)
         return H2O4GPU_KMEANS_EARG;
     }
-    const size_t kd = (size_t)k * d;
     // Centroid buffers are padded to a multiple of CENTROID_PAD rows (zeros) and the
     // norms to as many entries (+inf): the tiled MFMA kernels read whole centroid
     // blocks without bounds tests and the padding can never win an argmin.
@@ -2146,22 +2146,22 @@ static int predict_device_noalloc(size_t rows, size_t cols, int k, const T *dX, 
   // launches instead of four (1000 x 16, k = 8: 15.0 -> 5.2 us).
   const AssignInputs in = assign_inputs<T>((int64_t)rows, d, k);
   const int split = default_split<T>(SPLIT_ASSIGN, (int64_t)rows, d, k);
+  SplitScratch parts;
+  parts.near_ties = true;
   if (in != ASSIGN_FROM_MODEL) {
     if (in == ASSIGN_FROM_ROW_NORMS) KM_TRY(launch_row_norms<T>(stream, dX, xnorm, (int64_t)rows, d));
     return launch_assign<T>(stream, ASSIGN_AUTO, dX, in == ASSIGN_FROM_ROW_NORMS ? xnorm : (const T *)nullptr, dC,
                             (const T *)nullptr, d_labels, mind, (int64_t)rows, d, k, nd.num_cu, nullptr, false,
-                            StackShape(), split);
+                            StackShape(), split, parts);
   }
   hipLaunchKernelGGL((stage_model_kernel<T>), dim3((unsigned)(kpad / 4)), dim3(256), 0, stream, dC, Cpad, cnorm, k,
                      (int)kpad, d);
   KM_HIP_TRY(hipGetLastError());
   KM_TRY(launch_row_norms<T>(stream, dX, xnorm, (int64_t)rows, d));
-  // the centroids' bfloat16 parts go behind the rest where the array has room for them (without,
-  // the launch runs the float32 instructions)
-  SplitScratch parts;
+  // the centroids' bfloat16 parts and the list of near ties go behind the rest where the array has
+  // room for both (without, the launch runs the float32 instructions: the same labels)
   parts.ptr = nd.ptr + need;
   parts.bytes = (size_t)H2O4GPU_KMEANS_NOALLOC_SCRATCH_BYTES - need;
-  parts.near_ties = true;
   return launch_assign<T>(stream, ASSIGN_AUTO, dX, xnorm, Cpad, cnorm, d_labels, mind, (int64_t)rows, d,
                           k, nd.num_cu, nullptr, false, StackShape(), split, parts);
 }

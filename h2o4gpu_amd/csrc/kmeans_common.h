@@ -86,25 +86,24 @@ enum SplitUse { SPLIT_ASSIGN, SPLIT_FUSED, SPLIT_TRANSFORM };
 template <typename T>
 int default_split(SplitUse use, int64_t n, int d, int k);
 
-// Rows a split launch of the tiled kernel has found within rounding of a tie (near_ties_kernel).
+// Rows a split launch of the tiled kernel has found within rounding of a tie (near_ties_kernel). A launch
+// on the float32 instructions that is given one runs only if more rows were counted than it holds.
 struct NearTies {
-  int *count = nullptr;  // null: none are listed
+  unsigned *count = nullptr;  // null: none are listed (float32: the launch always runs)
   int *rows = nullptr;
   unsigned long long *keys = nullptr;
-  int cap = 0;
+  unsigned cap = 0;
   float margin = 0;  // relative to xx + cc
   unsigned mask = ~0u;  // bits of a distance that are compared (keys: 16 ulp)
 };
-size_t near_ties_bytes(int64_t n);
 
 // Device memory a launch with the bfloat16-parts option may write the centroids' parts to
-// (tiled kernel only; tiled_split_scratch_bytes() says how much a shape needs). A launch that
+// (tiled kernel only; tiled_split_scratch_bytes() says how much a launch needs). A launch that
 // is given less runs the float32 instructions.
 struct SplitScratch {
   void *ptr = nullptr;
   size_t bytes = 0;
-  // assignments: settle near ties as the float32 instructions do (tiled kernel: the scratch then holds
-  // near_ties_bytes(n) behind the parts, 256-aligned)
+  // assignments: settle near ties as the float32 instructions do
   bool near_ties = false;
   // every value of X is a bfloat16 (row_norms' check): the products with its other parts are zeros
   bool rows_bf16 = false;
@@ -163,11 +162,12 @@ const char *assign_variant_name(int variant);
 // instructions.
 template <typename T>
 int assign_split_products(int variant, int split, int64_t n, int d, int k, bool fused);
-// The tiled kernel takes the centroids' parts from device scratch of this many bytes
+// The tiled kernel keeps the centroids' parts in device scratch of this many bytes
 // (split_scratch of launch_assign / launch_transform), written anew by every launch; without
-// the scratch (or with 0 bytes needed) it runs the float32 instructions.
+// the scratch (or with 0 bytes needed) it runs the float32 instructions. ties: the rows of an
+// assignment whose near ties are settled (0: none are), whose list lies behind the parts.
 template <typename T>
-size_t tiled_split_scratch_bytes(int split, int d, int k);
+size_t tiled_split_scratch_bytes(int split, int d, int k, int64_t ties);
 
 // Fused assign + accumulate (row-stationary MFMA shapes and the small VALU shapes): labels/mindist as
 // launch_assign, plus per-workgroup partial sums psums[slot][k][d] and counts

@@ -330,10 +330,12 @@ int h2o4gpu_kmeans_bandwidth_probe(int gpu_id, int kind, size_t bytes, int reps,
  * of a process for a new kind of shape (a kernel instance that needs more than
  * 64 KB of LDS: wide rows, large models) sets that kernel's LDS limit once
  * (hipFuncSetAttribute): make one call per shape that will be used outside
- * graph capture first. The float32 arithmetic is always the float32 matrix
- * instructions': the environment variable H2O4GPU_KMEANS_FP32_SPLIT, which
- * switches handles to bfloat16 parts, is not read here, so with it set the
- * labels can differ from h2o4gpu_kmeans_predict_host's on near-tie rows.
+ * graph capture first. The labels are those of the float32 matrix instructions:
+ * where the array has room for it the call forms its products on the bfloat16
+ * matrix pipe as handles do by default ("fp32_split"; the centroids' parts and a
+ * list of near ties then lie behind the rest), which gives the same labels. The
+ * environment variable H2O4GPU_KMEANS_FP32_SPLIT is not read here; a handle it
+ * sets to 6 or 9 may label near-tie rows otherwise.
  * ------------------------------------------------------------------------- */
 #define H2O4GPU_KMEANS_NOALLOC_SCRATCH_BYTES (16u << 20)
 int h2o4gpu_kmeans_predict_device_noalloc(int elem_size, size_t rows, size_t cols,

@@ -3,6 +3,7 @@ float32 instructions bit for bit: rows within rounding of a tie are settled as t
 every kernel family and wherever a model or a tile ends."""
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -55,6 +56,47 @@ def test_labels_are_the_float32_instructions(hip, n, d, k, offset):
         assert not np.array_equal(run(hip, X, C, split=6, fuse=0)[0], want)
     scale = (X.astype(np.float64) ** 2).sum(1).max() + (C.astype(np.float64) ** 2).sum(1).max()
     assert np.abs(mind - wmind).max() <= (16 + 4 * np.sqrt(d) + 40) * np.finfo(np.float32).eps * scale
+
+
+@pytest.mark.parametrize("offset", [0.0, 4000.0])
+@pytest.mark.parametrize("n,d,k", TILED + [(5000, 132, 200), (4097, 131, 70), (20011, 298, 300), (3000, 784, 257), (20000, 160, 256)])
+def test_more_ties_than_the_list_holds(hip, n, d, k, offset):
+    """A third of the centroids in pairs, or data so far from the origin that most rows are ties: the
+    pass runs again on the float32 instructions, in each form the plain kernel has."""
+    X, C = near_tied(n, d, k, offset)
+    got, _, mind, products = run(hip, X, C)
+    want, _, wmind, _ = run(hip, X, C, split=0)
+    assert products == 6 and np.array_equal(got, want) and np.array_equal(mind, wmind)
+
+
+def test_parts_of_a_set_are_labelled_as_the_set(hip):
+    """labels of rows predicted in pieces, whatever ties each piece has, are those of the fit."""
+    X, C = near_tied(30000, 150, 200, every=8)
+    with hip.Handle(30000, 150, 200, np.float32) as h:
+        h.set_data(X)
+        h.set_centroids(C)
+        h.assign()
+        want = h.labels()
+        assert np.array_equal(h.predict(X), want)
+        for lo, hi in ((0, 40), (40, 5000), (5000, 30000)):
+            assert np.array_equal(h.predict(X[lo:hi]), want[lo:hi])
+
+
+# (65 features: the parts fit the fixed array in both cases, the list beside two million rows does not)
+@pytest.mark.parametrize("n,d,k", [(20000, 3, 27), (5000, 8, 60), (20001, 32, 256), (9000, 24, 1500), (5000, 65, 300), (3000, 300, 200),
+                                   (2000000, 65, 300), (3000, 784, 3000)])
+def test_calls_without_allocation_give_the_same_labels(hip, n, d, k):
+    X, C = near_tied(n, d, k, every=3 if n < 100000 else 60)
+    with hip.Handle(k, d, k, np.float32) as h:
+        h.set_centroids(C)
+        h.set_option("fp32_split", 0)
+        want = h.predict(X)
+    dX, dC = torch.from_numpy(X).cuda(), torch.from_numpy(C).cuda()
+    labels = torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    hip.predict_device_noalloc(np.float32, n, d, k, dX.data_ptr(), dC.data_ptr(), labels.data_ptr(),
+                               torch.cuda.current_stream().cuda_stream)
+    assert np.array_equal(labels.cpu().numpy(), want)
 
 
 @pytest.mark.parametrize("n,d,k", [(60000, 32, 256), (40000, 61, 40), (50000, 13, 200), (60000, 3, 27), (40000, 7, 60), (30000, 100, 400)])
