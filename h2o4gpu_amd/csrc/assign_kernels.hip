@@ -1439,11 +1439,14 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
     for (int q = 0; q < B_VECS; q++) breg[q] = fetch(xrow[q], false);
   };
   // (SPLIT) the three bfloat16 parts of a staged vector, 8 bytes each
+  unsigned low = 0;  // (XB) bits of the row values that a bfloat16 does not have
   auto store_parts = [&](unsigned char *dst, const vec_t &v) {
     if constexpr (SPLIT != 0) {
       typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
       if constexpr (XB) {
         uintx2 p;
+#pragma unroll
+        for (int w = 0; w < 4; w++) low |= __float_as_uint((float)v[w]);
 #pragma unroll
         for (int w = 0; w < 2; w++)
           p[w] = (__float_as_uint((float)v[2 * w]) >> 16) | (__float_as_uint((float)v[2 * w + 1]) & 0xFFFF0000u);
@@ -1678,6 +1681,11 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
       }
     }
   }
+  // (XB) Rows that are not bfloat16 values after all (rewritten in place since they were looked at):
+  // the float32 launch behind this one runs.
+  if constexpr (XB) {
+    if (__any((low & 0xFFFFu) != 0) && lane == 0) atomicOr(ties.count, 1u << 31);
+  }
   if (MODE == 0) {
     if constexpr (sizeof(T) == 4 && !EXACT) {
 #pragma unroll
@@ -1739,7 +1747,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
           if constexpr (SECOND) {
             // (all on the accumulators' scale of half a distance; xx[rt] is -xx / 2, and a centroid
             // this close has a norm of at most 2 xx + 2 distances; keys: and two buckets of 16 ulp)
-            if (ties.count && second[rt] - best[rt] <= ties.margin * (4 * best[rt] - 3 * xx[rt]) +
+            if (ties.rows && second[rt] - best[rt] <= ties.margin * (4 * best[rt] - 3 * xx[rt]) +
                                                            (EXACT ? (T)0 : (T)3.9e-6f * second[rt])) {
               const unsigned at = atomicAdd(ties.count, 1u);
               if (at < ties.cap) {
@@ -2760,7 +2768,7 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
 #undef KM_TILED
 #undef KM_TILED_X
   if constexpr (SPLIT != 0 && MODE == 0) {
-    if (ties.count) {
+    if (ties.rows) {
       hipLaunchKernelGGL(near_ties_kernel, dim3(512), dim3(WG), 0, s, X, xnorm, C, cnorm, d, k, ties);
       hipLaunchKernelGGL(near_ties_labels_kernel, dim3(std::min(64u, (ties.cap + WG - 1) / WG)), dim3(WG), 0, s,
                          labels, mindist, ties);
@@ -2861,19 +2869,23 @@ static int launch_tiled(hipStream_t s, const T *X, const T *xnorm, const T *C,
     if (need > 0 && scratch.ptr && scratch.bytes >= need) {
       const bool wide = tiled_split_wide(k);
       void *const parts = static_cast<unsigned char *>(scratch.ptr) + 256;
-      const NearTies ties = settle ? near_ties_at(scratch.ptr, n, d, k, exact) : NearTies();
+      const bool xb = split == 6 && wide && scratch.rows_bf16;
+      NearTies ties;
+      if (settle) ties = near_ties_at(scratch.ptr, n, d, k, exact);
+      else if (xb) ties.count = static_cast<unsigned *>(scratch.ptr);
       // rows of bfloat16 values: three products (500k x 784 8-bit pixels, k = 4096: 24.0 ms on
-      // the float32 instructions, 12.9 with six products, 8.2 with three)
+      // the float32 instructions, 12.9 with six products, 8.2 with three). The kernel looks at every
+      // value it stages, so the note that they are bfloat16 need not be up to date.
 #define KM_TILED_SPLIT(BCW, WIDE, SP, XB)                                                                   \
   KM_TRY((launch_tiled_bcw<T, MODE, BCW, WIDE, SP, XB>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, \
                                                        k, exact, parts, true, ties)))
-      if (split == 6 && wide && scratch.rows_bf16) KM_TILED_SPLIT(4, false, 6, true);
+      if (xb) KM_TILED_SPLIT(4, false, 6, true);
       else if (split == 6 && wide) KM_TILED_SPLIT(2, true, 6, false);
       else if (split == 6) KM_TILED_SPLIT(2, false, 6, false);
       else if (wide) KM_TILED_SPLIT(2, true, 9, false);
       else KM_TILED_SPLIT(2, false, 9, false);
 #undef KM_TILED_SPLIT
-      if (!settle) return 0;
+      if (!ties.count) return 0;
       return launch_tiled_plain<T, MODE>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn, d, k, exact, direct, ties);
     }
   }

@@ -87,10 +87,11 @@ template <typename T>
 int default_split(SplitUse use, int64_t n, int d, int k);
 
 // Rows a split launch of the tiled kernel has found within rounding of a tie (near_ties_kernel). A launch
-// on the float32 instructions that is given one runs only if more rows were counted than it holds.
+// on the float32 instructions that is given one runs only if more rows were counted than it holds, or
+// if the three-product form counted 2^31 for rows that are no bfloat16 values.
 struct NearTies {
-  unsigned *count = nullptr;  // null: none are listed (float32: the launch always runs)
-  int *rows = nullptr;
+  unsigned *count = nullptr;  // null: nothing is counted (float32: the launch always runs)
+  int *rows = nullptr;  // null: none are listed
   unsigned long long *keys = nullptr;
   unsigned cap = 0;
   float margin = 0;  // relative to xx + cc
@@ -105,7 +106,8 @@ struct SplitScratch {
   size_t bytes = 0;
   // assignments: settle near ties as the float32 instructions do
   bool near_ties = false;
-  // every value of X is a bfloat16 (row_norms' check): the products with its other parts are zeros
+  // every value of X was a bfloat16 when its norms were made (row_norms' check): the products with its
+  // other parts are zeros
   bool rows_bf16 = false;
   // tiled kernels: stage the operands through registers also where the direct-to-LDS form
   // applies (handle option "tiled_direct" = 0)

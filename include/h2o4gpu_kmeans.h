@@ -165,7 +165,11 @@ int h2o4gpu_kmeans_select_set(h2o4gpu_kmeans_handle *h, int set);
 int h2o4gpu_kmeans_set_iterations(h2o4gpu_kmeans_handle *h, int *iterations);
 
 /* Upload rows from host memory (copies) / adopt a device pointer (no copy,
- * caller keeps it alive). Row norms are computed on the device either way. */
+ * caller keeps it alive). Row norms are computed on the device either way, on a
+ * stream of the handle's own: adopted rows must be complete when the call is made
+ * (work that still writes them on another stream is not waited for), and rows that
+ * are rewritten later need another call, or distances are formed with the norms of
+ * the rows before. */
 int h2o4gpu_kmeans_set_data_host(h2o4gpu_kmeans_handle *h, const void *X);
 int h2o4gpu_kmeans_set_data_device(h2o4gpu_kmeans_handle *h, const void *d_X);
 
