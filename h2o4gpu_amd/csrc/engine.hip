@@ -2433,7 +2433,7 @@ KM_API int h2o4gpu_kmeans_set_option(h2o4gpu_kmeans_handle *h, const char *name,
     return 0;
   }
   if (strcmp(name, "fp32_split") == 0) {
-    if (value != 0 && value != 6 && value != 9) return H2O4GPU_KMEANS_EARG;
+    if (value != SPLIT_DEFAULT && value != 0 && value != 6 && value != 9) return H2O4GPU_KMEANS_EARG;
     h->opt_split = value;
     return 0;
   }

@@ -22,7 +22,10 @@ extern "C" {
 
 /* error codes */
 #define H2O4GPU_KMEANS_OK 0
-#define H2O4GPU_KMEANS_EALLOC (-1)   /* allocation failed (the reference's -1) */
+#define H2O4GPU_KMEANS_EALLOC (-1)   /* allocation failed (the reference's -1); besides create and
+                                      * set_data_host, the first call of a handle that seeds or updates
+                                      * centroids allocates, and init_parallel, predict_host and
+                                      * transform_host for the call's duration */
 #define H2O4GPU_KMEANS_EARG (-2)     /* bad argument */
 #define H2O4GPU_KMEANS_EDEVICE (-3)  /* HIP runtime error / no usable device */
 #define H2O4GPU_KMEANS_ESTATE (-4)   /* call order (e.g. fit before data) */
@@ -243,12 +246,13 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * "fp32_split" = 6 or 9 makes the float32 matrix-core kernels form their dot
  * products on the bfloat16 matrix pipe: every float is the exact sum of three bfloat16
  * parts (rounded to nearest), 9 runs all nine products of the parts (each exact,
- * accumulated in float32), 6 leaves out the three smallest (2^-25 of |x||c| and below); 0 runs the
- * float32 matrix instructions. A handle that nobody sets it for, and that asks for no kernel family
- * and no exact compare, runs 6 wherever that is the faster form (more than 64 centroids,
- * or d * k > 2048; from 17 centroids on for 3 or 4 features, 49 for 5 to 8): 1.4 to 2 times on
- * matrix-bound shapes, with distances as close to float64 as the float32 instructions' or
- * closer. Rows whose every value is a bfloat16 (8-bit pixels, small integers) need three of the six.
+ * accumulated in float32), 6 leaves out the three smallest (2^-24 of |x||c| at most, together); 0 runs
+ * the float32 matrix instructions. -1 (the default) runs 6 wherever that is the faster form (more than
+ * 64 centroids, or d * k > 2048; from 17 centroids on for 3 or 4 features, 49 for 5 to 8) on a handle
+ * that asks for no kernel family and no exact compare: 1.1 to 2 times on matrix-bound shapes. Rows
+ * within rounding of a tie are then settled as the float32 instructions settle them, so labels and
+ * centroids are those of 0, and distances are as close to float64 or closer. Rows whose every
+ * value is a bfloat16 (8-bit pixels, small integers) need three of the six.
  * Shapes it does not apply to (float64, k <= 16 && d <= 64, ...) run as without it.
  * h2o4gpu_kmeans_assign_variant() names a form that was asked for ("mfma_tiled_bf16x6", ...),
  * h2o4gpu_kmeans_step_products() says what runs. The environment variable

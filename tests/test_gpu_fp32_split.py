@@ -208,6 +208,18 @@ def test_stacked_sets_take_the_option(hip):
             assert h.inertia() == got[s][2]
 
 
+def test_a_handle_goes_back_to_the_default(hip):
+    X = blobs(2000, 32, 100, seed=1)
+    with hip.Handle(2000, 32, 100, np.float32) as h:
+        h.set_data(X)
+        h.set_centroids(X[:100])
+        assert h.step_products() == 6
+        h.set_option("fp32_split", 0)
+        assert h.step_products() == 0
+        h.set_option("fp32_split", -1)
+        assert h.step_products() == 6 and h.assign_variant() == "mfma_rowstat"
+
+
 def test_option_values(hip):
     with hip.Handle(100, 32, 4, np.float32) as h:
         for bad in (1, 3, 12, -9):
