@@ -1607,9 +1607,12 @@ struct Engine : h2o4gpu_kmeans_handle {
   hipEvent_t shift_ready[2] = {nullptr, nullptr};
   int fit_with_threshold(int max_iterations, double threshold, int *updates_out) {
     if (!host_shift) {
-      KM_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&host_shift), 2 * sizeof(T), hipHostMallocDefault));
+      // (a kernel stores the scalar there: coherent memory, whatever HIP_HOST_COHERENT says, and events
+      // that release to the system)
+      KM_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&host_shift), 2 * sizeof(T),
+                               hipHostMallocCoherent | hipHostMallocMapped));
       for (int i = 0; i < 2; i++)
-        KM_HIP_TRY(hipEventCreateWithFlags(&shift_ready[i], hipEventDisableTiming));
+        KM_HIP_TRY(hipEventCreateWithFlags(&shift_ready[i], hipEventDisableTiming | hipEventReleaseToSystem));
     }
     auto queue_iteration = [&](int i) -> int {
       log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);

@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(WG) void finalize_kernel(
   const T sum = sum_shift_partials<T>(shift_partials, (int)gridDim.x);
   if (tid == 0) {
     *shift2 = sum;
-    if (shift_host) *shift_host = sum;
+    if (shift_host) __hip_atomic_store(shift_host, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     *done = 0;  // for the next launch
   }
 }
@@ -1054,7 +1054,7 @@ __global__ __launch_bounds__(WG) void post_update_kernel(
     const T sum = sum_shift_partials<T>(shift_partials, n_partials);
     if (tid == 0) {
       *shift2 = sum;
-      if (shift_host) *shift_host = sum;
+      if (shift_host) __hip_atomic_store(shift_host, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     return;
   }
