@@ -1220,21 +1220,6 @@ struct TiledCfg {
   static constexpr size_t LDS_BYTES = OPERAND_BYTES + (size_t)2 * BC * sizeof(T);
 };
 
-// The distance the float32 matrix instructions of the tiled kernels give (xxh = -xx / 2): one chain of
-// fused multiply-adds, of every eight features 0 4 1 5 2 6 3 7.
-__device__ __forceinline__ float float32_distance(const float *x, const float *c, int d, float xxh, float cc) {
-  float acc = 0;
-#pragma unroll 1
-  for (int f = 0; f < d; f += 8) {
-#pragma unroll 1
-    for (int e = 0; e < 8; e++) {
-      const int j = f + (e & 1) * 4 + (e >> 1);
-      if (j < d) acc = fmaf(c[j], x[j], acc);
-    }
-  }
-  return 2.0f * fabsf(acc + fmaf(-0.5f, cc, xxh));
-}
-
 template <typename T, int MODE, bool VECLOAD, bool DTAIL, int BCW, bool EXACT = false, bool WIDE = false,
           int SPLIT = 0, bool XB = false>
 __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) void assign_tiled_kernel(
@@ -1603,15 +1588,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
           for (int rt = 0; rt < RT; rt++) {
             const int64_t row = row0 + (wr * RT + rt) * MT + r;
             const T a = acc[ct][rt][v] + fma((T)-0.5, cc, xx[rt]);
-            if (c < k && row < n) {
-              T dist = (T)2 * fabs(a);
-              // (SPLIT) the parts of an infinity are not finite either, and a float just below it rounds up
-              // to one: such distances come from the float32 chain, infinite or NaN as it has them
-              if constexpr (SPLIT != 0) {
-                if (!(dist <= argmin_start<T>())) dist = float32_distance((const float *)X + row * d, (const float *)C + (size_t)c * d, d, (float)xx[rt], (float)cc);
-              }
-              D[(size_t)c * ldn + row] = dist;
-            }
+            if (c < k && row < n) D[(size_t)c * ldn + row] = (T)2 * fabs(a);
           }
         }
       }
@@ -1681,10 +1658,23 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
       }
     }
   }
-  // (XB) Rows that are not bfloat16 values after all (rewritten in place since they were looked at):
-  // the float32 launch behind this one runs.
-  if constexpr (XB) {
-    if (__any((low & 0xFFFFu) != 0) && lane == 0) atomicOr(ties.count, 1u << 31);
+  // Cases for the float32 launch behind this one, which then runs. XB: rows that are not bfloat16 values
+  // after all (rewritten in place since they were looked at). MODE 1: infinite norms, whose distances
+  // may be infinite or NaN, and which the parts of an infinity cannot tell (100k x 784, k = 4096: 3.3
+  // ms, 8.9 with an infinite row, 5.1 on the float32 instructions alone). A NaN norm makes its distances
+  // NaN here as there. (Distances of finite norms come from finite sums in either form.)
+  if constexpr (SPLIT != 0 && (XB || MODE == 1)) {
+    bool rerun = (low & 0xFFFFu) != 0;
+    if (MODE == 1) {
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++) rerun |= fabs(xx[rt]) == pos_inf<T>();
+#pragma unroll
+      for (int ct = 0; ct < CT; ct++) {
+        const int c = c_begin + (wc * CT + ct) * MT + r;
+        rerun |= c < k && cnorm[c] == pos_inf<T>();
+      }
+    }
+    if (__any(rerun) && lane == 0) atomicOr(ties.count, 1u << 31);
   }
   if (MODE == 0) {
     if constexpr (sizeof(T) == 4 && !EXACT) {
@@ -2872,7 +2862,7 @@ static int launch_tiled(hipStream_t s, const T *X, const T *xnorm, const T *C,
       const bool xb = split == 6 && wide && scratch.rows_bf16;
       NearTies ties;
       if (settle) ties = near_ties_at(scratch.ptr, n, d, k, exact);
-      else if (xb) ties.count = static_cast<unsigned *>(scratch.ptr);
+      else if (xb || MODE == 1) ties.count = static_cast<unsigned *>(scratch.ptr);
       // rows of bfloat16 values: three products (500k x 784 8-bit pixels, k = 4096: 24.0 ms on
       // the float32 instructions, 12.9 with six products, 8.2 with three). The kernel looks at every
       // value it stages, so the note that they are bfloat16 need not be up to date.

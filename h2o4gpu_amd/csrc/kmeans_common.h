@@ -88,7 +88,7 @@ int default_split(SplitUse use, int64_t n, int d, int k);
 
 // Rows a split launch of the tiled kernel has found within rounding of a tie (near_ties_kernel). A launch
 // on the float32 instructions that is given one runs only if more rows were counted than it holds, or
-// if the three-product form counted 2^31 for rows that are no bfloat16 values.
+// if a split launch counted 2^31 for rows or norms that are not its.
 struct NearTies {
   unsigned *count = nullptr;  // null: nothing is counted (float32: the launch always runs)
   int *rows = nullptr;  // null: none are listed

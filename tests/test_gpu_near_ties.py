@@ -89,3 +89,33 @@ def test_transform_of_rows_that_are_not_finite(hip, d, k):
     finite = np.isfinite(want)
     assert np.array_equal(got[~finite], want[~finite], equal_nan=True) and np.isfinite(got[finite]).all()
     assert (~finite).sum() > 4 * k
+
+
+@pytest.mark.parametrize("d,k", [(20, 70), (150, 90), (130, 300)])
+def test_missing_values_cost_a_transform_no_second_pass(hip, d, k):
+    """NaN rows and centroids give NaN where they stand and leave the others as the bfloat16 products have
+    them; an infinite row or centroid has the whole transform run on the float32 instructions."""
+    rng = np.random.default_rng(d)
+    X, C = rng.standard_normal((5000, d)).astype(np.float32), rng.standard_normal((k, d)).astype(np.float32)
+    with hip.Handle(5000, d, k, np.float32) as h:
+        def both(X, C):
+            h.set_centroids(C)
+            h.set_option("fp32_split", 0)
+            want = h.transform(X)
+            h.set_option("fp32_split", -1)
+            return h.transform(X), want
+        plain, f32 = both(X, C)
+        assert not np.array_equal(plain, f32)
+        Y, E = X.copy(), C.copy()
+        Y[[3, 4000], [0, 7]] = np.nan
+        E[11, 5] = np.nan
+        got, _ = both(Y, E)
+        hurt = np.zeros(got.shape, bool)
+        hurt[:, [3, 4000]] = hurt[11] = True
+        assert np.isnan(got[hurt]).all() and np.array_equal(got[~hurt], plain[~hurt])
+        for bad in (np.inf, -np.inf, 3e30):
+            for where in "XC":
+                Y, E = X.copy(), C.copy()
+                (Y if where == "X" else E)[17, 2] = bad
+                got, want = both(Y, E)
+                assert np.array_equal(got, want, equal_nan=True) and not np.isfinite(want).all()
