@@ -1013,7 +1013,8 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
             low = fminf(low, (float)pm[rt]);
           }
           // (each lane group sees the second minimum of its own centroids: a row is tied if either says so)
-          const unsigned long long ties = __ballot(near_tie(low, second, (float)xx[rt], bound));
+          unsigned long long ties = __ballot(near_tie(low, second, (float)xx[rt], bound));
+          if (ties != 0) ties &= __ballot((float)xx[rt] <= argmin_start<float>());  // (no distance to settle)
           const bool again = ties != 0 || direct > 0;
           if (__builtin_expect(again, 0)) {
             const bool tie = direct > 0 || (((ties | ties >> 32) >> r) & 1) != 0;
@@ -1640,8 +1641,10 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
 #pragma unroll
           for (int rt = 0; rt < RT; rt++) {
             const T a = acc[ct][rt][v] + fma((T)-0.5, cc, xx[rt]);
+            // (a NaN distance is nobody's second: fmin makes it an infinity)
             if constexpr (SECOND)
-              second[rt] = __builtin_amdgcn_fmed3f((float)fabs(a), (float)fabs(best[rt]), (float)second[rt]);
+              second[rt] = __builtin_amdgcn_fmed3f(fminf((float)fabs(a), pos_inf<float>()), (float)fabs(best[rt]),
+                                                   (float)second[rt]);
             if (fabs(a) < fabs(best[rt])) {
               best[rt] = a;
               loc[rt] = ct * NACC + v;
@@ -1737,7 +1740,8 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
           if constexpr (SECOND) {
             // (all on the accumulators' scale of half a distance; xx[rt] is -xx / 2, and a centroid
             // this close has a norm of at most 2 xx + 2 distances; keys: and two buckets of 16 ulp)
-            if (ties.rows && second[rt] - best[rt] <= ties.margin * (4 * best[rt] - 3 * xx[rt]) +
+            // (a row whose norm is infinite has no distance to settle)
+            if (ties.rows && xx[rt] >= -argmin_start<T>() && second[rt] - best[rt] <= ties.margin * (4 * best[rt] - 3 * xx[rt]) +
                                                            (EXACT ? (T)0 : (T)3.9e-6f * second[rt])) {
               const unsigned at = atomicAdd(ties.count, 1u);
               if (at < ties.cap) {

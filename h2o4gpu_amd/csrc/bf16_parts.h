@@ -61,7 +61,7 @@ __device__ __forceinline__ unsigned two_smallest_keys(const unsigned (&key)[16],
 // Whether two distances of a row, compared at 16 ulp, lie so close that the bfloat16 products and the
 // float32 instructions may order them differently. settle_margin() bounds the rounding of both forms
 // relative to xx + cc, and a centroid at a distance `second` has a norm of at most 2 xx + 2 second; two
-// buckets of 16 ulp come on top. (A row whose norm is infinite counts as tied, a NaN never does.)
+// buckets of 16 ulp come on top. (A row whose norm is infinite is said to be tied as well, a NaN never is.)
 struct TieBound {
   float of_norm, of_second;  // tied when of_second * second - best <= of_norm * xx; of_norm -infinity: never
 };

@@ -199,7 +199,8 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
       // Near ties, settled as the float32 instructions settle them (assign_rowstat_kernel): a tile with
       // such a row is swept again by them, with the operands the row-stationary kernel gives them
       // (lane group 0 the features 0 to 3, group 1 the rest).
-      const unsigned long long ties = __ballot(near_tie(best, second, nrm[rt], bound));
+      unsigned long long ties = __ballot(near_tie(best, second, nrm[rt], bound));
+      if (ties != 0) ties &= __ballot(nrm[rt] <= argmin_start<float>());  // (no distance to settle)
       if (__builtin_expect(ties != 0, 0)) {
         const bool tie = (((ties | ties >> 32) >> r) & 1) != 0;
         unsigned fkey = 0x7F7FFFF0u;

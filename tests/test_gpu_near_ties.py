@@ -73,6 +73,29 @@ def test_rows_no_distance_exists_for(hip):
     assert np.array_equal(got, want) and (got[[3, 77, 2999]] == -1).all()
 
 
+@pytest.mark.parametrize("d", [150, 256])
+def test_rows_and_centroids_that_are_not_finite_are_no_ties(hip, d):
+    """A NaN centroid, or rows with infinite norms, beside rows that are near ties: only those are listed.
+    (Were more listed than the list holds, the float32 instructions would run again over all rows, and
+    every minimum distance would be theirs.)"""
+    rng = np.random.default_rng(d)
+    n, k = 8000, 120
+    C = rng.uniform(0, 200, size=(k, d)).astype(np.float32)
+    C[61] = C[60] + (1e-4 * rng.standard_normal(d)).astype(np.float32)
+    X = (C[rng.integers(0, k, size=n)] + 30 * rng.standard_normal((n, d))).astype(np.float32)
+    for case in "nan centroid", "infinite rows":
+        Y, E = X.copy(), C.copy()
+        if case == "nan centroid":
+            E[100, 5] = np.nan
+        else:
+            Y[::5, 3] = np.inf
+        got, mind, _ = labels_of(hip, Y, E)
+        want, wmind, _ = labels_of(hip, Y, E, split=0)
+        assert np.array_equal(got, want), case
+        assert not np.array_equal(labels_of(hip, Y, E, split=6)[0], want), case
+        assert (mind != wmind).mean() > 0.1, case
+
+
 @pytest.mark.parametrize("d,k", [(20, 70), (150, 90), (130, 300)])
 def test_transform_of_rows_that_are_not_finite(hip, d, k):
     """Infinite and NaN distances come out as the float32 instructions have them."""
