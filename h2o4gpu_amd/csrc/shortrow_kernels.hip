@@ -6,17 +6,18 @@
 // is the exact sum of three bfloat16 parts (bf16_parts.h), six products of parts make a product of
 // floats to float32 accuracy, and with so few features the six products of all of them lie side by
 // side in the 16-wide k-steps. A lane group holds NP pairs of features, group 0 the features
-// 0 .. 2NP-1, group 1 the rest, and its k-slots are, for every pair (a, b), twelve halves in six
-// registers
-//     row side       h h  m m  l l  h h  m m  h h      (h, m, l: the parts of a and of b)
-//     centroid side  H H  H H  H H  M M  M M  L L      (parts of -2c)
-// which is what splitting a pair yields in packed form anyway. The accumulators start at cc (the
-// instruction takes them from the registers that hold the tile's norms, nothing is moved), the
-// products bring them to the size of xx, and an instruction of its own adds the three parts of xx
-// against ones: every partial sum is rounded at half the size of xx + cc or below. Up to four
-// features the smallest products come after that, at the size of the distance itself. (Distances
-// against float64 at three to eight features, rms, over the float32 instructions': 0.89 to
-// 0.94 centred on the origin, 0.73 to 0.85 at an offset of three times the spread.)
+// 0 .. 2NP-1, group 1 the rest. A pair (a, b) packs into one register per part, and the k-steps are
+//     one for each pair, its small products    m m  l l  h h  m m    (h, m, l: the parts of a and of b)
+//                                       with   H H  H H  M M  M M    (parts of -2c)
+//     lane group 0 h h of all pairs with L L, lane group 1 the parts of xx and cc against ones
+//     lane group 0 h h of all pairs with H H, lane group 1 zeros
+// The instruction adds the eight products of lane group 0, then those of group 1, and rounds after
+// either at the size of the largest term (bf16_parts.h). The small products are thus summed at their own
+// size, and a distance is rounded twice at the size of xx + cc, where the float32 instructions round
+// once per feature and once for xx + cc. (Rms error of the minimum distances over the float32
+// instructions': 0.73 to 0.93 in the mean, 1.06 at worst over forty sets of columns with scales and
+// offsets of their own; 0.70 to 0.96 and 1.19 with the accumulators starting at cc and large and small
+// products side by side. The small products last: 0.86 to 1.02.)
 // Labels (16-ulp integer keys, lowest index on ties; near ties settled by the float32 instructions),
 // minimum distances, -1 where nothing is below FLT_MAX: as in the row-stationary kernel. xx is summed from the row in feature order with
 // separate multiply and add, the value row_norms stores, so the norm buffer is not read.
@@ -43,12 +44,12 @@ constexpr int SR_NW = SR_TPB / 64;
 constexpr int SR_MAX_D = 8;
 constexpr size_t SR_LDS_MAX = 150 * 1024;
 __host__ __device__ constexpr int sr_pairs(int d) { return d <= 4 ? 1 : 2; }
-__host__ __device__ constexpr int sr_steps(int d) { return d <= 4 ? 2 : 3; }  // k-steps of the products
+__host__ __device__ constexpr int sr_steps(int d) { return sr_pairs(d) + 1; }  // k-steps before the last
 
 // row tiles a wavefront keeps in flight: as many as its 128 registers hold beside the work
 __host__ __device__ constexpr int sr_ahead(int d) { return d <= 3 ? 8 : d == 4 ? 6 : d == 5 ? 4 : 2; }
 
-size_t sr_model_lds(int d, int k) { return (size_t)((k + 31) / 32) * (sr_steps(d) * 64 * 16 + 32 * 4); }
+size_t sr_model_lds(int d, int k) { return (size_t)((k + 31) / 32) * (sr_steps(d) * 64 + 32) * 16 + 16; }
 size_t sr_sums_lds(int d, int k) { return (size_t)k * (4 * sr_pairs(d) + 1) * sizeof(double); }
 
 template <int D, bool FUSE>
@@ -59,12 +60,12 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
   constexpr int NP = sr_pairs(D), NM = sr_steps(D), NV = 2 * NP;
   constexpr int SD = 2 * NV + 1;  // doubles per centroid of the sums, the count last
   constexpr int MT = 32, NACC = 16, ROWT = 2;
-  static_assert(D >= 1 && D <= 2 * NV && NM * 4 >= 6 * NP, "the features' products fit the k-steps");
+  static_assert(D >= 1 && D <= 2 * NV && 2 * NP <= 4, "a lane group holds the leading parts of all pairs");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int KT = (k + MT - 1) / MT;
-  uintx4 *cs = reinterpret_cast<uintx4 *>(smem_raw);                        // [KT][NM][64]
-  floatx4 *ccs = reinterpret_cast<floatx4 *>(cs + (size_t)KT * NM * 64);    // [KT][8] norms, four centroids each
-  double *sums = reinterpret_cast<double *>(ccs + (size_t)KT * 8);          // (FUSE) [ncopy][k][SD]
+  uintx4 *cs = reinterpret_cast<uintx4 *>(smem_raw);                     // [KT][NM][64]
+  uintx4 *lead = cs + (size_t)KT * NM * 64;                              // [KT][32] the last step, then zeros
+  double *sums = reinterpret_cast<double *>(lead + (size_t)KT * 32 + 1);  // (FUSE) [ncopy][k][SD]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane % MT, g = lane / MT;
   if (FUSE)
@@ -72,30 +73,39 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
   // the centroid side, one (tile, lane) per thread and turn
   for (int e = tid; e < KT * 64; e += SR_TPB) {
     const int t = e >> 6, l = e & 63, c = t * MT + l % MT, gg = l / MT;
-    float v[NV];
+    Bf16x3Pair s[2 * NP];
 #pragma unroll
-    for (int q = 0; q < NV; q++) {
-      const int f = gg * NV + q;
-      v[q] = (c < k && f < D) ? -2.0f * C[(size_t)c * D + f] : 0.0f;
+    for (int p = 0; p < 2 * NP; p++) {
+      float v[2];
+#pragma unroll
+      for (int q = 0; q < 2; q++) v[q] = (c < k && 2 * p + q < D) ? -2.0f * C[(size_t)c * D + 2 * p + q] : 0.0f;
+      s[p] = split_pair_bf16x3(v[0], v[1]);
     }
-    unsigned w[NM * 4];
-#pragma unroll
-    for (int q = 0; q < NM * 4; q++) w[q] = 0;
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-      const Bf16x3Pair s = split_pair_bf16x3(v[2 * p], v[2 * p + 1]);
-      w[6 * p] = w[6 * p + 1] = w[6 * p + 2] = s.h;
-      w[6 * p + 3] = w[6 * p + 4] = s.m;
-      w[6 * p + 5] = s.l;
+      const unsigned h = gg == 0 ? s[p].h : s[NP + p].h, m = gg == 0 ? s[p].m : s[NP + p].m;
+      const uintx4 q = {h, h, m, m};
+      cs[(size_t)(t * NM + p) * 64 + l] = q;
     }
-    // (a padding centroid is infinitely far)
-    if (gg == 0)
-      reinterpret_cast<float *>(ccs)[c] = c < k ? row_sqnorm<float>(C + (size_t)c * D, D) : pos_inf<float>();
+    uintx4 q = {0u, 0u, 0u, 0u}, last = q;
+    if (gg == 0) {
 #pragma unroll
-    for (int m = 0; m < NM; m++) {
-      const uintx4 q = {w[4 * m], w[4 * m + 1], w[4 * m + 2], w[4 * m + 3]};
-      cs[(size_t)(t * NM + m) * 64 + l] = q;
+      for (int p = 0; p < 2 * NP; p++) {
+        q[p] = s[p].l;
+        last[p] = s[p].h;
+      }
+      lead[c] = last;
+    } else {  // (a padding centroid is infinitely far)
+      const Bf16x3 n = split_norm_bf16x3(c < k ? row_sqnorm<float>(C + (size_t)c * D, D) : pos_inf<float>());
+      q[0] = n.h | (n.m << 16);
+      q[1] = n.l | (0x3F80u << 16);
+      q[2] = 0x3F803F80u;
     }
+    cs[(size_t)(t * NM + NP) * 64 + l] = q;
+  }
+  if (tid == 0) {
+    const uintx4 zero = {0u, 0u, 0u, 0u};
+    lead[KT * 32] = zero;
   }
   __syncthreads();
 
@@ -110,12 +120,12 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
 #pragma unroll
     for (int j = 0; j < D; j++) x[j] = src[j];
   };
-  // the centroid side of the instruction that adds xx
-  const uintx4 ones = {g == 0 ? 0x3F803F80u : 0u, g == 0 ? 0x3F80u : 0u, 0u, 0u};
+  const uintx4 *const my_lead = g == 0 ? lead + r : lead + KT * 32;
+  const int lead_step = g == 0 ? 32 : 0;
   auto work = [&](const float (&xr)[ROWT][D], int64_t row0) {
     float val[ROWT][NV];  // what this lane group holds of the row
     float nrm[ROWT];
-    uintx4 b[ROWT][NM], bn[ROWT];
+    uintx4 b[ROWT][NM];  // (the last step has the row side of the one before)
 #pragma unroll
     for (int rt = 0; rt < ROWT; rt++) {
       float x[4 * NP];
@@ -131,24 +141,21 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
       nrm[rt] = xx;
 #pragma unroll
       for (int q = 0; q < NV; q++) val[rt][q] = g == 0 ? x[q] : x[NV + q];
-      unsigned w[NM * 4];
-#pragma unroll
-      for (int q = 0; q < NM * 4; q++) w[q] = 0;
+      uintx4 lastq = {0u, 0u, 0u, 0u};
 #pragma unroll
       for (int p = 0; p < NP; p++) {
         const Bf16x3Pair s = split_pair_bf16x3(val[rt][2 * p], val[rt][2 * p + 1]);
-        w[6 * p] = w[6 * p + 3] = w[6 * p + 5] = s.h;
-        w[6 * p + 1] = w[6 * p + 4] = s.m;
-        w[6 * p + 2] = s.l;
-      }
-#pragma unroll
-      for (int m = 0; m < NM; m++) {
-        const uintx4 q = {w[4 * m], w[4 * m + 1], w[4 * m + 2], w[4 * m + 3]};
-        b[rt][m] = q;
+        const uintx4 q = {s.m, s.l, s.h, s.m};
+        b[rt][p] = q;
+        lastq[p] = s.h;
+        lastq[NP + p] = cvt_pk_bf16(x[NV + 2 * p], x[NV + 2 * p + 1]);
       }
       const Bf16x3 xp = split_norm_bf16x3(xx);
-      const uintx4 q = {g == 0 ? xp.h | (xp.m << 16) : 0u, g == 0 ? xp.l : 0u, 0u, 0u};
-      bn[rt] = q;
+      lastq[0] = g == 0 ? lastq[0] : 0x3F803F80u;
+      lastq[1] = g == 0 ? lastq[1] : 0x3F80u | (xp.h << 16);
+      lastq[2] = g == 0 ? lastq[2] : xp.m | (xp.l << 16);
+      lastq[3] = g == 0 ? lastq[3] : 0u;
+      b[rt][NP] = lastq;
     }
     unsigned bkey[ROWT], skey[ROWT];
     int btile[ROWT];
@@ -161,24 +168,15 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
       uintx4 a[NM];
 #pragma unroll
       for (int m = 0; m < NM; m++) a[m] = cs[(size_t)(t * NM + m) * 64 + lane];
-      floatx16 cc;  // accumulator v is centroid 8 (v / 4) + 4 g + v % 4 of the tile
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const floatx4 c4 = ccs[t * 8 + 2 * q + g];
-#pragma unroll
-        for (int e = 0; e < 4; e++) cc[4 * q + e] = c4[e];
-      }
+      const uintx4 al = my_lead[t * lead_step];
 #pragma unroll
       for (int rt = 0; rt < ROWT; rt++) {
-        floatx16 acc = mma_bf16(a[0], b[rt][0], cc);
-        if constexpr (NP == 1) {
-          acc = mma_bf16(ones, bn[rt], acc);
-          acc = mma_bf16(a[1], b[rt][1], acc);
-        } else {
+        floatx16 acc;
 #pragma unroll
-          for (int m = 1; m < NM; m++) acc = mma_bf16(a[m], b[rt][m], acc);
-          acc = mma_bf16(ones, bn[rt], acc);
-        }
+        for (int v = 0; v < NACC; v++) acc[v] = 0;
+#pragma unroll
+        for (int m = 0; m < NM; m++) acc = mma_bf16(a[m], b[rt][m], acc);
+        acc = mma_bf16(al, b[rt][NP], acc);
         unsigned key[NACC];
 #pragma unroll
         for (int v = 0; v < NACC; v++) key[v] = (__float_as_uint(acc[v]) & 0x7FFFFFF0u) | (unsigned)v;
@@ -209,19 +207,19 @@ __global__ __launch_bounds__(SR_TPB) void assign_shortrow_kernel(
         for (int t = 0; t < KT; t++) {
           floatx16 acc;
 #pragma unroll
-          for (int v = 0; v < NACC; v++)
-            acc[v] = nrm[rt] + reinterpret_cast<const float *>(ccs)[t * MT + Mfma<float>::acc_row(v, g)];
+          for (int v = 0; v < NACC; v++) {
+            const uintx4 p = cs[(size_t)(t * NM + NP) * 64 + MT + Mfma<float>::acc_row(v, g)];
+            acc[v] = nrm[rt] + ((bf16_low(p[0]) + bf16_high(p[0])) + bf16_low(p[1]));
+          }
 #pragma unroll
           for (int e = 0; e < 4; e++) {
-            // feature 4 g + e of this lane's centroid, from its parts' words 6 p, 6 p + 3 and 6 p + 5
-            auto part = [&](int w) {
-              const uintx4 *slot = cs + (size_t)(t * NM + w / 4) * 64 + (NP == 2 ? lane : r + e / 2 * MT);
-              const unsigned u = reinterpret_cast<const unsigned *>(slot)[w % 4];
+            // feature 4 g + e of this lane's centroid, from the words of its three parts
+            auto word = [&](int step, int at, int w) {
+              const unsigned u = reinterpret_cast<const unsigned *>(cs + (size_t)(t * NM + step) * 64 + at)[w];
               return e % 2 ? bf16_high(u) : bf16_low(u);
             };
-            constexpr int P = 6;
-            const int p = NP == 2 ? e / 2 : 0;
-            float a = (part(P * p) + part(P * p + 3)) + part(P * p + 5);
+            const int own = NP == 2 ? lane : r + e / 2 * MT, step = NP == 2 ? e / 2 : 0;
+            float a = (word(step, own, 0) + word(step, own, 2)) + word(NP, r, NP == 2 ? 2 * g + e / 2 : e / 2);
             float b = NP == 2 ? val[rt][e % NV] : (e < D ? xr[rt][e < D ? e : 0] : 0.0f);
             if (NP == 1 && g == 1) a = b = 0.0f;
             acc = Mfma<float>::mma(a, b, acc);
