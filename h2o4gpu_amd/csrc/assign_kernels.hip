@@ -1242,6 +1242,12 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
     int *__restrict__ labels, T *__restrict__ mindist, T *__restrict__ D,
     int64_t n, int64_t ldn, int d, int k, const uintx4 *__restrict__ Cparts, NearTies ties) {
   if (SPLIT == 0 && ties.count && *ties.count <= ties.cap) return;
+  // (SPLIT) the float32 launch behind this one is to run: nothing left to do here. Only workgroups that
+  // start late look (261k x 298, k = 1000, nearly every row a tie: 2.03 -> 1.82 ms; transform 100k x 784,
+  // k = 4096 with an infinite row: 7.2 -> 5.3).
+  if (SPLIT != 0 && blockIdx.x >= 1024 && ties.count &&
+      __hip_atomic_load(ties.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > ties.cap)
+    return;
   typedef Mfma<T> M;
   typedef TiledCfg<T, BCW, WIDE, SPLIT, XB> Cfg;
   static_assert(!XB || SPLIT == 6, "bfloat16 rows: a form of the split kernel");
@@ -1685,7 +1691,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
   // Cases for the float32 launch behind this one, which then runs. XB: rows that are not bfloat16 values
   // after all (rewritten in place since they were looked at). MODE 1: infinite norms, whose distances
   // may be infinite or NaN, and which the parts of an infinity cannot tell (100k x 784, k = 4096: 3.3
-  // ms, 8.9 with an infinite row, 5.1 on the float32 instructions alone). A NaN norm makes its distances
+  // ms, 5.5 with an infinite row, 5.1 on the float32 instructions alone). A NaN norm makes its distances
   // NaN here as there. (Distances of finite norms come from finite sums in either form.)
   if constexpr (SPLIT != 0 && (XB || MODE == 1)) {
     bool rerun = (low & 0xFFFFu) != 0;
