@@ -790,7 +790,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     KM_TRY(allocate(list, &slab));
     KM_HIP_TRY(hipMemsetAsync(slab, 0, (size_t)(reinterpret_cast<unsigned char *>(cnorm) - slab), stream));
     KM_TRY(launch_fill<T>(stream, cnorm, std::numeric_limits<T>::infinity(), (int64_t)kpad));
-    use_buckets = bucketed_update_applies(plan.k_chunks, k, d);
+    use_buckets = bucketed_update_applies(plan.k_chunks, n, k, d, sizeof(T));
     log_msg(verbose, LOG_DEBUG,
             "handle: rows=%lld cols=%d k=%d elem=%d device=%d CUs=%d update plan: "
             "row_blocks=%d kc=%d k_chunks=%d vec=%d",

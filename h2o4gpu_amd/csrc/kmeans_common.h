@@ -226,7 +226,7 @@ int launch_accumulate(hipStream_t s, const UpdatePlan &p, const T *X,
 // windows of the ordered rows (partials: [bucket_partial_slots(n, k)][d] double) into
 // gsum [k][d] double; counts receives the bucket sizes. Run-to-run reproducible for
 // both precisions. The result is consumed by launch_finalize with slots = 1.
-bool bucketed_update_applies(int k_chunks, int k, int d);
+bool bucketed_update_applies(int k_chunks, int64_t n, int k, int d, size_t elem);
 int bucket_blocks(int64_t n, int k);
 size_t bucket_partial_slots(int64_t n, int k);
 template <typename T>

@@ -845,7 +845,7 @@ __global__ __launch_bounds__(WG) void bucket_sum_kernel(const double *__restrict
 }
 
 size_t bucket_lds_bytes(int k) { return (size_t)bucket_waves(k) * k * sizeof(int); }
-bool bucketed_update_applies(int k_chunks, int k, int d) {
+bool bucketed_update_applies(int k_chunks, int64_t n, int k, int d, size_t elem) {
   if ((size_t)k * sizeof(int) > 128 * 1024) return false;
   // Short rows: up to 8 chunks of centroids the LDS kernel is ahead (2M x 32, k = 4096: 0.15 vs
   // 0.21 ms, 2M x 64, k = 1000: 0.19 vs 0.22).
@@ -855,7 +855,12 @@ bool bucketed_update_applies(int k_chunks, int k, int d) {
   // k = 100: 0.57 vs 0.45, 640k x 784, k = 100: 0.54 vs 0.45). With a single chunk (298 features, k = 48
   // 0.59 vs 0.47; 256, k = 48 0.47 vs 0.45) it would need counts that a handful of centroids, whose
   // buckets span thousands of windows each, does not have.
-  return d >= 96 && k_chunks > 1;
+  if (d < 96 || k_chunks <= 1) return false;
+  // Float64 rows beyond 256 features: the chunks read whole pages in a row, and on a table that is read
+  // from memory that is ahead of gathering (1M x 300, k = 100: 0.51 ordered, 0.47 in chunks; 300k x 784, k = 60
+  // 0.40 and 0.37, 200k x 2500, k = 8 0.89 and 0.74; but 300k x 300, k = 100 0.168 and 0.173, 100k x 784, k = 60
+  // 0.155 and 0.169, 1M x 256, k = 80 0.432 and 0.433, 1M x 160, k = 120 0.29 and 0.39).
+  return !(elem == 8 && d > 256 && (size_t)n * d * elem > ((size_t)1 << 30));
 }
 
 template <typename T>
