@@ -24,6 +24,12 @@ def test_step_and_labels(hip, oracle, n, d, k, offset):
     with hip.Handle(n, d, k, np.float32) as h:
         h.set_data(X)
         h.set_centroids(C)
+        # (the dispatch rule; d = 5 to 8 beyond its LDS runs the row-stationary kernel's float32 instructions)
+        h.set_option("fuse", 0)
+        assert h.step_products() == (6 if k > (16 if d <= 4 else 48) else 0)
+        h.set_option("fuse", 1)
+        if k <= 300:
+            assert h.step_products() == (6 if k > (16 if d <= 4 else 48) else 0)
         h.iterate(1)
         fused, counts, centres = h.labels(), h.counts(), h.centroids()
         h.set_centroids(C)
@@ -53,6 +59,7 @@ def test_distances_are_as_close_to_float64_as_the_float32_instructions(hip, d):
             h.set_data(X)
             h.set_centroids(C)
             h.set_option("assign", variant)
+            assert h.step_products() == (6 if variant == "auto" else 0)
             h.assign()
             err[variant] = np.sqrt(((h.min_distances() - truth) ** 2).mean())
     print("d=%d: rms error of the minimum distance %.3g, float32 instructions %.3g" % (d, err["auto"], err["mfma_rowstat"]))
