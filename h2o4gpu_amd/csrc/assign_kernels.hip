@@ -514,8 +514,8 @@ __device__ __forceinline__ float float32_chain(const float *x, const float *c, i
 // load per lane, then walks over row tiles. Each wavefront keeps ROWT tiles of
 // MT data rows in registers (plain 16-byte global loads, never through LDS)
 // and sweeps all centroid tiles over them: accumulators start at xx + cc, the
-// matrix core adds -2 x.c, and the epilogue folds |acc| into a per-lane running
-// (min, index). Lane groups holding different centroid subsets of the same row
+// matrix core adds -2 x.c (SPLIT: they start at zero and xx + cc joins on the way),
+// and the epilogue folds |acc| into a per-lane running (min, index). Lane groups holding different centroid subsets of the same row
 // are merged with one (f32) or two (f64) cross-lane exchanges per row tile.
 // ---------------------------------------------------------------------------
 //
@@ -531,7 +531,8 @@ __device__ __forceinline__ float float32_chain(const float *x, const float *c, i
 // 0: d below the vector width: scalar loads, zero padded.
 // SPLIT (float32 only; 0, 6 or 9): the dot products run on the bfloat16 matrix pipe as that
 // many products of bfloat16 parts per feature pair (see split_pair_bf16x3). 9: every product
-// exact. 6: the three smallest (below 2^-24 of |x||c|) left out. The centroid parts are
+// exact. 6: the three smallest (together at most 2^-24 of |x||c|) left out, and rows within rounding of a
+// tie swept once more by the float32 instructions where `bound` asks for it. The centroid parts are
 // staged in LDS in operand order, [tile][16-feature step][part][lane] 16 bytes each; the
 // data rows are split in registers once per row tile.
 template <typename T, int DP, int ROWT, int LOAD, bool FUSE, int NW, bool EXACT = false, int SPLIT = 0>
@@ -701,7 +702,7 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
     if (cnorm == nullptr) {
       // No norm buffer given: take the norms from the staged centroids. A staged value is
       // -2c; halving it is exact, so the sum below (j ascending, multiply and add rounded
-      // separately) is bit for bit what row_norms / post_update would have stored.
+      // separately) is bit for bit what row_norms would have stored.
 #pragma clang fp contract(off)
       for (int c = tid; c < k; c += TPB) {
         if ((c % kps) >= kset) continue;

@@ -8,7 +8,7 @@
 namespace kmhip {
 
 // Squared norm of one centroid row, j ascending, multiply and add rounded separately:
-// the value row_norms / post_update would store (kmeans_labels.h:187-199). The fused
+// the value row_norms would store (kmeans_labels.h:187-199). The fused
 // kernels call it when they are given no norm buffer, which spares the Lloyd loop a launch.
 template <typename T>
 __device__ __forceinline__ T row_sqnorm(const T *__restrict__ x, int d) {

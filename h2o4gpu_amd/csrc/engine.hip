@@ -650,13 +650,9 @@ struct Engine : h2o4gpu_kmeans_handle {
   int *rows_inexact = nullptr;
   unsigned *finalize_done = nullptr;  // workgroups of a finalize launch that have ended
   int *d_frozen = nullptr;  // [sets] flags of a stacked handle's sets that have converged
-  // (option fp32_split, tiled kernel) the centroids' bfloat16 parts, rewritten by every launch
+  // (tiled kernel, bfloat16 products) the centroids' parts and the list of near ties, rewritten by every launch
   unsigned char *d_split = nullptr;
   size_t split_bytes = 0;
-  // The scratch a launch with the option needs, allocated on first use (an in-flight launch
-  // may still read the old one: the stream is drained before it is replaced); null when the
-  // option is off or does not apply, and when the allocation fails (the launch then runs the
-  // float32 instructions).
   // bfloat16 products per feature pair a launch is asked to run with: the option's number or, left
   // alone, the rule of default_split() (which a kernel family or the exact compare asked for by
   // name switches off: they stand for the float32 instructions)
@@ -678,6 +674,9 @@ struct Engine : h2o4gpu_kmeans_handle {
     return products == 6 && rows_bf16 && k > 128 && pick_assign_variant<T>(opt_assign, n, d, k) == ASSIGN_TILED
                ? 3 : products;
   }
+  // The scratch a split launch needs, allocated on first use (an in-flight launch may still read the
+  // old one: the stream is drained before it is replaced); null when the products are off or do not apply,
+  // and when the allocation fails (the launch then runs the float32 instructions).
   // resident: the launch reads the handle's rows
   // ties: rows of an assignment whose near ties are settled (default rule only; 0: none)
   SplitScratch split_scratch(int split, int model_rows, bool resident, int64_t ties) {  // (the seeding runs models of other sizes)
@@ -875,7 +874,8 @@ struct Engine : h2o4gpu_kmeans_handle {
   }
 
   // Norms of the rows, and whether they are bfloat16 values (8-bit pixels, small integers), which the
-  // split kernels need half the products for: the pass over long rows looks at them on its way.
+  // split kernels need half the products for: the pass over long rows looks at them on its way. (The
+  // kernels look again at what they stage: adopted rows may change in place.)
   bool rows_bf16 = false;
   int data_changed() {
     const bool look = row_norms_check<T>(n, d);

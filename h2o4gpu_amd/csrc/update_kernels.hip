@@ -10,9 +10,11 @@
 //           atomics, no sort);
 //   pass 2  finalize   : sums the slots in slot order, applies the reference's
 //           rules (count < 1 keeps the old centroid; mean = sum * (1/count)),
-//           and emits per-block partials of sum((old-new)^2);
-//   pass 3  post_update: centroid norms for the next assign and the ordered
-//           sum of the shift partials.
+//           and emits per-block partials of sum((old-new)^2), which its last
+//           workgroup adds up in order when there are few;
+//   pass 3  post_update: the ordered sum of the shift partials when there are
+//           many, or of each set of a stacked model, with that set's centroid
+//           norms. (Norms of an ordinary model are made by whoever needs them.)
 #include <algorithm>
 
 #include "kmeans_common.h"
