@@ -251,7 +251,8 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * 64 centroids, or d * k > 2048; from 17 centroids on for 3 or 4 features, 49 for 5 to 8) on a handle
  * that asks for no kernel family and no exact compare: 1.1 to 2 times on matrix-bound shapes. Rows
  * within rounding of a tie are then settled as the float32 instructions settle them, so labels and
- * centroids are those of 0, and distances are as close to float64 or closer. Rows whose every
+ * centroids are those of 0 (asked for by number, 6 and 9 leave near ties as they fall), and the rms error
+ * of the distances against float64 is no larger. Rows whose every
  * value is a bfloat16 (8-bit pixels, small integers) need three of the six.
  * Shapes it does not apply to (float64, k <= 16 && d <= 64, ...) run as without it.
  * h2o4gpu_kmeans_assign_variant() names a form that was asked for ("mfma_tiled_bf16x6", ...),

@@ -133,3 +133,40 @@ def test_a_restart_is_the_fit_it_stands_for(hip, n, d, k, sets):
             labels, centres, _, products = run(hip, X, starts[s], steps=15)
             assert products == 6
             assert np.array_equal(h.labels(), labels) and np.array_equal(h.centroids(), centres)
+
+
+@pytest.mark.parametrize("n,d,k", [(5000, 8, 60), (20001, 32, 256), (9000, 24, 1500), (5000, 65, 300), (3000, 300, 200)])
+def test_captured_calls_settle_each_replay_anew(hip, n, d, k):
+    """The call without allocation recorded into a graph: replays on other rows, with few ties, with more
+    than the list holds, and with few again, give what the call gives outside the graph."""
+    few, C = near_tied(n, d, k, every=60)
+    dX, dC = torch.from_numpy(few).cuda(), torch.from_numpy(C).cuda()
+    labels = torch.empty(n, dtype=torch.int32, device="cuda")
+    side = torch.cuda.Stream()
+
+    def call(stream):
+        hip.predict_device_noalloc(np.float32, n, d, k, dX.data_ptr(), dC.data_ptr(), labels.data_ptr(), stream.cuda_stream)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(side)  # (a kernel's LDS limit is raised outside the capture)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(torch.cuda.current_stream())
+    tied = torch.from_numpy(C[np.random.default_rng(3).integers(0, 2, size=n)]).cuda() * 0.5 + 0.5 * dC[torch.arange(n, device="cuda") % k]
+    for rows in (torch.from_numpy(few).cuda(), tied, torch.from_numpy(few).cuda(), tied + 3000):
+        dX.copy_(rows)
+        torch.cuda.synchronize()
+        labels.fill_(-7)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = labels.cpu().numpy()
+        labels.fill_(-7)
+        torch.cuda.synchronize()
+        call(torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        assert np.array_equal(got, labels.cpu().numpy()) and (got >= 0).all()
+        with hip.Handle(k, d, k, np.float32) as h:
+            h.set_centroids(C)
+            h.set_option("fp32_split", 0)
+            assert np.array_equal(got, h.predict(dX.cpu().numpy()))
