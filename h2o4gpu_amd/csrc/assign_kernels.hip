@@ -490,18 +490,15 @@ __global__ __launch_bounds__(WG) void lloyd_valu_anyd_kernel(
 // times `scale` (a power of two).
 __device__ __forceinline__ float float32_chain(const float *x, const float *c, int d, float acc, float scale) {
 #pragma unroll 1
-  for (int f = 0; f < d; f += 16) {
-    float cv[16], xv[16];
+  for (int f = 0; f < d; f += 8) {
+    float cv[8], xv[8];
 #pragma unroll
-    for (int e = 0; e < 16; e++) {  // (all loads of a turn under way; a feature past the end adds 0 * 0)
+    for (int e = 0; e < 8; e++) {  // (all loads of a turn under way; a feature past the end adds 0 * 0)
       cv[e] = f + e < d ? scale * c[f + e] : 0.0f;
       xv[e] = f + e < d ? x[f + e] : 0.0f;
     }
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-      const int j = (e & 8) + (e & 1) * 4 + ((e & 7) >> 1);
-      acc = fmaf(cv[j], xv[j], acc);
-    }
+    for (int e = 0; e < 8; e++) acc = fmaf(cv[(e & 1) * 4 + (e >> 1)], xv[(e & 1) * 4 + (e >> 1)], acc);
   }
   return acc;
 }
@@ -1012,14 +1009,13 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
         if constexpr (SECOND) {
           // Near ties, settled as the float32 instructions settle them: the two forms round
           // differently, and a row whose two nearest centroids lie within rounding of each other
-          // would carry the difference into the next centroids. A tile with such a row is swept
-          // once more by the float32 instructions, with their operands (the sum of a float's parts is
-          // the float, but for parts below 2^-133) in their order. One tile in a thousand on
-          // clustered data (10M x 32, k = 256: 0.98 -> 0.97 ms a fused step; 2M x 16, k = 500, where the
-          // second minimum weighs most, 190 -> 214 us; the float32 instructions' 1.43 ms and 325 us). A
-          // few such tiles are a few microseconds at the end of a launch (300k x 32, k = 1500 in four
-          // launches: 168 -> 239 us, float32 296); where every tile has them (an offset of a hundred
-          // times the spread, 2M x 32, k = 256) a step takes 0.49 ms instead of 0.29 on float32.
+          // would carry the difference into the next centroids. Such rows are labelled once more with the
+          // float32 instructions' arithmetic: a few by scalar chains, a tile of many by the instructions
+          // themselves, with their operands (the sum of a float's parts is the float, but for parts below
+          // 2^-133) in their order. One tile in a thousand to one in a hundred on clustered data
+          // (300k x 32, k = 1500 in four launches 167 us without, 188 with, 240 with a sweep for every such
+          // tile; 10M x 32, k = 256 the same within 2 %). Where every tile has them (an offset of a hundred times the spread, 2M x 32,
+          // k = 256) a step takes 0.49 ms instead of 0.29 on float32.
           float second = fminf((float)fmax(own, other), __uint_as_float(skey[rt] & 0xFFFFFFF0u));
           float low = (float)best[rt];
           if (!FUSE && merge && pl[rt] >= 0) {
@@ -1031,52 +1027,109 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
           if (ties != 0) ties &= __ballot((float)xx[rt] <= argmin_start<float>());  // (no distance to settle)
           const bool again = ties != 0 || direct > 0;
           if (__builtin_expect(again, 0)) {
-            const bool tie = direct > 0 || (((ties | ties >> 32) >> r) & 1) != 0;
+            const unsigned tied_rows = (unsigned)(ties | ties >> 32);
+            const bool tie = direct > 0 || ((tied_rows >> r) & 1) != 0;
+            T fbest = __uint_as_float(0x7F7FFFF0u);
+            int fidx = -1;
             __builtin_amdgcn_s_setprio(3);
-            unsigned fkey = 0x7F7FFFF0u;
-            int ftile = -1;
-#pragma unroll 1
-            for (int t = set * tps; t < (set + 1) * tps; t++) {
-              acc_t acc;
+            if (direct == 0 && sets == 1 && __popc(tied_rows) <= 4) {
+              // a few rows: one after the other, the centroids dealt to the lanes, the chain of the
+              // instructions as scalar multiply-adds
+              for (unsigned left = tied_rows; left != 0; left &= left - 1) {
+                const int b = __ffs((int)left) - 1;
+                auto of_row = [&](T v, int gg) -> float {  // lane group gg's value of the row, for all lanes
+                  return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint((float)v), b + gg * MT));
+                };
+                const float xxb = of_row(xx[rt], 0);
+                unsigned long long low_key = ~0ull;
+                for (int c = lane; c < k; c += 64) {
+                  const float *cr = (const float *)C + (size_t)c * d;
+                  const uintx4 p = nps[(c / MT) * 64 + c % MT];
+                  float a = xxb + ((bf16_low(p[0]) + bf16_high(p[0])) + bf16_low(p[1]));
 #pragma unroll
-              for (int v = 0; v < NACC; v++) {
-                const uintx4 p = nps[t * 64 + M::acc_row(v, g)];
-                acc[v] = xx[rt] + (T)((bf16_low(p[0]) + bf16_high(p[0])) + bf16_low(p[1]));
-              }
-              typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+                  for (int q = 0; q < NV; q++) {
+                    if (LOAD == 1 || q < nq) {
+                      float cv[KL][4];
 #pragma unroll
-              for (int q = 0; q < NV; q++) {
-                if (LOAD == 1 || q < nq) {
-                  const unsigned char *part =
-                      smem_raw + ((size_t)((t * NS + q / 2) * 3) * 64 + lane) * 16 + (q % 2) * 8;
-                  const uintx2 ph = *reinterpret_cast<const uintx2 *>(part);
-                  const uintx2 pmid = *reinterpret_cast<const uintx2 *>(part + 64 * 16);
-                  const uintx2 plow = *reinterpret_cast<const uintx2 *>(part + 128 * 16);
+                      for (int gg = 0; gg < KL; gg++) {
+                        const int f = (q * KL + gg) * 4;
+                        if (LOAD == 1 || f + 4 <= d) {
+                          const floatx4_u u = *reinterpret_cast<const floatx4_u *>(cr + f);
 #pragma unroll
-                  for (int w = 0; w < 2; w++) {
-                    acc = M::mma((T)((bf16_low(ph[w]) + bf16_low(pmid[w])) + bf16_low(plow[w])),
-                                 x[rt][q * VW + 2 * w], acc);
-                    acc = M::mma((T)((bf16_high(ph[w]) + bf16_high(pmid[w])) + bf16_high(plow[w])),
-                                 x[rt][q * VW + 2 * w + 1], acc);
+                          for (int e = 0; e < 4; e++) cv[gg][e] = u[e];
+                        } else {
+#pragma unroll
+                          for (int e = 0; e < 4; e++) cv[gg][e] = f + e < d ? cr[f + e] : 0.0f;
+                        }
+                      }
+#pragma unroll
+                      for (int e = 0; e < 4; e++) {
+#pragma unroll
+                        for (int gg = 0; gg < KL; gg++)
+                          a = fmaf(-2.0f * cv[gg][e], of_row(x[rt][q * VW + e % VW], gg), a);
+                      }
+                    }
                   }
+                  const unsigned long long key =
+                      ((unsigned long long)(__float_as_uint(a) & 0x7FFFFFF0u) << 32) | (unsigned)c;
+                  low_key = key < low_key ? key : low_key;
+                }
+#pragma unroll
+                for (int off = 1; off < 64; off <<= 1) {
+                  const unsigned long long o = __shfl_xor(low_key, off, 64);
+                  low_key = o < low_key ? o : low_key;
+                }
+                if (r == b && (unsigned)(low_key >> 32) < 0x7F7FFFF0u) {
+                  fbest = __uint_as_float((unsigned)(low_key >> 32));
+                  fidx = (int)(unsigned)low_key;
                 }
               }
-              unsigned key[NACC];
+            } else {
+              unsigned fkey = 0x7F7FFFF0u;
+              int ftile = -1;
+#pragma unroll 1
+              for (int t = set * tps; t < (set + 1) * tps; t++) {
+                acc_t acc;
 #pragma unroll
-              for (int v = 0; v < NACC; v++) key[v] = (__float_as_uint((float)acc[v]) & 0x7FFFFFF0u) | (unsigned)v;
-              unsigned m = umin3(key[0], key[1], key[2]);
+                for (int v = 0; v < NACC; v++) {
+                  const uintx4 p = nps[t * 64 + M::acc_row(v, g)];
+                  acc[v] = xx[rt] + (T)((bf16_low(p[0]) + bf16_high(p[0])) + bf16_low(p[1]));
+                }
+                typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-              for (int v = 3; v + 1 < NACC; v += 2) m = umin3(m, key[v], key[v + 1]);
-              m = min(m, key[NACC - 1]);
-              if ((m | 15u) < fkey) {
-                fkey = m;
-                ftile = t;
+                for (int q = 0; q < NV; q++) {
+                  if (LOAD == 1 || q < nq) {
+                    const unsigned char *part =
+                        smem_raw + ((size_t)((t * NS + q / 2) * 3) * 64 + lane) * 16 + (q % 2) * 8;
+                    const uintx2 ph = *reinterpret_cast<const uintx2 *>(part);
+                    const uintx2 pmid = *reinterpret_cast<const uintx2 *>(part + 64 * 16);
+                    const uintx2 plow = *reinterpret_cast<const uintx2 *>(part + 128 * 16);
+#pragma unroll
+                    for (int w = 0; w < 2; w++) {
+                      acc = M::mma((T)((bf16_low(ph[w]) + bf16_low(pmid[w])) + bf16_low(plow[w])),
+                                   x[rt][q * VW + 2 * w], acc);
+                      acc = M::mma((T)((bf16_high(ph[w]) + bf16_high(pmid[w])) + bf16_high(plow[w])),
+                                   x[rt][q * VW + 2 * w + 1], acc);
+                    }
+                  }
+                }
+                unsigned key[NACC];
+#pragma unroll
+                for (int v = 0; v < NACC; v++) key[v] = (__float_as_uint((float)acc[v]) & 0x7FFFFFF0u) | (unsigned)v;
+                unsigned m = umin3(key[0], key[1], key[2]);
+#pragma unroll
+                for (int v = 3; v + 1 < NACC; v += 2) m = umin3(m, key[v], key[v + 1]);
+                m = min(m, key[NACC - 1]);
+                if ((m | 15u) < fkey) {
+                  fkey = m;
+                  ftile = t;
+                }
               }
+              fbest = __uint_as_float(fkey & 0xFFFFFFF0u);
+              fidx = ftile < 0 ? -1 : ftile * MT + key_row(fkey & 15u, g);
+              argmin_merge(fbest, fidx, (T)__shfl_xor(fbest, MT, 64), __shfl_xor(fidx, MT, 64));
             }
             __builtin_amdgcn_s_setprio(0);
-            T fbest = __uint_as_float(fkey & 0xFFFFFFF0u);
-            int fidx = ftile < 0 ? -1 : ftile * MT + key_row(fkey & 15u, g);
-            argmin_merge(fbest, fidx, (T)__shfl_xor(fbest, MT, 64), __shfl_xor(fidx, MT, 64));
             if (tie) {
               best[rt] = fbest;
               bidx[rt] = fidx;
