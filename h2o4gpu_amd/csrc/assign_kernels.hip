@@ -785,7 +785,7 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
   const int64_t wrow_first = ((int64_t)wave * gridDim.x + blockIdx.x) * ROWS_PER_WAVE;
   if (wrow_first < n) fetch_rows(wrow_first);
   int direct = 0;     // (SECOND) tiles to come that go straight to the float32 instructions
-  bool tied = false;  // the tile before had near ties
+  bool tied = false;  // the tile before had many near ties
   static_assert(!SECOND || ROWT == 1, "one row tile a wavefront");
   for (int64_t wrow0 = wrow_first; wrow0 < n; wrow0 += row_stride) {
     T x[ROWT][DCH];
@@ -1013,9 +1013,11 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
           // float32 instructions' arithmetic: a few by scalar chains, a tile of many by the instructions
           // themselves, with their operands (the sum of a float's parts is the float, but for parts below
           // 2^-133) in their order. One tile in a thousand to one in a hundred on clustered data
-          // (300k x 32, k = 1500 in four launches 167 us without, 188 with, 240 with a sweep for every such
-          // tile; 10M x 32, k = 256 the same within 2 %). Where every tile has them (an offset of a hundred times the spread, 2M x 32,
-          // k = 256) a step takes 0.49 ms instead of 0.29 on float32.
+          // (300k x 32, k = 1500 in four launches 167 us without, 189 with, 240 with a sweep for every such
+          // tile; 10M x 32, k = 256 0.875 ms a step without, 0.881 with; 2M x 16, k = 500, where the second
+          // minimum weighs most, 189 and 200 us). Rows left on a list for the end of the workgroup's walk
+          // were no faster. Where every tile has many (an offset of a hundred times the spread, 2M x 32,
+          // k = 256) a step takes 0.52 ms instead of 0.29 on float32.
           float second = fminf((float)fmax(own, other), __uint_as_float(skey[rt] & 0xFFFFFFF0u));
           float low = (float)best[rt];
           if (!FUSE && merge && pl[rt] >= 0) {
@@ -1141,10 +1143,11 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
                                          0x7FFFFFF0u);
             }
           }
-          // data whose every tile has ties (far from the origin, for instance): two in a row, and the
-          // next tiles go straight to the float32 instructions
-          if (sets == 1) direct = direct > 0 ? direct - 1 : (ties != 0 && tied ? 14 : 0);
-          tied = ties != 0;
+          // data whose every tile is full of ties (far from the origin, for instance): two in a row, and
+          // the next tiles go straight to the float32 instructions
+          const bool many = __popc((unsigned)(ties | ties >> 32)) > 4;
+          if (sets == 1) direct = direct > 0 ? direct - 1 : (many && tied ? 14 : 0);
+          tied = many;
         }
         if (g == 0 && row < n) {
           // A model too large for LDS is swept in chunks of centroids, one launch each:
