@@ -503,6 +503,41 @@ __device__ __forceinline__ float float32_chain(const float *x, const float *c, i
   return acc;
 }
 
+// The rows of a launch: all of them, or (LIST) those a RowBounds names.
+template <bool LIST>
+struct ListedRows {
+  int64_t count;
+  __device__ __forceinline__ ListedRows(const RowBounds &, int64_t n) : count(n) {}
+  __device__ __forceinline__ int64_t row(int64_t i) const { return i; }
+  __device__ __forceinline__ bool all() const { return true; }
+  __device__ __forceinline__ void label(int *labels, int64_t row, int c) const { labels[row] = c; }
+};
+template <>
+struct ListedRows<true> {
+  int64_t count;
+  const int *rows;  // null: all
+  unsigned *changed;
+  bool limits;  // the next step looks at them
+  __device__ __forceinline__ ListedRows(const RowBounds &rb, int64_t n)
+      : count(rb.ctl->full ? n : (int64_t)rb.ctl->count), rows(rb.ctl->full ? nullptr : rb.rows),
+        changed(&rb.ctl->changed), limits(rb.ctl->wait == 0) {}
+  __device__ __forceinline__ int64_t row(int64_t i) const { return rows ? (int64_t)rows[i] : i; }
+  __device__ __forceinline__ bool all() const { return rows == nullptr; }
+  __device__ __forceinline__ void label(int *labels, int64_t row, int c) const {
+    if (rows && labels[row] == c) return;
+    labels[row] = c;
+    if (rows) *changed = 1;  // (set already where all rows are measured)
+  }
+};
+// The second smallest magnitude once `a` joins a row whose smallest is `best`. (A NaN is nobody's second.)
+template <typename T>
+__device__ __forceinline__ T second_of(T a, T best, T second) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_amdgcn_fmed3f(fminf(fabsf(a), pos_inf<float>()), fabsf(best), second);
+  else
+    return fmin(second, fmax(fabs(a), fabs(best)));
+}
+
 // ---------------------------------------------------------------------------
 // MFMA row-stationary variant (d <= DP, all centroids resident in LDS).
 //
@@ -532,13 +567,22 @@ __device__ __forceinline__ float float32_chain(const float *x, const float *c, i
 // tie swept once more by the float32 instructions where `bound` asks for it. The centroid parts are
 // staged in LDS in operand order, [tile][16-feature step][part][lane] 16 bytes each; the
 // data rows are split in registers once per row tile.
-template <typename T, int DP, int ROWT, int LOAD, bool FUSE, int NW, bool EXACT = false, int SPLIT = 0>
+// LIST (with FUSE and SPLIT): the rows are those that rb names, and each is given its limit (row_bounds.h). The
+// sums are then what the step changes: a row with a new label is added to its sums and taken off
+// those of the label before (all rows measured: the whole sums, as without LIST).
+template <typename T, int DP, int ROWT, int LOAD, bool FUSE, int NW, bool EXACT = false, int SPLIT = 0, bool LIST = false>
 __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
     const T *__restrict__ X, const T *__restrict__ xnorm,
     const T *__restrict__ C, const T *__restrict__ cnorm,
     int *__restrict__ labels, T *__restrict__ mindist, int64_t n, int d, int k,
     int kp, double *__restrict__ psums, int *__restrict__ pcounts, int c_off, int merge,
-    int sets, int kps, int kset, int ncopy, TieBound bound) {
+    int sets, int kps, int kset, int ncopy, TieBound bound, RowBounds rb) {
+  static_assert(!LIST || (FUSE && SPLIT == 6), "listed rows: the fused split step");
+  const ListedRows<LIST> at(rb, n);
+  if constexpr (LIST) {
+    n = at.count;
+    if ((int64_t)blockIdx.x * ROWT * Mfma<T>::MT >= n) return;  // (finalize_kernel knows which workgroups had rows)
+  }
   constexpr int TPB = NW * 64;
   typedef Mfma<T> M;
   constexpr int MT = M::MT, KL = M::KL, NACC = M::NACC, VW = M::VW;
@@ -726,48 +770,65 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
     pmn[rt] = 0;
     pln[rt] = -1;
   }
+  // (LIST) the place of the row in the table, asked for one tile before its values, and its label so far
+  int rown[LIST ? ROWT : 1];
+  int oldn[LIST ? ROWT : 1];
+  auto fetch_places = [&](int64_t wrow0) {
+    if constexpr (LIST) {
+#pragma unroll
+      for (int rt = 0; rt < ROWT; rt++) rown[rt] = (int)at.row(min(wrow0 + rt * MT + r, n - 1));
+    }
+  };
+  // this lane's features of a row
+  auto load_values = [&](T (&to)[DCH], int64_t row) {
+    if (VECLOAD) {
+      const vec_t *src = reinterpret_cast<const vec_t *>(X + row * (int64_t)DP);
+#pragma unroll
+      for (int q = 0; q < NV; q++) {
+        vec_t v = src[q * KL + g];
+#pragma unroll
+        for (int e = 0; e < VW; e++) to[q * VW + e] = v[e];
+      }
+    } else if (LOAD == 2) {
+      const T *src = X + row * (int64_t)d;
+#pragma unroll
+      for (int q = 0; q < NV; q++) {
+        // (steps from nq on are never used, but their loads are issued all the same,
+        // clamped into the row: a branch here would make every load wait for the last)
+        const int f0 = (q * KL + g) * VW;
+        vec_t v;
+        if (d % VW == 0) {
+          // no vector straddles the end of the row: one that lies past it re-reads the
+          // row's last vector (finite x * 0 from the zero-padded centroid side adds
+          // nothing, and the padded columns of the fused sums are never written back)
+          const typename M::uvec_t u = *reinterpret_cast<const typename M::uvec_t *>(src + min(f0, d - VW));
+#pragma unroll
+          for (int e = 0; e < VW; e++) v[e] = u[e];
+        } else {
+          v = load_row_vector<T>(src, f0, d);
+        }
+#pragma unroll
+        for (int e = 0; e < VW; e++) to[q * VW + e] = v[e];
+      }
+    } else {
+      const T *src = X + row * (int64_t)d;
+#pragma unroll
+      for (int s = 0; s < DCH; s++) {
+        const int j = ((s / VW) * KL + g) * VW + s % VW;
+        to[s] = j < d ? src[j] : (T)0;
+      }
+    }
+  };
   auto fetch_rows = [&](int64_t wrow0) {
 #pragma unroll
     for (int rt = 0; rt < ROWT; rt++) {
       // rows past the end re-read the last row; their results are never stored
-      const int64_t row = min(wrow0 + rt * MT + r, n - 1);
-      if (VECLOAD) {
-        const vec_t *src = reinterpret_cast<const vec_t *>(X + row * (int64_t)DP);
-#pragma unroll
-        for (int q = 0; q < NV; q++) {
-          vec_t v = src[q * KL + g];
-#pragma unroll
-          for (int e = 0; e < VW; e++) xn[rt][q * VW + e] = v[e];
-        }
-      } else if (LOAD == 2) {
-        const T *src = X + row * (int64_t)d;
-#pragma unroll
-        for (int q = 0; q < NV; q++) {
-          // (steps from nq on are never used, but their loads are issued all the same,
-          // clamped into the row: a branch here would make every load wait for the last)
-          const int f0 = (q * KL + g) * VW;
-          vec_t v;
-          if (d % VW == 0) {
-            // no vector straddles the end of the row: one that lies past it re-reads the
-            // row's last vector (finite x * 0 from the zero-padded centroid side adds
-            // nothing, and the padded columns of the fused sums are never written back)
-            const typename M::uvec_t u = *reinterpret_cast<const typename M::uvec_t *>(src + min(f0, d - VW));
-#pragma unroll
-            for (int e = 0; e < VW; e++) v[e] = u[e];
-          } else {
-            v = load_row_vector<T>(src, f0, d);
-          }
-#pragma unroll
-          for (int e = 0; e < VW; e++) xn[rt][q * VW + e] = v[e];
-        }
-      } else {
-        const T *src = X + row * (int64_t)d;
-#pragma unroll
-        for (int s = 0; s < DCH; s++) {
-          const int j = ((s / VW) * KL + g) * VW + s % VW;
-          xn[rt][s] = j < d ? src[j] : (T)0;
-        }
+      int64_t row = min(wrow0 + rt * MT + r, n - 1);
+      if constexpr (LIST) {
+        row = rown[rt];
+        if (!at.all()) oldn[rt] = labels[row];
       }
+      load_values(xn[rt], row);
       xxn[rt] = xnorm[row];
       if (!FUSE && merge) {  // the row's result from the earlier chunks travels with the prefetch
         pmn[rt] = mindist[row];
@@ -783,7 +844,18 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
   const int64_t tile_stride = (int64_t)gridDim.x * NW;
   const int64_t row_stride = tile_stride * ROWS_PER_WAVE;
   const int64_t wrow_first = ((int64_t)wave * gridDim.x + blockIdx.x) * ROWS_PER_WAVE;
-  if (wrow_first < n) fetch_rows(wrow_first);
+  if (wrow_first < n) {
+    fetch_places(wrow_first);
+    fetch_rows(wrow_first);
+  }
+  int row_of[LIST ? ROWT : 1];
+  int old[LIST ? ROWT : 1];
+  int placen[LIST ? ROWT : 1];  // rown of the tile whose values are in xn
+  if constexpr (LIST) {
+#pragma unroll
+    for (int rt = 0; rt < ROWT; rt++) placen[rt] = rown[rt];
+    if (wrow_first + row_stride < n) fetch_places(wrow_first + row_stride);
+  }
   int direct = 0;     // (SECOND) tiles to come that go straight to the float32 instructions
   bool tied = false;  // the tile before had many near ties
   static_assert(!SECOND || ROWT == 1, "one row tile a wavefront");
@@ -799,8 +871,19 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
       xx[rt] = xxn[rt];
       pm[rt] = pmn[rt];
       pl[rt] = pln[rt];
+      if constexpr (LIST) {
+        row_of[rt] = placen[rt];
+        old[rt] = oldn[rt];
+      }
     }
-    if (wrow0 + row_stride < n) fetch_rows(wrow0 + row_stride);
+    if (wrow0 + row_stride < n) {
+      fetch_rows(wrow0 + row_stride);
+      if constexpr (LIST) {
+#pragma unroll
+        for (int rt = 0; rt < ROWT; rt++) placen[rt] = rown[rt];
+        if (wrow0 + 2 * row_stride < n) fetch_places(wrow0 + 2 * row_stride);
+      }
+    }
     // (SPLIT) the row tile's three bfloat16 parts, packed in operand order
     uintx4 xh[SPLIT ? ROWT : 1][SPLIT ? NS : 1], xm[SPLIT ? ROWT : 1][SPLIT ? NS : 1],
         xl[SPLIT ? ROWT : 1][SPLIT ? NS : 1];
@@ -981,6 +1064,12 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
         tile_argmin(acc, t);
       }
       __builtin_amdgcn_s_setprio(0);
+      // (LIST) the values are asked for once more instead of being kept through the sweep, where the places of
+      // rows and the old labels have their registers
+      if constexpr (LIST) {
+#pragma unroll
+        for (int rt = 0; rt < ROWT; rt++) load_values(x[rt], row_of[rt]);
+      }
       if constexpr (KEYS) {
 #pragma unroll
         for (int rt = 0; rt < ROWT; rt++) {
@@ -1006,6 +1095,7 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
           other = ob;
         }
         const int64_t row = wrow0 + rt * MT + r;
+        float to_second = 0, to_best = 0;  // (LIST) as the products have them
         if constexpr (SECOND) {
           // Near ties, settled as the float32 instructions settle them: the two forms round
           // differently, and a row whose two nearest centroids lie within rounding of each other
@@ -1023,6 +1113,10 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
           if (!FUSE && merge && pl[rt] >= 0) {
             second = fminf(second, fmaxf(low, (float)pm[rt]));
             low = fminf(low, (float)pm[rt]);
+          }
+          if constexpr (LIST) {
+            to_second = fminf(second, __shfl_xor(second, MT, 64));
+            to_best = low;
           }
           // (each lane group sees the second minimum of its own centroids: a row is tied if either says so)
           unsigned long long ties = __ballot(near_tie(low, second, (float)xx[rt], bound));
@@ -1149,7 +1243,14 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
           if (sets == 1) direct = direct > 0 ? direct - 1 : (many && tied ? 14 : 0);
           tied = many;
         }
-        if (g == 0 && row < n) {
+        if constexpr (LIST) {
+          if (g == 0 && row < n) {
+            if (at.limits)
+              rb.limit[row_of[rt]] = row_limit(to_best, to_second, (float)xx[rt], bidx[rt] >= 0 ? rb.drift[bidx[rt]] : 0.0f,
+                                             rb.noise, rb.grain);
+            if (at.all() || bidx[rt] != old[rt]) labels[row_of[rt]] = bidx[rt];
+          }
+        } else if (g == 0 && row < n) {
           // A model too large for LDS is swept in chunks of centroids, one launch each:
           // C and cnorm then point at the chunk, c_off is its first centroid, and from the
           // second chunk on (merge) the row's result so far is read back and kept unless
@@ -1161,7 +1262,8 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
           labels[(int64_t)set * n + row] = bi;
           if (mindist) mindist[(int64_t)set * n + row] = bv;
         }
-        if (FUSE && row < n && bidx[rt] >= 0) {
+        const bool whole = !LIST || at.all();
+        if (FUSE && row < n && bidx[rt] >= 0 && (whole || bidx[rt] != old[LIST ? rt : 0])) {
           double *srow = my_sums + (size_t)bidx[rt] * SD;
 #pragma unroll
           for (int q = 0; q < NV; q++) {
@@ -1174,6 +1276,22 @@ __global__ __launch_bounds__(NW * 64) void assign_rowstat_kernel(
             }
           }
           if (g == 0) atomicAdd(&my_cnt[bidx[rt]], 1);
+        }
+        if constexpr (LIST) {
+          if (!whole && row < n && old[rt] >= 0 && bidx[rt] != old[rt]) {
+            double *srow = my_sums + (size_t)old[rt] * SD;
+#pragma unroll
+            for (int q = 0; q < NV; q++) {
+              if (LOAD == 1 || q < nq) {
+#pragma unroll
+                for (int e = 0; e < VW; e++) {
+                  const int f = (q * KL + g) * VW + e;
+                  if (LOAD == 1 || f < d) unsafeAtomicAdd(srow + f, -(double)x[rt][q * VW + e]);
+                }
+              }
+            }
+            if (g == 0) atomicAdd(&my_cnt[old[rt]], -1);
+          }
         }
       }
     }  // centroid sets
@@ -1291,13 +1409,21 @@ struct TiledCfg {
   static constexpr size_t LDS_BYTES = OPERAND_BYTES + (size_t)2 * BC * sizeof(T);
 };
 
+// LIST: the rows are those that rb names, each gets its label and its limit (row_bounds.h), and no
+// minimum distances are written.
 template <typename T, int MODE, bool VECLOAD, bool DTAIL, int BCW, bool EXACT = false, bool WIDE = false,
-          int SPLIT = 0, bool XB = false>
+          int SPLIT = 0, bool XB = false, bool LIST = false>
 __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) void assign_tiled_kernel(
     const T *__restrict__ X, const T *__restrict__ xnorm,
     const T *__restrict__ C, const T *__restrict__ cnorm,
     int *__restrict__ labels, T *__restrict__ mindist, T *__restrict__ D,
-    int64_t n, int64_t ldn, int d, int k, const uintx4 *__restrict__ Cparts, NearTies ties) {
+    int64_t n, int64_t ldn, int d, int k, const uintx4 *__restrict__ Cparts, NearTies ties, RowBounds rb) {
+  static_assert(!LIST || MODE == 0, "listed rows are labelled");
+  const ListedRows<LIST> at(rb, n);
+  if constexpr (LIST) {
+    n = at.count;
+    if ((int64_t)blockIdx.x * 128 >= n) return;
+  }
   if (SPLIT == 0 && ties.count && *ties.count <= ties.cap) return;
   // (SPLIT) the float32 launch behind this one is to run: nothing left to do here. Only workgroups that
   // start late look (261k x 298, k = 1000, nearly every row a tie: 2.03 -> 1.82 ms; transform 100k x 784,
@@ -1420,7 +1546,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
   const T *xrow[B_VECS];
 #pragma unroll
   for (int q = 0; q < B_VECS; q++)
-    xrow[q] = X + min(row0 + rr0 + q * ROWS_PER_PASS, n - 1) * (int64_t)d;
+    xrow[q] = X + at.row(min(row0 + rr0 + q * ROWS_PER_PASS, n - 1)) * (int64_t)d;
 
   // The accumulators hold -1/2 of the reference's value: they start at -(xx + cc)/2 and the
   // matrix cores add +x.c with the centroids staged as they are, which spares the staging of
@@ -1431,7 +1557,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
   T xx[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
-    xx[rt] = (T)-0.5 * xnorm[min(row0 + (wr * RT + rt) * MT + r, n - 1)];
+    xx[rt] = (T)-0.5 * xnorm[at.row(min(row0 + (wr * RT + rt) * MT + r, n - 1))];
   T best[RT];
   int bidx[RT];
   unsigned bkey[RT];
@@ -1445,7 +1571,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
     return SPLIT != 0 ? fma((T)-0.5, cc, dot + xxh) : dot + fma((T)-0.5, cc, xxh);
   };
   // (SPLIT) the second smallest distance of the row, for the near-tie test at the end
-  constexpr bool SECOND = SPLIT != 0 && MODE == 0;
+  constexpr bool SECOND = (SPLIT != 0 && MODE == 0) || LIST;
   T second[RT];
   unsigned skey[RT];  // (integer keys: likewise)
 #pragma unroll
@@ -1726,9 +1852,7 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
           for (int rt = 0; rt < RT; rt++) {
             const T a = close(acc[ct][rt][v], cc, xx[rt]);
             // (a NaN distance is nobody's second: fmin makes it an infinity)
-            if constexpr (SECOND)
-              second[rt] = __builtin_amdgcn_fmed3f(fminf((float)fabs(a), pos_inf<float>()), (float)fabs(best[rt]),
-                                                   (float)second[rt]);
+            if constexpr (SECOND) second[rt] = second_of<T>(a, best[rt], second[rt]);
             if (fabs(a) < fabs(best[rt])) {
               best[rt] = a;
               loc[rt] = ct * NACC + v;
@@ -1817,22 +1941,33 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
             second[rt] = fmin(fmax(best[rt], mb[w * BR + lr]), fmin(second[rt], ms[w * BR + lr]));
           argmin_merge(best[rt], bidx[rt], mb[w * BR + lr], mi[w * BR + lr]);
         }
-        const int64_t row = row0 + lr;
-        if (row < n) {
-          labels[row] = bidx[rt];
-          if (mindist) mindist[row] = (T)2 * best[rt];
-          if constexpr (SECOND) {
+        if (row0 + lr < n) {
+          const int64_t row = at.row(row0 + lr);
+          bool listed = false;
+          if constexpr (SPLIT != 0) {
             // (all on the accumulators' scale of half a distance; xx[rt] is -xx / 2, and a centroid
             // this close has a norm of at most 2 xx + 2 distances; keys: and two buckets of 16 ulp)
             // (a row whose norm is infinite has no distance to settle)
             if (ties.rows && xx[rt] >= -argmin_start<T>() && second[rt] - best[rt] <= ties.margin * (4 * best[rt] - 3 * xx[rt]) +
                                                            (EXACT ? (T)0 : (T)3.9e-6f * second[rt])) {
-              const unsigned at = atomicAdd(ties.count, 1u);
-              if (at < ties.cap) {
-                ties.rows[at] = (int)row;
-                ties.keys[at] = ~0ull;
+              const unsigned at_tie = atomicAdd(ties.count, 1u);
+              listed = at_tie < ties.cap;
+              if (listed) {
+                ties.rows[at_tie] = (int)row;
+                ties.keys[at_tie] = ~0ull;
               }
             }
+          }
+          if constexpr (LIST) {
+            // (a near tie keeps the label it has until near_ties_labels_kernel knows better)
+            if (at.limits)
+              rb.limit[row] = listed ? -pos_inf<float>()
+                                   : row_limit((float)(2 * best[rt]), (float)(2 * second[rt]), (float)(-2 * xx[rt]),
+                                               bidx[rt] >= 0 ? rb.drift[bidx[rt]] : 0.0f, rb.noise, rb.grain);
+            if (!listed) at.label(labels, row, bidx[rt]);
+          } else {
+            labels[row] = bidx[rt];
+            if (mindist) mindist[row] = (T)2 * best[rt];
           }
         }
       }
@@ -1890,13 +2025,22 @@ __device__ __forceinline__ void dma_to_lds_16(const void *gsrc, void *lds) {
 // "do not wait")
 #define KM_WAIT_VMCNT(N) __builtin_amdgcn_s_waitcnt(0x0F70 | ((N) & 15) | (((N) >> 4) << 14))
 
-template <typename T, int MODE, int BCW, bool EXACT, bool WIDE, int BK, int NBUF, bool SPREAD>
+// LIST: as in assign_tiled_kernel. The listed rows lie anywhere in the table, so their loads take a
+// 64-bit address per lane.
+template <typename T, int MODE, int BCW, bool EXACT, bool WIDE, int BK, int NBUF, bool SPREAD, bool LIST = false>
 __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
     const T *__restrict__ X, const T *__restrict__ xnorm,
     const T *__restrict__ C, const T *__restrict__ cnorm,
     int *__restrict__ labels, T *__restrict__ mindist, T *__restrict__ D,
-    int64_t n, int64_t ldn, int d, int k, NearTies gate) {
-  if (gate.count && *gate.count <= gate.cap) return;
+    int64_t n, int64_t ldn, int d, int k, NearTies gate, RowBounds rb) {
+  static_assert(!LIST || (MODE == 0 && sizeof(T) == 8), "listed rows are labelled; float32 ones by the split kernel");
+  const ListedRows<LIST> at(rb, n);
+  if constexpr (LIST) {
+    n = at.count;
+    if ((int64_t)blockIdx.x * 128 >= n) return;
+  } else {
+    if (gate.count && *gate.count <= gate.cap) return;
+  }
   typedef Mfma<T> M;
   typedef DmaCfg<T, BCW, WIDE, BK, NBUF> Cfg;
   constexpr int MT = M::MT, KL = M::KL, NACC = M::NACC, VW = M::VW;
@@ -1940,16 +2084,18 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
   // wavefront is responsible for, as a byte offset from a base that is the same for the whole
   // workgroup (the block's first centroid, the workgroup's first row): the loads then take
   // their address as scalar base + 32-bit lane offset and cost no vector arithmetic.
-  unsigned aoff[A_TPW], boff[B_TPW];
+  typedef typename std::conditional<LIST, uint64_t, unsigned>::type row_off_t;
+  unsigned aoff[A_TPW];
+  row_off_t boff[B_TPW];
 #pragma unroll
   for (int t = 0; t < A_TPW; t++)
     aoff[t] = (unsigned)((((wave * A_TPW + t) * MT + r) * (size_t)d + g * VW) * sizeof(T));
 #pragma unroll
   for (int t = 0; t < B_TPW; t++) {
-    const int64_t row = min(row0 + (wave * B_TPW + t) * MT + r, n - 1);  // clamped: stays inside X
-    boff[t] = (unsigned)(((row - row0) * (int64_t)d + g * VW) * sizeof(T));
+    const int64_t row = at.row(min(row0 + (wave * B_TPW + t) * MT + r, n - 1));  // clamped: stays inside X
+    boff[t] = (row_off_t)(((row - (LIST ? 0 : row0)) * (int64_t)d + g * VW) * sizeof(T));
   }
-  const char *const xbase = reinterpret_cast<const char *>(X + row0 * (int64_t)d);
+  const char *const xbase = reinterpret_cast<const char *>(X + (LIST ? 0 : row0) * (int64_t)d);
   // the pipeline's fetch position: stage ist of block iblk goes to ring slot ibuf
   int iblk = 0, ist = 0, ibuf = 0, issued = 0;
   // The burst form takes the tiles one after the other, the NV vectors of a tile in a row:
@@ -2003,13 +2149,15 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
   T xxh[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; rt++)
-    xxh[rt] = (T)-0.5 * xnorm[min(row0 + (wr * RT + rt) * MT + r, n - 1)];
+    xxh[rt] = (T)-0.5 * xnorm[at.row(min(row0 + (wr * RT + rt) * MT + r, n - 1))];
   T best[RT];
   int bidx[RT];
   unsigned bkey[RT];
   int bblk[RT];
+  T second[RT];  // (LIST)
 #pragma unroll
   for (int rt = 0; rt < RT; rt++) {
+    second[rt] = pos_inf<T>();
     best[rt] = (T)0.5 * argmin_start<T>();  // the start value FLT_MAX on the accumulators' scale
     bidx[rt] = -1;
     bkey[rt] = 0x7EFFFFF0u;  // FLT_MAX / 2 with the index bits cleared
@@ -2140,6 +2288,7 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
 #pragma unroll
           for (int rt = 0; rt < RT; rt++) {
             const T a = acc[ct][rt][v] + fma((T)-0.5, cc, xxh[rt]);
+            if constexpr (LIST) second[rt] = second_of<T>(a, best[rt], second[rt]);
             if (fabs(a) < fabs(best[rt])) {
               best[rt] = a;
               loc[rt] = ct * NACC + v;
@@ -2177,18 +2326,24 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
       for (int off = MT; off < 64; off <<= 1) {
         const T ob = __shfl_xor(best[rt], off, 64);
         const int oi = __shfl_xor(bidx[rt], off, 64);
+        if constexpr (LIST) {
+          const T os = __shfl_xor(second[rt], off, 64);
+          second[rt] = fmin(fmax(best[rt], ob), fmin(second[rt], os));
+        }
         argmin_merge(best[rt], bidx[rt], ob, oi);
       }
     }
     __syncthreads();  // all waves are past their last LDS operand read
     T *mb = reinterpret_cast<T *>(smem_raw);                   // [BCW-1][BR]
-    int *mi = reinterpret_cast<int *>(mb + (BCW - 1) * BR);    // [BCW-1][BR]
+    T *ms = mb + (BCW - 1) * BR;                               // (LIST) [BCW-1][BR]
+    int *mi = reinterpret_cast<int *>(ms + (BCW - 1) * BR);    // [BCW-1][BR]
     if (wc > 0 && g == 0) {
 #pragma unroll
       for (int rt = 0; rt < RT; rt++) {
         const int lr = (wr * RT + rt) * MT + r;
         mb[(wc - 1) * BR + lr] = best[rt];
         mi[(wc - 1) * BR + lr] = bidx[rt];
+        if constexpr (LIST) ms[(wc - 1) * BR + lr] = second[rt];
       }
     }
     __syncthreads();
@@ -2197,12 +2352,19 @@ __global__ __launch_bounds__(2 * BCW * 64, 2) void assign_tiled_dma_kernel(
       for (int rt = 0; rt < RT; rt++) {
         const int lr = (wr * RT + rt) * MT + r;
 #pragma unroll
-        for (int w = 0; w < BCW - 1; w++)
+        for (int w = 0; w < BCW - 1; w++) {
+          if constexpr (LIST)
+            second[rt] = fmin(fmax(best[rt], mb[w * BR + lr]), fmin(second[rt], ms[w * BR + lr]));
           argmin_merge(best[rt], bidx[rt], mb[w * BR + lr], mi[w * BR + lr]);
-        const int64_t row = row0 + lr;
-        if (row < n) {
-          labels[row] = bidx[rt];
-          if (mindist) mindist[row] = (T)2 * best[rt];
+        }
+        if (row0 + lr < n) {
+          const int64_t row = at.row(row0 + lr);
+          at.label(labels, row, bidx[rt]);
+          if constexpr (LIST) {
+            if (at.limits)
+              rb.limit[row] = row_limit((float)(2 * best[rt]), (float)(2 * second[rt]), (float)(-2 * xxh[rt]),
+                                        bidx[rt] >= 0 ? rb.drift[bidx[rt]] : 0.0f, rb.noise, rb.grain);
+          } else if (mindist) mindist[row] = (T)2 * best[rt];
         }
       }
     }
@@ -2300,16 +2462,22 @@ __global__ __launch_bounds__(WG) void near_ties_kernel(const float *__restrict__
     }
   }
 }
+// changed (nullable): set where a label is not the one before.
 __global__ __launch_bounds__(WG) void near_ties_labels_kernel(int *__restrict__ labels, float *__restrict__ mindist,
-                                                             NearTies ties) {
-  if (*ties.count > ties.cap) return;
+                                                             NearTies ties, unsigned *__restrict__ changed) {
+  if (*ties.count > ties.cap) {  // (the launch behind labels all rows)
+    if (changed && blockIdx.x == 0 && threadIdx.x == 0) *changed = 1;
+    return;
+  }
   const int m = (int)*ties.count;
   for (int at = blockIdx.x * WG + threadIdx.x; at < m; at += gridDim.x * WG) {
     const unsigned long long key = ties.keys[at];
     const unsigned start = __float_as_uint(0.5f * argmin_start<float>()) & ties.mask;
     const unsigned bits = (unsigned)(key >> 32);
     const bool found = bits < start;  // (a NaN compares above)
-    labels[ties.rows[at]] = found ? (int)(unsigned)key : -1;
+    const int label = found ? (int)(unsigned)key : -1;
+    if (changed && labels[ties.rows[at]] != label) *changed = 1;
+    labels[ties.rows[at]] = label;
     if (mindist) mindist[ties.rows[at]] = 2.0f * __uint_as_float(found ? bits : start);
   }
 }
@@ -2444,7 +2612,7 @@ static int launch_rowstat_nw(hipStream_t s, const T *X, const T *xnorm, const T 
                              const T *cnorm, int *labels, T *mindist, int64_t n, int d,
                              int k, int num_cu, double *psums, int *pcounts, int *slots,
                              size_t lds, int c_off, int merge, bool exact, const StackShape &st,
-                             bool settle = false) {
+                             bool settle = false, const RowBounds *rb = nullptr) {
   const TieBound bound = settle_margin(d, settle);
   int ncopy = 1;
   // (the one workgroup of a CU; two 4-wave ones share its LDS. From 2048 rows a workgroup on: clearing
@@ -2475,11 +2643,15 @@ static int launch_rowstat_nw(hipStream_t s, const T *X, const T *xnorm, const T 
   const bool padvec = !vec && d >= Mfma<T>::VW;
 #define KM_RS_LAUNCH_X(LOAD, EXACT)                                                           \
   do {                                                                                        \
+    constexpr bool LISTS = FUSE && SPLIT == 6;                                                \
+    if (rb && !LISTS) return H2O4GPU_KMEANS_EARG;                                             \
     auto kern = assign_rowstat_kernel<T, DP, ROWT, LOAD, FUSE, NW, EXACT, SPLIT>;             \
+    if constexpr (LISTS)                                                                      \
+      if (rb) kern = assign_rowstat_kernel<T, DP, ROWT, LOAD, FUSE, NW, EXACT, SPLIT, true>;  \
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                    \
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), lds, s, X, xnorm, C, cnorm, \
                        labels, mindist, n, d, k, kp, psums, pcounts, c_off, merge, sets, kps, \
-                       kset, ncopy, bound);                                                   \
+                       kset, ncopy, bound, rb ? *rb : RowBounds());                           \
   } while (0)
   // the exact-compare form exists for the float32 assignment-only kernels
 #define KM_RS_LAUNCH(LOAD)                                       \
@@ -2533,14 +2705,15 @@ template <bool FUSE, int SPLIT>
 static int launch_rowstat_split(hipStream_t s, const float *X, const float *xnorm, const float *C,
                                 const float *cnorm, int *labels, float *mindist, int64_t n, int d,
                                 int k, int num_cu, double *psums, int *pcounts, int *slots,
-                                int c_off, int merge, const StackShape &st, bool settle) {
+                                int c_off, int merge, const StackShape &st, bool settle,
+                                const RowBounds *rb = nullptr) {
   const size_t lds = FUSE ? rowstat_fused_lds<float>(d, k, SPLIT) : rowstat_lds<float>(d, k, SPLIT);
 #define KM_SPLIT_CASE(DP, ROWT, NW)                                                              \
   case DP:                                                                                       \
     return launch_rowstat_nw<float, DP, ROWT, FUSE, NW, SPLIT>(s, X, xnorm, C, cnorm, labels,    \
                                                                mindist, n, d, k, num_cu, psums,  \
                                                                pcounts, slots, lds, c_off, merge, false, st, \
-                                                               settle)
+                                                               settle, rb)
   switch (rowstat_dp<float>(d)) {
     KM_SPLIT_CASE(16, 1, 16);
     KM_SPLIT_CASE(32, 1, 16);
@@ -2562,7 +2735,7 @@ struct RowstatDispatch<float, FUSE> {
                  const float *cnorm, int *labels, float *mindist, int64_t n, int d,
                  int k, int num_cu, double *psums, int *pcounts, int *slots, int c_off = 0,
                  int merge = 0, bool exact = false, const StackShape &st = StackShape(),
-                 int split = 0, bool settle = false) {
+                 int split = 0, bool settle = false, const RowBounds *rb = nullptr) {
     if (!exact) {
       split = rowstat_split<float>(split, d, k, FUSE);
       if (split == 9)
@@ -2570,8 +2743,9 @@ struct RowstatDispatch<float, FUSE> {
                                              psums, pcounts, slots, c_off, merge, st, false);
       if (split == 6)
         return launch_rowstat_split<FUSE, 6>(s, X, xnorm, C, cnorm, labels, mindist, n, d, k, num_cu,
-                                             psums, pcounts, slots, c_off, merge, st, settle);
+                                             psums, pcounts, slots, c_off, merge, st, settle, rb);
     }
+    if (rb) return H2O4GPU_KMEANS_EARG;  // (listed rows: the split kernels)
     switch (rowstat_dp<float>(d)) {
       KM_ROWSTAT_CASE(float, 8, 2);
       KM_ROWSTAT_CASE(float, 16, 2);
@@ -2748,7 +2922,7 @@ int launch_assign_accumulate(hipStream_t s, int variant, const T *X, const T *xn
 template <typename T, int MODE, int BCW, bool WIDE, int BK, int NBUF, bool SPREAD>
 static int launch_tiled_dma(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm,
                             int *labels, T *mindist, T *D, int64_t n, int64_t ldn, int d, int k,
-                            bool exact, const NearTies &gate) {
+                            bool exact, const NearTies &gate, const RowBounds *rb = nullptr) {
   typedef DmaCfg<T, BCW, WIDE, BK, NBUF> Cfg;
   const uintptr_t bits = reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(C) |
                          reinterpret_cast<uintptr_t>(cnorm);
@@ -2757,19 +2931,26 @@ static int launch_tiled_dma(hipStream_t s, const T *X, const T *xnorm, const T *
   const int64_t tiles = MODE == 1 ? row_tiles * ((k + Cfg::BC - 1) / Cfg::BC) : row_tiles;
   if (tiles > 2147483647ll) return H2O4GPU_KMEANS_EARG;
   const size_t lds = Cfg::LDS_BYTES;
-#define KM_DMA_X(EXACT)                                                                      \
+#define KM_DMA_X(...)                                                                        \
   do {                                                                                       \
-    auto kern = assign_tiled_dma_kernel<T, MODE, BCW, EXACT, WIDE, BK, NBUF, SPREAD>;        \
+    auto kern = assign_tiled_dma_kernel<T, MODE, BCW, __VA_ARGS__>;                          \
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                   \
     hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(Cfg::TPB), lds, s, X, xnorm, C,     \
-                       cnorm, labels, mindist, D, n, ldn, d, k, gate);                       \
+                       cnorm, labels, mindist, D, n, ldn, d, k, gate, rb ? *rb : RowBounds()); \
   } while (0)
+  if constexpr (sizeof(T) == 8 && MODE == 0) {
+    if (rb) {
+      KM_DMA_X(false, WIDE, BK, NBUF, SPREAD, true);
+      KM_HIP_TRY(hipGetLastError());
+      return 0;
+    }
+  }
   if (d >= 128) exact = true;  // as in launch_tiled_bcw
   if constexpr (MODE == 0 && sizeof(T) == 4) {
-    if (exact) KM_DMA_X(true);
-    else KM_DMA_X(false);
+    if (exact) KM_DMA_X(true, WIDE, BK, NBUF, SPREAD);
+    else KM_DMA_X(false, WIDE, BK, NBUF, SPREAD);
   } else {
-    KM_DMA_X(false);
+    KM_DMA_X(false, WIDE, BK, NBUF, SPREAD);
   }
 #undef KM_DMA_X
   KM_HIP_TRY(hipGetLastError());
@@ -2780,7 +2961,7 @@ template <typename T, int MODE, int BCW, bool WIDE = false, int SPLIT = 0, bool 
 static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *C,
                             const T *cnorm, int *labels, T *mindist, T *D, int64_t n,
                             int64_t ldn, int d, int k, bool exact, void *cparts = nullptr,
-                            bool direct = true, NearTies ties = NearTies()) {
+                            bool direct = true, NearTies ties = NearTies(), const RowBounds *rb = nullptr) {
   typedef TiledCfg<T, BCW, WIDE, SPLIT, XB> Cfg;
   const size_t lds = Cfg::LDS_BYTES;
   if constexpr (SPLIT != 0) {
@@ -2803,7 +2984,7 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
     int rc = 1;
     if constexpr (sizeof(T) == 8)
       rc = launch_tiled_dma<T, MODE, BCW, WIDE, 16, 2, false>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn,
-                                                              d, k, exact, ties);
+                                                              d, k, exact, ties, rb);
     else if constexpr (!WIDE)
       rc = launch_tiled_dma<T, MODE, BCW, WIDE, 32, 2, false>(s, X, xnorm, C, cnorm, labels, mindist, D, n, ldn,
                                                               d, k, exact, ties);
@@ -2820,10 +3001,16 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
   const bool tail = (d % Cfg::BK) != 0;
 #define KM_TILED_X(VEC, TAIL, EXACT)                                                         \
   do {                                                                                       \
-    auto kern = assign_tiled_kernel<T, MODE, VEC, TAIL, BCW, EXACT, WIDE, SPLIT, XB>;            \
+    /* (rows named by bounds: float32 with six products, float64) */                         \
+    constexpr bool LISTS = MODE == 0 && !XB && BCW == 2 && (sizeof(T) == 8 || SPLIT == 6);   \
+    auto kern = assign_tiled_kernel<T, MODE, VEC, TAIL, BCW, EXACT, WIDE, SPLIT, XB>;        \
+    if constexpr (LISTS)                                                                     \
+      if (rb) kern = assign_tiled_kernel<T, MODE, VEC, TAIL, BCW, EXACT, WIDE, SPLIT, XB, true>; \
+    if (rb && !LISTS) return H2O4GPU_KMEANS_EARG;                                            \
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds));                   \
     hipLaunchKernelGGL(kern, grid, dim3(Cfg::TPB), lds, s, X, xnorm, C, cnorm, labels,       \
-                       mindist, D, n, ldn, d, k, static_cast<const uintx4 *>(cparts), ties); \
+                       mindist, D, n, ldn, d, k, static_cast<const uintx4 *>(cparts), ties,  \
+                       rb ? *rb : RowBounds());                                              \
   } while (0)
   // From 128 features on the float32 argmin compares the distances themselves: the
   // epilogue is then about one per cent of the matrix work (2M x 256, k = 1024: 8.30 ->
@@ -2849,7 +3036,7 @@ static int launch_tiled_bcw(hipStream_t s, const T *X, const T *xnorm, const T *
     if (ties.rows) {
       hipLaunchKernelGGL(near_ties_kernel, dim3(512), dim3(WG), 0, s, X, xnorm, C, cnorm, d, k, ties);
       hipLaunchKernelGGL(near_ties_labels_kernel, dim3(std::min(64u, (ties.cap + WG - 1) / WG)), dim3(WG), 0, s,
-                         labels, mindist, ties);
+                         labels, mindist, ties, rb ? &rb->ctl->changed : (unsigned *)nullptr);
     }
   }
   KM_HIP_TRY(hipGetLastError());
@@ -3024,6 +3211,77 @@ int launch_assign(hipStream_t s, int variant, const T *X, const T *xnorm,
       return launch_longrow<T, false>(s, X, xnorm, C, cnorm, labels, mindist, n, d, k, num_cu, nullptr,
                                       nullptr, nullptr);
   }
+  return H2O4GPU_KMEANS_EARG;
+}
+
+// float32: the six products' kernels (rows of bfloat16 values keep theirs, which have no such form), with
+// room for parts and ties; float64: the 128-centroid block.
+template <typename T>
+bool bounded_assign_applies(int64_t n, int d, int k, int split, const SplitScratch &scratch) {
+  if (k <= 64 || k > MAX_BOUND_CENTROIDS || n > 2147483647 || pick_assign_variant<T>(ASSIGN_AUTO, n, d, k) != ASSIGN_TILED)
+    return false;
+  if (sizeof(T) == 8) return true;
+  return split == 6 && tiled_split<T>(split, d, k) == 6 && scratch.near_ties && scratch.ptr &&
+         scratch.bytes >= tiled_split_scratch_bytes<T>(split, d, k, n) && !(scratch.rows_bf16 && tiled_split_wide(k));
+}
+template bool bounded_assign_applies<float>(int64_t, int, int, int, const SplitScratch &);
+template bool bounded_assign_applies<double>(int64_t, int, int, int, const SplitScratch &);
+
+template <typename T>
+int launch_bounded_assign(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm, int *labels,
+                          int64_t n, int d, int k, SplitScratch scratch, const RowBounds &bounds) {
+  if (!bounded_assign_applies<T>(n, d, k, 6, scratch)) return H2O4GPU_KMEANS_EARG;
+  const bool direct = !scratch.through_registers;
+  RowBounds rb = bounds;
+  rb.noise = bound_noise<T>(d);
+  rb.grain = sizeof(T) == 4 && d < 128 ? 8e-6f : 0.0f;  // (keys, see launch_tiled_bcw)
+  T *const none = nullptr;
+  if constexpr (sizeof(T) == 4) {
+    void *const parts = static_cast<unsigned char *>(scratch.ptr) + 256;
+    const NearTies ties = near_ties_at(scratch.ptr, n, d, k, false);
+    if (tiled_split_wide(k))
+      KM_TRY((launch_tiled_bcw<T, 0, 2, true, 6>(s, X, xnorm, C, cnorm, labels, none, none, n, n, d, k, false, parts,
+                                                 true, ties, &rb)));
+    else
+      KM_TRY((launch_tiled_bcw<T, 0, 2, false, 6>(s, X, xnorm, C, cnorm, labels, none, none, n, n, d, k, false, parts,
+                                                  true, ties, &rb)));
+    // (more ties than the list holds: all rows, by the float32 instructions. Their limits stand: those of
+    // near ties are passed already.)
+    return launch_tiled_plain<T, 0>(s, X, xnorm, C, cnorm, labels, none, none, n, n, d, k, false, direct, ties);
+  } else {
+    return launch_tiled_bcw<T, 0, 2>(s, X, xnorm, C, cnorm, labels, none, none, n, n, d, k, false, nullptr, direct,
+                                     NearTies(), &rb);
+  }
+}
+template int launch_bounded_assign<float>(hipStream_t, const float *, const float *, const float *, const float *, int *,
+                                          int64_t, int, int, SplitScratch, const RowBounds &);
+template int launch_bounded_assign<double>(hipStream_t, const double *, const double *, const double *, const double *,
+                                           int *, int64_t, int, int, SplitScratch, const RowBounds &);
+
+template <>
+bool bounded_accumulate_applies<float>(int64_t n, int d, int k, int split, int num_cu) {
+  if (split != 6 || k > MAX_BOUND_CENTROIDS || n > 2147483647 || fused_slots<float>(ASSIGN_AUTO, n, d, k, num_cu) <= 0 ||
+      pick_assign_variant<float>(ASSIGN_AUTO, n, d, k) != ASSIGN_ROWSTAT)
+    return false;
+  return !shortrow_applies(d, k, true) && rowstat_split<float>(split, d, k, true) == 6;
+}
+template <>
+bool bounded_accumulate_applies<double>(int64_t, int, int, int, int) { return false; }
+
+template <>
+int launch_bounded_accumulate<float>(hipStream_t s, const float *X, const float *xnorm, const float *C, int *labels,
+                                     int64_t n, int d, int k, int num_cu, double *psums, int *pcounts, int *slots,
+                                     const RowBounds &bounds) {
+  if (!bounded_accumulate_applies<float>(n, d, k, 6, num_cu)) return H2O4GPU_KMEANS_EARG;
+  RowBounds rb = bounds;
+  rb.noise = bound_noise<float>(d);
+  rb.grain = 8e-6f;  // (keys)
+  return RowstatDispatch<float, true>::run(s, X, xnorm, C, nullptr, labels, nullptr, n, d, k, num_cu, psums, pcounts,
+                                           slots, 0, 0, false, StackShape(), 6, true, &rb);
+}
+template <>
+int launch_bounded_accumulate<double>(hipStream_t, const double *, const double *, const double *, int *, int64_t, int,
+                                      int, int, double *, int *, int *, const RowBounds &) {
   return H2O4GPU_KMEANS_EARG;
 }
 

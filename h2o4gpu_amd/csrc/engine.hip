@@ -241,6 +241,7 @@ struct h2o4gpu_kmeans_handle {
   int opt_transform_buffers = 2;  // sets of device buffers of a transform in several batches
   int opt_seed_matrix = 1;  // k-means||: distances between candidates as one matrix (0: a kernel per pick)
   int opt_tiled_direct = 1;  // tiled kernels: operands by direct-to-LDS loads where the shape allows
+  int opt_bounds = 1;  // fits: rows whose label cannot have changed are not measured (2: however little there is to measure)
   int opt_transform_batch_mb = 4096;  // device buffer of transform_host's output, per batch of rows
   int last_variant = ASSIGN_AUTO;
 
@@ -288,6 +289,7 @@ struct h2o4gpu_kmeans_handle {
   virtual int transform_host(size_t rows, const void *X, void *dist) = 0;
   virtual int transform_resident(void *d_dist) = 0;
   virtual int release() = 0;
+  virtual int rows_measured(long long *rows) = 0;
   // bfloat16 products per feature pair of the kernel a Lloyd step labels the rows with (0: none)
   virtual int step_products() const = 0;
   int kk() const { return sets > 1 ? kset : k; }  // centroids of one set
@@ -844,9 +846,9 @@ struct Engine : h2o4gpu_kmeans_handle {
       e = nullptr;
     }
     if (own_X && X) (void)hipFree(X);
-    for (void *p : {(void *)slab, (void *)work_slab, (void *)d_split})
+    for (void *p : {(void *)slab, (void *)work_slab, (void *)d_split, (void *)bound_slab})
       if (p) (void)hipFree(p);
-    slab = work_slab = d_split = nullptr;
+    slab = work_slab = d_split = bound_slab = nullptr;
     if (stream) (void)hipStreamDestroy(stream);
     stream = nullptr;
     return 0;
@@ -1391,16 +1393,17 @@ struct Engine : h2o4gpu_kmeans_handle {
     return 0;
   }
 
-  int update_async(bool want_shift = true, T *shift_host = nullptr) {
+  // changed (nullable, device): 0 when the labels are those of the update before
+  int update_async(bool want_shift = true, T *shift_host = nullptr, const unsigned *changed = nullptr) {
     KM_TRY(ensure_work());
     if (use_buckets && opt_buckets) {
       PROFILED("accumulate", launch_bucketed_accumulate<T>(stream, X, labels, order, order_label,
                                                            bucket_offsets, bucket_hist, bucket_seg,
                                                            bucket_total, bucket_partials, psums,
-                                                           pcounts, n, d, k));
+                                                           pcounts, n, d, k, changed));
       return finish_update(1, want_shift, shift_host);
     }
-    PROFILED("accumulate", launch_accumulate<T>(stream, plan, X, labels, psums, pcounts, n, d, k));
+    PROFILED("accumulate", launch_accumulate<T>(stream, plan, X, labels, psums, pcounts, n, d, k, changed));
     return finish_update(plan.row_blocks, want_shift, shift_host);
   }
 
@@ -1429,10 +1432,95 @@ struct Engine : h2o4gpu_kmeans_handle {
     return update_async(want_shift, shift_host);
   }
 
+  // Steps that measure only the rows whose label may have changed (row_bounds.h). The first of them
+  // measures all rows and leaves their limits.
+  static const int BOUNDS_FROM = 2;         // by then most centroids have found their place
+  static const int BOUNDS_ITERATIONS = 8;   // of a fit, at least
+  unsigned char *bound_slab = nullptr;
+  float *limit = nullptr, *moves = nullptr, *drift_float = nullptr;
+  int *found = nullptr, *found_counts = nullptr, *listed = nullptr;
+  double *drift[2] = {nullptr, nullptr};
+  BoundControl *bound_ctl[2] = {nullptr, nullptr};
+  int bound_cur = 0, bound_steps = 0;
+  bool bound_fused = false;  // the fused step
+  double *run_sums = nullptr;  // (fused) the sums behind the centroids, and the rows in them
+  int *run_counts[2] = {nullptr, nullptr};
+  bool bounds_begin(int max_iterations) {
+    bound_steps = 0;
+    if (!opt_bounds || (opt_bounds == 1 && max_iterations < BOUNDS_ITERATIONS) || sets > 1 || opt_assign != ASSIGN_AUTO || opt_exact ||
+        opt_split != SPLIT_DEFAULT)
+      return false;
+    // Three more launches and eight bytes a row are to be had for less than a tenth of the step.
+    if (opt_bounds == 1 && 2.0 * (double)n * k * d < (sizeof(T) == 4 ? 2e10 : 4e9)) return false;
+    bound_fused = opt_fuse && bounded_accumulate_applies<T>(n, d, k, split_for(SPLIT_FUSED, k), num_cu);
+    const int split = split_for(SPLIT_ASSIGN, k);
+    if (!bound_fused && !bounded_assign_applies<T>(n, d, k, split, split_scratch(split, k, true, n))) return false;
+    if (!bound_slab) {
+      std::vector<Want> list;
+      want(list, &limit, n);
+      want(list, &found, n);
+      want(list, &listed, n);
+      want(list, &found_counts, bound_segments(n));
+      want(list, &moves, k);
+      want(list, &drift_float, k);
+      for (int i = 0; i < 2; i++) {
+        want(list, &drift[i], k);
+        want(list, &run_counts[i], k);
+        want(list, &bound_ctl[i], 1);
+      }
+      want(list, &run_sums, (size_t)k * d);
+      if (allocate(list, &bound_slab) != 0) return false;  // (every row is measured, then)
+    }
+    return true;
+  }
+  int bounded_step(bool first, bool want_shift, T *shift_host = nullptr) {
+    KM_TRY(ensure_work());
+    if (!bound_fused) KM_TRY(ensure_cnorm());
+    const int was = bound_cur;
+    bound_cur ^= 1;
+    bound_steps++;
+    PROFILED("bounds", launch_bounds<T>(stream, C[cur ^ 1], C[cur], labels, limit, n, d, k, moves,
+                                        first ? (const double *)nullptr : drift[was], drift[bound_cur], drift_float, found,
+                                        found_counts, listed, bound_ctl[was], bound_ctl[bound_cur]));
+    RowBounds rb;
+    rb.rows = listed;
+    rb.ctl = bound_ctl[bound_cur];
+    rb.limit = limit;
+    rb.drift = drift_float;
+    if (bound_fused) {
+      int slots = 0;
+      PROFILED("assign_accumulate", launch_bounded_accumulate<T>(stream, X, xnorm, C[cur], labels, n, d, k, num_cu, psums,
+                                                                 pcounts, &slots, rb));
+      have_mindist = false;
+      RunningSums run;
+      run.sums = run_sums;
+      run.counts_old = run_counts[was];
+      run.counts_new = run_counts[bound_cur];
+      run.ctl = rb.ctl;
+      return finish_update(slots, want_shift, shift_host, run);
+    }
+    const int split = split_for(SPLIT_ASSIGN, k);
+    PROFILED("assign", launch_bounded_assign<T>(stream, X, xnorm, C[cur], cnorm, labels, n, d, k,
+                                                split_scratch(split, k, true, n), rb));
+    have_mindist = false;
+    return update_async(want_shift, shift_host, &rb.ctl->changed);
+  }
+
+  int rows_measured(long long *rows) override {
+    KM_HIP_TRY(hipSetDevice(dev));
+    *rows = -1;
+    if (bound_steps == 0) return 0;
+    BoundControl ctl;
+    KM_HIP_TRY(hipMemcpyAsync(&ctl, bound_ctl[bound_cur], sizeof(ctl), hipMemcpyDeviceToHost, stream));
+    KM_HIP_TRY(hipStreamSynchronize(stream));
+    *rows = ctl.full ? (long long)n : (long long)ctl.count;
+    return 0;
+  }
+
   // want_shift: the scalar sum((old - new)^2) of this step is left in shift2 (and in shift_host).
   // The norms of the new centroids are made by whoever needs them (ensure_cnorm): the fused kernels
   // do not.
-  int finish_update(int slots, bool want_shift, T *shift_host = nullptr) {
+  int finish_update(int slots, bool want_shift, T *shift_host = nullptr, RunningSums run = RunningSums()) {
     int nsp = 0;
     if (sets > 1 && want_shift) {
       // per-set convergence: frozen sets keep their centroids; every set's squared shift is
@@ -1450,7 +1538,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     PROFILED("finalize", launch_finalize<T>(stream, slots, psums, pcounts, C[cur], C[cur ^ 1],
                                             counts, shift_partials, &nsp, d, k, nullptr, 1,
-                                            want_shift ? finalize_done : (unsigned *)nullptr, shift2, shift_host));
+                                            want_shift ? finalize_done : (unsigned *)nullptr, shift2, shift_host, run));
     cnorm_stale = true;
     cur ^= 1;
     return 0;
@@ -1480,6 +1568,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     if (!have_data || !have_centroids) return H2O4GPU_KMEANS_ESTATE;
     maybe_install_signal_handlers();
     int updates = 0;
+    const bool bounded = bounds_begin(max_iterations);
     if (max_iterations <= 0) {
       // The reference's loop then never runs, its final relabel included, and the labels it
       // returns are the zeros its vector was created with (kmeans_impl.h:109-232,
@@ -1490,11 +1579,13 @@ struct Engine : h2o4gpu_kmeans_handle {
     } else if (sets > 1) {
       KM_TRY(fit_stacked(max_iterations, threshold, &updates));
     } else if (threshold > 0 && max_iterations > 0) {
-      KM_TRY(fit_with_threshold(max_iterations, threshold, &updates));
+      KM_TRY(fit_with_threshold(max_iterations, threshold, bounded, &updates));
     } else {
       for (int i = 0; i < max_iterations; i++) {
         log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
-        KM_TRY(step_async(false, false));  // (the final relabel below leaves the minimum distances)
+        // (the final relabel below leaves the minimum distances)
+        if (bounded && i >= BOUNDS_FROM) KM_TRY(bounded_step(i == BOUNDS_FROM, false));
+        else KM_TRY(step_async(false, false));
         updates++;
         bool done = false;
         if (g_stop_flag) {
@@ -1605,7 +1696,8 @@ struct Engine : h2o4gpu_kmeans_handle {
   // back and the centroid norms recomputed.
   T *host_shift = nullptr;            // [2] pinned
   hipEvent_t shift_ready[2] = {nullptr, nullptr};
-  int fit_with_threshold(int max_iterations, double threshold, int *updates_out) {
+  // (bounded: a queued iteration that measured some of the rows only is followed by a relabel of all.)
+  int fit_with_threshold(int max_iterations, double threshold, bool bounded, int *updates_out) {
     if (!host_shift) {
       // (a kernel stores the scalar there: coherent memory, whatever HIP_HOST_COHERENT says, and events
       // that release to the system)
@@ -1616,7 +1708,8 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     auto queue_iteration = [&](int i) -> int {
       log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
-      KM_TRY(step_async(true, true, host_shift + (i & 1)));
+      if (bounded && i >= BOUNDS_FROM) KM_TRY(bounded_step(i == BOUNDS_FROM, true, host_shift + (i & 1)));
+      else KM_TRY(step_async(true, true, host_shift + (i & 1)));
       KM_HIP_TRY(hipEventRecord(shift_ready[i & 1], stream));
       return 0;
     };
@@ -1640,6 +1733,7 @@ struct Engine : h2o4gpu_kmeans_handle {
         cur ^= 1;
         PROFILED("row_norms", launch_row_norms<T>(stream, C[cur], cnorm, k, d));
         cnorm_stale = false;
+        if (!have_mindist) KM_TRY(assign());
       } else {
         KM_TRY(assign());
       }
@@ -2450,6 +2544,11 @@ KM_API int h2o4gpu_kmeans_set_option(h2o4gpu_kmeans_handle *h, const char *name,
     h->opt_transform_buffers = value;
     return 0;
   }
+  if (strcmp(name, "bounds") == 0) {
+    if (value < 0 || value > 2) return H2O4GPU_KMEANS_EARG;
+    h->opt_bounds = value;
+    return 0;
+  }
   if (strcmp(name, "tiled_direct") == 0) {
     if (value != 0 && value != 1) return H2O4GPU_KMEANS_EARG;
     h->opt_tiled_direct = value;
@@ -2514,6 +2613,10 @@ KM_API const char *h2o4gpu_kmeans_assign_variant(h2o4gpu_kmeans_handle *h) {
 }
 
 KM_API int h2o4gpu_kmeans_step_products(h2o4gpu_kmeans_handle *h) { return h ? h->step_products() : 0; }
+
+KM_API int h2o4gpu_kmeans_rows_measured(h2o4gpu_kmeans_handle *h, long long *rows) {
+  return h && rows ? h->rows_measured(rows) : H2O4GPU_KMEANS_EARG;
+}
 
 KM_API int h2o4gpu_kmeans_bandwidth_probe(int gpu_id, int kind, size_t bytes, int reps, float *ms) {
   if (!ms || reps < 1 || bytes < 16 || kind < 0 || kind > 3) return H2O4GPU_KMEANS_EARG;

@@ -8,6 +8,7 @@
 #include <stdio.h>
 
 #include "../../include/h2o4gpu_kmeans.h"
+#include "row_bounds.h"
 
 namespace kmhip {
 
@@ -125,6 +126,31 @@ int launch_assign(hipStream_t s, int variant, const T *X, const T *xnorm,
                   const T *C, const T *cnorm, int *labels, T *mindist,
                   int64_t n, int d, int k, int num_cu, int *used, bool exact = false,
                   StackShape st = StackShape(), int split = 0, SplitScratch split_scratch = SplitScratch());
+// The assignment pass of a loop that keeps bounds (row_bounds.h): the rows rb names get their label and
+// their limit (where the next step will look at it), and rb.ctl->changed is set where a label is not the one before. No minimum distances.
+// Tiled shapes: float32 with six products (and their scratch, near ties settled), float64.
+template <typename T>
+bool bounded_assign_applies(int64_t n, int d, int k, int split, const SplitScratch &scratch);
+template <typename T>
+int launch_bounded_assign(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm, int *labels,
+                          int64_t n, int d, int k, SplitScratch scratch, const RowBounds &rb);
+// The fused step of such a loop (row-stationary float32 shapes with six products): labels and limits as
+// above; partial sums and counts of all rows where the control block says that all are measured, of
+// what the new labels change otherwise, for launch_finalize with RunningSums.
+template <typename T>
+bool bounded_accumulate_applies(int64_t n, int d, int k, int split, int num_cu);
+template <typename T>
+int launch_bounded_accumulate(hipStream_t s, const T *X, const T *xnorm, const T *C, int *labels, int64_t n, int d,
+                              int k, int num_cu, double *psums, int *pcounts, int *slots, const RowBounds &rb);
+// The step before such a pass: how far the centroids have moved, the drift that leaves (drift_old ->
+// drift_new; null: zeros, and every row is measured), the rows whose limit it has passed and the control block.
+// drift_float: drift_new, for the pass. found, listed: [n] int32 each; found_counts: [bound_segments(n)]; moves: [k].
+static const int MAX_BOUND_CENTROIDS = 8192;
+int bound_segments(int64_t n);
+template <typename T>
+int launch_bounds(hipStream_t s, const T *c_old, const T *c_new, const int *labels, const float *limit, int64_t n,
+                  int d, int k, float *moves, const double *drift_old, double *drift_new, float *drift_float, int *found,
+                  int *found_counts, int *listed, const BoundControl *ctl_old, BoundControl *ctl_new);
 // What launch_assign (variant ASSIGN_AUTO) needs beside the rows and the k centroids for a shape:
 enum AssignInputs {
   ASSIGN_FROM_ROWS,       // nothing: xnorm and cnorm may be null, C need not be padded
@@ -219,13 +245,14 @@ UpdatePlan plan_update(int64_t n, int d, int k, int num_cu);
 template <typename T>
 int launch_accumulate(hipStream_t s, const UpdatePlan &p, const T *X,
                       const int *labels, double *psums, int *pcounts, int64_t n,
-                      int d, int k);
+                      int d, int k, const unsigned *changed = nullptr);
 // Pass 1 for shapes whose sums need many LDS chunks: the rows are ordered by label with a
 // stable counting sort (order / order_label: [n] int32 each, offsets: [k] int32,
 // block_hist: [bucket_blocks(n, k)][k] int32, seg_hist: [32][k] int32) and summed in fixed
 // windows of the ordered rows (partials: [bucket_partial_slots(n, k)][d] double) into
 // gsum [k][d] double; counts receives the bucket sizes. Run-to-run reproducible for
-// both precisions. The result is consumed by launch_finalize with slots = 1.
+// both precisions. The result is consumed by launch_finalize with slots = 1. changed (nullable, device): 0
+// says that the labels are those of the pass before, whose gsum and counts are then left as they are.
 bool bucketed_update_applies(int k_chunks, int64_t n, int k, int d, size_t elem);
 int bucket_blocks(int64_t n, int k);
 size_t bucket_partial_slots(int64_t n, int k);
@@ -233,7 +260,7 @@ template <typename T>
 int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int *order,
                                int *order_label, int *offsets, int *block_hist, int *seg_hist,
                                int *total, double *partials, double *gsum, int *counts, int64_t n,
-                               int d, int k);
+                               int d, int k, const unsigned *changed = nullptr);
 
 // Pass 2: fixed-order reduction of the partials, empty clusters keep the old
 // centroid, mean = sum * (1/count), per-block partial of sum((old-new)^2).
@@ -248,12 +275,21 @@ static inline int max_shift_partials(int d, int k) {
   const int64_t kd = (int64_t)k * d;
   return (int)(kd <= FINALIZE_NARROW_KD ? (kd + 3) / 4 : (kd + 31) / 32);
 }
+// run (launch_bounded_accumulate): the partials are changes to sums kept here, unless its control block
+// says that all rows were measured; slots is what a launch over all rows writes.
+struct RunningSums {
+  double *sums = nullptr;           // [k][d], updated
+  const int *counts_old = nullptr;  // [k]
+  int *counts_new = nullptr;        // [k], another buffer
+  const BoundControl *ctl = nullptr;
+};
+static const int BOUND_TILE_ROWS = 32;  // listed rows a workgroup takes at a time: fewer tiles, fewer slots written
 template <typename T>
 int launch_finalize(hipStream_t s, int slots, const double *psums,
                     const int *pcounts, const T *c_old, T *c_new, int *counts,
                     T *shift_partials, int *n_shift_partials, int d, int k,
                     const int *frozen = nullptr, int kps = 1, unsigned *done = nullptr,
-                    T *shift2 = nullptr, T *shift_host = nullptr);
+                    T *shift2 = nullptr, T *shift_host = nullptr, RunningSums run = RunningSums());
 // Pass 3: cnorm of the new centroids and the fixed-order sum of the shift
 // partials into *shift2.
 template <typename T>

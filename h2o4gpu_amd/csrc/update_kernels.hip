@@ -344,7 +344,8 @@ template <typename T, int VEC, bool RAGGED, int TPB>
 __global__ __launch_bounds__(TPB) void accumulate_kernel(
     const T *__restrict__ X, const int *__restrict__ labels,
     double *__restrict__ psums, int *__restrict__ pcounts, int64_t n, int d, int k,
-    int kc, int64_t rows_per_block, int lpr, int sd) {
+    int kc, int64_t rows_per_block, int lpr, int sd, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double *sums = reinterpret_cast<double *>(smem_raw);         // [kc][sd]
   int *cnt = reinterpret_cast<int *>(sums + (size_t)kc * sd);  // [kc]
@@ -476,7 +477,7 @@ UpdatePlan plan_update(int64_t n, int d, int k, int num_cu) {
 template <typename T, int VEC, bool RAGGED>
 static int launch_accumulate_vec(hipStream_t s, const UpdatePlan &p, const T *X,
                                  const int *labels, double *psums, int *pcounts,
-                                 int64_t n, int d, int k) {
+                                 int64_t n, int d, int k, const unsigned *changed) {
   const int64_t rows_per_block = ((n + p.row_blocks - 1) / p.row_blocks + 63) / 64 * 64;
   int groups = (d + VEC - 1) / VEC;  // lanes wanted per row
   int lpr = 1;
@@ -487,7 +488,7 @@ static int launch_accumulate_vec(hipStream_t s, const UpdatePlan &p, const T *X,
     auto kern = accumulate_kernel<T, VEC, RAGGED, TPB>;                                         \
     KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(kern), p.lds_bytes));              \
     hipLaunchKernelGGL(kern, dim3(p.row_blocks, p.k_chunks), dim3(TPB), p.lds_bytes, s, X,      \
-                       labels, psums, pcounts, n, d, k, p.kc, rows_per_block, lpr, p.sd);       \
+                       labels, psums, pcounts, n, d, k, p.kc, rows_per_block, lpr, p.sd, changed);       \
   } while (0)
   if (p.threads == 1024) KM_ACC_LAUNCH(1024);
   else KM_ACC_LAUNCH(256);
@@ -501,20 +502,20 @@ static int launch_accumulate_vec(hipStream_t s, const UpdatePlan &p, const T *X,
 template <>
 int launch_accumulate<float>(hipStream_t s, const UpdatePlan &p, const float *X,
                              const int *labels, double *psums, int *pcounts,
-                             int64_t n, int d, int k) {
-  if (d >= 4 && d % 4 == 0) return launch_accumulate_vec<float, 4, false>(s, p, X, labels, psums, pcounts, n, d, k);
-  if (d >= 4) return launch_accumulate_vec<float, 4, true>(s, p, X, labels, psums, pcounts, n, d, k);
-  if (d == 2) return launch_accumulate_vec<float, 2, false>(s, p, X, labels, psums, pcounts, n, d, k);
-  if (d == 3) return launch_accumulate_vec<float, 2, true>(s, p, X, labels, psums, pcounts, n, d, k);
-  return launch_accumulate_vec<float, 1, false>(s, p, X, labels, psums, pcounts, n, d, k);
+                             int64_t n, int d, int k, const unsigned *changed) {
+  if (d >= 4 && d % 4 == 0) return launch_accumulate_vec<float, 4, false>(s, p, X, labels, psums, pcounts, n, d, k, changed);
+  if (d >= 4) return launch_accumulate_vec<float, 4, true>(s, p, X, labels, psums, pcounts, n, d, k, changed);
+  if (d == 2) return launch_accumulate_vec<float, 2, false>(s, p, X, labels, psums, pcounts, n, d, k, changed);
+  if (d == 3) return launch_accumulate_vec<float, 2, true>(s, p, X, labels, psums, pcounts, n, d, k, changed);
+  return launch_accumulate_vec<float, 1, false>(s, p, X, labels, psums, pcounts, n, d, k, changed);
 }
 template <>
 int launch_accumulate<double>(hipStream_t s, const UpdatePlan &p, const double *X,
                               const int *labels, double *psums, int *pcounts,
-                              int64_t n, int d, int k) {
-  if (d >= 2 && d % 2 == 0) return launch_accumulate_vec<double, 2, false>(s, p, X, labels, psums, pcounts, n, d, k);
-  if (d >= 2) return launch_accumulate_vec<double, 2, true>(s, p, X, labels, psums, pcounts, n, d, k);
-  return launch_accumulate_vec<double, 1, false>(s, p, X, labels, psums, pcounts, n, d, k);
+                              int64_t n, int d, int k, const unsigned *changed) {
+  if (d >= 2 && d % 2 == 0) return launch_accumulate_vec<double, 2, false>(s, p, X, labels, psums, pcounts, n, d, k, changed);
+  if (d >= 2) return launch_accumulate_vec<double, 2, true>(s, p, X, labels, psums, pcounts, n, d, k, changed);
+  return launch_accumulate_vec<double, 1, false>(s, p, X, labels, psums, pcounts, n, d, k, changed);
 }
 
 // ---------------------------------------------------------------------------
@@ -572,7 +573,8 @@ size_t bucket_partial_slots(int64_t n, int k) { return (size_t)(n / bucket_windo
 
 __global__ __launch_bounds__(WG) void bucket_hist_kernel(const int *__restrict__ labels,
                                                         int *__restrict__ bh, int64_t n, int k,
-                                                        int64_t rpb) {
+                                                        int64_t rpb, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   extern __shared__ int hist[];  // [k]
   const int tid = threadIdx.x;
   for (int c = tid; c < k; c += WG) hist[c] = 0;
@@ -591,7 +593,8 @@ __global__ __launch_bounds__(WG) void bucket_hist_kernel(const int *__restrict__
 // Level 1 of the scan over blocks: seg[s][c] = rows of label c in the blocks of segment s.
 __global__ __launch_bounds__(WG) void bucket_seg_kernel(const int *__restrict__ bh,
                                                        int *__restrict__ seg, int nb, int k,
-                                                       int per_seg) {
+                                                       int per_seg, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   const int c = blockIdx.x * WG + threadIdx.x;
   if (c >= k) return;
   const int b0 = blockIdx.y * per_seg, b1 = min(nb, b0 + per_seg);
@@ -610,7 +613,8 @@ __global__ __launch_bounds__(WG) void bucket_seg_kernel(const int *__restrict__ 
 __global__ __launch_bounds__(WG) void bucket_block_scan_kernel(int *__restrict__ bh,
                                                               const int *__restrict__ seg,
                                                               int *__restrict__ counts, int nb,
-                                                              int k, int per_seg) {
+                                                              int k, int per_seg, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   const int c = blockIdx.x * WG + threadIdx.x;
   if (c >= k) return;
   int run = 0;
@@ -637,7 +641,8 @@ __global__ __launch_bounds__(WG) void bucket_block_scan_kernel(int *__restrict__
 // offsets[c] = sum of counts[0..c), *total = sum of all; single workgroup.
 __global__ __launch_bounds__(WG) void bucket_scan_kernel(const int *__restrict__ counts,
                                                         int *__restrict__ offsets,
-                                                        int *__restrict__ total, int k) {
+                                                        int *__restrict__ total, int k, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   __shared__ int part[WG];
   const int tid = threadIdx.x;
   const int per = (k + WG - 1) / WG;
@@ -667,7 +672,8 @@ __global__ __launch_bounds__(WG) void bucket_scan_kernel(const int *__restrict__
 // [r0 + w*q, r0 + (w+1)*q) of the block, q = rpb / NWB, and its own counters wh[w][k].
 __global__ void bucket_scatter_kernel(const int *__restrict__ labels, const int *__restrict__ bh,
                                       const int *__restrict__ offsets, int *__restrict__ order,
-                                      int *__restrict__ order_label, int64_t n, int k, int64_t rpb) {
+                                      int *__restrict__ order_label, int64_t n, int k, int64_t rpb, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   extern __shared__ int wh[];  // [NWB][k]
   const int tid = threadIdx.x, tpb = blockDim.x;
   const int nwb = tpb >> 6, wave = tid >> 6, lane = tid & 63;
@@ -732,7 +738,8 @@ template <typename T, int VEC, int NVEC>
 __global__ __launch_bounds__(WG) void window_sum_kernel(
     const T *__restrict__ X, const int *__restrict__ order,
     const int *__restrict__ order_label, double *__restrict__ P,
-    const int *__restrict__ total, int d, int wm) {
+    const int *__restrict__ total, int d, int wm, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   const int64_t m = *total;
   const int lane = threadIdx.x & 63;
   const int64_t win = (int64_t)blockIdx.x * (WG / 64) + (threadIdx.x >> 6);
@@ -820,7 +827,8 @@ __global__ __launch_bounds__(WG) void window_sum_kernel(
 __global__ __launch_bounds__(WG) void bucket_sum_kernel(const double *__restrict__ P,
                                                        const int *__restrict__ offsets,
                                                        const int *__restrict__ counts,
-                                                       double *__restrict__ gsum, int d, int wpos) {
+                                                       double *__restrict__ gsum, int d, int wpos, const unsigned *changed) {
+  if (changed && *changed == 0) return;
   __shared__ double part[4][64];
   const int c = blockIdx.x;
   const int f = threadIdx.x & 63, strand = threadIdx.x >> 6;
@@ -869,7 +877,7 @@ template <typename T>
 int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int *order,
                                int *order_label, int *offsets, int *block_hist, int *seg_hist,
                                int *total, double *partials, double *gsum, int *counts, int64_t n,
-                               int d, int k) {
+                               int d, int k, const unsigned *changed) {
   const int64_t rpb = bucket_rows_per_block(n, k);
   const int nb = bucket_blocks(n, k);
   const int per_seg = (nb + BUCKET_SEGS - 1) / BUCKET_SEGS;
@@ -878,14 +886,14 @@ int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int
   KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(bucket_hist_kernel), lds1));
   KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(bucket_scatter_kernel), lds2));
   const unsigned kblocks = (unsigned)((k + WG - 1) / WG);
-  hipLaunchKernelGGL(bucket_hist_kernel, dim3(nb), dim3(WG), lds1, s, labels, block_hist, n, k, rpb);
+  hipLaunchKernelGGL(bucket_hist_kernel, dim3(nb), dim3(WG), lds1, s, labels, block_hist, n, k, rpb, changed);
   hipLaunchKernelGGL(bucket_seg_kernel, dim3(kblocks, segs), dim3(WG), 0, s, block_hist, seg_hist, nb, k,
-                     per_seg);
+                     per_seg, changed);
   hipLaunchKernelGGL(bucket_block_scan_kernel, dim3(kblocks, segs), dim3(WG), 0, s, block_hist, seg_hist,
-                     counts, nb, k, per_seg);
-  hipLaunchKernelGGL(bucket_scan_kernel, dim3(1), dim3(WG), 0, s, counts, offsets, total, k);
+                     counts, nb, k, per_seg, changed);
+  hipLaunchKernelGGL(bucket_scan_kernel, dim3(1), dim3(WG), 0, s, counts, offsets, total, k, changed);
   hipLaunchKernelGGL(bucket_scatter_kernel, dim3(nb), dim3(bucket_waves(k) * 64), lds2, s, labels,
-                     block_hist, offsets, order, order_label, n, k, rpb);
+                     block_hist, offsets, order, order_label, n, k, rpb, changed);
   // rows with a label outside [0, k) are not bucketed, so the ordered rows may be fewer
   // than n: the grid covers n positions and every wavefront bounds itself by the
   // device-side total
@@ -895,7 +903,7 @@ int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int
   // 16-byte loads for any d that holds a whole vector (rows need element alignment only)
 #define KM_SEG(VEC, NVEC)                                                                  \
   hipLaunchKernelGGL((window_sum_kernel<T, VEC, NVEC>), dim3(sblocks), dim3(WG), 0, s, X, \
-                     order, order_label, partials, total, d, wm)
+                     order, order_label, partials, total, d, wm, changed)
   if constexpr (sizeof(T) == 4) {
     if (d >= 4) {
       if (d <= 256) KM_SEG(4, 1);
@@ -915,7 +923,7 @@ int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int
   }
 #undef KM_SEG
   hipLaunchKernelGGL(bucket_sum_kernel, dim3((unsigned)k, (unsigned)((d + 63) / 64)), dim3(WG), 0, s,
-                     partials, offsets, counts, gsum, d, wm * 64);
+                     partials, offsets, counts, gsum, d, wm * 64, changed);
   KM_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -959,9 +967,11 @@ __global__ __launch_bounds__(WG) void finalize_kernel(
     const double *__restrict__ psums, const int *__restrict__ pcounts, int row_blocks,
     const T *__restrict__ c_old, T *__restrict__ c_new, int *__restrict__ counts,
     T *__restrict__ shift_partials, int d, int k, const int *__restrict__ frozen, int kps,
-    unsigned *__restrict__ done, T *__restrict__ shift2, T *__restrict__ shift_host) {
+    unsigned *__restrict__ done, T *__restrict__ shift2, T *__restrict__ shift_host, RunningSums run) {
 #pragma clang fp contract(off)
   constexpr int RS = WG / EPW;
+  const bool changes = run.sums != nullptr && run.ctl->full == 0;
+  if (changes) row_blocks = min(row_blocks, (int)((run.ctl->count + BOUND_TILE_ROWS - 1) / BOUND_TILE_ROWS));
   __shared__ double part[RS][EPW];
   __shared__ int cpart[RS][EPW];
   __shared__ T red[EPW];
@@ -1004,6 +1014,14 @@ __global__ __launch_bounds__(WG) void finalize_kernel(
     for (int q = 1; q < RS; q++) {
       tot = tot + part[q][el];
       ctot += cpart[q][el];
+    }
+    if (run.sums) {
+      if (changes) {
+        tot = run.sums[e] + tot;
+        ctot += run.counts_old[c];
+      }
+      run.sums[e] = tot;
+      if (e - (int64_t)c * d == 0) run.counts_new[c] = ctot;
     }
     const T oldv = c_old[e];
     T newv;
@@ -1080,7 +1098,7 @@ template <typename T>
 int launch_finalize(hipStream_t s, int slots, const double *psums,
                     const int *pcounts, const T *c_old, T *c_new, int *counts,
                     T *shift_partials, int *n_shift_partials, int d, int k, const int *frozen,
-                    int kps, unsigned *done, T *shift2, T *shift_host) {
+                    int kps, unsigned *done, T *shift2, T *shift_host, RunningSums run) {
   const int64_t kd = (int64_t)k * d;
   // (a stacked model always takes the wide form: its sets' partials must not share a block)
   const bool narrow = kd <= FINALIZE_NARROW_KD && slots >= 256 && frozen == nullptr;
@@ -1091,10 +1109,10 @@ int launch_finalize(hipStream_t s, int slots, const double *psums,
   if (sum_to) done = nullptr;
   if (narrow)
     hipLaunchKernelGGL((finalize_kernel<T, 4>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
-                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host);
+                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host, run);
   else
     hipLaunchKernelGGL((finalize_kernel<T, 32>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
-                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host);
+                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host, run);
   if (sum_to)
     hipLaunchKernelGGL((post_update_kernel<T>), dim3(1), dim3(WG), 0, s, c_new, (T *)nullptr, shift_partials,
                        blocks, sum_to, shift_host, d, k);
@@ -1190,17 +1208,17 @@ int launch_gather_rows(hipStream_t s, const T *X, const int *idx, T *C, int k, i
 
 template int launch_bucketed_accumulate<float>(hipStream_t, const float *, const int *, int *, int *,
                                                int *, int *, int *, int *, double *, double *, int *,
-                                               int64_t, int, int);
+                                               int64_t, int, int, const unsigned *);
 template int launch_bucketed_accumulate<double>(hipStream_t, const double *, const int *, int *, int *,
                                                 int *, int *, int *, int *, double *, double *, int *,
-                                                int64_t, int, int);
+                                                int64_t, int, int, const unsigned *);
 
 #define KM_INSTANTIATE(T)                                                            \
   template int launch_row_norms<T>(hipStream_t, const T *, T *, int64_t, int, int *);       \
   template UpdatePlan plan_update<T>(int64_t, int, int, int);                        \
   template int launch_finalize<T>(hipStream_t, int, const double *,                  \
                                   const int *, const T *, T *, int *, T *, int *,    \
-                                  int, int, const int *, int, unsigned *, T *, T *);                       \
+                                  int, int, const int *, int, unsigned *, T *, T *, RunningSums);                       \
   template int launch_post_update<T>(hipStream_t, const T *, T *, const T *, int,    \
                                      T *, int, int);                                 \
   template int launch_sum<T>(hipStream_t, const T *, int64_t, double *, int,         \

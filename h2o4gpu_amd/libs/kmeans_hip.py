@@ -78,6 +78,7 @@ PROTOTYPES = {
     "h2o4gpu_kmeans_kernel_time": (c_int, [c_void_p, c_char_p, P(c_int), P(c_double)]),
     "h2o4gpu_kmeans_assign_variant": (c_char_p, [c_void_p]),
     "h2o4gpu_kmeans_step_products": (c_int, [c_void_p]),
+    "h2o4gpu_kmeans_rows_measured": (c_int, [c_void_p, P(ctypes.c_longlong)]),
     "h2o4gpu_kmeans_copy_probe": (c_int, [c_int, c_size_t, c_int, P(c_float)]),
     "h2o4gpu_kmeans_bandwidth_probe": (c_int, [c_int, c_int, c_size_t, c_int, P(c_float)]),
     "h2o4gpu_kmeans_predict_device_noalloc": (c_int, [c_int, c_size_t, c_size_t, c_int, c_void_p,
@@ -310,6 +311,12 @@ class Handle:
 
     def assign_variant(self):
         return lib().h2o4gpu_kmeans_assign_variant(self._h).decode()
+
+    def rows_measured(self):
+        """Rows the last step of the last fit that kept bounds measured; -1 when no step kept any."""
+        rows = ctypes.c_longlong()
+        _check("rows_measured", lib().h2o4gpu_kmeans_rows_measured(self._h, ctypes.byref(rows)))
+        return rows.value
 
     def step_products(self):
         """Bfloat16 products per pair of float32 values in a Lloyd step's distance kernel (0: none)."""

@@ -273,6 +273,11 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * memory for the downloaded copy (M x M values for M candidates; when either allocation
  * fails the picks fall back to the other form); 0 runs one small kernel per pick, as
  * "assign" = 1 always does.
+ * "bounds" = 1 (default) lets a fit of eight steps or more keep, from its third step on, how far
+ * each row is from changing its label, and measure only rows that may have changed it (row_bounds.h:
+ * float32 and float64 shapes of the tiled kernels, where there is enough to measure). Labels and
+ * centroids are those of 0, which measures every row in every step; 2 does it for fits of any length and
+ * shapes of any size. Twelve bytes of device memory a row; where they cannot be had every row is measured.
  * Unknown names return EARG. */
 int h2o4gpu_kmeans_set_option(h2o4gpu_kmeans_handle *h, const char *name,
                               int value);
@@ -291,6 +296,9 @@ int h2o4gpu_kmeans_kernel_time(h2o4gpu_kmeans_handle *h, const char *kernel,
                                int *launches, double *milliseconds);
 /* Name of the assign kernel variant the handle's shape dispatches to. */
 const char *h2o4gpu_kmeans_assign_variant(h2o4gpu_kmeans_handle *h);
+/* Rows the last step of the last fit measured that kept bounds (option "bounds"); -1: no step did. */
+int h2o4gpu_kmeans_rows_measured(h2o4gpu_kmeans_handle *h, long long *rows);
+
 /* Bfloat16 products per pair of float32 values that the distance kernel of a Lloyd step runs
  * with (see "fp32_split"): 9, 6, 3, or 0 where it runs the float32 or float64 instructions. */
 int h2o4gpu_kmeans_step_products(h2o4gpu_kmeans_handle *h);
