@@ -1435,7 +1435,8 @@ struct Engine : h2o4gpu_kmeans_handle {
   // Steps that measure only the rows whose label may have changed (row_bounds.h). The first of them
   // measures all rows and leaves their limits.
   static const int BOUNDS_FROM = 2;         // by then most centroids have found their place
-  static const int BOUNDS_ITERATIONS = 8;   // of a fit, at least
+  // of a fit, at least: ten steps gain 1.3 to 1.8 times on clustered data, eight lose up to a tenth on noise
+  static const int BOUNDS_ITERATIONS = 10;
   unsigned char *bound_slab = nullptr;
   float *limit = nullptr, *moves = nullptr, *drift_float = nullptr;
   int *found = nullptr, *found_counts = nullptr, *listed = nullptr;
@@ -1450,9 +1451,12 @@ struct Engine : h2o4gpu_kmeans_handle {
     if (!opt_bounds || (opt_bounds == 1 && max_iterations < BOUNDS_ITERATIONS) || sets > 1 || opt_assign != ASSIGN_AUTO || opt_exact ||
         opt_split != SPLIT_DEFAULT)
       return false;
-    // Three more launches and eight bytes a row are to be had for less than a tenth of the step.
-    if (opt_bounds == 1 && 2.0 * (double)n * k * d < (sizeof(T) == 4 ? 2e10 : 4e9)) return false;
     bound_fused = opt_fuse && bounded_accumulate_applies<T>(n, d, k, split_for(SPLIT_FUSED, k), num_cu);
+    // Three more launches and eight bytes a row have to be small beside a step. Twenty steps on blobs and
+    // on noise: fused 200k x 32, k = 256 0.96 and 0.79 times as fast, 1M (16 GF) 1.54 and 0.94, 2M (33 GF)
+    // 1.93 and 1.00; tiled 20k x 256, k = 300 (3 GF) 1.99 and 0.94, 100k (15 GF) 1.88 and 0.96; float64
+    // 50k x 100, k = 300 (3 GF) 1.63 and 0.90, 200k (12 GF) 1.88 and 0.94.
+    if (opt_bounds == 1 && 2.0 * (double)n * k * d < (bound_fused ? 3e10 : 1e10)) return false;
     const int split = split_for(SPLIT_ASSIGN, k);
     if (!bound_fused && !bounded_assign_applies<T>(n, d, k, split, split_scratch(split, k, true, n))) return false;
     if (!bound_slab) {

@@ -273,9 +273,10 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * memory for the downloaded copy (M x M values for M candidates; when either allocation
  * fails the picks fall back to the other form); 0 runs one small kernel per pick, as
  * "assign" = 1 always does.
- * "bounds" = 1 (default) lets a fit of eight steps or more keep, from its third step on, how far
- * each row is from changing its label, and measure only rows that may have changed it (row_bounds.h:
- * float32 and float64 shapes of the tiled kernels, where there is enough to measure). Labels and
+ * "bounds" = 1 (default) lets a fit of ten steps or more keep, from its third step on, how far
+ * each row is from changing its label, and measure only rows that may have changed it (shapes of the
+ * tiled kernels, float32 shapes of the row-stationary one with six products, where there is enough to
+ * measure). Labels and
  * centroids are those of 0, which measures every row in every step; 2 does it for fits of any length and
  * shapes of any size. Twelve bytes of device memory a row; where they cannot be had every row is measured.
  * Unknown names return EARG. */
