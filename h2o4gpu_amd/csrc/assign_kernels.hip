@@ -503,32 +503,6 @@ __device__ __forceinline__ float float32_chain(const float *x, const float *c, i
   return acc;
 }
 
-// The rows of a launch: all of them, or (LIST) those a RowBounds names.
-template <bool LIST>
-struct ListedRows {
-  int64_t count;
-  __device__ __forceinline__ ListedRows(const RowBounds &, int64_t n) : count(n) {}
-  __device__ __forceinline__ int64_t row(int64_t i) const { return i; }
-  __device__ __forceinline__ bool all() const { return true; }
-  __device__ __forceinline__ void label(int *labels, int64_t row, int c) const { labels[row] = c; }
-};
-template <>
-struct ListedRows<true> {
-  int64_t count;
-  const int *rows;  // null: all
-  unsigned *changed;
-  bool limits;  // the next step looks at them
-  __device__ __forceinline__ ListedRows(const RowBounds &rb, int64_t n)
-      : count(rb.ctl->full ? n : (int64_t)rb.ctl->count), rows(rb.ctl->full ? nullptr : rb.rows),
-        changed(&rb.ctl->changed), limits(rb.ctl->wait == 0) {}
-  __device__ __forceinline__ int64_t row(int64_t i) const { return rows ? (int64_t)rows[i] : i; }
-  __device__ __forceinline__ bool all() const { return rows == nullptr; }
-  __device__ __forceinline__ void label(int *labels, int64_t row, int c) const {
-    if (rows && labels[row] == c) return;
-    labels[row] = c;
-    if (rows) *changed = 1;  // (set already where all rows are measured)
-  }
-};
 // The second smallest magnitude once `a` joins a row whose smallest is `best`. (A NaN is nobody's second.)
 template <typename T>
 __device__ __forceinline__ T second_of(T a, T best, T second) {
@@ -3260,6 +3234,8 @@ template int launch_bounded_assign<double>(hipStream_t, const double *, const do
 
 template <>
 bool bounded_accumulate_applies<float>(int64_t n, int d, int k, int split, int num_cu) {
+  if (pick_assign_variant<float>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW)
+    return k > 1 && n <= 2147483647 && fused_slots<float>(ASSIGN_AUTO, n, d, k, num_cu) > 0;
   if (split != 6 || k > MAX_BOUND_CENTROIDS || n > 2147483647 || fused_slots<float>(ASSIGN_AUTO, n, d, k, num_cu) <= 0 ||
       pick_assign_variant<float>(ASSIGN_AUTO, n, d, k) != ASSIGN_ROWSTAT)
     return false;
@@ -3271,17 +3247,23 @@ bool bounded_accumulate_applies<double>(int64_t, int, int, int, int) { return fa
 template <>
 int launch_bounded_accumulate<float>(hipStream_t s, const float *X, const float *xnorm, const float *C, int *labels,
                                      int64_t n, int d, int k, int num_cu, double *psums, int *pcounts, int *slots,
-                                     const RowBounds &bounds) {
+                                     int *tile_rows, const RowBounds &bounds) {
   if (!bounded_accumulate_applies<float>(n, d, k, 6, num_cu)) return H2O4GPU_KMEANS_EARG;
   RowBounds rb = bounds;
   rb.noise = bound_noise<float>(d);
+  if (pick_assign_variant<float>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW) {
+    *tile_rows = longrow_tile_rows<float>(d);
+    return launch_longrow<float, true, true>(s, X, xnorm, C, nullptr, labels, nullptr, n, d, k, num_cu, psums, pcounts,
+                                             slots, rb);
+  }
   rb.grain = 8e-6f;  // (keys)
+  *tile_rows = Mfma<float>::MT;
   return RowstatDispatch<float, true>::run(s, X, xnorm, C, nullptr, labels, nullptr, n, d, k, num_cu, psums, pcounts,
                                            slots, 0, 0, false, StackShape(), 6, true, &rb);
 }
 template <>
 int launch_bounded_accumulate<double>(hipStream_t, const double *, const double *, const double *, int *, int64_t, int,
-                                      int, int, double *, int *, int *, const RowBounds &) {
+                                      int, int, double *, int *, int *, int *, const RowBounds &) {
   return H2O4GPU_KMEANS_EARG;
 }
 

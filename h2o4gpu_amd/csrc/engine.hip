@@ -1456,7 +1456,11 @@ struct Engine : h2o4gpu_kmeans_handle {
     // on noise: fused 200k x 32, k = 256 0.96 and 0.79 times as fast, 1M (16 GF) 1.54 and 0.94, 2M (33 GF)
     // 1.93 and 1.00; tiled 20k x 256, k = 300 (3 GF) 1.99 and 0.94, 100k (15 GF) 1.88 and 0.96; float64
     // 50k x 100, k = 300 (3 GF) 1.63 and 0.90, 200k (12 GF) 1.88 and 0.94.
-    if (opt_bounds == 1 && 2.0 * (double)n * k * d < (bound_fused ? 3e10 : 1e10)) return false;
+    // Long rows with a handful of centroids are bound by reading them: 500k x 784 (1.6 GB), k = 10, twenty steps on
+    // blobs 8.77 -> 3.39 ms, on noise 8.73 -> 9.60; 1M x 68 (0.3 GB), k = 4 3.29 -> 3.90 on either.
+    const bool long_rows = pick_assign_variant<T>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW;
+    if (opt_bounds == 1 && (long_rows ? (double)n * d * sizeof(T) < 4e8 : 2.0 * (double)n * k * d < (bound_fused ? 3e10 : 1e10)))
+      return false;
     const int split = split_for(SPLIT_ASSIGN, k);
     if (!bound_fused && !bounded_assign_applies<T>(n, d, k, split, split_scratch(split, k, true, n))) return false;
     if (!bound_slab) {
@@ -1493,10 +1497,10 @@ struct Engine : h2o4gpu_kmeans_handle {
     rb.drift = drift_float;
     if (bound_fused) {
       int slots = 0;
-      PROFILED("assign_accumulate", launch_bounded_accumulate<T>(stream, X, xnorm, C[cur], labels, n, d, k, num_cu, psums,
-                                                                 pcounts, &slots, rb));
-      have_mindist = false;
       RunningSums run;
+      PROFILED("assign_accumulate", launch_bounded_accumulate<T>(stream, X, xnorm, C[cur], labels, n, d, k, num_cu, psums,
+                                                                 pcounts, &slots, &run.tile_rows, rb));
+      have_mindist = false;
       run.sums = run_sums;
       run.counts_old = run_counts[was];
       run.counts_new = run_counts[bound_cur];

@@ -134,14 +134,15 @@ bool bounded_assign_applies(int64_t n, int d, int k, int split, const SplitScrat
 template <typename T>
 int launch_bounded_assign(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm, int *labels,
                           int64_t n, int d, int k, SplitScratch scratch, const RowBounds &rb);
-// The fused step of such a loop (row-stationary float32 shapes with six products): labels and limits as
-// above; partial sums and counts of all rows where the control block says that all are measured, of
+// The fused step of such a loop (float32: row-stationary shapes with six products, long rows with a
+// handful of centroids): labels and limits as above; partial sums and counts of all rows where the control block says that all are measured, of
 // what the new labels change otherwise, for launch_finalize with RunningSums.
 template <typename T>
 bool bounded_accumulate_applies(int64_t n, int d, int k, int split, int num_cu);
 template <typename T>
 int launch_bounded_accumulate(hipStream_t s, const T *X, const T *xnorm, const T *C, int *labels, int64_t n, int d,
-                              int k, int num_cu, double *psums, int *pcounts, int *slots, const RowBounds &rb);
+                              int k, int num_cu, double *psums, int *pcounts, int *slots, int *tile_rows,
+                              const RowBounds &rb);
 // The step before such a pass: how far the centroids have moved, the drift that leaves (drift_old ->
 // drift_new; null: zeros, and every row is measured), the rows whose limit it has passed and the control block.
 // drift_float: drift_new, for the pass. found, listed: [n] int32 each; found_counts: [bound_segments(n)]; moves: [k].
@@ -169,10 +170,13 @@ template <typename T>
 bool longrow_applies(int d, int k);
 template <typename T>
 int longrow_max_slots(int d, int k, int num_cu);
-template <typename T, bool SUMS>
+// LIST (float32, SUMS): the rows rb names. longrow_tile_rows: rows a workgroup takes at a time.
+template <typename T, bool SUMS, bool LIST = false>
 int launch_longrow(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm, int *labels,
                    T *mindist, int64_t n, int d, int k, int num_cu, double *psums, int *pcounts,
-                   int *slots);
+                   int *slots, const RowBounds &rb = RowBounds());
+template <typename T>
+int longrow_tile_rows(int d);
 // The kernel for rows of three to eight float32 features and more than 16 centroids
 // (shortrow_kernels.hip): whether a shape is its, and the launch. It makes both norms itself and
 // reads the k centroids only; fused: partial sums and counts per workgroup, at most 2 * num_cu slots.
@@ -282,8 +286,8 @@ struct RunningSums {
   const int *counts_old = nullptr;  // [k]
   int *counts_new = nullptr;        // [k], another buffer
   const BoundControl *ctl = nullptr;
+  int tile_rows = 0;  // listed rows a workgroup takes at a time: fewer tiles, fewer slots written
 };
-static const int BOUND_TILE_ROWS = 32;  // listed rows a workgroup takes at a time: fewer tiles, fewer slots written
 template <typename T>
 int launch_finalize(hipStream_t s, int slots, const double *psums,
                     const int *pcounts, const T *c_old, T *c_new, int *counts,

@@ -38,6 +38,33 @@ struct RowBounds {
   float grain = 0;  // and compared at this relative resolution
 };
 
+// The rows of a launch: all of them, or (LIST) those a RowBounds names.
+template <bool LIST>
+struct ListedRows {
+  int64_t count;
+  __device__ __forceinline__ ListedRows(const RowBounds &, int64_t n) : count(n) {}
+  __device__ __forceinline__ int64_t row(int64_t i) const { return i; }
+  __device__ __forceinline__ bool all() const { return true; }
+  __device__ __forceinline__ void label(int *labels, int64_t row, int c) const { labels[row] = c; }
+};
+template <>
+struct ListedRows<true> {
+  int64_t count;
+  const int *rows;  // null: all
+  unsigned *changed;
+  bool limits;  // the next step looks at them
+  __device__ __forceinline__ ListedRows(const RowBounds &rb, int64_t n)
+      : count(rb.ctl->full ? n : (int64_t)rb.ctl->count), rows(rb.ctl->full ? nullptr : rb.rows),
+        changed(&rb.ctl->changed), limits(rb.ctl->wait == 0) {}
+  __device__ __forceinline__ int64_t row(int64_t i) const { return rows ? (int64_t)rows[i] : i; }
+  __device__ __forceinline__ bool all() const { return rows == nullptr; }
+  __device__ __forceinline__ void label(int *labels, int64_t row, int c) const {
+    if (rows && labels[row] == c) return;
+    labels[row] = c;
+    if (rows) *changed = 1;  // (set already where all rows are measured)
+  }
+};
+
 // The limit of a row whose nearest centroid (with this drift) is at the squared distance `best`, the
 // next one at `second`. A centroid at a squared distance D has a norm of at most 2 xx + 2 D, so D is known
 // to noise * (3 xx + 2 D). What a later pass needs to order the two as they are is e2 between their squares,

@@ -971,7 +971,7 @@ __global__ __launch_bounds__(WG) void finalize_kernel(
 #pragma clang fp contract(off)
   constexpr int RS = WG / EPW;
   const bool changes = run.sums != nullptr && run.ctl->full == 0;
-  if (changes) row_blocks = min(row_blocks, (int)((run.ctl->count + BOUND_TILE_ROWS - 1) / BOUND_TILE_ROWS));
+  if (changes) row_blocks = min(row_blocks, (int)((run.ctl->count + run.tile_rows - 1) / run.tile_rows));
   __shared__ double part[RS][EPW];
   __shared__ int cpart[RS][EPW];
   __shared__ T red[EPW];

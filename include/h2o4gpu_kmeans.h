@@ -275,9 +275,8 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * "assign" = 1 always does.
  * "bounds" = 1 (default) lets a fit of ten steps or more keep, from its third step on, how far
  * each row is from changing its label, and measure only rows that may have changed it (shapes of the
- * tiled kernels, float32 shapes of the row-stationary one with six products, where there is enough to
- * measure). Labels and
- * centroids are those of 0, which measures every row in every step; 2 does it for fits of any length and
+ * tiled kernels, float32 shapes of the row-stationary one with six products and of the one for long rows
+ * and a handful of centroids, where there is enough to measure). Labels and centroids are those of 0, which measures every row in every step; 2 does it for fits of any length and
  * shapes of any size. Twelve bytes of device memory a row; where they cannot be had every row is measured.
  * Unknown names return EARG. */
 int h2o4gpu_kmeans_set_option(h2o4gpu_kmeans_handle *h, const char *name,
