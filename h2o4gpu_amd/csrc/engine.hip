@@ -846,9 +846,9 @@ struct Engine : h2o4gpu_kmeans_handle {
       e = nullptr;
     }
     if (own_X && X) (void)hipFree(X);
-    for (void *p : {(void *)slab, (void *)work_slab, (void *)d_split, (void *)bound_slab})
+    for (void *p : {(void *)slab, (void *)work_slab, (void *)d_split, (void *)bound_slab, (void *)cell_slab})
       if (p) (void)hipFree(p);
-    slab = work_slab = d_split = bound_slab = nullptr;
+    slab = work_slab = d_split = bound_slab = cell_slab = nullptr;
     if (stream) (void)hipStreamDestroy(stream);
     stream = nullptr;
     return 0;
@@ -1514,9 +1514,76 @@ struct Engine : h2o4gpu_kmeans_handle {
     return update_async(want_shift, shift_host, &rb.ctl->changed);
   }
 
+  // Steps over rows ordered in space (cell_kernels.hip). Ordering them takes as long as eight to ten
+  // steps of the other kind, a step then a fifth to a half, so they are ordered where at least CELL_STEPS are to
+  // come (k = 27, 24 steps on blobs and on noise: 2M rows 0.99 and 0.96 times as fast, 4M 1.21 and 1.16, 10M 1.54
+  // and 1.36; 60 steps of 10M 2.18 and 1.88), and used if their blocks are small enough to leave little to measure.
+  static const int CELL_STEPS = 24;
+  static const int64_t CELL_ROWS = 4000000;
+  unsigned char *cell_slab = nullptr;
+  float *cell_rows = nullptr, *cell_range = nullptr;
+  int *cell_ids = nullptr, *cell_order = nullptr, *cell_order_id = nullptr;
+  int *cell_offsets = nullptr, *cell_counts = nullptr, *cell_hist = nullptr, *cell_seg = nullptr, *cell_total = nullptr;
+  CellBlock *cell_block = nullptr;
+  unsigned long long *cell_work = nullptr;
+  long long cell_measured = -1;  // rows the first such step of the last fit measured, in whole models' worth
+  bool cells_possible() const {
+    return sizeof(T) == 4 && opt_bounds && sets == 1 && opt_fuse && opt_assign == ASSIGN_AUTO && !opt_exact && settles() &&
+           cells_apply(n, d, k) && (opt_bounds == 2 || n >= CELL_ROWS);
+  }
+  // *use: the steps from here on may be made that way
+  int cells_begin(bool *use) {
+    *use = false;
+    if constexpr (sizeof(T) == 4) {
+      if (!cell_slab) {
+        std::vector<Want> list;
+        want(list, &cell_rows, (size_t)n * d);
+        want(list, &cell_block, (size_t)cell_blocks(n));
+        want(list, &cell_ids, n);
+        want(list, &cell_order, n);
+        want(list, &cell_order_id, n);
+        want(list, &cell_range, cell_range_values());
+        want(list, &cell_offsets, CELL_IDS);
+        want(list, &cell_counts, CELL_IDS);
+        want(list, &cell_hist, (size_t)bucket_blocks(n, CELL_IDS) * CELL_IDS);
+        want(list, &cell_seg, (size_t)32 * CELL_IDS);
+        want(list, &cell_total, 1);
+        want(list, &cell_work, 1);
+        if (allocate(list, &cell_slab) != 0) return 0;  // (every row is measured, then)
+      }
+      KM_TRY(ensure_work());
+      prof_begin("cells");
+      KM_TRY(launch_cell_ids(stream, X, n, d, cell_range, cell_ids));
+      KM_TRY(launch_bucket_rows(stream, cell_ids, cell_order, cell_order_id, cell_offsets, cell_hist, cell_seg, cell_total,
+                                cell_counts, n, CELL_IDS));
+      KM_TRY(launch_cell_windows(stream, X, n, d, cell_range, cell_order, cell_rows, cell_block));
+      prof_end();
+      // (the sums of this step are made again by the one that counts)
+      KM_TRY(launch_fill<int>(stream, reinterpret_cast<int *>(cell_work), 0, 2));
+      int slots = 0;
+      KM_TRY(launch_cell_step(stream, cell_rows, cell_block, n, C[cur], d, k, num_cu, psums, pcounts, &slots, cell_work));
+      unsigned long long work = 0;
+      KM_HIP_TRY(hipMemcpyAsync(&work, cell_work, sizeof(work), hipMemcpyDeviceToHost, stream));
+      KM_HIP_TRY(hipStreamSynchronize(stream));
+      cell_measured = (long long)(work * 64 / k);
+      // (centroids per row: 0.8 to 2.2 where a step was 1.9 to 2.2 times as fast, k = 27 and 60; 4.8 at 1.5 times, k = 100)
+      *use = opt_bounds == 2 || (double)work * 64 / n < 2 + k / 32.0;
+    }
+    return 0;
+  }
+  int cells_step(bool want_shift, T *shift_host = nullptr) {
+    int slots = 0;
+    if constexpr (sizeof(T) == 4) {
+      PROFILED("assign_accumulate", launch_cell_step(stream, cell_rows, cell_block, n, C[cur], d, k, num_cu, psums, pcounts,
+                                                     &slots, nullptr));
+    }
+    have_mindist = false;  // (nor labels: an assignment pass over all rows follows the loop)
+    return finish_update(slots, want_shift, shift_host);
+  }
+
   int rows_measured(long long *rows) override {
     KM_HIP_TRY(hipSetDevice(dev));
-    *rows = -1;
+    *rows = cell_measured;
     if (bound_steps == 0) return 0;
     BoundControl ctl;
     KM_HIP_TRY(hipMemcpyAsync(&ctl, bound_ctl[bound_cur], sizeof(ctl), hipMemcpyDeviceToHost, stream));
@@ -1577,6 +1644,8 @@ struct Engine : h2o4gpu_kmeans_handle {
     maybe_install_signal_handlers();
     int updates = 0;
     const bool bounded = bounds_begin(max_iterations);
+    bool cells = false, cells_wanted = cells_possible();
+    cell_measured = -1;
     if (max_iterations <= 0) {
       // The reference's loop then never runs, its final relabel included, and the labels it
       // returns are the zeros its vector was created with (kmeans_impl.h:109-232,
@@ -1592,7 +1661,12 @@ struct Engine : h2o4gpu_kmeans_handle {
       for (int i = 0; i < max_iterations; i++) {
         log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
         // (the final relabel below leaves the minimum distances)
-        if (bounded && i >= BOUNDS_FROM) KM_TRY(bounded_step(i == BOUNDS_FROM, false));
+        if (cells_wanted && i >= 1) {
+          if (opt_bounds == 2 || max_iterations - i >= CELL_STEPS) KM_TRY(cells_begin(&cells));
+          cells_wanted = false;
+        }
+        if (cells) KM_TRY(cells_step(false));
+        else if (bounded && i >= BOUNDS_FROM) KM_TRY(bounded_step(i == BOUNDS_FROM, false));
         else KM_TRY(step_async(false, false));
         updates++;
         bool done = false;
@@ -1714,9 +1788,23 @@ struct Engine : h2o4gpu_kmeans_handle {
       for (int i = 0; i < 2; i++)
         KM_HIP_TRY(hipEventCreateWithFlags(&shift_ready[i], hipEventDisableTiming | hipEventReleaseToSystem));
     }
+    bool cells = false, cells_wanted = cells_possible();
+    std::vector<double> shifts;
+    // steps to come, if the shift goes on falling as it did over the last four
+    auto steps_ahead = [&](int i) -> double {
+      if (shifts.size() < 5) return 0;
+      const double now = shifts.back(), was = shifts[shifts.size() - 5];
+      const double ahead = now < was ? 4 * std::log(now / threshold) / std::log(was / now) : max_iterations;
+      return std::min(ahead, (double)(max_iterations - i));
+    };
     auto queue_iteration = [&](int i) -> int {
       log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
-      if (bounded && i >= BOUNDS_FROM) KM_TRY(bounded_step(i == BOUNDS_FROM, true, host_shift + (i & 1)));
+      if (cells_wanted && i >= 1 && (opt_bounds == 2 || steps_ahead(i) >= CELL_STEPS)) {
+        KM_TRY(cells_begin(&cells));
+        cells_wanted = false;
+      }
+      if (cells) KM_TRY(cells_step(true, host_shift + (i & 1)));
+      else if (bounded && i >= BOUNDS_FROM) KM_TRY(bounded_step(i == BOUNDS_FROM, true, host_shift + (i & 1)));
       else KM_TRY(step_async(true, true, host_shift + (i & 1)));
       KM_HIP_TRY(hipEventRecord(shift_ready[i & 1], stream));
       return 0;
@@ -1729,6 +1817,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       KM_HIP_TRY(hipEventSynchronize(shift_ready[i & 1]));
       updates = i + 1;
       bool done = (double)host_shift[i & 1] < threshold;
+      if (cells_wanted) shifts.push_back((double)host_shift[i & 1]);
       if (done) log_msg(verbose, LOG_INFO, "Threshold triggered. Terminating early.");
       if (g_stop_flag) {
         fprintf(stderr, "Signal caught. Terminated early.\n");

@@ -183,6 +183,24 @@ int longrow_tile_rows(int d);
 bool shortrow_applies(int d, int k, bool fused);
 int launch_shortrow(hipStream_t s, const float *X, const float *C, int *labels, float *mindist, int64_t n, int d,
                     int k, int num_cu, bool fused, double *psums, int *pcounts, int *slots, bool settle);
+// Lloyd steps over such rows (three features) once they have been ordered in space and cut into
+// blocks of 64 (cell_kernels.hip). ids: a number below CELL_IDS per row, whose order (launch_bucket_rows) the
+// windows then refine; range: [cell_range_values()], Xs: [n][d], blocks: [cell_blocks(n)]. The step leaves
+// partial sums and counts of at most 2 * num_cu slots and no labels; measured (nullable, zero before): receives
+// how many centroids the blocks' rows were measured against, added up over the blocks.
+struct CellBlock {
+  float lo[4], hi[4];
+  double sum[4];
+};
+static const int CELL_IDS = 4096;
+bool cells_apply(int64_t n, int d, int k);
+int64_t cell_blocks(int64_t n);
+int cell_range_values();
+int launch_cell_ids(hipStream_t s, const float *X, int64_t n, int d, float *range, int *ids);
+int launch_cell_windows(hipStream_t s, const float *X, int64_t n, int d, const float *range, const int *order,
+                        float *Xs, CellBlock *blocks);
+int launch_cell_step(hipStream_t s, const float *Xs, const CellBlock *blocks, int64_t n, const float *C, int d, int k,
+                     int num_cu, double *psums, int *pcounts, int *slots, unsigned long long *measured);
 const char *assign_variant_name(int variant);
 // split (float32 matrix-core kernels; 0, 6 or 9): run the dot products on the bfloat16
 // matrix pipe as that many products of bfloat16 parts per feature pair (9: every product
@@ -260,6 +278,9 @@ int launch_accumulate(hipStream_t s, const UpdatePlan &p, const T *X,
 bool bucketed_update_applies(int k_chunks, int64_t n, int k, int d, size_t elem);
 int bucket_blocks(int64_t n, int k);
 size_t bucket_partial_slots(int64_t n, int k);
+// (the sort alone: order, order_label, counts and offsets, *total rows in all)
+int launch_bucket_rows(hipStream_t s, const int *labels, int *order, int *order_label, int *offsets, int *block_hist,
+                       int *seg_hist, int *total, int *counts, int64_t n, int k, const unsigned *changed = nullptr);
 template <typename T>
 int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int *order,
                                int *order_label, int *offsets, int *block_hist, int *seg_hist,

@@ -873,11 +873,8 @@ bool bucketed_update_applies(int k_chunks, int64_t n, int k, int d, size_t elem)
   return !(elem == 8 && d > 256 && (size_t)n * d * elem > ((size_t)1 << 30));
 }
 
-template <typename T>
-int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int *order,
-                               int *order_label, int *offsets, int *block_hist, int *seg_hist,
-                               int *total, double *partials, double *gsum, int *counts, int64_t n,
-                               int d, int k, const unsigned *changed) {
+int launch_bucket_rows(hipStream_t s, const int *labels, int *order, int *order_label, int *offsets, int *block_hist,
+                       int *seg_hist, int *total, int *counts, int64_t n, int k, const unsigned *changed) {
   const int64_t rpb = bucket_rows_per_block(n, k);
   const int nb = bucket_blocks(n, k);
   const int per_seg = (nb + BUCKET_SEGS - 1) / BUCKET_SEGS;
@@ -894,6 +891,16 @@ int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int
   hipLaunchKernelGGL(bucket_scan_kernel, dim3(1), dim3(WG), 0, s, counts, offsets, total, k, changed);
   hipLaunchKernelGGL(bucket_scatter_kernel, dim3(nb), dim3(bucket_waves(k) * 64), lds2, s, labels,
                      block_hist, offsets, order, order_label, n, k, rpb, changed);
+  KM_HIP_TRY(hipGetLastError());
+  return 0;
+}
+
+template <typename T>
+int launch_bucketed_accumulate(hipStream_t s, const T *X, const int *labels, int *order,
+                               int *order_label, int *offsets, int *block_hist, int *seg_hist,
+                               int *total, double *partials, double *gsum, int *counts, int64_t n,
+                               int d, int k, const unsigned *changed) {
+  KM_TRY(launch_bucket_rows(s, labels, order, order_label, offsets, block_hist, seg_hist, total, counts, n, k, changed));
   // rows with a label outside [0, k) are not bucketed, so the ordered rows may be fewer
   // than n: the grid covers n positions and every wavefront bounds itself by the
   // device-side total

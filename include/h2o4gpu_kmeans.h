@@ -278,6 +278,8 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * tiled kernels, float32 shapes of the row-stationary one with six products and of the one for long rows
  * and a handful of centroids, where there is enough to measure). Labels and centroids are those of 0, which measures every row in every step; 2 does it for fits of any length and
  * shapes of any size. Twelve bytes of device memory a row; where they cannot be had every row is measured.
+ * Float32 rows of three features and 17 to 128 centroids: long fits order a copy of the rows in space and
+ * measure only blocks of them that more than one centroid may be the nearest in (cell_kernels.hip; 26 bytes a row).
  * Unknown names return EARG. */
 int h2o4gpu_kmeans_set_option(h2o4gpu_kmeans_handle *h, const char *name,
                               int value);
@@ -296,7 +298,8 @@ int h2o4gpu_kmeans_kernel_time(h2o4gpu_kmeans_handle *h, const char *kernel,
                                int *launches, double *milliseconds);
 /* Name of the assign kernel variant the handle's shape dispatches to. */
 const char *h2o4gpu_kmeans_assign_variant(h2o4gpu_kmeans_handle *h);
-/* Rows the last step of the last fit measured that kept bounds (option "bounds"); -1: no step did. */
+/* Rows the last step of the last fit measured that kept bounds (option "bounds"); where rows were ordered in
+ * space, as many as its first such step's distances make. -1: no step did. */
 int h2o4gpu_kmeans_rows_measured(h2o4gpu_kmeans_handle *h, long long *rows);
 
 /* Bfloat16 products per pair of float32 values that the distance kernel of a Lloyd step runs
