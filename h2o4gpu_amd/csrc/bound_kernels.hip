@@ -30,13 +30,18 @@ __global__ __launch_bounds__(WG) void centroid_moves_kernel(const T *__restrict_
   if (c >= k) return;
   const T *a = c_old + (size_t)c * d, *b = c_new + (size_t)c * d;
   double s = 0;
+  bool moved = false;
   for (int j = lane; j < d; j += 64) {
     const double v = (double)b[j] - (double)a[j];
     s += v * v;
+    moved |= v != 0;
   }
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) moves[c] = (float)sqrt(s) * (1.0f + 1e-6f);
+  moved = __ballot(moved) != 0;
+  // (a move too small for its square or for a float is a move all the same)
+  const float m = (float)sqrt(s) * (1.0f + 1e-6f);
+  if (lane == 0) moves[c] = moved && m < 1.2e-38f ? 1.2e-38f : m;
 }
 
 __global__ __launch_bounds__(WG) void rows_to_measure_kernel(
@@ -148,14 +153,16 @@ __global__ __launch_bounds__(WG) void pack_rows_kernel(const int *__restrict__ f
                                                       const int *__restrict__ found_counts, int segments,
                                                       int64_t seg_rows, int64_t n, int *__restrict__ listed,
                                                       const BoundControl *__restrict__ ctl_old,
-                                                      BoundControl *__restrict__ ctl_new) {
+                                                      BoundControl *__restrict__ ctl_new, unsigned *news_host) {
   __shared__ unsigned before_s[WG / 64], all_s[WG / 64];
   const int tid = threadIdx.x, lane = tid & 63;
   const BoundControl was = *ctl_old;
   const unsigned still = ctl_new->still;
   if (still || was.wait > 0) {
-    if (blockIdx.x == 0 && tid == 0)
+    if (blockIdx.x == 0 && tid == 0) {
+      if (still && news_host) __hip_atomic_store(news_host + BOUND_STILL, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       *ctl_new = BoundControl{0u, still ? 0u : 1u, was.wait > 0 ? was.wait - 1 : 0u, was.fails, still ? 0u : 1u, still};
+    }
     return;
   }
   const int s0 = blockIdx.x * (WG / 64);
@@ -186,6 +193,8 @@ __global__ __launch_bounds__(WG) void pack_rows_kernel(const int *__restrict__ f
   const bool full = (int64_t)all * 8 > n * 5;
   if (blockIdx.x == 0 && tid == 0) {
     const unsigned fails = full ? was.fails + 1 : 0;
+    if (fails == BOUND_FAILS && news_host)
+      __hip_atomic_store(news_host + BOUND_FAILING, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     *ctl_new = BoundControl{all, full ? 1u : 0u, full ? (1u << (fails < 4 ? fails - 1 : 3)) - 1 : 0u, fails, full ? 1u : 0u, 0u};
   }
   if (full) return;
@@ -215,7 +224,7 @@ int bound_segments(int64_t n) {
 template <typename T>
 int launch_bounds(hipStream_t s, const T *c_old, const T *c_new, const int *labels, const float *limit, int64_t n,
                   int d, int k, float *moves, const double *drift_old, double *drift_new, float *drift_float, int *found,
-                  int *found_counts, int *listed, const BoundControl *ctl_old, BoundControl *ctl_new) {
+                  int *found_counts, int *listed, const BoundControl *ctl_old, BoundControl *ctl_new, unsigned *news_host) {
   if (n < 1 || n > 2147483647 || k < 1 || k > MAX_BOUND_CENTROIDS) return H2O4GPU_KMEANS_EARG;
   if (drift_old == nullptr) {
     hipLaunchKernelGGL(first_bounds_kernel, dim3(1), dim3(WG), 0, s, drift_new, drift_float, k, ctl_new);
@@ -230,15 +239,15 @@ int launch_bounds(hipStream_t s, const T *c_old, const T *c_new, const int *labe
                      segment_rows(n), moves, drift_old, drift_new, drift_float, found, found_counts,
                      ctl_old, ctl_new);
   hipLaunchKernelGGL(pack_rows_kernel, dim3(groups), dim3(WG), 0, s, found, found_counts, segments, segment_rows(n), n,
-                     listed, ctl_old, ctl_new);
+                     listed, ctl_old, ctl_new, news_host);
   KM_HIP_TRY(hipGetLastError());
   return 0;
 }
 template int launch_bounds<float>(hipStream_t, const float *, const float *, const int *, const float *, int64_t, int,
                                   int, float *, const double *, double *, float *, int *, int *, int *, const BoundControl *,
-                                  BoundControl *);
+                                  BoundControl *, unsigned *);
 template int launch_bounds<double>(hipStream_t, const double *, const double *, const int *, const float *, int64_t,
                                    int, int, float *, const double *, double *, float *, int *, int *, int *,
-                                   const BoundControl *, BoundControl *);
+                                   const BoundControl *, BoundControl *, unsigned *);
 
 }  // namespace kmhip

@@ -146,12 +146,17 @@ int launch_bounded_accumulate(hipStream_t s, const T *X, const T *xnorm, const T
 // The step before such a pass: how far the centroids have moved, the drift that leaves (drift_old ->
 // drift_new; null: zeros, and every row is measured), the rows whose limit it has passed and the control block.
 // drift_float: drift_new, for the pass. found, listed: [n] int32 each; found_counts: [bound_segments(n)]; moves: [k].
+// news_host (nullable, pinned): [BOUND_STILL] receives 1 where no centroid has moved, [BOUND_FAILING] where
+// most rows had to be measured at BOUND_FAILS looks in a row.
+enum BoundNews { BOUND_STILL, BOUND_FAILING, BOUND_NEWS };
+static const unsigned BOUND_FAILS = 3;
 static const int MAX_BOUND_CENTROIDS = 8192;
 int bound_segments(int64_t n);
 template <typename T>
 int launch_bounds(hipStream_t s, const T *c_old, const T *c_new, const int *labels, const float *limit, int64_t n,
                   int d, int k, float *moves, const double *drift_old, double *drift_new, float *drift_float, int *found,
-                  int *found_counts, int *listed, const BoundControl *ctl_old, BoundControl *ctl_new);
+                  int *found_counts, int *listed, const BoundControl *ctl_old, BoundControl *ctl_new,
+                  unsigned *news_host = nullptr);
 // What launch_assign (variant ASSIGN_AUTO) needs beside the rows and the k centroids for a shape:
 enum AssignInputs {
   ASSIGN_FROM_ROWS,       // nothing: xnorm and cnorm may be null, C need not be padded

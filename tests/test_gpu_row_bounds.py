@@ -88,7 +88,7 @@ def test_fits_that_converge(hip, dtype, n, d, k):
 
 
 @pytest.mark.parametrize("dtype,n,d,k", TILED + FUSED + CELLS)
-@pytest.mark.parametrize("what", ["noise", "far", "twins", "not finite", "small", "large", "empty"])
+@pytest.mark.parametrize("what", ["noise", "far", "twins", "not finite", "small", "large", "empty", "tiny"])
 def test_whatever_the_data(hip, dtype, n, d, k, what):
     X, C = blobs(n, d, k, dtype, seed=2, offset=3000.0 if what == "far" else 0.0)
     rng = np.random.default_rng(5)
@@ -103,6 +103,8 @@ def test_whatever_the_data(hip, dtype, n, d, k, what):
         X[5, 2], X[17, 0], X[n - 1, d - 1] = np.nan, np.inf, -np.inf
     elif what == "small":
         X, C = (X * 2.0 ** -50).astype(dtype), (C * 2.0 ** -50).astype(dtype)
+    elif what == "tiny" and dtype == "float64":  # moves that no float holds
+        X, C = X * 2.0 ** -200, C * 2.0 ** -200
     elif what == "large":
         X, C = (X * 2.0 ** 53).astype(dtype), (C * 2.0 ** 53).astype(dtype)
     elif what == "empty":  # centroids that never get a row, one of them at infinity
