@@ -3201,6 +3201,15 @@ bool bounded_assign_applies(int64_t n, int d, int k, int split, const SplitScrat
 template bool bounded_assign_applies<float>(int64_t, int, int, int, const SplitScratch &);
 template bool bounded_assign_applies<double>(int64_t, int, int, int, const SplitScratch &);
 
+// keys: fused kernels, and tiled ones up to 128 features (see launch_tiled_bcw)
+template <typename T>
+float bound_grain(int64_t n, int d, int k, bool fused) {
+  if (fused) return pick_assign_variant<T>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW ? 0.0f : 8e-6f;
+  return sizeof(T) == 4 && d < 128 ? 8e-6f : 0.0f;
+}
+template float bound_grain<float>(int64_t, int, int, bool);
+template float bound_grain<double>(int64_t, int, int, bool);
+
 template <typename T>
 int launch_bounded_assign(hipStream_t s, const T *X, const T *xnorm, const T *C, const T *cnorm, int *labels,
                           int64_t n, int d, int k, SplitScratch scratch, const RowBounds &bounds) {
@@ -3208,7 +3217,7 @@ int launch_bounded_assign(hipStream_t s, const T *X, const T *xnorm, const T *C,
   const bool direct = !scratch.through_registers;
   RowBounds rb = bounds;
   rb.noise = bound_noise<T>(d);
-  rb.grain = sizeof(T) == 4 && d < 128 ? 8e-6f : 0.0f;  // (keys, see launch_tiled_bcw)
+  rb.grain = bound_grain<T>(n, d, k, false);
   T *const none = nullptr;
   if constexpr (sizeof(T) == 4) {
     void *const parts = static_cast<unsigned char *>(scratch.ptr) + 256;
@@ -3256,7 +3265,7 @@ int launch_bounded_accumulate<float>(hipStream_t s, const float *X, const float 
     return launch_longrow<float, true, true>(s, X, xnorm, C, nullptr, labels, nullptr, n, d, k, num_cu, psums, pcounts,
                                              slots, rb);
   }
-  rb.grain = 8e-6f;  // (keys)
+  rb.grain = bound_grain<float>(n, d, k, true);
   *tile_rows = Mfma<float>::MT;
   return RowstatDispatch<float, true>::run(s, X, xnorm, C, nullptr, labels, nullptr, n, d, k, num_cu, psums, pcounts,
                                            slots, 0, 0, false, StackShape(), 6, true, &rb);

@@ -1442,8 +1442,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   // of a fit, at least: ten steps gain 1.3 to 1.8 times on clustered data, eight lose up to a tenth on noise
   static const int BOUNDS_ITERATIONS = 10;
   unsigned char *bound_slab = nullptr;
-  float *limit = nullptr, *moves = nullptr, *drift_float = nullptr;
-  int *found = nullptr, *found_counts = nullptr, *listed = nullptr;
+  BoundBuffers bound;
   double *drift[2] = {nullptr, nullptr};
   BoundControl *bound_ctl[2] = {nullptr, nullptr};
   int bound_cur = 0, bound_steps = 0;
@@ -1468,13 +1467,22 @@ struct Engine : h2o4gpu_kmeans_handle {
     const int split = split_for(SPLIT_ASSIGN, k);
     if (!bound_fused && !bounded_assign_applies<T>(n, d, k, split, split_scratch(split, k, true, n))) return false;
     if (!bound_slab) {
+      // (Rows of the fused kernels are measured against all centroids in the time it takes to look at a few
+      // of them: 10M x 32, k = 256 0.9 ms and 1.4.)
+      const bool neighbours = !bound_fused && neighbours_apply(n, d, k);
       std::vector<Want> list;
-      want(list, &limit, n);
-      want(list, &found, n);
-      want(list, &listed, n);
-      want(list, &found_counts, bound_segments(n));
-      want(list, &moves, k);
-      want(list, &drift_float, k);
+      want(list, &bound.limit, n);
+      want(list, &bound.found, n);
+      want(list, &bound.listed, n);
+      want(list, &bound.found_counts, bound_counts(n));
+      want(list, &bound.moves, k);
+      want(list, &bound.drift_float, k);
+      want(list, &bound.mid, 1);
+      if (neighbours) {
+        want(list, &bound.near.matrix, (size_t)k * k);
+        want(list, &bound.near.dist, (size_t)k * (NEAREST + 1));
+        want(list, &bound.near.at, (size_t)k * (NEAREST + 1));
+      }
       for (int i = 0; i < 2; i++) {
         want(list, &drift[i], k);
         want(list, &run_counts[i], k);
@@ -1503,7 +1511,7 @@ struct Engine : h2o4gpu_kmeans_handle {
                                hipHostMallocCoherent | hipHostMallocMapped));
       for (auto &ev : news_ready) KM_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     }
-    for (int i = 0; i < BOUND_NEWS; i++) const_cast<volatile unsigned *>(news_host)[i] = 0;  // (nothing is under way)
+    for (int i = 0; i < BOUND_NEWS; i++) const_cast<volatile unsigned *>(news_host)[i] = i == BOUND_LISTED ? ~0u : 0u;  // (nothing is under way)
     bounds_at = BOUNDS_FROM;
     bounds_pause = 16;
     return 0;
@@ -1526,21 +1534,43 @@ struct Engine : h2o4gpu_kmeans_handle {
     KM_HIP_TRY(hipEventRecord(ev, stream));
     return 0;
   }
+  // (a handle's options may change between fits)
+  BoundBuffers bound_buffers() const {
+    BoundBuffers b = bound;
+    // (short lists have no use for the neighbours, and their launches are not for nothing)
+    if (bound_fused || news(BOUND_LISTED) < DECIDE_ROWS) b.near = Neighbours();
+    return b;
+  }
+  // The step before the first of them, where that looks at rows already: it leaves labels.
+  bool bound_fresh = false;
+  int bounds_prime(bool want_shift, T *shift_host = nullptr) {
+    const BoundBuffers b = bound_buffers();
+    bound_fresh = b.near.matrix != nullptr;
+    if (bound_fresh) {
+      bound_cur ^= 1;
+      KM_TRY((launch_bounds<T>(stream, b, BOUNDS_FRESH, X, xnorm, C[cur ^ 1], C[cur], labels, n, d, k, drift[0],
+                               drift[bound_cur], bound_ctl[0], bound_ctl[bound_cur], nullptr, 0.0f)));
+    }
+    return step_async(want_shift, shift_host != nullptr, shift_host);
+  }
   int bounded_step(bool first, bool want_shift, T *shift_host = nullptr) {
     KM_TRY(ensure_work());
     if (!bound_fused) KM_TRY(ensure_cnorm());
     const int was = bound_cur;
     bound_cur ^= 1;
     bound_steps++;
-    PROFILED("bounds", launch_bounds<T>(stream, C[cur ^ 1], C[cur], labels, limit, n, d, k, moves,
-                                        first ? (const double *)nullptr : drift[was], drift[bound_cur], drift_float, found,
-                                        found_counts, listed, bound_ctl[was], bound_ctl[bound_cur],
-                                        news_host));
+    BoundBuffers b = bound_buffers();
+    // (news may have come in since the step before)
+    if (first) b.near = bound_fresh ? bound.near : Neighbours();
+    const BoundStart start = first && !bound_fresh ? BOUNDS_FIRST : BOUNDS_GO;
+    PROFILED("bounds", launch_bounds<T>(stream, b, start, X, xnorm, C[cur ^ 1], C[cur], labels, n, d, k, drift[was],
+                                        drift[bound_cur], bound_ctl[was], bound_ctl[bound_cur], news_host,
+                                        bound_grain<T>(n, d, k, bound_fused)));
     RowBounds rb;
-    rb.rows = listed;
+    rb.rows = bound.listed;
     rb.ctl = bound_ctl[bound_cur];
-    rb.limit = limit;
-    rb.drift = drift_float;
+    rb.limit = bound.limit;
+    rb.drift = bound.drift_float;
     if (bound_fused) {
       int slots = 0;
       RunningSums run;
@@ -1719,6 +1749,7 @@ struct Engine : h2o4gpu_kmeans_handle {
         if (cells) KM_TRY(cells_step(false));
         else if (still) {}  // (the step would change nothing)
         else if (bounded && i >= bounds_at) KM_TRY(bounded_step(i == bounds_at, false));
+        else if (bounded && i == bounds_at - 1) KM_TRY(bounds_prime(false));
         else KM_TRY(step_async(false, false));
         updates++;
         bool done = false;
@@ -1857,6 +1888,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       }
       if (cells) KM_TRY(cells_step(true, host_shift + (i & 1)));
       else if (bounded && i >= bounds_at) KM_TRY(bounded_step(i == bounds_at, true, host_shift + (i & 1)));
+      else if (bounded && i == bounds_at - 1) KM_TRY(bounds_prime(true, host_shift + (i & 1)));
       else KM_TRY(step_async(true, true, host_shift + (i & 1)));
       KM_HIP_TRY(hipEventRecord(shift_ready[i & 1], stream));
       return 0;

@@ -143,20 +143,25 @@ template <typename T>
 int launch_bounded_accumulate(hipStream_t s, const T *X, const T *xnorm, const T *C, int *labels, int64_t n, int d,
                               int k, int num_cu, double *psums, int *pcounts, int *slots, int *tile_rows,
                               const RowBounds &rb);
-// The step before such a pass: how far the centroids have moved, the drift that leaves (drift_old ->
-// drift_new; null: zeros, and every row is measured), the rows whose limit it has passed and the control block.
-// drift_float: drift_new, for the pass. found, listed: [n] int32 each; found_counts: [bound_segments(n)]; moves: [k].
-// news_host (nullable, pinned): [BOUND_STILL] receives 1 where no centroid has moved, [BOUND_FAILING] where
-// most rows had to be measured at BOUND_FAILS looks in a row.
-enum BoundNews { BOUND_STILL, BOUND_FAILING, BOUND_NEWS };
+// The launches before such a pass: how far the centroids have moved, the drift that leaves (drift_old ->
+// drift_new), the rows whose limit it has passed, those of them that the centroids' neighbours do not decide,
+// and the control block. BOUNDS_FIRST: zeros, and every row is measured. BOUNDS_FRESH: that, for a step that
+// leaves no limits; the next one's rows are all looked at. news_host (nullable, pinned): [BOUND_STILL]
+// receives 1 where no centroid has moved, [BOUND_FAILING] where most rows had to be measured at BOUND_FAILS looks
+// in a row, [BOUND_LISTED] the rows whose limit the drift had passed. grain: see RowBounds.
+enum BoundNews { BOUND_STILL, BOUND_FAILING, BOUND_LISTED, BOUND_NEWS };
 static const unsigned BOUND_FAILS = 3;
 static const int MAX_BOUND_CENTROIDS = 8192;
-int bound_segments(int64_t n);
+enum BoundStart { BOUNDS_GO, BOUNDS_FIRST, BOUNDS_FRESH };
+int bound_counts(int64_t n);
+bool neighbours_apply(int64_t n, int d, int k);
 template <typename T>
-int launch_bounds(hipStream_t s, const T *c_old, const T *c_new, const int *labels, const float *limit, int64_t n,
-                  int d, int k, float *moves, const double *drift_old, double *drift_new, float *drift_float, int *found,
-                  int *found_counts, int *listed, const BoundControl *ctl_old, BoundControl *ctl_new,
-                  unsigned *news_host = nullptr);
+int launch_bounds(hipStream_t s, const BoundBuffers &b, BoundStart start, const T *X, const T *xnorm, const T *c_old,
+                  const T *c_new, int *labels, int64_t n, int d, int k, const double *drift_old, double *drift_new,
+                  const BoundControl *ctl_old, BoundControl *ctl_new, unsigned *news_host, float grain);
+// The resolution distances are compared at by the two passes above.
+template <typename T>
+float bound_grain(int64_t n, int d, int k, bool fused);
 // What launch_assign (variant ASSIGN_AUTO) needs beside the rows and the k centroids for a shape:
 enum AssignInputs {
   ASSIGN_FROM_ROWS,       // nothing: xnorm and cnorm may be null, C need not be padded

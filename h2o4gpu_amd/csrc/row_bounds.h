@@ -27,6 +27,33 @@ struct BoundControl {
   unsigned fails;    // steps in a row whose list held most rows
   unsigned changed;  // 1: some row has a new label
   unsigned still;    // 1: no centroid has moved, and no row is measured
+  unsigned fresh;    // 1: no row has a limit yet
+  unsigned look;     // 1: decide_rows_kernel goes through the rows
+  unsigned listed;   // rows whose limit the drift had passed
+};
+
+// The nearest centroids of each centroid (bound_kernels.hip). matrix null: none are kept.
+// A pass over fewer listed rows than DECIDE_ROWS leaves CUs idle and takes as long whatever is taken from the list
+// (128 rows a workgroup; 261k x 298, k = 1000: 117 us, looking for neighbours 35 and through the list 50). What a
+// step needs the neighbours for is known when they have been found, so the list before it is asked as well.
+static const int NEAREST = 8;
+static const unsigned DECIDE_ROWS = 32768;
+struct Neighbours {
+  float *matrix = nullptr;  // [k][k] squared distances
+  float *dist = nullptr;    // [k][NEAREST + 1] ascending, rounded down; the last is that of the next one
+  int *at = nullptr;        // [k][NEAREST + 1]
+};
+
+// What a loop keeps beside the drift and the control blocks.
+struct BoundBuffers {
+  float *limit = nullptr;        // [n]
+  int *found = nullptr;          // [n]
+  int *listed = nullptr;         // [n]
+  int *found_counts = nullptr;   // [bound_counts(n)]
+  float *moves = nullptr;        // [k]
+  float *drift_float = nullptr;  // [k] the drift, for the pass
+  Neighbours near;
+  BoundControl *mid = nullptr;   // between the two packings of a step
 };
 
 struct RowBounds {

@@ -12,6 +12,12 @@ TILED = [("float32", 20003, 70, 260), ("float32", 9001, 101, 300), ("float32", 3
          ("float32", 5000, 160, 257), ("float32", 300, 67, 230), ("float32", 20000, 780, 66), ("float64", 20003, 80, 700),
          ("float64", 9001, 101, 130), ("float64", 12345, 96, 300), ("float64", 300, 75, 70)]
 
+# lists long enough for the centroids' neighbours to be asked in later steps too: models staged in LDS and not,
+# rows of whole 16-byte vectors and not, each number of lanes and pieces a row is dealt to
+TILED += [("float32", 100003, 68, 260), ("float32", 70001, 101, 300), ("float32", 70001, 130, 300), ("float32", 70001, 298, 100),
+          ("float32", 70001, 260, 100), ("float32", 36001, 601, 66), ("float64", 70001, 70, 300), ("float64", 70001, 33, 900),
+          ("float64", 70001, 129, 100), ("float64", 40001, 300, 70), ("float64", 36001, 601, 66)]
+
 # rows of whole 16-byte vectors and not, a model of one and several tiles, two wavefronts' layouts (d > 32),
 # the smallest k, sums with and without copies, less than a tile of rows
 FUSED = [("float32", 20003, 16, 140), ("float32", 30001, 32, 256), ("float32", 9001, 13, 300), ("float32", 12345, 30, 70),
