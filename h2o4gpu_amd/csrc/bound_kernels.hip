@@ -549,6 +549,55 @@ __global__ __launch_bounds__(decide_threads<LOCAL>()) void decide_rows_kernel(
   if (lane == 0) found_counts[seg] = cnt;
 }
 
+// mindist[i] = |x - c|^2 of each row and the centroid it is labelled with, from the differences (a row without
+// a label: the start value of the passes). Rows of LPR lanes, NV pieces of VW values a lane. Bound by reading the
+// rows.
+template <typename T, int VW, int LPR, int NV>
+__global__ __launch_bounds__(WG) void own_distances_kernel(const T *__restrict__ X, const T *__restrict__ C,
+                                                          const int *__restrict__ labels, T *__restrict__ mindist,
+                                                          int64_t n, int d, int k) {
+  constexpr int RPW = 64 / LPR, U = VW * NV * (int)sizeof(T) <= 16 ? 4 : 2;
+  typedef T vec_t __attribute__((ext_vector_type(VW), aligned(sizeof(T))));
+  const int lane = threadIdx.x & 63, sub = lane % LPR, pieces = (d + VW - 1) / VW;
+  const int64_t waves = (int64_t)gridDim.x * (WG / 64);
+  for (int64_t i0 = ((int64_t)blockIdx.x * (WG / 64) + (threadIdx.x >> 6)) * (RPW * U); i0 < n; i0 += waves * (RPW * U)) {
+    int own[U];
+    T s[U];
+    vec_t x[U][NV];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int64_t row = min(i0 + u * RPW + lane / LPR, n - 1);
+      own[u] = labels[row];
+#pragma unroll
+      for (int v = 0; v < NV; v++)
+        x[u][v] = *reinterpret_cast<const vec_t *>(X + row * d + (size_t)min(v * LPR + sub, pieces - 1) * VW);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const T *src = C + (size_t)((unsigned)own[u] < (unsigned)k ? own[u] : 0) * d;
+      s[u] = 0;
+#pragma unroll
+      for (int v = 0; v < NV; v++) {
+        if (v * LPR + sub < pieces) {
+          const vec_t cv = *reinterpret_cast<const vec_t *>(src + (size_t)(v * LPR + sub) * VW);
+#pragma unroll
+          for (int q = 0; q < VW; q++) {
+            const T e = x[u][v][q] - cv[q];
+            s[u] = fma(e, e, s[u]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+#pragma unroll
+      for (int off = 1; off < LPR; off <<= 1) s[u] += __shfl_xor(s[u], off, 64);
+      const int64_t row = i0 + u * RPW + lane / LPR;
+      if (sub == 0 && row < n) mindist[row] = (unsigned)own[u] < (unsigned)k ? s[u] : argmin_start<T>();
+    }
+  }
+}
+
 __global__ void first_bounds_kernel(double *__restrict__ drift, float *__restrict__ drift_float, int k,
                                     BoundControl *__restrict__ ctl, bool fresh) {
   for (int c = threadIdx.x; c < k; c += blockDim.x) drift[c] = drift_float[c] = 0.0f;
@@ -605,6 +654,38 @@ int launch_decide(hipStream_t s, const BoundBuffers &b, const T *X, const T *xno
 }
 
 }  // namespace
+
+template <typename T>
+int launch_own_distances(hipStream_t s, const T *X, const T *C, const int *labels, T *mindist, int64_t n, int d, int k,
+                         int num_cu) {
+  if (n < 1 || k < 1 || !own_distances_apply(d)) return H2O4GPU_KMEANS_EARG;
+  constexpr int VW = Mfma<T>::VW;
+#define KM_OWN(VW, LPR, NV)                                                                                         \
+  hipLaunchKernelGGL((own_distances_kernel<T, VW, LPR, NV>), dim3((unsigned)std::min<int64_t>(                      \
+                         (int64_t)num_cu * 8, (n + WG / LPR - 1) / (WG / LPR))), dim3(WG), 0, s, X, C, labels, mindist, n, d, k)
+  if (d % VW == 0) {
+    const int v = d / VW;
+    if (v <= 8) KM_OWN(VW, 8, 1);
+    else if (v <= 16) KM_OWN(VW, 16, 1);
+    else if (v <= 32) KM_OWN(VW, 32, 1);
+    else if (v <= 64) KM_OWN(VW, 64, 1);
+    else if (v <= 128) KM_OWN(VW, 64, 2);
+    else if (v <= 256) KM_OWN(VW, 64, 4);
+    else KM_OWN(VW, 64, 8);
+  } else {
+    if (d <= 64) KM_OWN(1, 16, 4);
+    else if (d <= 256) KM_OWN(1, 64, 4);
+    else if (d <= 512) KM_OWN(1, 64, 8);
+    else KM_OWN(1, 64, 16);
+  }
+#undef KM_OWN
+  KM_HIP_TRY(hipGetLastError());
+  return 0;
+}
+bool own_distances_apply(int d) { return d >= 1 && d <= 1024; }
+template int launch_own_distances<float>(hipStream_t, const float *, const float *, const int *, float *, int64_t, int, int, int);
+template int launch_own_distances<double>(hipStream_t, const double *, const double *, const int *, double *, int64_t, int, int,
+                                          int);
 
 int bound_segments(int64_t n) {
   const int64_t per = segment_rows(n);

@@ -1461,8 +1461,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     // 50k x 100, k = 300 (3 GF) 1.63 and 0.90, 200k (12 GF) 1.88 and 0.94.
     // Long rows with a handful of centroids are bound by reading them: 500k x 784 (1.6 GB), k = 10, twenty steps on
     // blobs 8.77 -> 3.39 ms, on noise 8.73 -> 9.60; 1M x 68 (0.3 GB), k = 4 3.29 -> 3.90 on either.
-    const bool long_rows = pick_assign_variant<T>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW;
-    if (opt_bounds == 1 && (long_rows ? (double)n * d * sizeof(T) < 4e8 : 2.0 * (double)n * k * d < (bound_fused ? 3e10 : 1e10)))
+    if (opt_bounds == 1 && (long_rows() ? (double)n * d * sizeof(T) < 4e8 : 2.0 * (double)n * k * d < (bound_fused ? 3e10 : 1e10)))
       return false;
     const int split = split_for(SPLIT_ASSIGN, k);
     if (!bound_fused && !bounded_assign_applies<T>(n, d, k, split, split_scratch(split, k, true, n))) return false;
@@ -1553,7 +1552,8 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     return step_async(want_shift, shift_host != nullptr, shift_host);
   }
-  int bounded_step(bool first, bool want_shift, T *shift_host = nullptr) {
+  // The assignment pass of a step (fused: with its sums, in *slots, for *run).
+  int bounded_pass(bool first, RunningSums *run, int *slots) {
     KM_TRY(ensure_work());
     if (!bound_fused) KM_TRY(ensure_cnorm());
     const int was = bound_cur;
@@ -1571,24 +1571,45 @@ struct Engine : h2o4gpu_kmeans_handle {
     rb.ctl = bound_ctl[bound_cur];
     rb.limit = bound.limit;
     rb.drift = bound.drift_float;
+    have_mindist = false;
     if (bound_fused) {
-      int slots = 0;
-      RunningSums run;
       PROFILED("assign_accumulate", launch_bounded_accumulate<T>(stream, X, xnorm, C[cur], labels, n, d, k, num_cu, psums,
-                                                                 pcounts, &slots, &run.tile_rows, rb));
-      have_mindist = false;
-      run.sums = run_sums;
-      run.counts_old = run_counts[was];
-      run.counts_new = run_counts[bound_cur];
-      run.ctl = rb.ctl;
-      return finish_update(slots, want_shift, shift_host, run);
+                                                                 pcounts, slots, &run->tile_rows, rb));
+      run->sums = run_sums;
+      run->counts_old = run_counts[was];
+      run->counts_new = run_counts[bound_cur];
+      run->ctl = rb.ctl;
+      return 0;
     }
     const int split = split_for(SPLIT_ASSIGN, k);
     PROFILED("assign", launch_bounded_assign<T>(stream, X, xnorm, C[cur], cnorm, labels, n, d, k,
                                                 split_scratch(split, k, true, n), rb));
-    have_mindist = false;
-    return update_async(want_shift, shift_host, &rb.ctl->changed);
+    return 0;
   }
+  int bounded_step(bool first, bool want_shift, T *shift_host = nullptr) {
+    RunningSums run;
+    int slots = 0;
+    KM_TRY(bounded_pass(first, &run, &slots));
+    if (bound_fused) return finish_update(slots, want_shift, shift_host, run);
+    return update_async(want_shift, shift_host, &bound_ctl[bound_cur]->changed);
+  }
+  // The relabel behind the last step of a bounded fit: the rows whose label may have changed, then every row's
+  // distance to its own centroid, for which the rows are read once (2M x 256, k = 1024 float64: 15.8 ms for a
+  // pass over all rows and centroids, 0.3 + 0.85 this way; 10M x 32, k = 256 0.82, 0.15 + 0.28).
+  // labelled: the labels are the final ones already.
+  int bounded_relabel(bool labelled) {
+    if (long_rows() || !own_distances_apply(d)) return assign();
+    if (!labelled) {
+      RunningSums run;
+      int slots = 0;
+      KM_TRY(bounded_pass(false, &run, &slots));
+    }
+    PROFILED("assign", launch_own_distances<T>(stream, X, C[cur], labels, mindist, n, d, k, num_cu));
+    have_mindist = true;
+    return 0;
+  }
+  // (bound by reading them, whatever is done with a row)
+  bool long_rows() const { return pick_assign_variant<T>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW; }
 
   // Steps over rows ordered in space (cell_kernels.hip). Ordering them takes as long as eight to ten
   // steps of the other kind, a step then a fifth to a half, so they are ordered where at least CELL_STEPS are to
@@ -1759,7 +1780,8 @@ struct Engine : h2o4gpu_kmeans_handle {
           done = true;
         }
         if (done || i == max_iterations - 1) {
-          KM_TRY(assign());  // final relabel with the final centroids
+          // final relabel with the final centroids
+          KM_TRY(bounded && i >= bounds_at ? bounded_relabel(still) : assign());
           break;
         }
       }
@@ -1916,9 +1938,9 @@ struct Engine : h2o4gpu_kmeans_handle {
         cur ^= 1;
         PROFILED("row_norms", launch_row_norms<T>(stream, C[cur], cnorm, k, d));
         cnorm_stale = false;
-        if (!have_mindist) KM_TRY(assign());
+        if (!have_mindist) KM_TRY(bounded && i + 1 >= bounds_at ? bounded_relabel(true) : assign());
       } else {
-        KM_TRY(assign());
+        KM_TRY(bounded && i >= bounds_at ? bounded_relabel(false) : assign());
       }
       break;
     }

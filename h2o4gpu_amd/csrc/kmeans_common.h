@@ -159,6 +159,11 @@ template <typename T>
 int launch_bounds(hipStream_t s, const BoundBuffers &b, BoundStart start, const T *X, const T *xnorm, const T *c_old,
                   const T *c_new, int *labels, int64_t n, int d, int k, const double *drift_old, double *drift_new,
                   const BoundControl *ctl_old, BoundControl *ctl_new, unsigned *news_host, float grain);
+// The squared distance of every row to the centroid it is labelled with, from the differences.
+bool own_distances_apply(int d);
+template <typename T>
+int launch_own_distances(hipStream_t s, const T *X, const T *C, const int *labels, T *mindist, int64_t n, int d, int k,
+                         int num_cu);
 // The resolution distances are compared at by the two passes above.
 template <typename T>
 float bound_grain(int64_t n, int d, int k, bool fused);
