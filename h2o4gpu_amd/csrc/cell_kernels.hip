@@ -270,7 +270,9 @@ __global__ __launch_bounds__(CELL_WG) void cell_step_kernel(const float *__restr
                                                            const CellBlock *__restrict__ blocks, int64_t n,
                                                            const float *__restrict__ C, int k,
                                                            double *__restrict__ psums, int *__restrict__ pcounts,
-                                                           int ncopy, unsigned long long *__restrict__ measured) {
+                                                           int ncopy, unsigned long long *__restrict__ measured,
+                                                           const unsigned *__restrict__ stopped) {
+  if (stopped != nullptr && *stopped != 0) return;
   constexpr int SD = D + 1;
   const int stride = cell_copy_stride(D, k);
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -440,7 +442,8 @@ int launch_cell_windows(hipStream_t s, const float *X, int64_t n, int d, const f
 }
 
 int launch_cell_step(hipStream_t s, const float *Xs, const CellBlock *blocks, int64_t n, const float *C, int d, int k,
-                     int num_cu, double *psums, int *pcounts, int *slots, unsigned long long *measured) {
+                     int num_cu, double *psums, int *pcounts, int *slots, unsigned long long *measured,
+                     const unsigned *stopped) {
   if (!cells_apply(n, d, k)) return H2O4GPU_KMEANS_EARG;
   // copies of the sums: what fits beside a second workgroup's
   int ncopy = 1;
@@ -449,7 +452,7 @@ int launch_cell_step(hipStream_t s, const float *Xs, const CellBlock *blocks, in
   const int grid = (int)std::min<int64_t>(2 * num_cu, cell_blocks(n));
   KM_TRY(ensure_dynamic_lds(reinterpret_cast<const void *>(cell_step_kernel<3>), lds));
   hipLaunchKernelGGL(cell_step_kernel<3>, dim3(grid), dim3(CELL_WG), lds, s, Xs, blocks, n, C, k, psums, pcounts, ncopy,
-                     measured);
+                     measured, stopped);
   KM_HIP_TRY(hipGetLastError());
   *slots = grid;
   return 0;

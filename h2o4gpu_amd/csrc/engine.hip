@@ -1623,6 +1623,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   int *cell_offsets = nullptr, *cell_counts = nullptr, *cell_hist = nullptr, *cell_seg = nullptr, *cell_total = nullptr;
   CellBlock *cell_block = nullptr;
   unsigned long long *cell_work = nullptr;
+  unsigned *cell_stop = nullptr;
   long long cell_measured = -1;  // rows the first such step of the last fit measured, in whole models' worth
   bool cells_possible() const {
     return sizeof(T) == 4 && opt_bounds && sets == 1 && opt_fuse && opt_assign == ASSIGN_AUTO && !opt_exact && settles() &&
@@ -1646,6 +1647,7 @@ struct Engine : h2o4gpu_kmeans_handle {
         want(list, &cell_seg, (size_t)32 * CELL_IDS);
         want(list, &cell_total, 1);
         want(list, &cell_work, 1);
+        want(list, &cell_stop, 1);
         if (allocate(list, &cell_slab) != 0) return 0;  // (every row is measured, then)
       }
       KM_TRY(ensure_work());
@@ -1668,14 +1670,51 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     return 0;
   }
-  int cells_step(bool want_shift, T *shift_host = nullptr) {
+  int cells_step(bool want_shift, StopRule stop = StopRule()) {
     int slots = 0;
     if constexpr (sizeof(T) == 4) {
       PROFILED("assign_accumulate", launch_cell_step(stream, cell_rows, cell_block, n, C[cur], d, k, num_cu, psums, pcounts,
-                                                     &slots, nullptr));
+                                                     &slots, nullptr, stop.stopped));
     }
     have_mindist = false;  // (nor labels: an assignment pass over all rows follows the loop)
-    return finish_update(slots, want_shift, shift_host);
+    return finish_update(slots, want_shift, nullptr, RunningSums(), stop);
+  }
+  // The rest of a fit with a convergence test, from iteration `first` on. A step takes no longer than the
+  // event and the wake-up that a host waiting for its scalar costs (some 6 us), so the device does the test, and
+  // the host looks at every eighth iteration, eight behind (10.1M x 3, k = 27, some 260 steps: 11.4 -> 10.9 ms a fit).
+  int cells_loop(int first, int max_iterations, double threshold, int *updates) {
+    KM_TRY(news_begin());
+    KM_TRY(launch_fill<int>(stream, reinterpret_cast<int *>(cell_stop), 0, 1));
+    const int start = cur;
+    int queued = 0;
+    while (first + queued < max_iterations) {
+      log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", first + queued, max_iterations);
+      StopRule stop;
+      stop.stopped = cell_stop;
+      stop.step_host = news_host + LOOP_STOPPED;
+      stop.threshold = threshold;
+      stop.step = (unsigned)(first + ++queued);
+      KM_TRY(cells_step(true, stop));
+      if (queued % 8 == 0) {
+        hipEvent_t *const ev = news_ready;
+        KM_HIP_TRY(hipEventRecord(ev[queued / 8 & 1], stream));
+        if (queued >= 16) KM_HIP_TRY(hipEventSynchronize(ev[(queued / 8 & 1) ^ 1]));
+        if (news(LOOP_STOPPED)) break;
+      }
+      if (g_stop_flag) {
+        fprintf(stderr, "Signal caught. Terminated early.\n");
+        g_stop_flag = 0;
+        break;
+      }
+    }
+    KM_HIP_TRY(hipStreamSynchronize(stream));
+    *updates = first + queued;
+    if (const unsigned step = news(LOOP_STOPPED)) {
+      log_msg(verbose, LOG_INFO, "Threshold triggered. Terminating early.");
+      *updates = (int)step;
+      cur = start ^ ((*updates - first) & 1);  // (what was queued behind it has changed nothing)
+    }
+    return 0;
   }
 
   int rows_measured(long long *rows) override {
@@ -1692,7 +1731,8 @@ struct Engine : h2o4gpu_kmeans_handle {
   // want_shift: the scalar sum((old - new)^2) of this step is left in shift2 (and in shift_host).
   // The norms of the new centroids are made by whoever needs them (ensure_cnorm): the fused kernels
   // do not.
-  int finish_update(int slots, bool want_shift, T *shift_host = nullptr, RunningSums run = RunningSums()) {
+  int finish_update(int slots, bool want_shift, T *shift_host = nullptr, RunningSums run = RunningSums(),
+                    StopRule stop = StopRule()) {
     int nsp = 0;
     if (sets > 1 && want_shift) {
       // per-set convergence: frozen sets keep their centroids; every set's squared shift is
@@ -1710,7 +1750,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     PROFILED("finalize", launch_finalize<T>(stream, slots, psums, pcounts, C[cur], C[cur ^ 1],
                                             counts, shift_partials, &nsp, d, k, nullptr, 1,
-                                            want_shift ? finalize_done : (unsigned *)nullptr, shift2, shift_host, run));
+                                            want_shift ? finalize_done : (unsigned *)nullptr, shift2, shift_host, run, stop));
     cnorm_stale = true;
     cur ^= 1;
     return 0;
@@ -1904,12 +1944,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     };
     auto queue_iteration = [&](int i) -> int {
       log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
-      if (cells_wanted && i >= 1 && (opt_bounds == 2 || steps_ahead(i) >= CELL_STEPS)) {
-        KM_TRY(cells_begin(&cells));
-        cells_wanted = false;
-      }
-      if (cells) KM_TRY(cells_step(true, host_shift + (i & 1)));
-      else if (bounded && i >= bounds_at) KM_TRY(bounded_step(i == bounds_at, true, host_shift + (i & 1)));
+      if (bounded && i >= bounds_at) KM_TRY(bounded_step(i == bounds_at, true, host_shift + (i & 1)));
       else if (bounded && i == bounds_at - 1) KM_TRY(bounds_prime(true, host_shift + (i & 1)));
       else KM_TRY(step_async(true, true, host_shift + (i & 1)));
       KM_HIP_TRY(hipEventRecord(shift_ready[i & 1], stream));
@@ -1919,7 +1954,12 @@ struct Engine : h2o4gpu_kmeans_handle {
     KM_TRY(queue_iteration(0));
     int updates = 0;
     for (int i = 0; i < max_iterations; i++) {
-      const bool queued_next = i + 1 < max_iterations;
+      bool queued_next = i + 1 < max_iterations;
+      if (queued_next && cells_wanted && (opt_bounds == 2 || steps_ahead(i + 1) >= CELL_STEPS)) {
+        KM_TRY(cells_begin(&cells));
+        cells_wanted = false;
+        if (cells) queued_next = false;
+      }
       if (bounded && i + 1 >= bounds_at) bounds_failing(i + 1, max_iterations);
       if (queued_next) KM_TRY(queue_iteration(i + 1));
       KM_HIP_TRY(hipEventSynchronize(shift_ready[i & 1]));
@@ -1933,6 +1973,7 @@ struct Engine : h2o4gpu_kmeans_handle {
         done = true;
       }
       if (!done && queued_next) continue;
+      if (!done && cells) KM_TRY(cells_loop(i + 1, max_iterations, threshold, &updates));
       if (queued_next) {
         // labels and minimum distances of the queued iteration are the final relabel
         cur ^= 1;

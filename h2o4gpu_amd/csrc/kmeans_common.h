@@ -148,8 +148,8 @@ int launch_bounded_accumulate(hipStream_t s, const T *X, const T *xnorm, const T
 // and the control block. BOUNDS_FIRST: zeros, and every row is measured. BOUNDS_FRESH: that, for a step that
 // leaves no limits; the next one's rows are all looked at. news_host (nullable, pinned): [BOUND_STILL]
 // receives 1 where no centroid has moved, [BOUND_FAILING] where most rows had to be measured at BOUND_FAILS looks
-// in a row, [BOUND_LISTED] the rows whose limit the drift had passed. grain: see RowBounds.
-enum BoundNews { BOUND_STILL, BOUND_FAILING, BOUND_LISTED, BOUND_NEWS };
+// in a row, [BOUND_LISTED] the rows whose limit the drift had passed. ([LOOP_STOPPED]: StopRule's step.) grain: see RowBounds.
+enum BoundNews { BOUND_STILL, BOUND_FAILING, BOUND_LISTED, LOOP_STOPPED, BOUND_NEWS };
 static const unsigned BOUND_FAILS = 3;
 static const int MAX_BOUND_CENTROIDS = 8192;
 enum BoundStart { BOUNDS_GO, BOUNDS_FIRST, BOUNDS_FRESH };
@@ -202,7 +202,7 @@ int launch_shortrow(hipStream_t s, const float *X, const float *C, int *labels, 
 // blocks of 64 (cell_kernels.hip). ids: a number below CELL_IDS per row, whose order (launch_bucket_rows) the
 // windows then refine; range: [cell_range_values()], Xs: [n][d], blocks: [cell_blocks(n)]. The step leaves
 // partial sums and counts of at most 2 * num_cu slots and no labels; measured (nullable, zero before): receives
-// how many centroids the blocks' rows were measured against, added up over the blocks.
+// how many centroids the blocks' rows were measured against, added up over the blocks; stopped: see StopRule.
 struct CellBlock {
   float lo[4], hi[4];
   double sum[4];
@@ -215,7 +215,8 @@ int launch_cell_ids(hipStream_t s, const float *X, int64_t n, int d, float *rang
 int launch_cell_windows(hipStream_t s, const float *X, int64_t n, int d, const float *range, const int *order,
                         float *Xs, CellBlock *blocks);
 int launch_cell_step(hipStream_t s, const float *Xs, const CellBlock *blocks, int64_t n, const float *C, int d, int k,
-                     int num_cu, double *psums, int *pcounts, int *slots, unsigned long long *measured);
+                     int num_cu, double *psums, int *pcounts, int *slots, unsigned long long *measured,
+                     const unsigned *stopped = nullptr);
 const char *assign_variant_name(int variant);
 // split (float32 matrix-core kernels; 0, 6 or 9): run the dot products on the bfloat16
 // matrix pipe as that many products of bfloat16 parts per feature pair (9: every product
@@ -324,12 +325,21 @@ struct RunningSums {
   const BoundControl *ctl = nullptr;
   int tile_rows = 0;  // listed rows a workgroup takes at a time: fewer tiles, fewer slots written
 };
+// A loop that is queued ahead of its convergence test: the update whose shift is below the threshold says so, and
+// the launches behind it that are given the flag do nothing.
+struct StopRule {
+  unsigned *stopped = nullptr;    // device, 0 at first; null: no such test
+  unsigned *step_host = nullptr;  // pinned: receives `step`
+  double threshold = 0;
+  unsigned step = 0;
+};
 template <typename T>
 int launch_finalize(hipStream_t s, int slots, const double *psums,
                     const int *pcounts, const T *c_old, T *c_new, int *counts,
                     T *shift_partials, int *n_shift_partials, int d, int k,
                     const int *frozen = nullptr, int kps = 1, unsigned *done = nullptr,
-                    T *shift2 = nullptr, T *shift_host = nullptr, RunningSums run = RunningSums());
+                    T *shift2 = nullptr, T *shift_host = nullptr, RunningSums run = RunningSums(),
+                    StopRule stop = StopRule());
 // Pass 3: cnorm of the new centroids and the fixed-order sum of the shift
 // partials into *shift2.
 template <typename T>

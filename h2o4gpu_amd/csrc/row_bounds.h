@@ -10,9 +10,9 @@
 //
 // 10M x 32, k = 256 blobs from random rows: the third step measures all rows (1.05 ms, 0.88 without limits),
 // the fifth 30 %, the ninth 10, the thirtieth 5 (0.10 ms, a third of it looking for them); thirty steps
-// 30.3 -> 11.5 ms. 261k x 298, k = 1000, a hundred steps 93 -> 16.5 ms, 2M x 256, k = 1024 float64, twenty
-// 350 -> 138. Data without clusters (normal noise) keeps all rows on the list and pays for the limits:
-// 1 to 6 % of twenty steps, 1 to 12 % of eight.
+// 30.3 -> 11.4 ms. 261k x 298, k = 1000, a hundred steps 93 -> 12.2 ms, 2M x 256, k = 1024 float64, twenty
+// 350 -> 81, 500k x 784, k = 10, twenty 9.8 -> 3.9. Data without clusters (normal noise) keeps all rows on the list and
+// pays for the limits: 0 to 5 % of twenty steps, 8 where a step is no more than reading long rows.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -969,13 +969,24 @@ __device__ __forceinline__ T sum_shift_partials(const T *shift_partials, int n) 
   return red[0];
 }
 
+template <typename T>
+__device__ __forceinline__ void leave_shift(T sum, T *shift2, T *shift_host, const StopRule &stop) {
+  *shift2 = sum;
+  if (shift_host) __hip_atomic_store(shift_host, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (stop.stopped != nullptr && (double)sum < stop.threshold) {
+    *stop.stopped = 1;
+    __hip_atomic_store(stop.step_host, stop.step, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 template <typename T, int EPW>
 __global__ __launch_bounds__(WG) void finalize_kernel(
     const double *__restrict__ psums, const int *__restrict__ pcounts, int row_blocks,
     const T *__restrict__ c_old, T *__restrict__ c_new, int *__restrict__ counts,
     T *__restrict__ shift_partials, int d, int k, const int *__restrict__ frozen, int kps,
-    unsigned *__restrict__ done, T *__restrict__ shift2, T *__restrict__ shift_host, RunningSums run) {
+    unsigned *__restrict__ done, T *__restrict__ shift2, T *__restrict__ shift_host, RunningSums run, StopRule stop) {
 #pragma clang fp contract(off)
+  if (stop.stopped != nullptr && *stop.stopped != 0) return;
   constexpr int RS = WG / EPW;
   const bool changes = run.sums != nullptr && run.ctl->full == 0;
   if (changes) row_blocks = min(row_blocks, (int)((run.ctl->count + run.tile_rows - 1) / run.tile_rows));
@@ -1064,8 +1075,7 @@ __global__ __launch_bounds__(WG) void finalize_kernel(
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   const T sum = sum_shift_partials<T>(shift_partials, (int)gridDim.x);
   if (tid == 0) {
-    *shift2 = sum;
-    if (shift_host) __hip_atomic_store(shift_host, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    leave_shift(sum, shift2, shift_host, stop);
     *done = 0;  // for the next launch
   }
 }
@@ -1079,15 +1089,13 @@ template <typename T>
 __global__ __launch_bounds__(WG) void post_update_kernel(
     const T *__restrict__ c_new, T *__restrict__ cnorm,
     const T *__restrict__ shift_partials, int n_partials, T *__restrict__ shift2,
-    T *__restrict__ shift_host, int d, int k) {
+    T *__restrict__ shift_host, int d, int k, StopRule stop) {
 #pragma clang fp contract(off)
+  if (stop.stopped != nullptr && *stop.stopped != 0) return;
   const int tid = threadIdx.x;
   if (blockIdx.x == gridDim.x - 1) {
     const T sum = sum_shift_partials<T>(shift_partials, n_partials);
-    if (tid == 0) {
-      *shift2 = sum;
-      if (shift_host) __hip_atomic_store(shift_host, sum, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (tid == 0) leave_shift(sum, shift2, shift_host, stop);
     return;
   }
   const int c = blockIdx.x * WG + tid;
@@ -1105,7 +1113,7 @@ template <typename T>
 int launch_finalize(hipStream_t s, int slots, const double *psums,
                     const int *pcounts, const T *c_old, T *c_new, int *counts,
                     T *shift_partials, int *n_shift_partials, int d, int k, const int *frozen,
-                    int kps, unsigned *done, T *shift2, T *shift_host, RunningSums run) {
+                    int kps, unsigned *done, T *shift2, T *shift_host, RunningSums run, StopRule stop) {
   const int64_t kd = (int64_t)k * d;
   // (a stacked model always takes the wide form: its sets' partials must not share a block)
   const bool narrow = kd <= FINALIZE_NARROW_KD && slots >= 256 && frozen == nullptr;
@@ -1116,13 +1124,13 @@ int launch_finalize(hipStream_t s, int slots, const double *psums,
   if (sum_to) done = nullptr;
   if (narrow)
     hipLaunchKernelGGL((finalize_kernel<T, 4>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
-                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host, run);
+                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host, run, stop);
   else
     hipLaunchKernelGGL((finalize_kernel<T, 32>), dim3(blocks), dim3(WG), 0, s, psums, pcounts,
-                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host, run);
+                       slots, c_old, c_new, counts, shift_partials, d, k, frozen, kps, done, shift2, shift_host, run, stop);
   if (sum_to)
     hipLaunchKernelGGL((post_update_kernel<T>), dim3(1), dim3(WG), 0, s, c_new, (T *)nullptr, shift_partials,
-                       blocks, sum_to, shift_host, d, k);
+                       blocks, sum_to, shift_host, d, k, stop);
   KM_HIP_TRY(hipGetLastError());
   *n_shift_partials = blocks;
   return 0;
@@ -1138,7 +1146,7 @@ int launch_post_update(hipStream_t s, const T *c_new, T *cnorm,
   const int blocks = separate_norms ? 1 : (k + WG - 1) / WG + 1;
   hipLaunchKernelGGL((post_update_kernel<T>), dim3(blocks), dim3(WG), 0, s, c_new,
                      separate_norms ? (T *)nullptr : cnorm, shift_partials, n_shift_partials,
-                     shift2, (T *)nullptr, d, k);
+                     shift2, (T *)nullptr, d, k, StopRule());
   KM_HIP_TRY(hipGetLastError());
   if (separate_norms) return launch_row_norms<T>(s, c_new, cnorm, k, d);
   return 0;
@@ -1225,7 +1233,7 @@ template int launch_bucketed_accumulate<double>(hipStream_t, const double *, con
   template UpdatePlan plan_update<T>(int64_t, int, int, int);                        \
   template int launch_finalize<T>(hipStream_t, int, const double *,                  \
                                   const int *, const T *, T *, int *, T *, int *,    \
-                                  int, int, const int *, int, unsigned *, T *, T *, RunningSums);                       \
+                                  int, int, const int *, int, unsigned *, T *, T *, RunningSums, StopRule);                       \
   template int launch_post_update<T>(hipStream_t, const T *, T *, const T *, int,    \
                                      T *, int, int);                                 \
   template int launch_sum<T>(hipStream_t, const T *, int64_t, double *, int,         \
