@@ -274,12 +274,15 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * fails the picks fall back to the other form); 0 runs one small kernel per pick, as
  * "assign" = 1 always does.
  * "bounds" = 1 (default) lets a fit of ten steps or more keep, from its third step on, how far
- * each row is from changing its label, and measure only rows that may have changed it (shapes of the
- * tiled kernels, float32 shapes of the row-stationary one with six products and of the one for long rows
- * and a handful of centroids, where there is enough to measure). Labels and centroids are those of 0, which measures every row in every step; 2 does it for fits of any length and
- * shapes of any size. Twelve bytes of device memory a row; where they cannot be had every row is measured.
- * Float32 rows of three features and 17 to 128 centroids: long fits order a copy of the rows in space and
- * measure only blocks of them that more than one centroid may be the nearest in (cell_kernels.hip; 26 bytes a row).
+ * each row is from changing its label, and measure only rows that may have changed it
+ * (row_bounds.h: shapes of the tiled kernels, float32 shapes of the row-stationary one with six
+ * products and of the one for long rows and a handful of centroids, where there is enough to
+ * measure). Labels and centroids are those of 0, which measures every row in every step; 2 does
+ * it for fits of any length and shapes of any size. Twelve bytes of device memory a row, and four
+ * per pair of up to 4096 centroids in tiled shapes; where they cannot be had every row is measured.
+ * Minimum distances of such fits are made from the differences. Float32 rows of three features and
+ * 17 to 128 centroids: long fits order a copy of the rows in space and measure only blocks of
+ * them that more than one centroid may be the nearest in (cell_kernels.hip; 26 bytes a row).
  * Unknown names return EARG. */
 int h2o4gpu_kmeans_set_option(h2o4gpu_kmeans_handle *h, const char *name,
                               int value);
