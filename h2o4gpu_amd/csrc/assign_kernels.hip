@@ -1401,10 +1401,16 @@ __global__ __launch_bounds__((XB ? 1 : 2) * BCW * 64, BCW == 4 && !XB ? 1 : 2) v
   if (SPLIT == 0 && ties.count && *ties.count <= ties.cap) return;
   // (SPLIT) the float32 launch behind this one is to run: nothing left to do here. Only workgroups that
   // start late look (261k x 298, k = 1000, nearly every row a tie: 2.03 -> 1.82 ms; transform 100k x 784,
-  // k = 4096 with an infinite row: 7.2 -> 5.3).
+  // k = 4096 with an infinite row: 7.2 -> 5.3). (LIST) That launch makes labels and no limits: the rows are to
+  // be measured again.
   if (SPLIT != 0 && blockIdx.x >= 1024 && ties.count &&
-      __hip_atomic_load(ties.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > ties.cap)
+      __hip_atomic_load(ties.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > ties.cap) {
+    if constexpr (LIST) {
+      const int64_t i = (int64_t)blockIdx.x * 128 + threadIdx.x;
+      if (threadIdx.x < 128 && i < n) rb.limit[at.row(i)] = -pos_inf<float>();
+    }
     return;
+  }
   typedef Mfma<T> M;
   typedef TiledCfg<T, BCW, WIDE, SPLIT, XB> Cfg;
   static_assert(!XB || SPLIT == 6, "bfloat16 rows: a form of the split kernel");
@@ -3228,8 +3234,8 @@ int launch_bounded_assign(hipStream_t s, const T *X, const T *xnorm, const T *C,
     else
       KM_TRY((launch_tiled_bcw<T, 0, 2, false, 6>(s, X, xnorm, C, cnorm, labels, none, none, n, n, d, k, false, parts,
                                                   true, ties, &rb)));
-    // (more ties than the list holds: all rows, by the float32 instructions. Their limits stand: those of
-    // near ties are passed already.)
+    // (more ties than the list holds: all rows, by the float32 instructions. The limits that the split launch has
+    // left stand: those of near ties, and of rows it has not come to, are passed already.)
     return launch_tiled_plain<T, 0>(s, X, xnorm, C, cnorm, labels, none, none, n, n, d, k, false, direct, ties);
   } else {
     return launch_tiled_bcw<T, 0, 2>(s, X, xnorm, C, cnorm, labels, none, none, n, n, d, k, false, nullptr, direct,

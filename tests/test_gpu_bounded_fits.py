@@ -1,0 +1,75 @@
+"""Fits that measure only the rows whose label may have changed, where their parts meet: rows that no pass
+has given a limit, steps that go without limits and begin anew, sums carried from step to step, handles that
+are used again, the rule that makes fits bounded by themselves, and what they need memory for."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def run(h, X, C, steps, bounds=None, tol=0.0):
+    if bounds is not None:
+        h.set_option("bounds", bounds)
+    h.set_centroids(C)
+    it = h.fit(steps, tol)
+    return dict(it=it, labels=h.labels(), centers=h.centroids(), mind=h.min_distances(), counts=h.counts(),
+                measured=h.rows_measured())
+
+
+def fit(hip, X, C, steps, bounds=None, tol=0.0):
+    with hip.Handle(X.shape[0], X.shape[1], C.shape[0], X.dtype) as h:
+        h.set_data(X)
+        return run(h, X, C, steps, bounds, tol)
+
+
+def same(got, want, exact=True):
+    """exact False: float64 sums made in LDS, in the order their rows arrive (off by up to the rows' number in
+    eps of the largest value)."""
+    assert got["it"] == want["it"]
+    assert np.array_equal(got["labels"], want["labels"])
+    assert np.array_equal(got["counts"], want["counts"])
+    if exact:
+        assert np.array_equal(got["centers"], want["centers"], equal_nan=True)
+    else:
+        big = np.abs(want["centers"]).max()
+        assert np.allclose(got["centers"], want["centers"], rtol=0, atol=1000 * np.finfo(np.float64).eps * big)
+
+
+def border_after_two_steps(q, tied, z):
+    """Between two centroids of the rows z and of so many rows at q."""
+    z, w = np.concatenate([[q], z]), np.concatenate([[tied], np.ones(len(z))])
+    c = np.array([0.0, 0.02])
+    for _ in range(2):
+        right = z > c.mean()
+        c = np.array([np.average(z[~right], weights=w[~right]), np.average(z[right], weights=w[right])])
+    return c.mean()
+
+
+def test_near_ties_that_fill_their_list_once(hip):
+    """The first step that leaves limits finds more near ties than their list holds (a seventh of the rows, on the
+    border of two centroids that moves on), so that the pass ends early and another one labels the rows. The rows it
+    had not come to have no limit from it, and must not be held to what the memory says: here the limits of
+    a fit before, with centroids so far apart that they are good for the whole fit."""
+    n, d, k, tied, line = 200003, 68, 3200, 30000, 60000
+    rng = np.random.default_rng(0)
+    z_line, z_rest = rng.uniform(0, 1, line), rng.uniform(3, 4, n - tied - line)
+    q, width = 0.4, 0.2  # the place that is the border after two steps, if the tied rows are there
+    for _ in range(3):
+        places = np.linspace(q - width, q + width, 201)
+        off = [abs(border_after_two_steps(p, tied, z_line) - p) for p in places]
+        q, width = places[int(np.argmin(off))], width / 50
+    assert min(off) < 1e-5  # (rows within some 1e-4 of the border are near ties)
+    X = np.full((n, d), 0.5, np.float32)
+    X[:, 0] = np.concatenate([np.full(tied, q), z_line, z_rest])
+    C = np.full((k, d), 0.5, np.float32)
+    C[:, 0] = np.concatenate([[0.0, 0.02], 3 + np.linspace(0, 0.02, 40), 1000 + np.arange(k - 42)])
+    far = C.copy()
+    far[:42, 0] = 2000 + np.arange(42) * 10
+    far[0, 0], far[2, 0] = 0.3, 3.5
+    with hip.Handle(n, d, k, np.float32) as h:
+        h.set_data(X)
+        assert run(h, X, far, 6, 2)["measured"] < n
+        got = run(h, X, C, 12, 2)
+    want = fit(hip, X, C, 12, 0)
+    assert np.array_equal(got["labels"], want["labels"])
+    same(got, want)
