@@ -1459,8 +1459,10 @@ struct Engine : h2o4gpu_kmeans_handle {
     // on noise: fused 200k x 32, k = 256 0.96 and 0.79 times as fast, 1M (16 GF) 1.54 and 0.94, 2M (33 GF)
     // 1.93 and 1.00; tiled 20k x 256, k = 300 (3 GF) 1.99 and 0.94, 100k (15 GF) 1.88 and 0.96; float64
     // 50k x 100, k = 300 (3 GF) 1.63 and 0.90, 200k (12 GF) 1.88 and 0.94.
-    // Long rows with a handful of centroids are bound by reading them: 500k x 784 (1.6 GB), k = 10, twenty steps on
-    // blobs 8.77 -> 3.39 ms, on noise 8.73 -> 9.60; 1M x 68 (0.3 GB), k = 4 3.29 -> 3.90 on either.
+    // Long rows with a handful of centroids are bound by reading them: twenty steps on blobs and on noise, 784
+    // features, 1.6 GB, k = 2 to 16 2.4 to 4.7 and 0.93 to 0.97 times as fast, 256 features, 0.5 GB, k = 3 and 8 4.1
+    // and 2.0, 0.92 and 0.96; below the line 0.3 GB, d = 132 to 784, k = 3 to 12 1.7 to 3.7 and 0.80 to 0.91, 0.1 GB
+    // 1.1 to 3.1 and 0.84 to 0.90. (68 features, k = 3 and 4, 0.2 to 0.8 GB gain on noise too: 1.2 to 1.5.)
     if (opt_bounds == 1 && (long_rows() ? (double)n * d * sizeof(T) < 4e8 : 2.0 * (double)n * k * d < (bound_fused ? 3e10 : 1e10)))
       return false;
     const int split = split_for(SPLIT_ASSIGN, k);

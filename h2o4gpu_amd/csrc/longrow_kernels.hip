@@ -204,9 +204,10 @@ __global__ __launch_bounds__(lr_threads<T>(NVL)) void lloyd_longrow_kernel(
         bidx = my_k;
       }
     }
-    // the lanes of a row differ in lane bits 2..5
+    // the lanes of a row differ in lane bits 2 to NB - 1; from bit NB on they hold copies, which a second minimum
+    // must not meet
 #pragma unroll
-    for (int m = 4; m < 64; m <<= 1) {
+    for (int m = 4; m < (1 << NB); m <<= 1) {
       const T ob = __shfl_xor(best, m, 64);
       const int oi = __shfl_xor(bidx, m, 64);
       if constexpr (LIST) {

@@ -73,3 +73,35 @@ def test_near_ties_that_fill_their_list_once(hip):
     want = fit(hip, X, C, 12, 0)
     assert np.array_equal(got["labels"], want["labels"])
     same(got, want)
+
+
+def strips(n, d, k, dtype, seed):
+    """Rows along lines of eight centroids each, the lines far apart, whose centroids go on moving a little for many
+    steps; sums of such values are exact."""
+    rng = np.random.default_rng(seed)
+    at = rng.integers(0, k, n)
+    X = np.round(rng.standard_normal((n, d)) * 64) / 1024
+    C = np.zeros((k, d))
+    X[:, 0] = np.round((8 * (at % 8) + rng.uniform(0, 8, n)) * 4096) / 4096
+    C[:, 0] = 8.0 * (np.arange(k) % 8) + rng.uniform(3, 5, k)
+    for A, c in ((X, at), (C, np.arange(k))):
+        line = c // 8 - 1
+        A[np.arange(len(A))[line >= 0], 1 + line[line >= 0] % (d - 1)] += 40.0 * (1 + line[line >= 0] // (d - 1))
+    return X.astype(dtype), C.astype(dtype)
+
+
+# each form of the long-row kernel (sums of 4, 8 and 16 centroids, one to four vectors a lane), the row-stationary
+# one, tiled ones with and without the centroids' neighbours
+ALONE = [("float32", 20003, d, k) for d, k in ((68, 2), (68, 3), (784, 4), (132, 5), (516, 8), (132, 8), (784, 10), (260, 16))]
+ALONE += [("float32", 30001, 32, 80), ("float32", 70001, 13, 300), ("float32", 70001, 132, 130), ("float32", 70001, 101, 300),
+          ("float64", 20003, 80, 130), ("float64", 40001, 101, 130)]
+
+
+@pytest.mark.parametrize("dtype,n,d,k", ALONE)
+def test_rows_are_left_alone_while_centroids_move(hip, dtype, n, d, k):
+    X, C = strips(n, d, k, dtype, 3)
+    fits = [fit(hip, X, C, s, 2) for s in range(4, 25)]
+    moving = [i for i in range(20) if not np.array_equal(fits[i]["centers"], fits[i + 1]["centers"])]
+    assert any(0 < fits[i]["measured"] < n / 2 for i in moving), [fits[i]["measured"] for i in moving]
+    for i in (0, 3, 8, 15):
+        same(fits[i], fit(hip, X, C, 4 + i, 0), dtype == "float32")
