@@ -695,7 +695,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       if (d_split) (void)hipFree(d_split);
       d_split = nullptr;
       split_bytes = 0;
-      if (dalloc(&d_split, need) != 0) return sc;
+      if (dalloc(&d_split, need, true) != 0) return sc;
       split_bytes = need;
     }
     sc.ptr = d_split;
@@ -712,13 +712,15 @@ struct Engine : h2o4gpu_kmeans_handle {
   size_t set_off() const { return sets > 1 ? (size_t)cur_set * kps : 0; }  // first model row of the set
   size_t row_off() const { return sets > 1 ? (size_t)cur_set * (size_t)n : 0; }  // its block of labels
 
+  // optional: the call goes on without it, and has nothing to report
   template <typename U>
-  int dalloc(U **p, size_t count) {
+  int dalloc(U **p, size_t count, bool optional = false) {
     *p = nullptr;
     if (count == 0) count = 1;
     hipError_t e = hipMalloc(reinterpret_cast<void **>(p), count * sizeof(U));
     if (e != hipSuccess) {
       (void)hipGetLastError();
+      if (optional) return H2O4GPU_KMEANS_EALLOC;
       // the reference's message and level (log_error(verbose, ...), kmeans_impl.h:81-94):
       // printed when verbose >= 200, and the call returns -1
       log_msg(verbose, LOG_ERROR,
@@ -746,10 +748,10 @@ struct Engine : h2o4gpu_kmeans_handle {
     list.push_back(Want{reinterpret_cast<void **>(p), std::max<size_t>(count, 1) * sizeof(U)});
   }
   static size_t slab_step(size_t bytes) { return (bytes + 255) / 256 * 256; }
-  int allocate(const std::vector<Want> &list, unsigned char **slab) {
+  int allocate(const std::vector<Want> &list, unsigned char **slab, bool optional = false) {
     size_t total = 0;
     for (const Want &w : list) total += slab_step(w.bytes);
-    KM_TRY(dalloc(slab, total));
+    KM_TRY(dalloc(slab, total, optional));
     unsigned char *at = *slab;
     for (const Want &w : list) {
       *w.ptr = at;
@@ -1451,7 +1453,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   int *run_counts[2] = {nullptr, nullptr};
   bool bounds_begin(int max_iterations) {
     bound_steps = 0;
-    if (!opt_bounds || (opt_bounds == 1 && max_iterations < BOUNDS_ITERATIONS) || sets > 1 || opt_assign != ASSIGN_AUTO || opt_exact ||
+    if (max_iterations < (opt_bounds == 1 ? BOUNDS_ITERATIONS : 1) || !opt_bounds || sets > 1 || opt_assign != ASSIGN_AUTO || opt_exact ||
         opt_split != SPLIT_DEFAULT)
       return false;
     bound_fused = opt_fuse && bounded_accumulate_applies<T>(n, d, k, split_for(SPLIT_FUSED, k), num_cu);
@@ -1467,6 +1469,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       return false;
     const int split = split_for(SPLIT_ASSIGN, k);
     if (!bound_fused && !bounded_assign_applies<T>(n, d, k, split, split_scratch(split, k, true, n))) return false;
+    if (!news_possible()) return false;
     if (!bound_slab) {
       // (Rows of the fused kernels are measured against all centroids in the time it takes to look at a few
       // of them: 10M x 32, k = 256 0.9 ms and 1.4.)
@@ -1490,7 +1493,7 @@ struct Engine : h2o4gpu_kmeans_handle {
         want(list, &bound_ctl[i], 1);
       }
       want(list, &run_sums, (size_t)k * d);
-      if (allocate(list, &bound_slab) != 0) return false;  // (every row is measured, then)
+      if (allocate(list, &bound_slab, true) != 0) return false;  // (every row is measured, then)
     }
     return true;
   }
@@ -1506,16 +1509,21 @@ struct Engine : h2o4gpu_kmeans_handle {
   hipEvent_t news_ready[2] = {nullptr, nullptr};
   int bounds_at = 0, bounds_pause = 0;  // the step that begins to keep bounds, and how long the next pause is
   unsigned news(BoundNews what) const { return const_cast<volatile unsigned *>(news_host)[what]; }
-  int news_begin() {
-    if (!news_host) {
-      KM_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&news_host), BOUND_NEWS * sizeof(unsigned),
-                               hipHostMallocCoherent | hipHostMallocMapped));
-      for (auto &ev : news_ready) KM_HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  bool news_possible() {
+    for (auto &ev : news_ready) {
+      if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) ev = nullptr;
     }
+    if (!news_host && hipHostMalloc(reinterpret_cast<void **>(&news_host), BOUND_NEWS * sizeof(unsigned),
+                                    hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess)
+      news_host = nullptr;
+    if (news_host && news_ready[0] && news_ready[1]) return true;
+    (void)hipGetLastError();
+    return false;
+  }
+  void news_begin() {
     for (int i = 0; i < BOUND_NEWS; i++) const_cast<volatile unsigned *>(news_host)[i] = i == BOUND_LISTED ? ~0u : 0u;  // (nothing is under way)
     bounds_at = BOUNDS_FROM;
     bounds_pause = 16;
-    return 0;
   }
   // before bounded step i: (a kernel says so once, and then not before bounds are begun anew)
   void bounds_failing(int i, int max_iterations) {
@@ -1635,6 +1643,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   int cells_begin(bool *use) {
     *use = false;
     if constexpr (sizeof(T) == 4) {
+      if (!news_possible()) return 0;
       if (!cell_slab) {
         std::vector<Want> list;
         want(list, &cell_rows, (size_t)n * d);
@@ -1650,9 +1659,8 @@ struct Engine : h2o4gpu_kmeans_handle {
         want(list, &cell_total, 1);
         want(list, &cell_work, 1);
         want(list, &cell_stop, 1);
-        if (allocate(list, &cell_slab) != 0) return 0;  // (every row is measured, then)
+        if (allocate(list, &cell_slab, true) != 0) return 0;  // (every row is measured, then)
       }
-      KM_TRY(ensure_work());
       prof_begin("cells");
       KM_TRY(launch_cell_ids(stream, X, n, d, cell_range, cell_ids));
       KM_TRY(launch_bucket_rows(stream, cell_ids, cell_order, cell_order_id, cell_offsets, cell_hist, cell_seg, cell_total,
@@ -1685,7 +1693,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   // event and the wake-up that a host waiting for its scalar costs (some 6 us), so the device does the test, and
   // the host looks at every eighth iteration, eight behind (10.1M x 3, k = 27, some 260 steps: 11.4 -> 10.9 ms a fit).
   int cells_loop(int first, int max_iterations, double threshold, int *updates) {
-    KM_TRY(news_begin());
+    news_begin();
     KM_TRY(launch_fill<int>(stream, reinterpret_cast<int *>(cell_stop), 0, 1));
     const int start = cur;
     int queued = 0;
@@ -1782,6 +1790,8 @@ struct Engine : h2o4gpu_kmeans_handle {
     if (!have_data || !have_centroids) return H2O4GPU_KMEANS_ESTATE;
     maybe_install_signal_handlers();
     int updates = 0;
+    // (what the steps cannot do without, before anything that only makes them faster)
+    if (max_iterations > 0) KM_TRY(ensure_work());
     const bool bounded = bounds_begin(max_iterations);
     bool cells = false, cells_wanted = cells_possible(), still = false;
     cell_measured = -1;
@@ -1797,7 +1807,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     } else if (threshold > 0 && max_iterations > 0) {
       KM_TRY(fit_with_threshold(max_iterations, threshold, bounded, &updates));
     } else {
-      if (bounded) KM_TRY(news_begin());
+      if (bounded) news_begin();
       for (int i = 0; i < max_iterations; i++) {
         log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
         if (bounded && i >= bounds_at && !still) {
@@ -1952,7 +1962,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       KM_HIP_TRY(hipEventRecord(shift_ready[i & 1], stream));
       return 0;
     };
-    if (bounded) KM_TRY(news_begin());
+    if (bounded) news_begin();
     KM_TRY(queue_iteration(0));
     int updates = 0;
     for (int i = 0; i < max_iterations; i++) {

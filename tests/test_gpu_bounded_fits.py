@@ -105,3 +105,39 @@ def test_rows_are_left_alone_while_centroids_move(hip, dtype, n, d, k):
     assert any(0 < fits[i]["measured"] < n / 2 for i in moving), [fits[i]["measured"] for i in moving]
     for i in (0, 3, 8, 15):
         same(fits[i], fit(hip, X, C, 4 + i, 0), dtype == "float32")
+
+
+def free_bytes():
+    from h2o4gpu_amd.libs import ch2o4gpu_gpu as shim
+    free = np.zeros(16, np.uint64)
+    status, n = shim.get_gpu_info_c(0, 0, 0, 0, 1, 0, 0, 0, 0, None, None, free, None, None, None,
+                                    None, None, None, None, None, None)
+    assert status == 0 and n >= 1 and free[0] > 0
+    return int(free[0])
+
+
+def test_a_fit_that_has_no_memory_to_spare_measures_every_row(hip, capfd):
+    """Twelve bytes a row and the centroids' distances (116 MB here) are only taken from what the steps themselves
+    leave: with some 60 MB more free than those need, the fit is made without limits, and has nothing to report."""
+    n, d, k = 4000000, 66, 4096
+    X = np.random.default_rng(1).standard_normal((n, d), dtype=np.float32)
+    with hip.Handle(n, d, k, np.float32) as h:  # what a fit of each kind takes beside the handle
+        h.set_data(X)
+        before = free_bytes()
+        want = run(h, X, X[:k], 4, 0)
+        plain = before - free_bytes()
+        same(run(h, X, X[:k], 4, 2), want)
+        assert before - free_bytes() > plain + (100 << 20)
+    with hip.Handle(n, d, k, np.float32, verbose=200) as h:
+        h.set_data(X)
+        hogs, left = [], plain + (60 << 20)
+        while free_bytes() > left + (8 << 20):  # (a handle's two models)
+            kh = min(free_bytes() - left, 32 << 30) // (2 * 4 * 4096) // 256 * 256
+            hogs.append(hip.Handle(kh, 4096, kh, np.float32))
+        capfd.readouterr()
+        got = run(h, X, X[:k], 4, 2)
+        err = capfd.readouterr().err
+        for hog in hogs:
+            hog.close()
+    same(got, want)
+    assert got["measured"] == -1 and err == ""
