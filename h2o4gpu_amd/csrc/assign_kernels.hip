@@ -3265,8 +3265,9 @@ int launch_bounded_accumulate<float>(hipStream_t s, const float *X, const float 
                                      int *tile_rows, const RowBounds &bounds) {
   if (!bounded_accumulate_applies<float>(n, d, k, 6, num_cu)) return H2O4GPU_KMEANS_EARG;
   RowBounds rb = bounds;
-  rb.noise = bound_noise<float>(d);
-  if (pick_assign_variant<float>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW) {
+  const bool long_rows = pick_assign_variant<float>(ASSIGN_AUTO, n, d, k) == ASSIGN_LONGROW;
+  rb.noise = bound_noise<float>(d, long_rows);
+  if (long_rows) {
     *tile_rows = longrow_tile_rows<float>(d);
     return launch_longrow<float, true, true>(s, X, xnorm, C, nullptr, labels, nullptr, n, d, k, num_cu, psums, pcounts,
                                              slots, rb);

@@ -115,11 +115,17 @@ __device__ __forceinline__ float row_limit(float best, float second, float xx, f
   return gap > 0.0f && at < 3e38f ? at : -__builtin_huge_valf();
 }
 
-// Rounding of a squared distance by whichever kernel measures it. float32: 18 times the rms error and
-// more (0.13 sqrt(d) eps (xx + cc), 3 to 784 features). float64: the worst case.
+// What a squared distance can be off by at most, relative to xx + cc, by whichever kernel measures it (u = half an eps
+// is a rounding). Norms are sums of d rounded squares one after the other: d u, and as much for any data whose
+// roundings all go the same way, equal features for one. Then the dot product, on a scale where no partial sum is
+// above xx + cc and each rounding counts twice: d of them on the float32 instructions, and fewer on the bfloat16 parts (six
+// instructions per 16 features, one truncation each). Long rows (a lane adds up to 16 products, a tree of six levels the
+// lanes) have 23 instead. Of 1200 eps at 784 features equal ones show 213, random ones some 4; a multiple of the random
+// error, 2 sqrt(d) eps, left rows of equal features with limits that rounding can pass. 10M x 32, k = 256, and 261k x 298,
+// k = 1000, take the same time with either, 500k x 784, k = 10, twenty steps 3.29 and 3.34 ms.
 template <typename T>
-static inline float bound_noise(int d) {
-  if (sizeof(T) == 4) return (8.0f + 2.0f * sqrtf((float)d)) * 1.1920929e-7f;
+static inline float bound_noise(int d, bool long_rows = false) {
+  if (sizeof(T) == 4) return (long_rows ? 16.0f + 0.5f * (float)d : 24.0f + 1.5f * (float)d) * 1.1920929e-7f;
   return (2.0f * (float)d + 16.0f) * 2.3e-16f;
 }
 

@@ -141,3 +141,16 @@ def test_a_fit_that_has_no_memory_to_spare_measures_every_row(hip, capfd):
             hog.close()
     same(got, want)
     assert got["measured"] == -1 and err == ""
+
+
+# (a centroid of equal features has a norm whose roundings all go the same way, and by how much hangs on its last bits:
+# up to d / 2 eps, where random features show some 0.13 sqrt(d))
+@pytest.mark.parametrize("n,d,k", [(20003, 784, 10), (20003, 1024, 3), (20003, 300, 16), (30001, 32, 80), (30001, 61, 70),
+                                   (30001, 298, 130), (30001, 780, 66)])
+def test_rows_of_equal_features(hip, n, d, k):
+    rng = np.random.default_rng(d)
+    X = np.empty((n, d), np.float32)
+    X[:] = rng.uniform(1.0, 1.4, (n, 1)).astype(np.float32)
+    C = X[rng.permutation(n)[:k]].copy()
+    for steps in (5, 8, 12, 20, 40):
+        same(fit(hip, X, C, steps, 2), fit(hip, X, C, steps, 0))
