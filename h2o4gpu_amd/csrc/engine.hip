@@ -1451,6 +1451,9 @@ struct Engine : h2o4gpu_kmeans_handle {
   bool bound_fused = false;  // the fused step
   double *run_sums = nullptr;  // (fused) the sums behind the centroids, and the rows in them
   int *run_counts[2] = {nullptr, nullptr};
+  double *run_least = nullptr;
+  float *run_range = nullptr;
+  SumsLimit *run_limit = nullptr;
   bool bounds_begin(int max_iterations) {
     bound_steps = 0;
     if (max_iterations < (opt_bounds == 1 ? BOUNDS_ITERATIONS : 1) || !opt_bounds || sets > 1 || opt_assign != ASSIGN_AUTO || opt_exact ||
@@ -1493,6 +1496,9 @@ struct Engine : h2o4gpu_kmeans_handle {
         want(list, &bound_ctl[i], 1);
       }
       want(list, &run_sums, (size_t)k * d);
+      want(list, &run_least, d);
+      want(list, &run_range, sizeof(T) == 4 ? least_sums_values(n, d) : 1);
+      want(list, &run_limit, 1);
       if (allocate(list, &bound_slab, true) != 0) return false;  // (every row is measured, then)
     }
     return true;
@@ -1576,6 +1582,9 @@ struct Engine : h2o4gpu_kmeans_handle {
     PROFILED("bounds", launch_bounds<T>(stream, b, start, X, xnorm, C[cur ^ 1], C[cur], labels, n, d, k, drift[was],
                                         drift[bound_cur], bound_ctl[was], bound_ctl[bound_cur], news_host,
                                         bound_grain<T>(n, d, k, bound_fused)));
+    if constexpr (sizeof(T) == 4) {
+      if (bound_fused && first) PROFILED("bounds", launch_sums_limit(stream, xnorm, n, run_limit));
+    }
     RowBounds rb;
     rb.rows = bound.listed;
     rb.ctl = bound_ctl[bound_cur];
@@ -1589,6 +1598,12 @@ struct Engine : h2o4gpu_kmeans_handle {
       run->counts_old = run_counts[was];
       run->counts_new = run_counts[bound_cur];
       run->ctl = rb.ctl;
+      run->least = run_least;
+      if constexpr (sizeof(T) == 4) run->X = X;
+      run->labels = labels;
+      run->n = n;
+      run->limit = run_limit;
+      run->news_host = news_host;
       return 0;
     }
     const int split = split_for(SPLIT_ASSIGN, k);
@@ -1600,7 +1615,13 @@ struct Engine : h2o4gpu_kmeans_handle {
     RunningSums run;
     int slots = 0;
     KM_TRY(bounded_pass(first, &run, &slots));
-    if (bound_fused) return finish_update(slots, want_shift, shift_host, run);
+    if (bound_fused) {
+      KM_TRY(finish_update(slots, want_shift, shift_host, run));
+      if constexpr (sizeof(T) == 4) {
+        if (first) PROFILED("bounds", launch_least_sums(stream, X, xnorm, n, d, run_range, run_least, run_limit));
+      }
+      return 0;
+    }
     return update_async(want_shift, shift_host, &bound_ctl[bound_cur]->changed);
   }
   // The relabel behind the last step of a bounded fit: the rows whose label may have changed, then every row's

@@ -318,13 +318,39 @@ static inline int max_shift_partials(int d, int k) {
 }
 // run (launch_bounded_accumulate): the partials are changes to sums kept here, unless its control block
 // says that all rows were measured; slots is what a launch over all rows writes.
+//
+// A value that leaves a sum leaves its rounding behind, up to the last bit of the largest sum it has been part of. That
+// is of no account to a float32 mean unless the sum is a 2^-24th of what it may have been, rows times the largest value:
+// such a sum is made anew, from the rows. No value is larger than the largest row's norm, which is enough for
+// most data; where the first sums have smaller ones (features of sizes of their own, features that are zero throughout a
+// cluster) the features' values are looked at (launch_least_sums), once a fit.
+struct SumsLimit {
+  unsigned anew;       // workgroups that made sums anew since the bounds were begun
+  unsigned look;       // 1: the features are to be looked at
+  unsigned norm_bits;  // the largest finite norm of a row
+};
 struct RunningSums {
   double *sums = nullptr;           // [k][d], updated
   const int *counts_old = nullptr;  // [k]
   int *counts_new = nullptr;        // [k], another buffer
   const BoundControl *ctl = nullptr;
   int tile_rows = 0;  // listed rows a workgroup takes at a time: fewer tiles, fewer slots written
+  const double *least = nullptr;    // [d]
+  const float *X = nullptr;         // [n][d], with the labels the new centroids are made from
+  const int *labels = nullptr;
+  int64_t n = 0;
+  SumsLimit *limit = nullptr;
+  unsigned *news_host = nullptr;    // (pinned) [BOUND_FAILING] is set when `anew` comes to SUMS_ANEW
 };
+static const unsigned SUMS_ANEW = 4;
+// Before the step that begins the bounds, and behind it.
+int launch_sums_limit(hipStream_t s, const float *xnorm, int64_t n, SumsLimit *limit);
+// least[f]: a sum of m rows is made anew below m * |least[f]|; 0: never (the sums of the feature are exact in whatever
+// order they are made). Negative: also where the partials say that it is what it was.
+// scratch: [least_sums_values(n, d)].
+size_t least_sums_values(int64_t n, int d);
+int launch_least_sums(hipStream_t s, const float *X, const float *xnorm, int64_t n, int d, float *scratch, double *least,
+                      const SumsLimit *limit);
 // A loop that is queued ahead of its convergence test: the update whose shift is below the threshold says so, and
 // the launches behind it that are given the flag do nothing.
 struct StopRule {
