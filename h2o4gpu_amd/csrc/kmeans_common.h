@@ -320,10 +320,12 @@ static inline int max_shift_partials(int d, int k) {
 // says that all rows were measured; slots is what a launch over all rows writes.
 //
 // A value that leaves a sum leaves its rounding behind, up to the last bit of the largest sum it has been part of. That
-// is of no account to a float32 mean unless the sum is a 2^-24th of what it may have been, rows times the largest value:
-// such a sum is made anew, from the rows. No value is larger than the largest row's norm, which is enough for
-// most data; where the first sums have smaller ones (features of sizes of their own, features that are zero throughout a
-// cluster) the features' values are looked at (launch_least_sums), once a fit.
+// is of no account to a float32 mean unless the sum is a 2^-28th of what it may have been, rows times the largest value:
+// such a sum is made anew, from the rows. (One value that leaves some rows has left 2^-53 of it, and a few times that
+// where it met many of them in one workgroup: 2^-25 of a sum at this line. At 2^-24 one fit in fifty of 10M x 32, k = 256, had a
+// sum that was small by chance, at 4 ms for each.) No value is larger than the largest row's norm, which is
+// enough for most data; where the first sums have smaller ones (features of sizes of their own, features that are zero
+// throughout a cluster) the features' values are looked at (launch_least_sums).
 struct SumsLimit {
   unsigned anew;       // workgroups that made sums anew since the bounds were begun
   unsigned look;       // 1: the features are to be looked at

@@ -998,7 +998,7 @@ __device__ __forceinline__ void test_shift(T sum, const StopRule &stop) {
 }
 
 __device__ __forceinline__ double least_by_norm(const SumsLimit &limit) {
-  return 6e-8 * sqrt((double)__uint_as_float(limit.norm_bits));  // (2^-24, and more than a norm can be off by)
+  return 3.8e-9 * sqrt((double)__uint_as_float(limit.norm_bits));  // (2^-28, and more than a norm can be off by)
 }
 
 // The sums of a workgroup's EPW coordinates (e, of centroid c, of thread tid % EPW) from the rows that are labelled with their
@@ -1408,7 +1408,7 @@ __global__ __launch_bounds__(WG) void least_sums_kernel(const float *__restrict_
   if (tid == 0) {
     const double big = red[0][0], small = red[1][0], last = red[2][0];
     const bool exact = big == 0 || (double)n * big <= 4503599627370496.0 * last;  // (2^52)
-    const double below = big * 5.9604644775390625e-8;                            // (2^-24)
+    const double below = big * 3.7252902984619140625e-9;                         // (2^-28)
     least[f] = exact ? 0.0 : (small * 1099511627776.0 >= big ? below : -below);
   }
 }
