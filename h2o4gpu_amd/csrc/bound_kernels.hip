@@ -275,7 +275,7 @@ __global__ __launch_bounds__(WG) void pack_rows_kernel(const int *__restrict__ f
                                                       const int *__restrict__ found_counts, int segments,
                                                       int64_t seg_rows, int64_t n, int *__restrict__ listed,
                                                       const BoundControl *__restrict__ ctl_old,
-                                                      BoundControl *__restrict__ ctl_new, unsigned *news_host,
+                                                      BoundControl *__restrict__ ctl_new, StepNews *news_host,
                                                       bool decides) {
   __shared__ unsigned before_s[WG / 64], all_s[WG / 64];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(WG) void pack_rows_kernel(const int *__restrict__ f
     if (still || was.wait > 0) {
       if (one) {
         if (still && news_host)
-          __hip_atomic_store(news_host + BOUND_STILL, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          __hip_atomic_store(&news_host->still, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         BoundControl c = {};
         c.full = c.changed = still ? 0u : 1u;
         c.wait = was.wait > 0 ? was.wait - 1 : 0u;
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(WG) void pack_rows_kernel(const int *__restrict__ f
     BoundControl c = {};
     const unsigned fails = full ? was.fails + 1 : 0;
     if (fails == BOUND_FAILS && !look && news_host)
-      __hip_atomic_store(news_host + BOUND_FAILING, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&news_host->failing, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     c.count = all;
     c.full = full;
     c.fails = look ? was.fails : fails;
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(WG) void pack_rows_kernel(const int *__restrict__ f
     c.look = look;
     c.listed = AGAIN ? was.listed : all;
     if (!AGAIN && news_host)
-      __hip_atomic_store(news_host + BOUND_LISTED, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(&news_host->listed, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     *ctl_new = c;
   }
   if (full) return;
@@ -699,7 +699,7 @@ bool neighbours_apply(int64_t n, int d, int k) { return k >= 2 && k <= 4096 && d
 template <typename T>
 int launch_bounds(hipStream_t s, const BoundBuffers &b, BoundStart start, const T *X, const T *xnorm, const T *c_old,
                   const T *c_new, int *labels, int64_t n, int d, int k, const double *drift_old, double *drift_new,
-                  const BoundControl *ctl_old, BoundControl *ctl_new, unsigned *news_host, float grain) {
+                  const BoundControl *ctl_old, BoundControl *ctl_new, StepNews *news_host, float grain) {
   if (n < 1 || n > 2147483647 || k < 1 || k > MAX_BOUND_CENTROIDS) return H2O4GPU_KMEANS_EARG;
   if (start != BOUNDS_GO) {
     hipLaunchKernelGGL(first_bounds_kernel, dim3(1), dim3(WG), 0, s, drift_new, b.drift_float, k, ctl_new,
@@ -732,7 +732,7 @@ int launch_bounds(hipStream_t s, const BoundBuffers &b, BoundStart start, const 
 #define KM_INST(T)                                                                                                  \
   template int launch_bounds<T>(hipStream_t, const BoundBuffers &, BoundStart, const T *, const T *, const T *, const T *, \
                                 int *, int64_t, int, int, const double *, double *, const BoundControl *, BoundControl *,  \
-                                unsigned *, float)
+                                StepNews *, float)
 KM_INST(float);
 KM_INST(double);
 #undef KM_INST

@@ -1510,16 +1510,26 @@ struct Engine : h2o4gpu_kmeans_handle {
   // Where most rows have to be measured all the same, the limits are an expense; after BOUND_FAILS looks in vain
   // the next steps do without, sixteen at first, then twice as many (noise, 500k x 784, k = 10: twenty
   // steps 8.77 -> 9.43 ms, 9.60 without pauses, sixty 25.6 -> 26.8).
-  static const int NEWS_BEHIND = 4;
-  unsigned *news_host = nullptr;  // pinned
+  // The host looks at a step's news once an event says that the step has ended, and at those of no later one: which
+  // steps keep bounds hangs on the rows alone, and not on how far ahead of the device the host is.
+  static const int NEWS_BEHIND = 4, NEWS_STEPS = 8;
+  struct HostNews {
+    StepNews step[NEWS_STEPS];  // of step i: [i % NEWS_STEPS]
+    unsigned stopped;           // StopRule's step
+  };
+  HostNews *news_host = nullptr;  // pinned
   hipEvent_t news_ready[2] = {nullptr, nullptr};
   int bounds_at = 0, bounds_pause = 0;  // the step that begins to keep bounds, and how long the next pause is
-  unsigned news(BoundNews what) const { return const_cast<volatile unsigned *>(news_host)[what]; }
+  int news_next = 0;                    // the first step whose news have not been looked at
+  bool news_still = false;
+  unsigned news_listed = 0;
   bool news_possible() {
     for (auto &ev : news_ready) {
+      // (the kernels store past the caches; an event that releases to the system would write them back: 500k x 784, k = 10,
+      // twenty steps 3.3 -> 3.5 ms)
       if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) ev = nullptr;
     }
-    if (!news_host && hipHostMalloc(reinterpret_cast<void **>(&news_host), BOUND_NEWS * sizeof(unsigned),
+    if (!news_host && hipHostMalloc(reinterpret_cast<void **>(&news_host), sizeof(HostNews),
                                     hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess)
       news_host = nullptr;
     if (news_host && news_ready[0] && news_ready[1]) return true;
@@ -1527,24 +1537,46 @@ struct Engine : h2o4gpu_kmeans_handle {
     return false;
   }
   void news_begin() {
-    for (int i = 0; i < BOUND_NEWS; i++) const_cast<volatile unsigned *>(news_host)[i] = i == BOUND_LISTED ? ~0u : 0u;  // (nothing is under way)
-    bounds_at = BOUNDS_FROM;
+    const_cast<volatile unsigned &>(news_host->stopped) = 0;  // (nothing is under way)
+    bounds_at = news_next = BOUNDS_FROM;
     bounds_pause = 16;
+    news_still = false;
+    news_listed = ~0u;
   }
-  // before bounded step i: (a kernel says so once, and then not before bounds are begun anew)
-  void bounds_failing(int i, int max_iterations) {
-    if (!news(BOUND_FAILING)) return;
-    const_cast<volatile unsigned *>(news_host)[BOUND_FAILING] = 0;
+  // for step i, about to be queued (the one before in its place has been looked at)
+  StepNews *news_of(int i) {
+    StepNews *const to = news_host->step + i % NEWS_STEPS;
+    volatile StepNews *const news = to;
+    news->still = news->failing = 0;
+    news->listed = ~0u;
+    return to;
+  }
+  // the news of the steps up to `last`, which have ended; whether one of them says that bounds are of no use
+  bool news_take(int last) {
+    bool failing = false;
+    for (; news_next <= last; news_next++) {
+      const volatile StepNews *const news = news_host->step + news_next % NEWS_STEPS;
+      news_still |= news->still != 0;
+      failing |= news->failing != 0;
+      if (news->listed != ~0u) news_listed = news->listed;
+    }
+    return failing;
+  }
+  // before bounded step i
+  int bounds_give_up(int i, int max_iterations) {
+    KM_HIP_TRY(hipStreamSynchronize(stream));  // (what the steps under way still have to tell is not waited for later)
     bounds_at = bounds_pause < max_iterations - i - BOUNDS_ITERATIONS ? i + bounds_pause : max_iterations;
+    news_next = bounds_at;
     bounds_pause *= 2;
+    return 0;
   }
   // before bounded step i of a fit whose steps are queued without waiting; an event every other step
-  int news_look(int i, bool *still) {
+  int news_look(int i, int max_iterations) {
     if (i % (NEWS_BEHIND / 2) != 0) return 0;
     hipEvent_t ev = news_ready[i / (NEWS_BEHIND / 2) % 2];
     if (i >= bounds_at + NEWS_BEHIND) {
-      KM_HIP_TRY(hipEventSynchronize(ev));
-      *still = news(BOUND_STILL) != 0;
+      KM_HIP_TRY(hipEventSynchronize(ev));  // (recorded before step i - NEWS_BEHIND)
+      if (news_take(i - NEWS_BEHIND - 1)) return bounds_give_up(i, max_iterations);
     }
     KM_HIP_TRY(hipEventRecord(ev, stream));
     return 0;
@@ -1553,7 +1585,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   BoundBuffers bound_buffers() const {
     BoundBuffers b = bound;
     // (short lists have no use for the neighbours, and their launches are not for nothing)
-    if (bound_fused || news(BOUND_LISTED) < DECIDE_ROWS) b.near = Neighbours();
+    if (bound_fused || news_listed < DECIDE_ROWS) b.near = Neighbours();
     return b;
   }
   // The step before the first of them, where that looks at rows already: it leaves labels.
@@ -1569,18 +1601,17 @@ struct Engine : h2o4gpu_kmeans_handle {
     return step_async(want_shift, shift_host != nullptr, shift_host);
   }
   // The assignment pass of a step (fused: with its sums, in *slots, for *run).
-  int bounded_pass(bool first, RunningSums *run, int *slots) {
+  int bounded_pass(bool first, RunningSums *run, int *slots, StepNews *news) {
     KM_TRY(ensure_work());
     if (!bound_fused) KM_TRY(ensure_cnorm());
     const int was = bound_cur;
     bound_cur ^= 1;
     bound_steps++;
     BoundBuffers b = bound_buffers();
-    // (news may have come in since the step before)
     if (first) b.near = bound_fresh ? bound.near : Neighbours();
     const BoundStart start = first && !bound_fresh ? BOUNDS_FIRST : BOUNDS_GO;
     PROFILED("bounds", launch_bounds<T>(stream, b, start, X, xnorm, C[cur ^ 1], C[cur], labels, n, d, k, drift[was],
-                                        drift[bound_cur], bound_ctl[was], bound_ctl[bound_cur], news_host,
+                                        drift[bound_cur], bound_ctl[was], bound_ctl[bound_cur], news,
                                         bound_grain<T>(n, d, k, bound_fused)));
     if constexpr (sizeof(T) == 4) {
       if (bound_fused && first) PROFILED("bounds", launch_sums_limit(stream, xnorm, n, run_limit));
@@ -1603,7 +1634,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       run->labels = labels;
       run->n = n;
       run->limit = run_limit;
-      run->news_host = news_host;
+      run->news_host = news;
       return 0;
     }
     const int split = split_for(SPLIT_ASSIGN, k);
@@ -1611,10 +1642,11 @@ struct Engine : h2o4gpu_kmeans_handle {
                                                 split_scratch(split, k, true, n), rb));
     return 0;
   }
-  int bounded_step(bool first, bool want_shift, T *shift_host = nullptr) {
+  int bounded_step(int i, bool want_shift, T *shift_host = nullptr) {
+    const bool first = i == bounds_at;
     RunningSums run;
     int slots = 0;
-    KM_TRY(bounded_pass(first, &run, &slots));
+    KM_TRY(bounded_pass(first, &run, &slots, news_of(i)));
     if (bound_fused) {
       KM_TRY(finish_update(slots, want_shift, shift_host, run));
       if constexpr (sizeof(T) == 4) {
@@ -1633,7 +1665,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     if (!labelled) {
       RunningSums run;
       int slots = 0;
-      KM_TRY(bounded_pass(false, &run, &slots));
+      KM_TRY(bounded_pass(false, &run, &slots, nullptr));
     }
     PROFILED("assign", launch_own_distances<T>(stream, X, C[cur], labels, mindist, n, d, k, num_cu));
     have_mindist = true;
@@ -1715,6 +1747,7 @@ struct Engine : h2o4gpu_kmeans_handle {
   // the host looks at every eighth iteration, eight behind (10.1M x 3, k = 27, some 260 steps: 11.4 -> 10.9 ms a fit).
   int cells_loop(int first, int max_iterations, double threshold, int *updates) {
     news_begin();
+    auto stopped = [&]() -> unsigned { return const_cast<volatile unsigned &>(news_host->stopped); };
     KM_TRY(launch_fill<int>(stream, reinterpret_cast<int *>(cell_stop), 0, 1));
     const int start = cur;
     int queued = 0;
@@ -1722,7 +1755,7 @@ struct Engine : h2o4gpu_kmeans_handle {
       log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", first + queued, max_iterations);
       StopRule stop;
       stop.stopped = cell_stop;
-      stop.step_host = news_host + LOOP_STOPPED;
+      stop.step_host = &news_host->stopped;
       stop.threshold = threshold;
       stop.step = (unsigned)(first + ++queued);
       KM_TRY(cells_step(true, stop));
@@ -1730,7 +1763,7 @@ struct Engine : h2o4gpu_kmeans_handle {
         hipEvent_t *const ev = news_ready;
         KM_HIP_TRY(hipEventRecord(ev[queued / 8 & 1], stream));
         if (queued >= 16) KM_HIP_TRY(hipEventSynchronize(ev[(queued / 8 & 1) ^ 1]));
-        if (news(LOOP_STOPPED)) break;
+        if (stopped()) break;
       }
       if (g_stop_flag) {
         fprintf(stderr, "Signal caught. Terminated early.\n");
@@ -1740,7 +1773,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     }
     KM_HIP_TRY(hipStreamSynchronize(stream));
     *updates = first + queued;
-    if (const unsigned step = news(LOOP_STOPPED)) {
+    if (const unsigned step = stopped()) {
       log_msg(verbose, LOG_INFO, "Threshold triggered. Terminating early.");
       *updates = (int)step;
       cur = start ^ ((*updates - first) & 1);  // (what was queued behind it has changed nothing)
@@ -1814,7 +1847,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     // (what the steps cannot do without, before anything that only makes them faster)
     if (max_iterations > 0) KM_TRY(ensure_work());
     const bool bounded = bounds_begin(max_iterations);
-    bool cells = false, cells_wanted = cells_possible(), still = false;
+    bool cells = false, cells_wanted = cells_possible();
     cell_measured = -1;
     if (max_iterations <= 0) {
       // The reference's loop then never runs, its final relabel included, and the labels it
@@ -1831,10 +1864,8 @@ struct Engine : h2o4gpu_kmeans_handle {
       if (bounded) news_begin();
       for (int i = 0; i < max_iterations; i++) {
         log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
-        if (bounded && i >= bounds_at && !still) {
-          KM_TRY(news_look(i, &still));
-          bounds_failing(i, max_iterations);
-        }
+        if (bounded && i >= bounds_at && !news_still) KM_TRY(news_look(i, max_iterations));
+        const bool still = bounded && news_still;
         // (the final relabel below leaves the minimum distances)
         if (cells_wanted && i >= 1) {
           if (opt_bounds == 2 || max_iterations - i >= CELL_STEPS) KM_TRY(cells_begin(&cells));
@@ -1842,7 +1873,7 @@ struct Engine : h2o4gpu_kmeans_handle {
         }
         if (cells) KM_TRY(cells_step(false));
         else if (still) {}  // (the step would change nothing)
-        else if (bounded && i >= bounds_at) KM_TRY(bounded_step(i == bounds_at, false));
+        else if (bounded && i >= bounds_at) KM_TRY(bounded_step(i, false));
         else if (bounded && i == bounds_at - 1) KM_TRY(bounds_prime(false));
         else KM_TRY(step_async(false, false));
         updates++;
@@ -1977,7 +2008,7 @@ struct Engine : h2o4gpu_kmeans_handle {
     };
     auto queue_iteration = [&](int i) -> int {
       log_msg(verbose, LOG_VERBOSE, "KMeans - Iteration %d/%d", i, max_iterations);
-      if (bounded && i >= bounds_at) KM_TRY(bounded_step(i == bounds_at, true, host_shift + (i & 1)));
+      if (bounded && i >= bounds_at) KM_TRY(bounded_step(i, true, host_shift + (i & 1)));
       else if (bounded && i == bounds_at - 1) KM_TRY(bounds_prime(true, host_shift + (i & 1)));
       else KM_TRY(step_async(true, true, host_shift + (i & 1)));
       KM_HIP_TRY(hipEventRecord(shift_ready[i & 1], stream));
@@ -1993,7 +2024,8 @@ struct Engine : h2o4gpu_kmeans_handle {
         cells_wanted = false;
         if (cells) queued_next = false;
       }
-      if (bounded && i + 1 >= bounds_at) bounds_failing(i + 1, max_iterations);
+      // (the wait for the shift of step i - 1 was one for its news)
+      if (bounded && i + 1 >= bounds_at && news_take(i - 1)) KM_TRY(bounds_give_up(i + 1, max_iterations));
       if (queued_next) KM_TRY(queue_iteration(i + 1));
       KM_HIP_TRY(hipEventSynchronize(shift_ready[i & 1]));
       updates = i + 1;

@@ -146,10 +146,13 @@ int launch_bounded_accumulate(hipStream_t s, const T *X, const T *xnorm, const T
 // The launches before such a pass: how far the centroids have moved, the drift that leaves (drift_old ->
 // drift_new), the rows whose limit it has passed, those of them that the centroids' neighbours do not decide,
 // and the control block. BOUNDS_FIRST: zeros, and every row is measured. BOUNDS_FRESH: that, for a step that
-// leaves no limits; the next one's rows are all looked at. news_host (nullable, pinned): [BOUND_STILL]
-// receives 1 where no centroid has moved, [BOUND_FAILING] where most rows had to be measured at BOUND_FAILS looks
-// in a row, [BOUND_LISTED] the rows whose limit the drift had passed. ([LOOP_STOPPED]: StopRule's step.) grain: see RowBounds.
-enum BoundNews { BOUND_STILL, BOUND_FAILING, BOUND_LISTED, LOOP_STOPPED, BOUND_NEWS };
+// leaves no limits; the next one's rows are all looked at. news_host (nullable, pinned) receives the step's news.
+// grain: see RowBounds.
+struct StepNews {
+  unsigned still;    // 1: no centroid has moved
+  unsigned failing;  // 1: most rows had to be measured at BOUND_FAILS looks in a row (or see SumsLimit)
+  unsigned listed;   // the rows whose limit the drift had passed, where it was looked at
+};
 static const unsigned BOUND_FAILS = 3;
 static const int MAX_BOUND_CENTROIDS = 8192;
 enum BoundStart { BOUNDS_GO, BOUNDS_FIRST, BOUNDS_FRESH };
@@ -158,7 +161,7 @@ bool neighbours_apply(int64_t n, int d, int k);
 template <typename T>
 int launch_bounds(hipStream_t s, const BoundBuffers &b, BoundStart start, const T *X, const T *xnorm, const T *c_old,
                   const T *c_new, int *labels, int64_t n, int d, int k, const double *drift_old, double *drift_new,
-                  const BoundControl *ctl_old, BoundControl *ctl_new, unsigned *news_host, float grain);
+                  const BoundControl *ctl_old, BoundControl *ctl_new, StepNews *news_host, float grain);
 // The squared distance of every row to the centroid it is labelled with, from the differences.
 bool own_distances_apply(int d);
 template <typename T>
@@ -342,7 +345,7 @@ struct RunningSums {
   const int *labels = nullptr;
   int64_t n = 0;
   SumsLimit *limit = nullptr;
-  unsigned *news_host = nullptr;    // (pinned) [BOUND_FAILING] is set when `anew` comes to SUMS_ANEW
+  StepNews *news_host = nullptr;    // (pinned) `failing` is set when `anew` comes to SUMS_ANEW
 };
 static const unsigned SUMS_ANEW = 4;
 // Before the step that begins the bounds, and behind it.

@@ -1018,7 +1018,7 @@ __device__ double sums_from_rows(const RunningSums &run, int d, int64_t e, int c
 #pragma unroll
   for (int off = 1; off < EPW; off <<= 1) last = max(last, __shfl_xor(last, off, 64));
   if (tid == 0 && atomicAdd(&run.limit->anew, 1u) + 1 == SUMS_ANEW && run.news_host)
-    __hip_atomic_store(run.news_host + BOUND_FAILING, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(&run.news_host->failing, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   double acc = 0;
   int2 *const mine = queue[tid >> 6];
   int waiting = 0;
