@@ -644,7 +644,6 @@ int launch_decide(hipStream_t s, const BoundBuffers &b, const T *X, const T *xno
   } else {
     if (d <= 64) KM_DECIDE(1, 16, 4);
     else if (d <= 256) KM_DECIDE(1, 64, 4);
-    else if (d <= 320) KM_DECIDE(1, 64, 5);
     else if (d <= 512) KM_DECIDE(1, 64, 8);
     else KM_DECIDE(1, 64, 16);
   }
