@@ -264,3 +264,55 @@ def test_fits_come_out_the_same_every_time(hip, dtype, n, d, k):
                 for g in f[1:]:
                     same(g, f[0], dtype == "float32")
                     assert dtype == "float64" or np.array_equal(g["mind"], f[0]["mind"])
+
+
+@pytest.mark.parametrize("dtype,n,d,k", NOISE)
+def test_bounds_given_up_and_begun_anew(hip, dtype, n, d, k):
+    """Three looks in vain from the third step on, sixteen steps without limits, three more, then 32 without:
+    fits that end in each stretch, and in the first steps of the next one."""
+    X, C = noise(dtype, n, d, k)
+    with hip.Handle(n, d, k, X.dtype) as h:
+        h.set_data(X)
+        for steps in (16, 24, 30, 41, 64, 80):
+            want = run(h, X, C, steps, 0)
+            for tol in (0.0, 1e-30):
+                got = run(h, X, C, steps, 2, tol)
+                assert got["it"] == steps or tol > 0
+                if got["it"] != steps:  # (at rest)
+                    want = run(h, X, C, steps, 0, tol)
+                same(got, want, dtype == "float32")
+
+
+# a little above the line from which fits keep bounds by themselves: the row-stationary step, tiled kernels of both
+# precisions, long rows with a handful of centroids
+DEFAULT = [("float32", 2000003, 32, 256), ("float32", 80001, 132, 500), ("float64", 60001, 101, 900), ("float32", 140001, 784, 10)]
+
+
+@pytest.mark.parametrize("dtype,n,d,k", DEFAULT)
+def test_fits_keep_bounds_by_themselves(hip, dtype, n, d, k):
+    """Through a handle that nobody sets an option for, and through the estimator."""
+    from h2o4gpu_amd import KMeans
+    X, C = strips(n, d, k, dtype, 5)
+    want = fit(hip, X, C, 12, 0)
+    got = fit(hip, X, C, 12)
+    assert want["measured"] == -1 and 0 <= got["measured"] < n / 2
+    same(got, want, dtype == "float32")
+    assert fit(hip, X, C, 9)["measured"] == -1
+    model = KMeans(n_clusters=k, init=C, n_init=1, max_iter=12, tol=0.0).fit(X)
+    assert np.array_equal(model.labels_, want["labels"])
+    big = np.abs(want["centers"]).max()
+    off = 0 if dtype == "float32" else 1000 * np.finfo(np.float64).eps * big
+    assert np.allclose(model.cluster_centers_, want["centers"], rtol=0, atol=off)
+
+
+@pytest.mark.parametrize("k", [17, 27, 100])
+def test_blocks_of_one_centroid_are_not_measured(hip, k):
+    """Rows ordered in space, clusters far apart: hardly a block has rows of two."""
+    n = 300007
+    rng = np.random.default_rng(k)
+    places = np.stack(np.meshgrid(*[np.arange(5) * 16.0] * 3), -1).reshape(-1, 3)[rng.permutation(125)[:k]]
+    X = (places[rng.integers(0, k, n)] + np.round(rng.standard_normal((n, 3)) * 256) / 256).astype(np.float32)
+    C = (places + 1).astype(np.float32)
+    got, want = fit(hip, X, C, 12, 2), fit(hip, X, C, 12, 0)
+    assert want["measured"] == -1 and 0 <= got["measured"] < n / 10
+    same(got, want)
