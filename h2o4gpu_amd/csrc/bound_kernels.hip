@@ -387,7 +387,7 @@ __global__ __launch_bounds__(decide_threads<LOCAL>()) void decide_rows_kernel(
     const T *__restrict__ X, const T *__restrict__ xnorm, const T *__restrict__ C, int *__restrict__ labels,
     float *__restrict__ limit, int64_t n, int d, int k, const int *__restrict__ listed, const float *__restrict__ near_dist,
     const int *__restrict__ near_at, const float *__restrict__ drift, int *__restrict__ found,
-    int *__restrict__ found_counts, BoundControl *ctl, float noise, float grain) {
+    int *__restrict__ found_counts, BoundControl *ctl, Rounding noise, float grain) {
   constexpr int TPB = decide_threads<LOCAL>();
   constexpr int RPW = 64 / LPR;
   constexpr int PIECES = VW * NV * (int)sizeof(T) / 4;  // registers of a row's part
@@ -613,7 +613,7 @@ __global__ void first_bounds_kernel(double *__restrict__ drift, float *__restric
 template <typename T>
 int launch_decide(hipStream_t s, const BoundBuffers &b, const T *X, const T *xnorm, const T *C, int *labels, int64_t n,
                   int d, int k, float grain) {
-  const float noise = bound_noise<T>(d);
+  const Rounding noise = bound_noise<T>(d);
   constexpr int VW = Mfma<T>::VW;
   // a model within half a CU's LDS is staged there
   const size_t lds = (size_t)k * (decide_row_stride<T>(d) * sizeof(T) + (NEAREST + 1) * 8);

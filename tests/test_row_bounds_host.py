@@ -17,7 +17,17 @@ static float norm(const float *x, int d) {
   for (int j = 0; j < d; j++) { volatile float p = x[j] * x[j]; s = s + p; }
   return s;
 }
-extern "C" float noise(int d, int long_rows) { return kmhip::bound_noise<float>(d, long_rows != 0); }
+extern "C" float noise(int d, int long_rows) {
+  const kmhip::Rounding r = kmhip::bound_noise<float>(d, long_rows != 0);
+  return r.products + r.norms;
+}
+extern "C" float limit(float best, float second, float xx, int d, int long_rows, float share) {
+  kmhip::Rounding r = kmhip::bound_noise<float>(d, long_rows != 0);
+  r.products *= share;
+  r.norms *= share;
+  return kmhip::row_limit(best, second, xx, 0.0f, r, 0.0f);
+}
+extern "C" float square(const float *x, int d) { return norm(x, d); }
 // the float32 instructions: half a distance, one multiply-add per feature
 extern "C" float chain(const float *x, const float *c, int d) {
   float a = fmaf(-0.5f, norm(c, d), -0.5f * norm(x, d));
@@ -43,7 +53,7 @@ def model(tmp_path_factory):
     subprocess.check_call(["g++", "-O2", "-ffp-contract=off", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-w", "-I" + CSRC,
                            "-I/opt/rocm/include", "-o", str(so), str(src)])
     lib = ctypes.CDLL(str(so))
-    for name in ("noise", "chain", "lanes"):
+    for name in ("noise", "chain", "lanes", "limit", "square"):
         getattr(lib, name).restype = ctypes.c_float
     return lib
 
@@ -70,3 +80,49 @@ def test_noise_covers_the_rounding(model, form, d):
         worst = max(worst, off)
     assert worst <= bound, (worst * 2 ** 23, bound * 2 ** 23)
     assert worst > bound / 50  # (what equal features show)
+
+
+def labels_that_change(model, form, d, share):
+    """How many rows with a limit change sides although the two centroids have not used it up: one moves away from the
+    row or towards it, the other towards the row. Rows and centroids of equal features, on which roundings add up, and
+    of any, far from the origin and near, near their centroid and not, the centroids at all but the same distance."""
+    f, rng, changed, limits = getattr(model, form), np.random.default_rng(d), 0, 0
+    for trial in range(3000):
+        away = 10.0 ** rng.uniform(-3, 0.5)
+        if trial % 3:
+            x = np.full(d, rng.uniform(1, 2))
+            side, other = np.full(d, 1.0), np.full(d, -1.0)
+        else:
+            x = rng.standard_normal(d) + rng.uniform(0, 3)
+            side, other = rng.standard_normal((2, d))
+        x = x.astype(np.float32)
+        x64 = x.astype(np.float64)
+        scale = away * np.sqrt((x64 ** 2).mean() * d)
+        side, other = (v / np.sqrt((v ** 2).sum()) * scale for v in (side, other))
+        more = 1 + 10.0 ** rng.uniform(-5, 0)
+        a, b = (x64 + side).astype(np.float32), (x64 + other * more).astype(np.float32)
+        best, second = f(ptr(x), ptr(a), d), f(ptr(x), ptr(b), d)
+        if best > second:
+            a, b, side, other, best, second = b, a, other, side, second, best
+        lim = model.limit(ctypes.c_float(best), ctypes.c_float(second), ctypes.c_float(model.square(ptr(x), d)), d,
+                          form == "lanes", ctypes.c_float(share))
+        if not lim > 0:
+            continue
+        limits += 1
+        for part in (0.0, 0.3, 1.0, -0.3, -1.0):  # of the limit, the row's own centroid
+            to = side / np.sqrt((side ** 2).sum()) * lim * 0.9999
+            fro = other / np.sqrt((other ** 2).sum()) * lim * 0.9999
+            a2 = (a + part * to).astype(np.float32)
+            b2 = (b - (1 - abs(part)) * fro).astype(np.float32)
+            used = sum(np.sqrt(((p.astype(np.float64) - q) ** 2).sum()) for p, q in ((a, a2), (b, b2)))
+            if used <= lim:
+                changed += not f(ptr(x), ptr(a2), d) < f(ptr(x), ptr(b2), d)
+    assert limits > 300
+    return changed
+
+
+@pytest.mark.parametrize("form,d", [("chain", d) for d in (5, 61, 298, 1024)] + [("lanes", d) for d in (68, 300, 784)])
+def test_rows_within_their_limit_keep_their_label(model, form, d):
+    assert labels_that_change(model, form, d, 1.0) == 0
+    if d >= 298:  # (and the rows above are such that it matters)
+        assert labels_that_change(model, form, d, 0.03) > 0
