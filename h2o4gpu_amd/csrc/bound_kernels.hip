@@ -642,9 +642,13 @@ int launch_decide(hipStream_t s, const BoundBuffers &b, const T *X, const T *xno
     else if (v <= 256) KM_DECIDE(VW, 64, 4);
     else KM_DECIDE(VW, 64, 8);
   } else {
+    // (A piece beyond the row is loaded all the same. 261k x 298, k = 1000, five lists 1199 us with eight pieces, 1115 with six;
+    // 150k rows of 601 and 701, 4.94 ms with sixteen, 4.82 with twelve.)
     if (d <= 64) KM_DECIDE(1, 16, 4);
     else if (d <= 256) KM_DECIDE(1, 64, 4);
+    else if (d <= 384) KM_DECIDE(1, 64, 6);
     else if (d <= 512) KM_DECIDE(1, 64, 8);
+    else if (d <= 768) KM_DECIDE(1, 64, 12);
     else KM_DECIDE(1, 64, 16);
   }
 #undef KM_DECIDE
