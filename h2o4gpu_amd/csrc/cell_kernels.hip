@@ -12,13 +12,15 @@
 // Centroids are those of steps that measure every row, bit for bit: a row's label is that of the chain of
 // multiply-adds the float32 instructions make (compared at 16 ulp, lowest index first), a centroid is
 // ruled out only where it is further by more than any rounding of that chain, and sums of float32 values in
-// double do not depend on their order.
+// double do not depend on their order where they are exact (colours, coordinates of less than some 14 binades; others
+// differ by some 2^-50 of the largest value, as two orders do. Each step makes its sums from the blocks'.)
 //
 // Bound by latency and by the additions in LDS: a block's test reads 64 bytes and takes some 20 instructions per
 // centroid, an undecided block's rows (a third of them with k = 27) are measured against two to four centroids.
-// A step, 10M rows: k = 27 84 -> 17 us on pixels, k = 60 110 -> 38 on blobs; putting the rows in order 0.65 ms, of which
+// A step, 10M rows: k = 27 84 -> 18 us on pixels, k = 60 110 -> 38 on blobs; putting the rows in order 0.65 ms, of which
 // 0.28 each for the sort and for the windows. (Rows of four features had fewer blocks decided: 1.3 to 1.7 times as
-// fast on blobs, 0.6 to 1.1 on noise; models of 300 centroids 1.1 and 0.8.)
+// fast on blobs, 0.6 to 1.1 on noise; models of 300 centroids 1.1 and 0.8. Rows
+// of two features and float64 rows have not been tried.)
 #include <algorithm>
 
 #include "bf16_parts.h"

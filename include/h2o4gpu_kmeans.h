@@ -277,10 +277,13 @@ int h2o4gpu_kmeans_transform_resident(h2o4gpu_kmeans_handle *h, void *d_dist);
  * each row is from changing its label, and measure only rows that may have changed it
  * (row_bounds.h: shapes of the tiled kernels, float32 shapes of the row-stationary one with six
  * products and of the one for long rows and a handful of centroids, where there is enough to
- * measure). Labels and centroids are those of 0, which measures every row in every step; 2 does
- * it for fits of any length and shapes of any size. Twelve bytes of device memory a row, and four
+ * measure). Labels and centroids are those of 0, which measures every row in every step; float32
+ * sums that one-pass kernels carry from step to step may differ in the last bit of a mean where they are
+ * not exact in double (a feature spanning more than some 14 binades in a cluster), float64 sums as two fits
+ * do. 2 does it for fits of any length and shapes of any size. Twelve bytes of device memory a row, and four
  * per pair of up to 4096 centroids in tiled shapes; where they cannot be had every row is measured.
- * Minimum distances of such fits are made from the differences. Float32 rows of three features and
+ * Minimum distances of such fits are made from the differences (nearer to float64 than the norms and
+ * products of other fits, from which an inertia differs by some 1e-6). Float32 rows of three features and
  * 17 to 128 centroids: long fits order a copy of the rows in space and measure only blocks of
  * them that more than one centroid may be the nearest in (cell_kernels.hip; 26 bytes a row).
  * Unknown names return EARG. */
