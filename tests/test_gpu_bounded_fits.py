@@ -316,3 +316,21 @@ def test_blocks_of_one_centroid_are_not_measured(hip, k):
     got, want = fit(hip, X, C, 12, 2), fit(hip, X, C, 12, 0)
     assert want["measured"] == -1 and 0 <= got["measured"] < n / 10
     same(got, want)
+
+
+def test_a_stop_signal_ends_a_fit_that_does_not_measure_every_row(hip):
+    """Runs in a child process: the handler is process-wide and must not replace pytest's. The labels are those of
+    the centroids the fit has come to."""
+    import json
+    import os
+    import subprocess
+    import sys
+    here = os.path.dirname(os.path.abspath(__file__))
+    proc = subprocess.run([sys.executable, os.path.join(here, "signal_stop_bounds_check.py")],
+                          capture_output=True, text=True, timeout=100)
+    assert proc.returncode == 0, proc.stdout + proc.stderr
+    fits = [json.loads(line) for line in proc.stdout.strip().splitlines()]
+    assert len(fits) == 4
+    for f in fits:
+        assert f["stopped"] and f["bounds"] and f["labels"] and f["counts"], fits
+    assert proc.stderr.count("Signal caught") == 4, fits
